@@ -100,6 +100,24 @@ def test_plan_and_group(lib):
         assert gs[len(order)] == start
 
 
+@pytest.mark.parametrize("n,distinct", ((64, 20), (65, 1), (65, 65), (127, 40), (128, 100), (191, 191), (255, 60), (256, 3), (256, 256)))
+def test_groups_of_many_entries(lib, n, distinct):
+    """Entry counts around the waves' edges, one group to a group an entry, blobs that agree in one half of their address, null blobs."""
+    rng = np.random.default_rng(n + distinct)
+    blobs = (rng.integers(1, 4, distinct) << 32) + 4096 * (1 + rng.permutation(distinct)).astype(np.int64)
+    p = blobs[np.concatenate([np.arange(distinct), rng.integers(0, distinct, n - distinct)])]
+    rng.shuffle(p)
+    p[rng.random(n) < 0.1] = 0
+    gp, gs, ge, ng = [t.cpu().numpy() for t in lib.group(torch.from_numpy(p).cuda())]
+    order = list(dict.fromkeys(int(b) for b in p if b))
+    members = [np.flatnonzero(p == b) for b in order]
+    assert ng[0] == len(order) and np.array_equal(gp[:len(order)], np.array(order, dtype=np.int64))
+    assert np.array_equal(gs[:len(order) + 1], np.cumsum([0] + [len(m) for m in members]))
+    want = np.concatenate(members + [np.full(int((p == 0).sum()), -1)])
+    assert np.array_equal(ge, want)
+
+
+
 # ---- the sigmoid router (router_sigmoid / moe_route's selection): ids bit-exact with the CPU checker, weights to the
 # reference's bar of 1e-5 (src/kernels/router_sigmoid_parity.cpp:137-143), on that test's case shapes and wider ones
 
