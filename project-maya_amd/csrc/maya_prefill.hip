@@ -26,79 +26,99 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------------------------- the plan
-// One workgroup: counts per expert and per segment (a wave's contiguous share of the entries), the prefix sums, then
-// every wave walks its segment in order so that an expert's rows keep the entries' order.
-// dynamic LDS: seg[kPlanWaves][n_expert] counts -> bases, base[n_expert + 1]
+// An expert's rows keep the entries' order: entry e sits behind every entry of a lower expert and behind the earlier entries of
+// its own.  Each workgroup scatters one share of the entries, its waves a contiguous run of them each, and counts ALL entries
+// for itself - those in front of its share, its waves' own, those behind - so nothing passes between workgroups and the plan
+// stays one launch with no scratch: an entry costs a load and an LDS add a workgroup, the scatter (a chain of LDS steps a
+// 64-entry chunk) runs on as many workgroups as there are runs of 1024 entries.  32768 entries over 288 experts: 193 us with
+// one workgroup scattering all 32 chunks a wave, 11.9 us like this; 4096 entries over 256: 12 us, 7.5 us.
+// dynamic LDS: [kPlanWaves][n_expert] 64-bit lane masks (with_masks), seg[kPlanWaves][n_expert] counts -> bases,
+// before[n_expert], total[n_expert], base[n_expert + 1], tbase[n_expert + 1]
+constexpr int kPlanMaxGroups = 64;   // (at 1 << 20 entries the counting would outweigh the scatter)
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_t* __restrict__ ids, int n_entries,
                                                                     const uint64_t* __restrict__ table, int n_expert,
                                                                     maya_prefill_plan p, int max_tiles, int with_masks) {
     extern __shared__ __attribute__((aligned(16))) int32_t sm[];
-    int32_t* seg = sm;                               // [kPlanWaves][n_expert]
-    int32_t* base = sm + kPlanWaves * n_expert;      // [n_expert + 1]
-    // (with_masks: [kPlanWaves][n_expert] 64-bit words behind base, 8-byte aligned)
-    unsigned long long* mask = with_masks ? (unsigned long long*) (sm + ((kPlanWaves * n_expert + n_expert + 1 + 1) & ~1)) : nullptr;
-    __shared__ int32_t s_tiles;
+    unsigned long long* mask = with_masks ? (unsigned long long*) sm : nullptr;
+    int32_t* seg = sm + (with_masks ? 2 * kPlanWaves * n_expert : 0);
+    int32_t* before = seg + kPlanWaves * n_expert;
+    int32_t* total = before + n_expert;              // (first the count of the entries behind the share)
+    int32_t* base = total + n_expert;
+    int32_t* tbase = base + n_expert + 1;
+    __shared__ unsigned long long resident[MAYA_MAX_EXPERTS / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    for (int i = tid; i < kPlanWaves * n_expert; i += kPlanThreads) seg[i] = 0;
+    {
+        const unsigned long long r = __ballot(tid < n_expert && table[tid] != 0ull);   // (n_expert <= kPlanThreads: checked on the host)
+        if (lane == 0) resident[wave] = r;
+    }
+    for (int i = tid; i < (kPlanWaves + 2) * n_expert; i += kPlanThreads) seg[i] = 0;
     if (mask != nullptr)
         for (int i = tid; i < kPlanWaves * n_expert; i += kPlanThreads) mask[i] = 0ull;
-    if (tid == 0) s_tiles = 0;
     __syncthreads();
-    const int per = (((n_entries + kPlanWaves - 1) / kPlanWaves) + 63) & ~63;   // a wave's share, whole chunks of 64
-    const int lo = wave * per, hi = min(n_entries, lo + per);
+    const int per = (((n_entries + kPlanWaves * (int) gridDim.x - 1) / (kPlanWaves * (int) gridDim.x)) + 63) & ~63;   // whole chunks of 64
+    const int lo = ((int) blockIdx.x * kPlanWaves + wave) * per, hi = min(n_entries, lo + per);
     auto expert_of = [&](int e) {
         const int x = ids[e];
-        return (x >= 0 && x < n_expert && table[x] != 0ull) ? x : -1;
+        return (x >= 0 && x < n_expert && ((resident[x >> 6] >> (x & 63)) & 1ull)) ? x : -1;
     };
-    for (int e = lo + lane; e < hi; e += 64) {
-        const int x = expert_of(e);
-        if (x >= 0) atomicAdd(&seg[wave * n_expert + x], 1);
-    }
+    auto count = [&](int from, int to, int step, int32_t* into) {   // (several loads in flight: the adds wait for none of their own)
+        for (int e0 = from; e0 < to; e0 += 8 * step) {
+            int x[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = e0 + i * step < to ? ids[e0 + i * step] : -1;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (x[i] >= 0 && x[i] < n_expert && ((resident[x[i] >> 6] >> (x[i] & 63)) & 1ull)) atomicAdd(&into[x[i]], 1);
+        }
+    };
+    const int first = min(n_entries, (int) blockIdx.x * kPlanWaves * per), last = min(n_entries, first + kPlanWaves * per);
+    count(tid, first, kPlanThreads, before);
+    count(lo + lane, hi, 64, seg + wave * n_expert);
+    count(last + tid, n_entries, kPlanThreads, total);
     __syncthreads();
-    // per expert: the segments' counts -> exclusive offsets, the total into base[x + 1]
+    // per expert: the waves' counts -> offsets from the expert's first row, and the total
     for (int x = tid; x < n_expert; x += kPlanThreads) {
-        int run = 0;
+        int run = before[x];
         for (int w = 0; w < kPlanWaves; ++w) {
             const int c = seg[w * n_expert + x];
             seg[w * n_expert + x] = run;
             run += c;
         }
-        base[x + 1] = run;
+        total[x] += run;
     }
     __syncthreads();
-    // base[x + 1] = the experts' running total: wave 0, a lane a run of experts, a scan over the lanes between two passes
-    if (tid < 64) {
-        const int per_lane = (n_expert + 63) >> 6, x0 = tid * per_lane;
+    // the experts' first rows (wave 0) and first tiles (wave 1): a lane a run of experts, a scan over the lanes between two passes
+    if (wave < 2) {
+        const int per_lane = (n_expert + 63) >> 6, x0 = lane * per_lane;
+        int32_t* o = wave ? tbase : base;
+        auto size = [&](int x) { return wave ? (total[x] + kPfRows - 1) / kPfRows : total[x]; };
         int local = 0;
         for (int i = 0; i < per_lane; ++i)
-            if (x0 + i < n_expert) local += base[x0 + i + 1];
+            if (x0 + i < n_expert) local += size(x0 + i);
         int incl = local;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const int up = __shfl_up(incl, d, 64);
-            if (tid >= d) incl += up;
+            if (lane >= d) incl += up;
         }
         int run = incl - local;
         for (int i = 0; i < per_lane; ++i)
             if (x0 + i < n_expert) {
-                run += base[x0 + i + 1];
-                base[x0 + i + 1] = run;
+                o[x0 + i] = run;
+                run += size(x0 + i);
+                if (x0 + i == n_expert - 1) o[n_expert] = run;
             }
-        if (tid == 0) base[0] = 0;
     }
     __syncthreads();
-    for (int x = tid; x <= n_expert; x += kPlanThreads) p.bounds[x] = base[x];
-    // tiles: expert x's rows in runs of kPfRows
-    for (int x = tid; x < n_expert; x += kPlanThreads) {
-        const int r0 = base[x], r1 = base[x + 1];
-        const int nt = (r1 - r0 + kPfRows - 1) / kPfRows;
-        if (nt > 0) {
-            const int t0 = atomicAdd(&s_tiles, nt);
-            for (int i = 0; i < nt && t0 + i < max_tiles; ++i) {
-                p.tile_expert[t0 + i] = x;
-                p.tile_row0[t0 + i] = r0 + i * kPfRows;
+    if (blockIdx.x == 0) {
+        for (int x = tid; x <= n_expert; x += kPlanThreads) p.bounds[x] = base[x];
+        // tiles: expert x's rows in runs of kPfRows
+        for (int x = tid; x < n_expert; x += kPlanThreads)
+            for (int t = tbase[x]; t < min(tbase[x + 1], max_tiles); ++t) {
+                p.tile_expert[t] = x;
+                p.tile_row0[t] = base[x] + (t - tbase[x]) * kPfRows;
             }
-        }
+        if (tid == 0) *p.n_tiles = min(tbase[n_expert], max_tiles);
     }
     // the stable scatter: 64 entries a step, a lane's rank = the earlier lanes of the step with its expert
     for (int c0 = lo; c0 < hi; c0 += 64) {
@@ -142,8 +162,6 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_s_waitcnt(0);
     }
-    __syncthreads();
-    if (tid == 0) *p.n_tiles = min(s_tiles, max_tiles);
 }
 
 // ------------------------------------------------------------------------------------------ activation quantizer
@@ -730,13 +748,15 @@ int maya_moe_prefill_plan(const int32_t* ids, int n_entries, const uint64_t* exp
     if (!ids || !expert_table || !plan_ok(plan)) return fail(MAYA_E_ARG, "prefill_plan: null pointer");
     if (n_entries <= 0 || n_entries > (1 << 20) || n_expert <= 0 || n_expert > MAYA_MAX_EXPERTS)
         return fail(MAYA_E_SHAPE, "prefill_plan: entries %d experts %d", n_entries, n_expert);
-    // (up to 256 experts: a wave's 64-bit lane masks per expert ride along, 8 bytes x 16 waves an expert)
-    const int with_masks = n_expert <= 256;
-    size_t lds = sizeof(int32_t) * ((size_t) kPlanWaves * n_expert + n_expert + 1);
-    if (with_masks) lds = ((lds + 7) & ~(size_t) 7) + sizeof(unsigned long long) * (size_t) kPlanWaves * n_expert;
+    // (a wave's 64-bit lane masks an expert ride along while LDS holds them: up to 780 experts; ballots beyond)
+    size_t lds = sizeof(int32_t) * ((size_t) (kPlanWaves + 4) * n_expert + 2);
+    const size_t masks = sizeof(unsigned long long) * (size_t) kPlanWaves * n_expert;
+    const int with_masks = lds + masks + 1024 <= (size_t) st->lds_limit;
+    if (with_masks) lds += masks;
     if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) prefill_plan_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
-    hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPlanThreads), lds, as_stream(stream), ids, n_entries, expert_table,
-                       n_expert, *plan, maya_moe_prefill_max_tiles(n_entries, n_expert), with_masks);
+    const int groups = (n_entries + kPlanThreads - 1) / kPlanThreads;
+    hipLaunchKernelGGL(prefill_plan_kernel, dim3(groups < kPlanMaxGroups ? groups : kPlanMaxGroups), dim3(kPlanThreads), lds, as_stream(stream),
+                       ids, n_entries, expert_table, n_expert, *plan, maya_moe_prefill_max_tiles(n_entries, n_expert), with_masks);
     MAYA_LAUNCHED("prefill_plan_kernel");
     return MAYA_OK;
 }

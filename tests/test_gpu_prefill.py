@@ -33,7 +33,9 @@ def make_blobs(oracle, n_expert, n_embd, n_ff, seed, encoded=False):
     return blobs
 
 
-PLAN_CASES = [(1, 1, 4, 0), (37, 2, 8, 1), (64, 8, 256, 2), (512, 8, 256, 3), (300, 3, 7, 4), (1000, 4, 1024, 5)]
+PLAN_CASES = [(1, 1, 4, 0), (37, 2, 8, 1), (64, 8, 256, 2), (512, 8, 256, 3), (300, 3, 7, 4), (1000, 4, 1024, 5),
+              # entries shared out over several workgroups: one past a workgroup's run, waves with nothing, the most of a call
+              (1025, 1, 288, 6), (3000, 8, 640, 7), (8191, 8, 1000, 8)]
 
 
 @pytest.mark.parametrize("n_tokens,k,n_expert,seed", PLAN_CASES)
