@@ -2,216 +2,206 @@
 // maya_prefill.hip inside namespace maya; the skeleton - tiles, the activations' copies, the barriers - is pf_tile's).
 // out[row][n] = 1/8 sum over blocks b of (d_w[n][b] d_x[row][b]) * sum over the block's 16-value groups j of (2 ls_j +
 // 1) (w_j . c_j), w = the grid magnitudes with their signs: the integer sums of the CPU path's IQ2_S x Q8_K row dot
-// (src/kernels/cpu/iq_avx2.cpp:160-176, 225-250).  The scale belongs to 16 values and (2 ls + 1) x 43 does not fit
-// int8, so a 32-deep matrix instruction takes ONE group: a lane (row ln, k-group kg) decodes grid entry kg of a sub-
-// block - 8 signed bytes (the grid's magnitudes and a sign-mask table sit in LDS), its whole operand - and the two
-// groups of a sub-block come from two instructions whose operands are zero in the lanes of the other group (kg < 2:
-// values 0..15, kg >= 2: 16..31).  The vector ALU then adds (2 ls + 1) x the group's sums to the block's int32 sums:
-// two multiply-adds an output a sub-block.  Weights go global -> LDS without registers, one super-block ahead: per
-// tile of 16 rows (4 quads) the 8 sub-blocks' index + sign words (1024 bytes: one 16-byte copy a lane) and their qh /
-// scale bytes (256 bytes: one 4-byte copy a lane), each lane's source chosen so that LDS holds [sub-block][quad][row]:
-// the 16 rows of a read then sit in 16 different bank pairs.  The block scales (2 bytes a row a block) come through a
-// register.
+// (src/kernels/cpu/iq_avx2.cpp:160-176, 225-250).
+//
+// A weight is one of six values of its group, +-(2 ls + 1) x {8, 25, 43} (at most 1333), so it is taken as two int8
+// digits, u = 256 hi + lo, and each digit as a byte looked up by v_perm_b32 in the group's six: a 16-entry table in LDS
+// gives a lane its group's eight bytes of either digit, the grid (its magnitudes as 0 / 1 / 2) joined with a sign table (4 in
+// the bytes of set bits) gives the selectors, and one v_perm_b32 a digit makes four weights, signed and scaled.  The two
+// digits' products with the codes then run through the 32x32x32 matrix instructions over the whole 256-value block, as
+// Q4_K's two planes do (pf_tile): no scaled sums outside the matrix cores, one convert and two multiplies an output a block.
+// The form before this one gave a matrix instruction the magnitudes of ONE 16-value group (the operand's other half zero) and
+// added (2 ls + 1) x its sums on the vector ALU: 41 vector instructions to decode 512 weights and two multiply-adds an
+// output every 32 values, 79 % of the cycles in vector issue.  A 75-token chunk on
+// 160 experts of 6144 x 1536 735 -> 535 us; gate/up IQ2_S with Q4_K down, 1187 tokens on 256 of 7168 x 2048, 2830 -> 2190 us.
+constexpr int kIqMags = 0, kIqSigns = 8192, kIqScales = kIqSigns + 2048, kIqTables = kIqScales + 256;   // byte offsets in LDS
 
-constexpr int kIqTileBytes = 1280, kIqWaveBytes = 2 * kIqTileBytes, kIqBufBytes = 4 * kIqWaveBytes;
+struct IqLook {   // the LDS look-ups of one sub-block: selectors and signs of the lane's two grid entries, its group's digits
+    pf_i2 m0, m1, s0, s1;
+    v4i sc;       // the low digits of +{8, 25, 43}, of -{8, 25, 43}, then the high ones
+};
+template <int BUT, int NM> __device__ __forceinline__ void iq_wait(IqLook& l, v4i (&x)[NM]) {
+    static_assert(NM == 1 || NM == 2, "1 or 2 row groups");
+    if constexpr (NM == 1)
+        asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(l.m0), "+v"(l.m1), "+v"(l.s0), "+v"(l.s1), "+v"(l.sc), "+v"(x[0]) : "n"(BUT));
+    else
+        asm volatile("s_waitcnt lgkmcnt(%7)" : "+v"(l.m0), "+v"(l.m1), "+v"(l.s0), "+v"(l.s1), "+v"(l.sc), "+v"(x[0]), "+v"(x[1]) : "n"(BUT));
+}
+template <int BUT> __device__ __forceinline__ void iq_wait_tail(v4f (&d)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]) : "n"(BUT));
+}
 
-template <bool GU, int NMT>
-__device__ __forceinline__ void pf_tile_iq2s(const PfGemm& a, uint8_t* b0, uint8_t* b1, uint8_t* b2, uint8_t* w0, uint8_t* w1,
-                                             uint32_t grid_lds, int ex, int row0, int nrows) {
+template <bool GU, int NM>
+__device__ __forceinline__ void pf_tile_iq2s(const PfGemm& a, uint8_t* b0, uint8_t* b1, uint8_t* b2, int ex, int row0, int nrows) {
     typedef const __attribute__((address_space(1))) uint8_t* wptr;
-    const uint64_t blob = a.table[ex];
-    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 15, kg = lane >> 4;
+    typedef uint32_t w2 __attribute__((ext_vector_type(2)));
+    constexpr int NMT = 2 * NM;
+    wptr blob = (wptr) a.table[ex];
+    const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nsb = (int) (a.k >> 8), nu = nsb * 8;
-    const uint32_t qb = 4u * (uint32_t) nsb * 82u;   // bytes of a quad of rows
+    const int nsb = (int) (a.k >> 8);
+    const size_t qb = 4u * (size_t) nsb * 82u;   // bytes of a quad of rows
 
+    wptr quad;
     int64_t n0;   // the wave's first feature (gate/up) or output row (down)
-    uint64_t base[2];   // the first quad of each of the wave's two tiles
     if constexpr (GU) {
         n0 = (int64_t) blockIdx.x * 64 + wave * 16;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) base[t] = blob + a.off[t] + (uint64_t) (n0 >> 2) * qb;
+        quad = blob + a.off[ln >> 4] + (size_t) ((n0 + (ln & 15)) >> 2) * qb;
     } else {
         n0 = (int64_t) blockIdx.x * 128 + wave * 32;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) base[t] = blob + a.off[0] + (uint64_t) ((n0 + 16 * t) >> 2) * qb;
+        quad = blob + a.off[0] + (size_t) ((n0 + ln) >> 2) * qb;
     }
     const bool wave_on = n0 < a.n;   // (a.n is a multiple of the wave's rows: checked on the host)
 
-    v4f acc[2][NMT];
-    v4i isum[2][NMT];
+    pf_v16f acc[NM];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int m = 0; m < NM; ++m)
 #pragma unroll
-        for (int m = 0; m < NMT; ++m) acc[t][m] = v4f{0.0f, 0.0f, 0.0f, 0.0f}, isum[t][m] = v4i{0, 0, 0, 0};
+        for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
 
     PfDma<NMT, false> dma;
     dma.init(a, row0, nrows, wave, lane);
-    // the weights' copies: lane L fills LDS piece L = [sub-block L >> 3][quad (L >> 1) & 3][row pair L & 1]
-    __amdgpu_buffer_rsrc_t wr[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) base[t]);
-        const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (base[t] >> 32));
-        wr[t] = __builtin_amdgcn_make_buffer_rsrc((void*) (((uint64_t) hi << 32) | lo), 0, (int) (4u * qb), 0x00020000);
-    }
-    const uint32_t cu = (uint32_t) (lane >> 3), cq = (uint32_t) ((lane >> 1) & 3), cp = (uint32_t) (lane & 1);
-    const uint32_t oi = cq * qb + 8u * (4u * cu + 2u * cp), oh = cq * qb + 32u * (uint32_t) nu + 2u * (4u * cu + 2u * cp);
-    auto wcopy = [&](uint8_t* wbuf, int sb) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            uint8_t* dst = wbuf + wave * kIqWaveBytes + t * kIqTileBytes;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr[t], (pf_lptr) dst, 16, oi, sb * 256, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr[t], (pf_lptr) (dst + 1024), 4, oh, sb * 64, 0, 0);
-        }
-    };
-    // the block scale of the lane's row: 2 bytes at 40 nu + 2 (4 b + r) of its quad
-    wptr dp[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) dp[t] = (wptr) base[t] + (size_t) (ln >> 2) * qb + 40u * (uint32_t) nu + 2u * (uint32_t) (ln & 3);
-    uint32_t dh[2] = {0u, 0u}, dhn[2] = {0u, 0u};
-    auto load_d = [&](int sb, uint32_t (&o)[2]) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) o[t] = *(const __attribute__((address_space(1))) uint16_t*) (dp[t] + 8 * sb);
-    };
-
     dma.copy(b0, 0);
     if (nsb > 1) dma.copy(b1, 1);
-    if (wave_on) {
-        wcopy(w0, 0);
-        load_d(0, dh);
-    }
-    // lane constants of the decode: the entry's byte and its two high bits, the group masks, the activations' place
-    const uint32_t sh8 = 8u * (uint32_t) kg, sh2 = 2u * (uint32_t) kg;
-    const uint32_t m0 = kg < 2 ? 0xffffffffu : 0u, m1 = ~m0;
-    const uint32_t w_rd = (uint32_t) (wave * kIqWaveBytes + (ln >> 2) * 32 + (ln & 3) * 8);
-    const uint32_t h_rd = (uint32_t) (wave * kIqWaveBytes + 1024 + (ln >> 2) * 8 + (ln & 3) * 2);
-    const int a_base = ln * 256 + 8 * (kg & 1), a_swz = (ln ^ (kg >> 1)) << 4;
+
+    // The weights of a super-block, one ahead in registers: lane (ln, kh) of row ln loads the (index, sign) words and the
+    // (high bits, scales) pairs of sub-blocks 4 kh .. 4 kh + 3, and one half-wave swap a pair of words then leaves every lane
+    // with its own half - the entries 2 kh and 2 kh + 1, the group kh - of all eight.
+    wptr pi = quad + 128 * kh + 8 * (ln & 3), ph = quad + 256 * (size_t) nsb + 32 * kh + 2 * (ln & 3),
+         pd = quad + 320 * (size_t) nsb + 2 * (ln & 3);
+    w2 is[4];
+    uint32_t hs[4], dn;
+    auto load_block = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) is[i] = *(const __attribute__((address_space(1))) w2*) (pi + 32 * i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) hs[i] = *(const __attribute__((address_space(1))) uint16_t*) (ph + 8 * i);
+        dn = *(const __attribute__((address_space(1))) uint16_t*) pd;
+        pi += 256, ph += 64, pd += 8;
+    };
+    uint32_t v[8], g[8];   // a sub-block: the two index bytes, then the two sign bytes; the high bits << 11 and ls << 19
+    float d = 0.0f;
+    auto unpack = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const auto r = __builtin_amdgcn_permlane32_swap(__builtin_amdgcn_perm(is[i].y, is[i].x, 0x05040100u),
+                                                            __builtin_amdgcn_perm(is[i].y, is[i].x, 0x07060302u), false, false);
+            v[i] = r[0], v[4 + i] = r[1];
+            const auto q = __builtin_amdgcn_permlane32_swap((hs[i] << 11) & 0x787800u, (hs[i] << 7) & 0x787800u, false, false);
+            g[i] = q[0], g[4 + i] = q[1];
+        }
+        d = f16_bits_to_f32((uint16_t) dn);
+    };
+    if (wave_on) load_block();
+    const int a_base = ln * 256, a_swz = ((ln & 15) ^ kh) << 4;   // (a lane's 16 codes of sub-block j: chunk 2 j + kh of the row)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if (wave_on) unpack();
 
-    auto step = [&](int sb, const uint8_t* buf, uint8_t* buf2, const uint8_t* wbuf, uint8_t* wbuf2) {
-        const bool more = sb + 2 < nsb;
-        if (wave_on && sb + 1 < nsb) {
-            load_d(sb + 1, dhn);
-            wcopy(wbuf2, sb + 1);
-        }
-        // (after the weights' copies, so that waiting for everything but these copies covers the weights too)
-        if (more) dma.copy(buf2, sb + 2);
+    auto step = [&](int sb, const uint8_t* buf, uint8_t* buf2) {   // super-block sb from buf; sb + 2 is copied into buf2
+        if (wave_on && sb + 1 < nsb) load_block();
+        // (after the weights' loads, so that waiting for everything but these copies covers the weights too)
+        if (sb + 2 < nsb) dma.copy(buf2, sb + 2);
         if (wave_on) {
-            const uint32_t lbuf = pf_lds_addr(buf), lw = pf_lds_addr(wbuf);
-#pragma unroll 1
-            for (int u = 0; u < 8; ++u) {
-                // the activations' 8 codes of this lane's k-group: chunk 2 u + (kg >> 1) of the row, its half kg & 1
-                pf_i2 xr[NMT];
-                {
-                    const uint32_t at = lbuf + a_base + (a_swz ^ (32 * u));
-                    pf_for_m<0, NMT>([&](auto mc) {
+            const uint32_t lbuf = pf_lds_addr(buf);
+            pf_v16i dot[NM][2];
+            v4i xr[2][NM];
+            IqLook lk[2];
+            auto read_x = [&](int j, v4i (&dst)[NM]) {
+                const uint32_t at = lbuf + a_base + (a_swz ^ ((2 * j) << 4));
+                pf_for_m<0, NM>([&](auto mc) {
+                    constexpr int m = decltype(mc)::value;
+                    dst[m] = pf_lds_i32x4<m * 8192>(at);
+                });
+            };
+            auto look = [&](int j, IqLook& o) {
+                const uint32_t x = v[j], h = g[j];
+                o.m0 = pf_lds_b64<kIqMags>(((x << 3) & 0x7f8u) | (h & 0x1800u));
+                o.m1 = pf_lds_b64<kIqMags>(((x >> 5) & 0x7f8u) | ((h >> 2) & 0x1800u));
+                o.s0 = pf_lds_b64<kIqSigns>((x >> 13) & 0x7f8u);
+                o.s1 = pf_lds_b64<kIqSigns>((x >> 21) & 0x7f8u);
+                o.sc = pf_lds_i32x4<kIqScales>((h >> 15) & 0xf0u);
+            };
+            v4f dxr[NM][4];
+            look(0, lk[0]);
+            read_x(0, xr[0]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                IqLook& l = lk[j & 1];
+                if (j < 7) {   // the next sub-block's look-ups go out under this one's arithmetic
+                    look(j + 1, lk[(j + 1) & 1]);
+                    read_x(j + 1, xr[(j + 1) & 1]);
+                    iq_wait<5 + NM>(l, xr[j & 1]);
+                } else {       // and the closing stage's block scales before the last one's
+                    pf_for_m<0, NM>([&](auto mc) {
                         constexpr int m = decltype(mc)::value;
-                        xr[m] = pf_lds_b64<m * 4096>(at);
+                        const uint32_t at = lbuf + 16 * kh;
+                        dxr[m][0] = pf_lds_f32x4<kPfDOffNoS + m * 128>(at);
+                        dxr[m][1] = pf_lds_f32x4<kPfDOffNoS + m * 128 + 32>(at);
+                        dxr[m][2] = pf_lds_f32x4<kPfDOffNoS + m * 128 + 64>(at);
+                        dxr[m][3] = pf_lds_f32x4<kPfDOffNoS + m * 128 + 96>(at);
                     });
+                    iq_wait<4 * NM>(l, xr[j & 1]);
                 }
-                pf_i2 iw[2];
-                uint32_t hs[2];
-                iw[0] = pf_lds_b64<0>(lw + w_rd + 128 * u);
-                iw[1] = pf_lds_b64<kIqTileBytes>(lw + w_rd + 128 * u);
-                hs[0] = pf_lds_u16<0>(lw + h_rd + 32 * u);
-                hs[1] = pf_lds_u16<kIqTileBytes>(lw + h_rd + 32 * u);
-                pf_lds_wait(iw);
-                pf_lds_wait(hs);
-                pf_i2 gr[2];
+                const uint32_t q[4] = {(uint32_t) (l.m0.x | l.s0.x), (uint32_t) (l.m0.y | l.s0.y), (uint32_t) (l.m1.x | l.s1.x), (uint32_t) (l.m1.y | l.s1.y)};
+                v4i wl, wh;
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const uint32_t idx = __builtin_amdgcn_ubfe((uint32_t) iw[t].x, sh8, 8u), hi2 = __builtin_amdgcn_ubfe(hs[t], sh2, 2u);
-                    const uint32_t ga = grid_lds + ((idx | (hi2 << 8)) << 3);
-                    gr[t] = pf_lds_b64<0>(ga);
+                for (int i = 0; i < 4; ++i) {
+                    wl[i] = (int) __builtin_amdgcn_perm((uint32_t) l.sc[1], (uint32_t) l.sc[0], q[i]);
+                    wh[i] = (int) __builtin_amdgcn_perm((uint32_t) l.sc[3], (uint32_t) l.sc[2], q[i]);
                 }
-                // the signs: the entry's sign byte -> 0xff in the bytes of its set bits (a 256-entry table beside the grid)
-                pf_i2 sm[2];
-                int s0[2], s1[2];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const uint32_t sbyte = __builtin_amdgcn_ubfe((uint32_t) iw[t].y, sh8, 8u);
-                    sm[t] = pf_lds_b64<8192>(grid_lds + (sbyte << 3));
-                    const uint32_t sc = hs[t] >> 8;
-                    s0[t] = (int) (2u * (sc & 15u) + 1u);
-                    s1[t] = (int) (2u * (sc >> 4) + 1u);
+                for (int m = 0; m < NM; ++m) {
+                    const pf_v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                    dot[m][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[j & 1][m], wl, j ? dot[m][0] : z, 0, 0, 0);
+                    dot[m][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[j & 1][m], wh, j ? dot[m][1] : z, 0, 0, 0);
                 }
-                pf_lds_wait(gr);
-                pf_lds_wait(sm);
-                pf_lds_wait(xr);
+            }
+            // once a block: lo + 256 hi = the block's integer sum, times the two block scales (blocks of 8 rows past the tile's
+            // last row are skipped)
+            pf_for_m<0, NM>([&](auto mc) {
+                constexpr int m = decltype(mc)::value;
+                iq_wait_tail<4 * (NM - 1 - m)>(dxr[m]);
+                const int nb = (nrows - 32 * m + 7) >> 3;
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    // the marked bytes negated: (g ^ 0xff) + 1 a byte, no carry (no magnitude is 0)
-                    const uint32_t ma = (uint32_t) sm[t].x, mb = (uint32_t) sm[t].y;
-                    const uint32_t wa = ((uint32_t) gr[t].x ^ ma) + (ma & 0x01010101u), wb = ((uint32_t) gr[t].y ^ mb) + (mb & 0x01010101u);
-                    const long o0 = (long) (((uint64_t) (wb & m0) << 32) | (uint64_t) (wa & m0));
-                    const long o1 = (long) (((uint64_t) (wb & m1) << 32) | (uint64_t) (wa & m1));
+                for (int b = 0; b < 4; ++b) {
+                    if (b < nb) {
 #pragma unroll
-                    for (int m = 0; m < NMT; ++m) {
-                        const long xa = (long) (((uint64_t) (uint32_t) xr[m].y << 32) | (uint64_t) (uint32_t) xr[m].x);
-                        const v4i z = {0, 0, 0, 0};
-                        const v4i d0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, o0, z, 0, 0, 0);
-                        const v4i d1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(xa, o1, z, 0, 0, 0);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                        {   // two 24-bit multiply-adds (kept apart: joined, the compiler makes two multiplies and a 3-way add)
-                            int v = __mul24(s0[t], d0[i]) + isum[t][m][i];
-                            asm("" : "+v"(v));
-                            isum[t][m][i] = __mul24(s1[t], d1[i]) + v;
+                        for (int r = 0; r < 4; ++r) {
+                            const int i = 4 * b + r;
+                            acc[m][i] = fmaf(__fmul_rn(dxr[m][b][r], d), (float) (dot[m][0][i] + 256 * dot[m][1][i]), acc[m][i]);
                         }
                     }
                 }
-            }
-            // once a block: the integer sums times the two block scales
-            v4f dxr[NMT];
-            pf_for_m<0, NMT>([&](auto mc) {
-                constexpr int m = decltype(mc)::value;
-                dxr[m] = pf_lds_f32x4<kPfDOffNoS + m * 64>(lbuf + 16 * kg);
             });
-            float d[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) d[t] = f16_bits_to_f32((uint16_t) dh[t]);
-            pf_lds_wait(dxr);
-#pragma unroll
-            for (int m = 0; m < NMT; ++m) {
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        acc[t][m][i] = fmaf(__fmul_rn(dxr[m][i], d[t]), (float) isum[t][m][i], acc[t][m][i]);
-                        isum[t][m][i] = 0;
-                    }
-                }
-            }
-            dh[0] = dhn[0], dh[1] = dhn[1];
+            if (sb + 1 < nsb) unpack();
         }
-        // super-block sb + 1 (activations and weights) has landed once only this iteration's activation copies (of
-        // sb + 2) may still be in flight; without such copies everything must have landed
-        if (more) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NMT) : "memory");
+        // super-block sb + 1 has landed once only the wave's youngest NMT operations - this iteration's copies (of sb + 2), in the
+        // last steps some of the nine weight loads, which `unpack` has waited for - may still be in flight; a wave that
+        // holds no weight rows has nothing younger than its last copies then and waits for all
+        if (sb + 2 < nsb || wave_on) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NMT) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
-    for (int sb = 0; sb < nsb; sb += 6) {
-        step(sb, b0, b2, w0, w1);
-        if (sb + 1 < nsb) step(sb + 1, b1, b0, w1, w0);
-        if (sb + 2 < nsb) step(sb + 2, b2, b1, w0, w1);
-        if (sb + 3 < nsb) step(sb + 3, b0, b2, w1, w0);
-        if (sb + 4 < nsb) step(sb + 4, b1, b0, w0, w1);
-        if (sb + 5 < nsb) step(sb + 5, b2, b1, w1, w0);
+    for (int sb = 0; sb < nsb; sb += 3) {
+        step(sb, b0, b2);
+        if (sb + 1 < nsb) step(sb + 1, b1, b0);
+        if (sb + 2 < nsb) step(sb + 2, b2, b1);
     }
     if (!wave_on) return;
 
-    // outputs: lane (ln, kg) holds weight row ln of each tile for the tokens 16 m + 4 kg + i
+    // outputs: lane (ln, kh) holds weight row ln for the tile's rows 32 m + 8 b + 4 kh + r (i = 4 b + r)
 #pragma unroll
-    for (int m = 0; m < NMT; ++m) {
+    for (int m = 0; m < NM; ++m) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = 16 * m + 4 * kg + i;
-            if (r >= nrows) continue;
-            float* o = a.out + (size_t) (row0 + r) * a.n + n0 + ln;
-            const float v0 = __fmul_rn(acc[0][m][i], 0.125f), v1 = __fmul_rn(acc[1][m][i], 0.125f);
-            if constexpr (GU) o[0] = pf_swiglu(v0, v1, a.limit);
-            else o[0] = v0, o[16] = v1;
+        for (int i = 0; i < 16; ++i) {
+            const int r = 32 * m + 8 * (i >> 2) + 4 * kh + (i & 3);
+            const float val = __fmul_rn(acc[m][i], 0.125f);
+            if constexpr (GU) {
+                const float up = __shfl(val, (lane + 16) & 63, kWave);   // the up row of a feature sits 16 lanes above its gate row
+                if (ln < 16 && r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = pf_swiglu(val, up, a.limit);
+            } else {
+                if (r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = val;
+            }
         }
     }
 }
@@ -219,26 +209,37 @@ __device__ __forceinline__ void pf_tile_iq2s(const PfGemm& a, uint8_t* b0, uint8
 // grid (bands of weight rows, tiles at most)
 template <bool GU>
 __global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebooks cb) {
-    __shared__ __attribute__((aligned(16))) uint8_t b0[kPfBufBytesNoS], b1[kPfBufBytesNoS], b2[kPfBufBytesNoS];
-    __shared__ __attribute__((aligned(16))) uint8_t w0[kIqBufBytes], w1[kIqBufBytes];
-    __shared__ __attribute__((aligned(16))) uint64_t grid[1024 + 256];   // the magnitudes, then the sign masks
+    // ONE array, so that it starts at LDS address 0 and the tables' addresses need no base added (five additions a sub-block)
+    __shared__ __attribute__((aligned(256))) uint8_t lds[kIqTables + 3 * kPfBufBytesNoS];
+    uint8_t *tables = lds, *b0 = lds + kIqTables, *b1 = b0 + kPfBufBytesNoS, *b2 = b1 + kPfBufBytesNoS;
+    if (pf_lds_addr(lds) != 0) return;   // (never: the kernel has no other LDS)
     const int tile = blockIdx.y;
     if (tile >= *a.plan.n_tiles) return;
-    for (int i = threadIdx.x; i < 1024; i += 256) grid[i] = cb.iq2s[i];
+    const int tid = threadIdx.x;
+    // the magnitudes 8, 25, 43 as 0, 1, 2 (their bits 4 and 5)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ((uint64_t*) (tables + kIqMags))[tid + 256 * i] = (cb.iq2s[tid + 256 * i] >> 4) & 0x0303030303030303ull;
     {
         uint64_t m = 0ull;
 #pragma unroll
         for (int b = 0; b < 8; ++b)
-            if (threadIdx.x & (1 << b)) m |= 0xffull << (8 * b);
-        grid[1024 + threadIdx.x] = m;
+            if (tid & (1 << b)) m |= 4ull << (8 * b);
+        ((uint64_t*) (tables + kIqSigns))[tid] = m;
+    }
+    if (tid < 16) {
+        v4i e = {0, 0, 0, 0};
+        const int mag[3] = {8, 25, 43};
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            const int u = (2 * tid + 1) * (i < 3 ? mag[i] : -mag[i - 3]), lo = (int) (int8_t) (u & 255), hi = (u - lo) >> 8;
+            const int at = 8 * (i % 3);
+            e[i / 3] |= (lo & 255) << at;
+            e[2 + i / 3] |= (hi & 255) << at;
+        }
+        ((v4i*) (tables + kIqScales))[tid] = e;
     }
     const int ex = a.plan.tile_expert[tile], row0 = a.plan.tile_row0[tile];
     const int nrows = min(kPfRows, a.plan.bounds[ex + 1] - row0);
-    const uint32_t gl = pf_lds_addr(grid);
-    switch ((nrows + 15) >> 4) {
-        case 1: pf_tile_iq2s<GU, 1>(a, b0, b1, b2, w0, w1, gl, ex, row0, nrows); break;
-        case 2: pf_tile_iq2s<GU, 2>(a, b0, b1, b2, w0, w1, gl, ex, row0, nrows); break;
-        case 3: pf_tile_iq2s<GU, 3>(a, b0, b1, b2, w0, w1, gl, ex, row0, nrows); break;
-        default: pf_tile_iq2s<GU, 4>(a, b0, b1, b2, w0, w1, gl, ex, row0, nrows); break;
-    }
+    if (nrows <= 32) pf_tile_iq2s<GU, 1>(a, b0, b1, b2, ex, row0, nrows);
+    else pf_tile_iq2s<GU, 2>(a, b0, b1, b2, ex, row0, nrows);
 }

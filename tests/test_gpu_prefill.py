@@ -198,6 +198,13 @@ IQ_CASES = [
     (22, 12, 1024, 768, 5, 2, 70, 0.0, ()),          # IQ2_S gate / up with Q4_K down (the mixed experts)
     (12, 22, 768, 1024, 4, 3, 90, 0.0, ()),          # and the other way round: 90-row experts, two tiles each
     (22, 22, 7168, 2048, 3, 2, 20, 0.0, ()),         # the full expert shape
+    # one expert of 1, 8, 9, 32, 33 and 65 rows: the edges of a closing block, of a row group and of a tile
+    (22, 22, 512, 1024, 1, 1, 1, 0.0, ()),
+    (22, 22, 512, 1024, 1, 1, 8, 0.0, ()),
+    (22, 22, 512, 1024, 1, 1, 9, 0.0, ()),
+    (22, 22, 512, 1024, 1, 1, 32, 0.0, ()),
+    (22, 22, 512, 1024, 1, 1, 33, 0.0, ()),
+    (22, 22, 512, 1024, 1, 1, 65, 0.0, ()),
 ]
 
 
