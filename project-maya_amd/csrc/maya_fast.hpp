@@ -310,9 +310,9 @@ struct QuadIQ2S {
 struct QuadOffs {  // byte offsets of the lane's fields inside a quad; quads advance through the scalar offset
     uint32_t is, hs, d;
 };
-template <int NU>
-__device__ __forceinline__ QuadOffs quad_offs(uint32_t mat_off, int u) {
-    return QuadOffs{mat_off + 32u * u, mat_off + 32u * NU + 8u * u, mat_off + 40u * NU + 8u * (u >> 3)};
+// (nu: sub-blocks a row)
+__device__ __forceinline__ QuadOffs quad_offs(uint32_t mat_off, int nu, int u) {
+    return QuadOffs{mat_off + 32u * u, mat_off + 32u * nu + 8u * u, mat_off + 40u * nu + 8u * (u >> 3)};
 }
 // A raw buffer resource over `bytes` of weights at `base`: loads take a per-lane 32-bit offset plus a scalar offset
 // (no vector address arithmetic in the row loop), and a load past `bytes` returns zero instead of faulting.
@@ -326,6 +326,12 @@ __device__ __forceinline__ QuadIQ2S load_quad(__amdgpu_buffer_rsrc_t rs, const Q
     q.hs = __builtin_amdgcn_raw_buffer_load_b64(rs, o.hs, quad_off, 0);
     q.d = __builtin_amdgcn_raw_buffer_load_b64(rs, o.d, quad_off, 0);
     return q;
+}
+// a lane past the row's last position: no codes, no scale
+__device__ __forceinline__ void idle_lane_zero(bool on, int (&y)[8], float& d) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = on ? y[i] : 0;
+    d = on ? d : 0.0f;
 }
 template <int R>
 __device__ __forceinline__ RawIQ2S quad_row(const QuadIQ2S& q) {
@@ -384,12 +390,17 @@ __device__ __forceinline__ void quad_values(const QuadIQ2S& q, const uint2* grid
 #undef MAYA_ROW
 }
 
-// ---- gate/up, one token, n_embd = 1024 NW: a workgroup of NW waves = the 2 * 32 NW sub-block positions of a
-// (gate row, up row) pair; grid (n_ff / ROWS, k).  DEPTH rows are in flight per lane.
-template <int NW, int ROWS, int DEPTH, int MINW>
+// ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the sub-block positions of a (gate row, up row) pair; grid
+// (n_ff / ROWS, entries).  DEPTH rows are in flight per lane.
+// Rows of any multiple of 256 values: NW = n_embd / 1024 rounded up, at least 2 (pos_waves), and a lane past the row's last
+// position reads that position's weights again - a line its neighbours ask for anyway - and meets them with zero codes and
+// a zero scale, so the sums are the same lane by lane.  The kernels took whole multiples of 1024 before; rows in
+// between, and down rows of other than 1024, 1536 and 2048 values, went to the general kernels at two to five times the time.
+// FIT: n_embd = 1024 NW, every lane has a position (known to the compiler, 0.3 to 1 us less a launch).
+template <int NW, int ROWS, int DEPTH, int MINW, bool FIT>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq2s_pos_kernel(maya_moe_args a, Codebooks cb) {
     static_assert(ROWS % 8 == 0 && (DEPTH == 1 || DEPTH == 2), "a batch is two quads; the ring holds one or two");
-    constexpr int NU = 32 * NW;  // sub-blocks a row
+    constexpr int NU = 32 * NW;  // the lanes of a row
     __shared__ __align__(16) int lds[kFastLdsWords];
     __shared__ float part[2][2 * NW][8];
     if (a.skip && *a.skip) return;
@@ -403,23 +414,26 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq2s_pos_kernel(maya_mo
     const uint2* stab = (const uint2*) (lds + 2048);
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int u = is_up ? t - NU : t;
+    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
+    const bool on = FIT || lu < nu;
+    const int u = on ? lu : nu - 1;
     const int tok = e / a.k;   // the entry's token: its activation row
     int y[8];
     {
-        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * NU));
+        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * nu));
         const int4 ya = q[2 * u], yb = q[2 * u + 1];
         y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
     }
+    float dy8 = a.x.d[(size_t) tok * nu + u] * 0.125f;
+    idle_lane_zero(on, y, dy8);
     int yn[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) yn[i] = neg4(y[i]);
-    const float dy8 = a.x.d[(size_t) tok * NU + u] * 0.125f;
-    constexpr uint32_t qb = NU / 8 * 82 * 4;  // bytes of a quad of rows
+    const uint32_t qb = (uint32_t) nu * 41u;  // bytes of a quad of rows: 4 x 82 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
     // one resource over the expert's gate and up rows; the up rows ride in the lane offset
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
-    const QuadOffs qo = quad_offs<NU>(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, u);
+    const QuadOffs qo = quad_offs(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     QuadIQ2S ring[DEPTH];
@@ -492,10 +506,11 @@ struct LayerHeadIn {
 // call - while the waves with gate lanes round their positions' x to Q8_K in registers (a 256-value block is 8 lanes: the
 // lane of position u holds the values o0 .. o0 + 15 and o1 .. o1 + 15 of x, o0 < o1 inside one block) and hand codes and
 // scale to the up lanes through LDS.  y: the position's 32 codes in that order, d: its block's scale, blob: the expert of
-// slot blockIdx.y.  False: the thread has nothing more to do in this launch.
+// slot blockIdx.y.  A lane past the row's last position (`on` false; u is then its own index, o0 and o1 the last
+// position's) gets zero codes and a zero scale.  False: the thread has nothing more to do in this launch.
 template <int NW>
-__device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent, const int32_t* skip, bool is_up, int u, int o0, int o1,
-                                                int (&y)[8], float& d, uint64_t& blob) {
+__device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent, const int32_t* skip, bool is_up, bool on, int u, int o0,
+                                                int o1, int (&y)[8], float& d, uint64_t& blob) {
     constexpr int NU = 32 * NW;
     __shared__ uint64_t s_blob[MAYA_MAX_K];
     __shared__ float s_lv[256];
@@ -597,6 +612,7 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
     // (a wave with a gate lane rounds: the block's 8 lanes are all gate lanes or all up lanes, NU being a multiple of 8)
     if (64 * (t >> 6) < NU) {
         q8k_round_lane32(v, [&](int i) { return i < 16 ? (o0 & 255) + i : (o1 & 255) + i - 16; }, y, d);
+        idle_lane_zero(on, y, d);   // (a block's 8 lanes are all on or all off: whole blocks a row)
         if (!is_up) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) s_y[i][u] = y[i];
@@ -619,8 +635,9 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
 // The leading arguments are what the kernel asks of memory first; as plain pointers and integers at the head of the
 // argument list they arrive in scalar registers with the dispatch (a structure passed by value is read from memory
 // first).  HEAD: p0 = the logits [n_expert], p1 = the table [n_expert] of blob addresses (0 = absent), p2 = x [n_embd] of
-// dtype `mode & 255`, bias = the sigmoid router's (`mode >> 8` = 1: the sigmoid router) or NULL; else p0 = the plan's blob
-// addresses (a.plan_ptr), p1 = the codes of x (a.x.q), p2 = their scales (a.x.d).
+// dtype `mode & 255`, bias = the sigmoid router's (bit 8 of mode: the sigmoid router) or NULL; else p0 = the plan's blob
+// addresses (a.plan_ptr), p1 = the codes of x (a.x.q), p2 = their scales (a.x.d).  mode >> 16 = n_embd / 32, the
+// sub-blocks a row.
 template <int NW, int MINW, bool HEAD>
 __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_kernel(const void* __restrict__ p0, const void* __restrict__ p1,
                                                                                       const void* __restrict__ p2,
@@ -629,7 +646,7 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
                                                                                       const int32_t* __restrict__ skip, int n_expert,
                                                                                       int mode, int n_ent, maya_moe_args a,
                                                                                       LayerHead hd) {
-    constexpr int NU = 32 * NW;  // sub-blocks a row
+    constexpr int NU = 32 * NW;  // the lanes of a row
     __shared__ __align__(16) int lds[kFastLdsWords];
     __shared__ float part[2][2 * NW][8];
     __shared__ uint64_t s_blob[HEAD ? MAYA_MAX_K : 1];
@@ -640,7 +657,9 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
     const uint2* stab = (const uint2*) (lds + 2048);
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int u = is_up ? t - NU : t;
+    const int nu = mode >> 16, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
+    const bool on = lu < nu;
+    const int u = on ? lu : nu - 1;
     // (n_ent = a.k: one token, entry = plan slot)
     int y[8];
     float dy8;
@@ -655,7 +674,7 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
         const uint64_t* table = (const uint64_t*) p1;
         const bool picker = t >= 64 * (NW - 1);
         const int x_dtype = mode & 255;
-        const bool sigm = (mode >> 8) != 0;
+        const bool sigm = (mode & 256) != 0;
         float lv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         uint64_t tab[4] = {0ull, 0ull, 0ull, 0ull};
         if (picker) {
@@ -754,17 +773,18 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
             float d;
             q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
             dy8 = d * 0.125f;
+            idle_lane_zero(on, y, dy8);   // (a block's 8 lanes are all on or all off: whole blocks a row)
             if (!is_up) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) s_y[i][u] = y[i];
-                s_y[8][u] = __float_as_int(dy8);
+                for (int i = 0; i < 8; ++i) s_y[i][lu] = y[i];
+                s_y[8][lu] = __float_as_int(dy8);
             }
         }
         __syncthreads();
         if (is_up) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = s_y[i][u];
-            dy8 = __int_as_float(s_y[8][u]);
+            for (int i = 0; i < 8; ++i) y[i] = s_y[i][lu];
+            dy8 = __int_as_float(s_y[8][lu]);
         }
     } else {
         // everything the first tile needs is requested side by side: no load waits on another
@@ -775,16 +795,17 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
             y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
         }
         dy8 = ((const float*) p2)[u] * 0.125f;
+        idle_lane_zero(on, y, dy8);
         if (skipv) return;
     }
     int yn[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) yn[i] = neg4(y[i]);
-    constexpr uint32_t qb = NU / 8 * 82 * 4;  // bytes of a quad of rows
+    const uint32_t qb = (uint32_t) nu * 41u;  // bytes of a quad of rows: 4 x 82 a block
     const int n_ff = a.layout.n_ff;
     const int tiles_per_entry = n_ff >> 3, n_tiles = n_ent * tiles_per_entry;
     const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
-    const QuadOffs qo = quad_offs<NU>(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, u);
+    const QuadOffs qo = quad_offs(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
     // the resource of a tile's expert (an absent expert: an empty resource, whose loads read as zero and touch nothing);
     // the entry is the same for the whole workgroup: its blob address is a scalar load (HEAD: read from LDS and moved to
     // scalar registers)
@@ -859,23 +880,22 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
 #undef MAYA_TROW
 }
 
-// ---- down + combine, one token, n_ff = 32 NU <= 2048 (NU sub-blocks a row on the first NU lanes of one wave; NU a
-// multiple of 8, the lanes past it idle): wave w = plan slot w, rows in batches of 8; grid (n_embd / ROWS).  The slots' rows
-// meet in LDS and are summed in slot order.
-template <int ROWS, int DEPTH, int MINW, int NU = 64>
-__global__ __launch_bounds__(512, MINW) void down_iq2s_pos_kernel(const uint64_t* __restrict__ plan_ptr, const float* __restrict__ plan_w,
+// ---- down + combine, n_ff = 32 nu <= 2048 (nu sub-blocks a row on the first nu lanes of one wave, the lanes past them idle):
+// wave w = plan slot w of at most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  The slots' rows meet in LDS and
+// are summed in slot order.  NU: nu where the compiler knows it (64), else 0.
+template <int ROWS, int DEPTH, int MINW, int SLOTS, int NU>
+__global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq2s_pos_kernel(const uint64_t* __restrict__ plan_ptr, const float* __restrict__ plan_w,
                                                                   const float* __restrict__ h, const uint64_t* __restrict__ iq2s_grid,
                                                                   const int32_t* __restrict__ skip, const int8_t* __restrict__ hq_q, int k,
-                                                                  int n_embd, maya_moe_args a, Codebooks cb) {
-    // (the leading arguments repeat a.plan_ptr, a.plan_w, a.h, cb.iq2s, a.skip, a.hq.q, a.k, a.layout.n_embd: plain pointers
+                                                                  int n_embd, int n_pos, maya_moe_args a, Codebooks cb) {
+    // (the leading arguments repeat a.plan_ptr, a.plan_w, a.h, cb.iq2s, a.skip, a.hq.q, a.k, a.layout.n_embd, n_ff / 32: plain pointers
     // and integers at the head of the argument list arrive in scalar registers with the dispatch, a structure passed by
     // value is read from memory first - and everything the kernel asks of memory at its start hangs on these)
     static_assert(ROWS % 4 == 0 && DEPTH >= 1 && DEPTH <= ROWS / 4, "a batch is two quads (the last may be one); the ring holds DEPTH quads");
-    static_assert(NU % 8 == 0 && NU >= 8 && NU <= 64, "whole 256-value blocks on one wave");
     __shared__ __align__(16) int lds[kFastLdsWords];
-    __shared__ float part[8][ROWS];
-    __shared__ float s_w[8];
-    __shared__ int s_on[8];
+    __shared__ float part[SLOTS][ROWS];
+    __shared__ float s_w[SLOTS];
+    __shared__ int s_on[SLOTS];
     const uint2* grid = (const uint2*) lds;
     const uint2* stab = (const uint2*) (lds + 2048);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -889,24 +909,25 @@ __global__ __launch_bounds__(512, MINW) void down_iq2s_pos_kernel(const uint64_t
     const int skipv = skip ? *skip : 0;
     const int ent = e0 + min(wave, k - 1);
     uint64_t blob = plan_ptr[ent];   // (asked for first: loads come back in order, and the weights' request waits for this one)
-    TablePieces<2048, 512> tp;
+    TablePieces<2048, 64 * SLOTS> tp;
     table_request(iq2s_grid, tp);
-    const int ci = e0 + min((int) threadIdx.x & 7, k - 1);
+    const int ci = e0 + min((int) threadIdx.x & (SLOTS - 1), k - 1);
     const uint64_t c_ptr = plan_ptr[ci];
     const float c_w = plan_w[ci];
-    const bool on = NU == 64 || lane < NU;   // (an idle lane reads the last position's data and uses zeros)
-    const int pos = on ? lane : NU - 1;
+    const int nu = NU ? NU : n_pos;
+    const bool on = NU == 64 || lane < nu;   // (an idle lane reads the last position's data and uses zeros)
+    const int pos = on ? lane : nu - 1;
     const bool rounded = hq_q != nullptr;
     int y[8];
     float dy8 = 0.0f;
     float v[32];
     if (rounded) {
-        const int4* q = (const int4*) (hq_q + (size_t) ent * (32 * NU));
+        const int4* q = (const int4*) (hq_q + (size_t) ent * (32 * nu));
         const int4 ya = q[2 * pos], yb = q[2 * pos + 1];
         y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-        dy8 = a.hq.d[(size_t) ent * NU + pos] * 0.125f;
+        dy8 = a.hq.d[(size_t) ent * nu + pos] * 0.125f;
     } else {
-        const float4* hv = (const float4*) (h + (size_t) ent * (32 * NU) + 32 * pos);
+        const float4* hv = (const float4*) (h + (size_t) ent * (32 * nu) + 32 * pos);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float4 t = hv[i];
@@ -915,14 +936,14 @@ __global__ __launch_bounds__(512, MINW) void down_iq2s_pos_kernel(const uint64_t
     }
     if (skipv) return;
     if (wave >= k) blob = 0ull;
-    constexpr uint32_t qb = NU / 8 * 82 * 4;
+    const uint32_t qb = (uint32_t) nu * 41u;   // bytes of a quad of rows: 4 x 82 a block
     // the wave's blob address is wave-uniform; readfirstlane (a signed int: widened through uint32_t) moves it to
     // scalar registers for the buffer resource (no blob: an empty resource, whose loads read as zero and touch nothing)
     const uint64_t mat = blob ? blob + a.layout.down_off : 0ull;
     const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
     const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (mat_lo | mat_hi) != 0u ? (uint32_t) (n_embd >> 2) * qb : 0u);
-    const QuadOffs qo = quad_offs<NU>(0u, pos);
+    const QuadOffs qo = quad_offs(0u, nu, pos);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     // the first rows' weights are requested before the tables are stored and h is rounded: one trip to memory for the
@@ -930,9 +951,9 @@ __global__ __launch_bounds__(512, MINW) void down_iq2s_pos_kernel(const uint64_t
     QuadIQ2S ring[DEPTH];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) ring[d] = load_quad(rs, qo, quad0 + (uint32_t) d * qb);
-    store_iq2s_selectors<512>(lds);
+    store_iq2s_selectors<64 * SLOTS>(lds);
     table_store(lds, tp);
-    if (threadIdx.x < 8) {
+    if (threadIdx.x < SLOTS) {
         s_on[threadIdx.x] = (int) threadIdx.x < k && c_ptr != 0ull;
         s_w[threadIdx.x] = c_w;
     }
@@ -989,7 +1010,7 @@ __global__ __launch_bounds__(512, MINW) void down_iq2s_pos_kernel(const uint64_t
         float sum = 0.0f;
         bool first = true;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {   // the present slots in slot order; the first product starts the sum
+        for (int i = 0; i < SLOTS; ++i) {   // the present slots in slot order; the first product starts the sum
             const bool have = s_on[i] != 0;
             const float p = __fmul_rn(part[i][c], s_w[i]);
             const float t = first ? p : __fadd_rn(sum, p);

@@ -38,9 +38,8 @@ struct QuadIQ1S {
 struct QuadOffs1 {
     uint32_t i4, qh, d;
 };
-template <int NU>
-__device__ __forceinline__ QuadOffs1 quad_offs1(uint32_t mat_off, int u) {
-    return QuadOffs1{mat_off + 16u * u, mat_off + 16u * NU + 8u * u, mat_off + 24u * NU + 8u * (u >> 3)};
+__device__ __forceinline__ QuadOffs1 quad_offs1(uint32_t mat_off, int nu, int u) {
+    return QuadOffs1{mat_off + 16u * u, mat_off + 16u * nu + 8u * u, mat_off + 24u * nu + 8u * (u >> 3)};
 }
 __device__ __forceinline__ QuadIQ1S load_quad1(__amdgpu_buffer_rsrc_t rs, const QuadOffs1& o, uint32_t quad_off) {
     QuadIQ1S q;
@@ -82,10 +81,11 @@ __device__ __forceinline__ int sum32_codes(const int (&y)[8]) {
     return s;
 }
 
-// ---- gate/up, n_embd = 1024 NW: a workgroup of NW waves = the 2 * 32 NW sub-block positions of a (gate row, up row) pair;
+// ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the sub-block positions of a (gate row, up row) pair (lanes past
+// the row's last position idle, as in the IQ2_S kernels);
 // grid (n_ff / ROWS, entries); entry e = token e / k, slot e % k.  Rows in batches of 8 (two quads), a quad ahead.
 // HEAD (one token): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k).
-template <int NW, int ROWS, int MINW, bool HEAD = false>
+template <int NW, int ROWS, int MINW, bool FIT, bool HEAD = false>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(maya_moe_args a, Codebooks cb, LayerHeadIn hd) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
     constexpr int NU = 32 * NW;
@@ -93,32 +93,35 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(maya_mo
     __shared__ float part[2][2 * NW][8];
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int u = is_up ? t - NU : t;
+    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
+    const bool on = FIT || lu < nu;
+    const int u = on ? lu : nu - 1;
     const int e = blockIdx.y;
     uint64_t blob;
     int y[8];
     float dy8;
     if constexpr (HEAD) {
         float d;
-        if (!head_in_gate_up<NW>(hd, a.k, a.skip, is_up, u, 32 * u, 32 * u + 16, y, d, blob)) return;
+        if (!head_in_gate_up<NW>(hd, a.k, a.skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob)) return;
         dy8 = d * 0.125f;
     } else {
         if (a.skip && *a.skip) return;
         blob = a.plan_ptr[e];
         if (blob == 0ull) return;
         const int tok = e / a.k;
-        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * NU));
+        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * nu));
         const int4 ya = q[2 * u], yb = q[2 * u + 1];
         y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-        dy8 = a.x.d[(size_t) tok * NU + u] * 0.125f;
+        dy8 = a.x.d[(size_t) tok * nu + u] * 0.125f;
+        idle_lane_zero(on, y, dy8);
     }
     stage_iq1s_table<64 * NW>(lds, cb);
     const uint2* grid = (const uint2*) lds;
     const int sy = sum32_codes(y);
-    constexpr uint32_t qb = NU / 8 * 50 * 4;  // bytes of a quad of rows
+    const uint32_t qb = (uint32_t) nu * 25u;  // bytes of a quad of rows: 4 x 50 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
-    const QuadOffs1 qo = quad_offs1<NU>(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, u);
+    const QuadOffs1 qo = quad_offs1(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     QuadIQ1S nxt = load_quad1(rs, qo, quad0);
@@ -153,47 +156,46 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(maya_mo
     }
 }
 
-// ---- down + combine, n_ff = 2048 (64 sub-blocks a row = one wave): wave w = slot w of token blockIdx.y, rows in batches
-// of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.  The
+// ---- down + combine, n_ff = 32 nu <= 2048 (a row on the first nu lanes of one wave): wave w = slot w of token blockIdx.y, of at
+// most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.  The
 // slots' rows meet in LDS and are summed in slot order.
-template <int ROWS, int MINW, int NU = 64>
-__global__ __launch_bounds__(512, MINW) void down_iq1s_pos_kernel(maya_moe_args a, Codebooks cb) {
+template <int ROWS, int MINW, int SLOTS, int NU>
+__global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1s_pos_kernel(maya_moe_args a, Codebooks cb) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
-    static_assert(NU % 8 == 0 && NU >= 8 && NU <= 64, "whole 256-value blocks on one wave");
     __shared__ __align__(16) int lds[kFast1LdsWords];
-    __shared__ float part[8][ROWS];
+    __shared__ float part[SLOTS][ROWS];
     if (a.skip && *a.skip) return;
-    stage_iq1s_table<512>(lds, cb);
+    stage_iq1s_table<64 * SLOTS>(lds, cb);
     const uint2* grid = (const uint2*) lds;
-    const int n_embd = a.layout.n_embd;
+    const int n_embd = a.layout.n_embd, nu = NU ? NU : a.layout.n_ff >> 5;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r0 = blockIdx.x * ROWS;
     const int e0 = blockIdx.y * a.k, ent = e0 + wave;
     const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
     __syncthreads();
     if (blob != 0ull) {
-        constexpr uint32_t qb = NU / 8 * 50 * 4;
+        const uint32_t qb = (uint32_t) nu * 25u;   // bytes of a quad of rows
         const uint64_t mat = blob + a.layout.down_off;
         const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
         const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
         const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) (n_embd >> 2) * qb);
-        // (an idle lane - past the row's NU positions - reads the last position's weights again and meets them with zero
+        // (an idle lane - past the row's nu positions - reads the last position's weights again and meets them with zero
         // activations)
-        const bool on = NU == 64 || lane < NU;
-        const int pos = on ? lane : NU - 1;
-        const QuadOffs1 qo = quad_offs1<NU>(0u, pos);
+        const bool on = NU == 64 || lane < nu;
+        const int pos = on ? lane : nu - 1;
+        const QuadOffs1 qo = quad_offs1(0u, nu, pos);
         const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
         constexpr int NQ = ROWS / 4;
         QuadIQ1S nxt = load_quad1(rs, qo, quad0);
         int y[8];
         float dy8;
         if (a.hq.q) {
-            const int4* q = (const int4*) (a.hq.q + (size_t) ent * (32 * NU));
+            const int4* q = (const int4*) (a.hq.q + (size_t) ent * (32 * nu));
             const int4 ya = q[2 * pos], yb = q[2 * pos + 1];
             y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-            dy8 = a.hq.d[(size_t) ent * NU + pos] * 0.125f;
+            dy8 = a.hq.d[(size_t) ent * nu + pos] * 0.125f;
         } else {
-            const float4* hv = (const float4*) (a.h + (size_t) ent * (32 * NU) + 32 * pos);
+            const float4* hv = (const float4*) (a.h + (size_t) ent * (32 * nu) + 32 * pos);
             float v[32];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -208,11 +210,7 @@ __global__ __launch_bounds__(512, MINW) void down_iq1s_pos_kernel(maya_moe_args 
             q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
             dy8 = d * 0.125f;
         }
-        if (!on) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = 0;
-            dy8 = 0.0f;
-        }
+        idle_lane_zero(on, y, dy8);
         const int sy = sum32_codes(y);
         float acc[8];
 #pragma unroll 1
@@ -264,9 +262,8 @@ struct QuadIQ1M {
 struct QuadOffsM {
     uint32_t i4, qh, d;
 };
-template <int NU>
-__device__ __forceinline__ QuadOffsM quad_offsm(uint32_t mat_off, int u) {
-    return QuadOffsM{mat_off + 16u * u, mat_off + 16u * NU + 8u * u, mat_off + 24u * NU + 32u * (u >> 3)};
+__device__ __forceinline__ QuadOffsM quad_offsm(uint32_t mat_off, int nu, int u) {
+    return QuadOffsM{mat_off + 16u * u, mat_off + 16u * nu + 8u * u, mat_off + 24u * nu + 32u * (u >> 3)};
 }
 __device__ __forceinline__ QuadIQ1M load_quadm(__amdgpu_buffer_rsrc_t rs, const QuadOffsM& o, uint32_t quad_off) {
     QuadIQ1M q;
@@ -314,9 +311,10 @@ __device__ __forceinline__ void sums8_codes(const int (&y)[8], int (&sy8)[4]) {
     for (int l = 0; l < 4; ++l) sy8[l] = dot4(0x01010101, y[2 * l], dot4(0x01010101, y[2 * l + 1], 0));
 }
 
-// ---- gate/up, n_embd = 1024 NW: a workgroup of NW waves = the 2 * 32 NW sub-block positions of a (gate row, up row) pair;
+// ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the sub-block positions of a (gate row, up row) pair (lanes past
+// the row's last position idle, as in the IQ2_S kernels);
 // grid (n_ff / ROWS, entries); entry e = token e / k, slot e % k.  Rows in batches of 8 (two quads), a quad ahead.
-template <int NW, int ROWS, int MINW>
+template <int NW, int ROWS, int MINW, bool FIT>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1m_pos_kernel(maya_moe_args a, Codebooks cb) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
     constexpr int NU = 32 * NW;
@@ -330,22 +328,25 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1m_pos_kernel(maya_mo
     const uint2* grid = (const uint2*) lds;
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int u = is_up ? t - NU : t;
+    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
+    const bool on = FIT || lu < nu;
+    const int u = on ? lu : nu - 1;
     const int tok = e / a.k;
     int y[8];
     {
-        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * NU));
+        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * nu));
         const int4 ya = q[2 * u], yb = q[2 * u + 1];
         y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
     }
+    float dy8 = a.x.d[(size_t) tok * nu + u] * 0.125f;
+    idle_lane_zero(on, y, dy8);
     int sy8[4];
     sums8_codes(y, sy8);
     const int sh = 16 + 6 * (u & 7);
-    const float dy8 = a.x.d[(size_t) tok * NU + u] * 0.125f;
-    constexpr uint32_t qb = NU / 8 * 56 * 4;  // bytes of a quad of rows
+    const uint32_t qb = (uint32_t) nu * 28u;  // bytes of a quad of rows: 4 x 56 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
-    const QuadOffsM qo = quad_offsm<NU>(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, u);
+    const QuadOffsM qo = quad_offsm(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     QuadIQ1M nxt = load_quadm(rs, qo, quad0);
@@ -380,47 +381,46 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1m_pos_kernel(maya_mo
     }
 }
 
-// ---- down + combine, n_ff = 2048 (64 sub-blocks a row = one wave): wave w = slot w of token blockIdx.y, rows in batches
-// of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.  The
+// ---- down + combine, n_ff = 32 nu <= 2048 (a row on the first nu lanes of one wave): wave w = slot w of token blockIdx.y, of at
+// most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.  The
 // slots' rows meet in LDS and are summed in slot order.
-template <int ROWS, int MINW, int NU = 64>
-__global__ __launch_bounds__(512, MINW) void down_iq1m_pos_kernel(maya_moe_args a, Codebooks cb) {
+template <int ROWS, int MINW, int SLOTS, int NU>
+__global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1m_pos_kernel(maya_moe_args a, Codebooks cb) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
-    static_assert(NU % 8 == 0 && NU >= 8 && NU <= 64, "whole 256-value blocks on one wave");
     __shared__ __align__(16) int lds[kFast1LdsWords];
-    __shared__ float part[8][ROWS];
+    __shared__ float part[SLOTS][ROWS];
     if (a.skip && *a.skip) return;
-    stage_iq1s_table<512>(lds, cb);
+    stage_iq1s_table<64 * SLOTS>(lds, cb);
     const uint2* grid = (const uint2*) lds;
-    const int n_embd = a.layout.n_embd;
+    const int n_embd = a.layout.n_embd, nu = NU ? NU : a.layout.n_ff >> 5;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r0 = blockIdx.x * ROWS;
     const int e0 = blockIdx.y * a.k, ent = e0 + wave;
     const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
     __syncthreads();
     if (blob != 0ull) {
-        constexpr uint32_t qb = NU / 8 * 56 * 4;
+        const uint32_t qb = (uint32_t) nu * 28u;   // bytes of a quad of rows
         const uint64_t mat = blob + a.layout.down_off;
         const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
         const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
         const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) (n_embd >> 2) * qb);
-        // (an idle lane - past the row's NU positions - reads the last position's weights again and meets them with zero
+        // (an idle lane - past the row's nu positions - reads the last position's weights again and meets them with zero
         // activations)
-        const bool on = NU == 64 || lane < NU;
-        const int pos = on ? lane : NU - 1;
-        const QuadOffsM qo = quad_offsm<NU>(0u, pos);
+        const bool on = NU == 64 || lane < nu;
+        const int pos = on ? lane : nu - 1;
+        const QuadOffsM qo = quad_offsm(0u, nu, pos);
         const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
         constexpr int NQ = ROWS / 4;
         QuadIQ1M nxt = load_quadm(rs, qo, quad0);
         int y[8];
         float dy8;
         if (a.hq.q) {
-            const int4* q = (const int4*) (a.hq.q + (size_t) ent * (32 * NU));
+            const int4* q = (const int4*) (a.hq.q + (size_t) ent * (32 * nu));
             const int4 ya = q[2 * pos], yb = q[2 * pos + 1];
             y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-            dy8 = a.hq.d[(size_t) ent * NU + pos] * 0.125f;
+            dy8 = a.hq.d[(size_t) ent * nu + pos] * 0.125f;
         } else {
-            const float4* hv = (const float4*) (a.h + (size_t) ent * (32 * NU) + 32 * pos);
+            const float4* hv = (const float4*) (a.h + (size_t) ent * (32 * nu) + 32 * pos);
             float v[32];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -435,11 +435,7 @@ __global__ __launch_bounds__(512, MINW) void down_iq1m_pos_kernel(maya_moe_args 
             q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
             dy8 = d * 0.125f;
         }
-        if (!on) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = 0;
-            dy8 = 0.0f;
-        }
+        idle_lane_zero(on, y, dy8);
         int sy8[4];
         sums8_codes(y, sy8);
         const int sh = 16 + 6 * (lane & 7);

@@ -40,6 +40,13 @@ __device__ __forceinline__ void pos_q4k_codes(PosQ4K& p, int u, const int8_t* q,
         p.shi = dot4(0x01010101, p.yhi[0], dot4(0x01010101, p.yhi[1], dot4(0x01010101, p.yhi[2], dot4(0x01010101, p.yhi[3], 0))));
     }
 }
+// a lane past the row's last position: no codes, no scale
+__device__ __forceinline__ void pos_q4k_idle(PosQ4K& p, bool on) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p.ylo[i] = on ? p.ylo[i] : 0, p.yhi[i] = on ? p.yhi[i] : 0;
+    p.slo = on ? p.slo : 0, p.shi = on ? p.shi : 0;
+    p.dx = on ? p.dx : 0.0f;
+}
 // one row's value at this position: dx (d (sc0 t0 + sc1 t1) - dmin (m0 s0 + m1 s1))
 __device__ __forceinline__ float pos_q4k_value(const PosQ4K& p, const u32x4 hdr, const u32x4 q) {
     // the 6-bit scales / minimums of the lane's two sub-blocks (get_scale_min_k4: include/strata/artifact/dequant.hpp:162-172)
@@ -59,12 +66,12 @@ __device__ __forceinline__ float pos_q4k_value(const PosQ4K& p, const u32x4 hdr,
     return __fmul_rn(p.dx, __fsub_rn(__fmul_rn(d, (float) is), __fmul_rn(dmin, (float) ms)));
 }
 
-// ---- gate/up: a workgroup of NW waves = the 2 * 32 NW positions of a (gate row, up row) pair of n_embd = 1024 NW values;
-// grid (n_ff / ROWS, entries); entry e = token e / k, slot e % k.  Rows in batches of 8, one row ahead in registers.
+// ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the positions of a (gate row, up row) pair (lanes past the row's
+// last position idle, as in the IQ2_S kernels); grid (n_ff / ROWS, entries); entry e = token e / k, slot e % k.  Rows in batches of 8, one row ahead in registers.
 // AHEAD (8 rows): all of a lane's rows are requested up front - the launches of a few entries, whose workgroups do not fill
 // the chip and would otherwise run at the memory's latency a row.
 // HEAD (one token): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k).
-template <int NW, int ROWS, int MINW, bool AHEAD = false, bool HEAD = false>
+template <int NW, int ROWS, int MINW, bool FIT, bool AHEAD = false, bool HEAD = false>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe_args a, LayerHeadIn hd) {
     static_assert(ROWS % 8 == 0, "rows come in batches of 8");
     static_assert(!AHEAD || ROWS == 8, "every row up front: one batch");
@@ -72,7 +79,9 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
     __shared__ float part[2][2 * NW][8];
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int u = is_up ? t - NU : t;
+    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // positions a row; the lane's among 32 NW
+    const bool on = FIT || lu < nu;
+    const int u = on ? lu : nu - 1;
     PosQ4K p;
     pos_q4k_init(p, u, is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u);
     int e;
@@ -83,7 +92,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
         int y[8];
         float d;
         e = (int) blockIdx.y;
-        if (!head_in_gate_up<NW>(hd, a.k, a.skip, is_up, u, v0, v0 + 32, y, d, blob)) return;
+        if (!head_in_gate_up<NW>(hd, a.k, a.skip, is_up, on, lu, v0, v0 + 32, y, d, blob)) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i) p.ylo[i] = y[i], p.yhi[i] = y[4 + i];
         p.dx = d;
@@ -97,9 +106,10 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
         blob = a.plan_ptr[e];
         if (blob == 0ull) return;
         const int tok = e / a.k;
-        pos_q4k_codes(p, u, a.x.q + (size_t) tok * (32 * NU), a.x.d + (size_t) tok * NU, a.x.bsums + (size_t) tok * (2 * NU));
+        pos_q4k_codes(p, u, a.x.q + (size_t) tok * (32 * nu), a.x.d + (size_t) tok * nu, a.x.bsums + (size_t) tok * (2 * nu));
+        pos_q4k_idle(p, on);
     }
-    constexpr uint32_t rb = NU / 8 * 144;   // bytes of a row
+    const uint32_t rb = (uint32_t) nu * 18u;   // bytes of a row: 144 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
     u32x4 hn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, (uint32_t) r0 * rb, 0);
@@ -146,19 +156,18 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
     }
 }
 
-// ---- down + combine, n_ff = 32 NU <= 2048 (NU positions a row on the first NU lanes of one wave; NU a multiple of 8, the
-// lanes past it idle): wave w = slot w of token blockIdx.y, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a
+// ---- down + combine, n_ff = 32 nu <= 2048 (nu positions a row on the first nu lanes of one wave, the lanes past them idle):
+// wave w = slot w of token blockIdx.y, of at most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a
 // rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.
 // AHEAD: all ROWS rows of the wave are requested before anything else is done (one or two slots on one token: a few
 // hundred waves on the whole chip, each with one row in flight, run at the memory's latency a row).
-template <int ROWS, int MINW, int NU = 64, bool AHEAD = false>
-__global__ __launch_bounds__(512, MINW) void down_q4k_pos_kernel(maya_moe_args a) {
+template <int ROWS, int MINW, int SLOTS, int NU, bool AHEAD = false>
+__global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(maya_moe_args a) {
     static_assert(ROWS % 8 == 0, "rows come in batches of 8");
     static_assert(!AHEAD || ROWS == 8, "every row up front: one batch");
-    static_assert(NU % 8 == 0 && NU >= 8 && NU <= 64, "whole 256-value blocks on one wave");
-    __shared__ float part[8][ROWS];
+    __shared__ float part[SLOTS][ROWS];
     if (a.skip && *a.skip) return;
-    const int n_embd = a.layout.n_embd;
+    const int n_embd = a.layout.n_embd, nu = NU ? NU : a.layout.n_ff >> 5;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int bx, by;
     down_block_of_grid(bx, by);
@@ -167,12 +176,12 @@ __global__ __launch_bounds__(512, MINW) void down_q4k_pos_kernel(maya_moe_args a
     const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
     if (blob != 0ull) {
         // (an idle lane reads the last position's weights again and meets them with zero activations)
-        const bool on = NU == 64 || lane < NU;
-        const int pos = on ? lane : NU - 1;
+        const bool on = NU == 64 || lane < nu;
+        const int pos = on ? lane : nu - 1;
         PosQ4K p;
         pos_q4k_init(p, pos, 0u);
         // the first row's weights are requested before h is rounded: their latency hides behind that arithmetic
-        constexpr uint32_t rb = NU / 8 * 144;
+        const uint32_t rb = (uint32_t) nu * 18u;   // bytes of a row: 144 a block
         const uint64_t mat = blob + a.layout.down_off;
         const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
         const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
@@ -188,13 +197,13 @@ __global__ __launch_bounds__(512, MINW) void down_q4k_pos_kernel(maya_moe_args a
             }
         }
         if (a.hq.q) {
-            pos_q4k_codes(p, pos, a.hq.q + (size_t) ent * (32 * NU), a.hq.d + (size_t) ent * NU, a.hq.bsums + (size_t) ent * (2 * NU));
+            pos_q4k_codes(p, pos, a.hq.q + (size_t) ent * (32 * nu), a.hq.d + (size_t) ent * nu, a.hq.bsums + (size_t) ent * (2 * nu));
         } else {
             // Q8_K of h in registers (quant_q8k_block's arithmetic): the lane's 32 values are two runs of 16, a block is
             // 8 lanes; the block's signed maximum is the value at the FIRST largest magnitude, so candidates carry their index
             const int piece = pos & 7, j = piece >> 1, half = piece & 1;
             const int v0 = 256 * (pos >> 3) + 64 * j + 16 * half;
-            const float* hrow = a.h + (size_t) ent * (32 * NU);
+            const float* hrow = a.h + (size_t) ent * (32 * nu);
             float v[32];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -215,12 +224,7 @@ __global__ __launch_bounds__(512, MINW) void down_q4k_pos_kernel(maya_moe_args a
             p.slo = dot4(0x01010101, p.ylo[0], dot4(0x01010101, p.ylo[1], dot4(0x01010101, p.ylo[2], dot4(0x01010101, p.ylo[3], 0))));
             p.shi = dot4(0x01010101, p.yhi[0], dot4(0x01010101, p.yhi[1], dot4(0x01010101, p.yhi[2], dot4(0x01010101, p.yhi[3], 0))));
         }
-        if (!on) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) p.ylo[i] = p.yhi[i] = 0;
-            p.slo = p.shi = 0;
-            p.dx = 0.0f;
-        }
+        pos_q4k_idle(p, on);
         float acc[8];
         if constexpr (AHEAD) {
             ha[0] = hn, qa[0] = qn;

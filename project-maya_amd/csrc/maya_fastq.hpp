@@ -45,9 +45,9 @@ __device__ __forceinline__ void q80_values(const u32x4 qa, const u32x4 qb, uint3
     }
 }
 
-// ---- gate/up: a workgroup of NW waves = the 2 * 32 NW block positions of a (gate row, up row) pair of n_embd = 1024 NW
-// values; grid (n_ff / ROWS, groups).  A step takes 8 / NT row pairs for NT tokens.
-template <int NW, int NT, int ROWS>
+// ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the block positions of a (gate row, up row) pair (lanes past the
+// row's last position idle, as in the IQ2_S kernels); grid (n_ff / ROWS, groups).  A step takes 8 / NT row pairs for NT tokens.
+template <int NW, int NT, int ROWS, bool FIT>
 __global__ __launch_bounds__(64 * NW) void gate_up_q80_pos_kernel(maya_moe_args a) {
     constexpr int NU = 32 * NW, R = 8 / NT;
     static_assert(ROWS % R == 0, "whole steps");
@@ -56,17 +56,21 @@ __global__ __launch_bounds__(64 * NW) void gate_up_q80_pos_kernel(maya_moe_args 
     if (!group_of(a, blockIdx.y, gr)) return;
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int u = is_up ? t - NU : t;
-    const int k = 32 * NU, n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
-    constexpr uint32_t rb = NU * 34;   // bytes of a row
+    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // blocks a row; the lane's position among 32 NW
+    const bool on = FIT || lu < nu;
+    const int u = on ? lu : nu - 1;
+    const int k = 32 * nu, n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
+    const uint32_t rb = (uint32_t) nu * 34u;   // bytes of a row
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(gr.blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
     const uint32_t mat = is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u;
-    const uint32_t oq = mat + 32u * u, od = mat + 32u * NU + 2u * u;
+    const uint32_t oq = mat + 32u * u, od = mat + 32u * nu + 2u * u;
     int step = 0;
     for (int c0 = 0; c0 < gr.ne; c0 += NT) {
         int ents[NT], y[NT][8];
         float dx[NT];
         q80_chunk<NT>(a, gr, c0, a.x, true, k, u, ents, y, dx);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) idle_lane_zero(on, y[i], dx[i]);
         for (int r = 0; r < ROWS; r += R, ++step) {
             float acc[8];
 #pragma unroll
@@ -95,37 +99,31 @@ __global__ __launch_bounds__(64 * NW) void gate_up_q80_pos_kernel(maya_moe_args 
     }
 }
 
-// ---- down, n_ff = 32 NU <= 2048 (NU block positions a row on the first NU lanes of one wave, the lanes past it idle):
+// ---- down, n_ff = 32 nu <= 2048 (nu block positions a row on the first nu lanes of one wave, the lanes past them idle):
 // every wave takes its own rows (wg_rows / 8 of them), a step 8 / NT rows for NT entries of the group; writes
 // part[entry][row]; grid (n_embd / wg_rows, groups)
-template <int NT, int NU = 64>
+template <int NT, int NU>
 __global__ __launch_bounds__(512) void down_q80_pos_kernel(maya_moe_args a, int wg_rows) {
     constexpr int R = 8 / NT;
-    static_assert(NU % 8 == 0 && NU >= 8 && NU <= 64, "a row on one wave");
     GroupRef gr;
     if (!group_of(a, blockIdx.y, gr)) return;
     const int wave = threadIdx.x >> 6, lane0 = threadIdx.x & 63;
     // (an idle lane reads the last position's weights again and meets them with zero activations)
-    const bool on = NU == 64 || lane0 < NU;
-    const int lane = on ? lane0 : NU - 1;
-    const int n_embd = a.layout.n_embd, k = 32 * NU;
+    const int nu = NU ? NU : a.layout.n_ff >> 5;
+    const bool on = NU == 64 || lane0 < nu;
+    const int lane = on ? lane0 : nu - 1;
+    const int n_embd = a.layout.n_embd, k = 32 * nu;
     const int per_wave = wg_rows >> 3, r0 = blockIdx.x * wg_rows + wave * per_wave;
-    constexpr uint32_t rb = NU * 34;
+    const uint32_t rb = (uint32_t) nu * 34u;
     const uint64_t mat = gr.blob + a.layout.down_off;
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(mat, (uint32_t) n_embd * rb);
-    const uint32_t oq = 32u * lane, od = 32u * NU + 2u * lane;
+    const uint32_t oq = 32u * lane, od = 32u * nu + 2u * lane;
     for (int c0 = 0; c0 < gr.ne; c0 += NT) {
         int ents[NT], y[NT][8];
         float dx[NT];
         q80_chunk<NT>(a, gr, c0, a.hq, false, k, lane, ents, y, dx);
-        if (!on) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) y[t][i] = 0;
-                dx[t] = 0.0f;
-            }
-        }
+        for (int i = 0; i < NT; ++i) idle_lane_zero(on, y[i], dx[i]);
         for (int r = 0; r < per_wave; r += R) {
             float acc[8];
 #pragma unroll

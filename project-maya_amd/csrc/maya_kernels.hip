@@ -1614,6 +1614,15 @@ int launch_down_t(const maya_moe_args& a, const DeviceState& st, hipStream_t s) 
     return MAYA_OK;
 }
 
+// The rows the position-mapped gate/up kernels take: any number of whole 256-value blocks up to 8192 values, on pos_waves
+// waves a (gate row, up row) pair; the down rows: up to 2048 values, a row on one wave, up to 16 slots.  What lies
+// between whole multiples of 1024 (n_ff: outside 1024, 1536, 2048), and more than 8 slots, went to the general kernels before:
+// Q4_K 2048 x 768 top-8, one token, 25.2 us a layer, 16.6 like this; IQ2_S 2816 x 768 29.7 -> 15.7; Q4_K 6912 x 1280 top-10, five
+// tokens, 733 -> 143; IQ2_S gate/up with Q4_K down 4864 x 1280, eight tokens, 430 -> 89; Q8_0 2560 x 1280, six tokens, 148 -> 81.
+static bool pos_row_ok(int n_embd) { return n_embd % 256 == 0 && n_embd >= 256 && n_embd <= 8192; }
+static int pos_waves(int n_embd) { return n_embd <= 2048 ? 2 : (n_embd + 1023) / 1024; }
+static bool down_pos_nff_ok(int n_ff) { return n_ff % 256 == 0 && n_ff >= 256 && n_ff <= 2048; }
+
 bool fast_1tok(const maya_moe_args& a) { return a.n_tokens == 1 && a.grp_ptr == nullptr; }
 
 int launch_gate_up_iq2s_gguf(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
@@ -1633,38 +1642,44 @@ template <int NW>
 int launch_gate_up_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
     constexpr int kRows = 16;
     const dim3 grid((unsigned) (a.layout.n_ff / kRows), (unsigned) (a.n_tokens * a.k));   // an entry a column of the grid
-    hipLaunchKernelGGL((gate_up_iq2s_pos_kernel<NW, kRows, 1, 8>), grid, dim3(64 * NW), 0, s, a, st.cb);
+    if (a.layout.n_embd == 1024 * NW) hipLaunchKernelGGL((gate_up_iq2s_pos_kernel<NW, kRows, 1, 8, true>), grid, dim3(64 * NW), 0, s, a, st.cb);
+    else hipLaunchKernelGGL((gate_up_iq2s_pos_kernel<NW, kRows, 1, 8, false>), grid, dim3(64 * NW), 0, s, a, st.cb);
     MAYA_LAUNCHED("gate_up_iq2s_pos_kernel");
     return MAYA_OK;
 }
 // One token: the tile-streaming form, launched with the workgroups the chip holds at once (asked of the runtime once a
 // shape), at most three a compute unit: measured on 7168 x 2048, top-8, 768 workgroups 18.5 us, 1024 (all resident, two
 // tiles each) 20.1 us, 512 20.4 us, 256 24.1 us - a workgroup's cold start is paid per workgroup, latency hiding per wave.
-// The kernel is compiled for 6 waves a SIMD - three workgroups of up to 8 waves a compute unit, what is launched - not 8:
+// (The layer at 4096 x 2048: 20.2 us with three a compute unit, 21.2 with six; 3072 x 1024: 15.6 and 15.7 with eight; only the
+// two-wave workgroups, whose three would leave a compute unit six waves, take twelve: 2048 x 2048 18.9 -> 16.8 us.)
+// The kernel is compiled for 6 waves a SIMD - three workgroups of up to 8 waves a compute unit, what is launched; the small
+// workgroups of two and three waves for 5, which their registers want - not 8:
 // with the head's prologue in it the kernel needs 73-77 registers, and at 64 it spilled 36 bytes a lane to scratch
 // memory: 6.8 MB written and read back a launch, 2.1 us of the layer.  Windows keep gate_up_iq2s_pos_kernel: the tile
 // stream with the resident workgroups shared out among the tokens (a token's codes in a workgroup's registers) was built
 // and is slower there (configs[2]: 260 us against 234).
 template <int NW>
 int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd = nullptr) {
+    constexpr int kMinW = NW <= 3 ? 5 : 6, kMostPerCu = NW == 2 ? 12 : 3;
     static int per_cu = 0;
     if (per_cu == 0) {
         int n = 0, m = 0;
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gate_up_iq2s_tiles_kernel<NW, 6, false>, 64 * NW, 0));
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, 6, true>, 64 * NW, 0));
+        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gate_up_iq2s_tiles_kernel<NW, kMinW, false>, 64 * NW, 0));
+        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, kMinW, true>, 64 * NW, 0));
         n = m < n ? m : n;
-        per_cu = n > 3 ? 3 : n > 0 ? n : 1;
+        per_cu = n > kMostPerCu ? kMostPerCu : n > 0 ? n : 1;
     }
     const int n_tiles = a.k * (a.layout.n_ff / 8);
     const int wgs = per_cu * st.n_cu;
     const unsigned walkers = (unsigned) (wgs < n_tiles ? wgs : n_tiles);
+    const int nu = a.layout.n_embd >> 5;   // sub-blocks a row, in the upper half of `mode`
     if (hd) {   // workgroup 0 routes, the others walk the tiles
-        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, 6, true>), dim3(walkers + 1), dim3(64 * NW), 0, s, (const void*) hd->logits,
-                           (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias, a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8), a.k, a,
+        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, true>), dim3(walkers + 1), dim3(64 * NW), 0, s, (const void*) hd->logits,
+                           (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias, a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a,
                            hd->out);
     } else {
-        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, 6, false>), dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
-                           (const void*) a.x.q, (const void*) a.x.d, st.cb.iq2s, (const float*) nullptr, a.skip, 0, 0, a.k, a, LayerHead{});
+        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, false>), dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
+                           (const void*) a.x.q, (const void*) a.x.d, st.cb.iq2s, (const float*) nullptr, a.skip, 0, nu << 16, a.k, a, LayerHead{});
     }
     MAYA_LAUNCHED("gate_up_iq2s_tiles_kernel");
     return MAYA_OK;
@@ -1683,11 +1698,10 @@ static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& r
         return false;
     if (l.gate_type == kQ4_K) return gate_up_q4k_pos_ok(a);
     if (l.gate_type == kIQ1_S) return gate_up_iq1s_pos_ok(a);
-    return l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && l.n_ff % 16 == 0 && l.n_embd % 1024 == 0 &&
-           l.n_embd >= 2048 && l.n_embd <= 8192;
+    return l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && l.n_ff % 16 == 0 && pos_row_ok(l.n_embd);
 }
 static int launch_layer_gate_up_iq2s(const maya_moe_args& a, const LayerHeadIn& hd, const DeviceState& st, hipStream_t s) {
-    switch (a.layout.n_embd / 1024) {
+    switch (pos_waves(a.layout.n_embd)) {
         case 2: return launch_gate_up_iq2s_tiles<2>(a, st, s, &hd);
         case 3: return launch_gate_up_iq2s_tiles<3>(a, st, s, &hd);
         case 4: return launch_gate_up_iq2s_tiles<4>(a, st, s, &hd);
@@ -1697,8 +1711,6 @@ static int launch_layer_gate_up_iq2s(const maya_moe_args& a, const LayerHeadIn& 
         default: return launch_gate_up_iq2s_tiles<8>(a, st, s, &hd);
     }
 }
-// the rows the position-mapped down kernels take on one wave: n_ff = 1024, 1536 or 2048
-static bool down_pos_nff_ok(int n_ff) { return n_ff == 1024 || n_ff == 1536 || n_ff == 2048; }
 int launch_down_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
     // One quad of rows in flight a wave: with 2, 4 or all 7 of a wave's quads requested ahead the 7168 x 2048 launch took
     // 12.6, 14.0 and 15.9 us against 11.9.
@@ -1706,14 +1718,16 @@ int launch_down_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStrea
     // SIMD the same number of rows, and half as many waves rounding h as with 16), else 16.
     const int n_embd = a.layout.n_embd;
     const int wide = n_embd % 1024 == 0 && n_embd >= 5120 && n_embd <= 8192 ? n_embd / 256 : 16;
-#define MAYA_DN_HEAD a.plan_ptr, a.plan_w, a.h, st.cb.iq2s, a.skip, a.hq.q, a.k, a.layout.n_embd
-#define MAYA_ROWS(R, MINW)                                                                                             \
-    {                                                                                                                  \
-        const dim3 grid((unsigned) (n_embd / R), (unsigned) a.n_tokens);                                               \
-        if (a.layout.n_ff == 1024) hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, MINW, 32>), grid, dim3(512), 0, s, MAYA_DN_HEAD, a, st.cb);      \
-        else if (a.layout.n_ff == 1536) hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, MINW, 48>), grid, dim3(512), 0, s, MAYA_DN_HEAD, a, st.cb); \
-        else hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, MINW>), grid, dim3(512), 0, s, MAYA_DN_HEAD, a, st.cb);                  \
+#define MAYA_ROWS(R, MINW)                                                                                                    \
+    {                                                                                                                         \
+        const dim3 grid((unsigned) (n_embd / R), (unsigned) a.n_tokens);                                                      \
+        if (a.k <= 8 && a.layout.n_ff == 2048)                                                                                \
+            hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, MINW, 8, 64>), grid, dim3(512), 0, s, MAYA_DN_HEAD, a, st.cb);     \
+        else if (a.k <= 8)                                                                                                    \
+            hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, MINW, 8, 0>), grid, dim3(512), 0, s, MAYA_DN_HEAD, a, st.cb);      \
+        else hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, 4, 16, 0>), grid, dim3(1024), 0, s, MAYA_DN_HEAD, a, st.cb);       \
     }
+#define MAYA_DN_HEAD a.plan_ptr, a.plan_w, a.h, st.cb.iq2s, a.skip, a.hq.q, a.k, n_embd, a.layout.n_ff >> 5
     switch (wide) {
         case 20: MAYA_ROWS(20, 4) break;
         case 24: MAYA_ROWS(24, 4) break;
@@ -1747,7 +1761,7 @@ int try_gate_up_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStre
     if (l.packing == MAYA_PACK_STREAM) {
         if (l.n_ff % 16 != 0) return 0;
         if (a.n_tokens == 1) {
-            switch (l.n_embd / 1024 * (l.n_embd % 1024 == 0)) {
+            switch (pos_row_ok(l.n_embd) ? pos_waves(l.n_embd) : 0) {
                 case 2: *rc = launch_gate_up_iq2s_tiles<2>(a, st, s); return 1;
                 case 3: *rc = launch_gate_up_iq2s_tiles<3>(a, st, s); return 1;
                 case 4: *rc = launch_gate_up_iq2s_tiles<4>(a, st, s); return 1;
@@ -1758,7 +1772,7 @@ int try_gate_up_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStre
                 default: return 0;
             }
         }
-        switch (l.n_embd / 1024 * (l.n_embd % 1024 == 0)) {
+        switch (pos_row_ok(l.n_embd) ? pos_waves(l.n_embd) : 0) {
             case 2: *rc = launch_gate_up_iq2s_pos<2>(a, st, s); return 1;
             case 3: *rc = launch_gate_up_iq2s_pos<3>(a, st, s); return 1;
             case 4: *rc = launch_gate_up_iq2s_pos<4>(a, st, s); return 1;
@@ -1777,37 +1791,42 @@ int try_gate_up_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStre
 bool gate_up_iq1s_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (!((l.gate_type == kIQ1_S || l.gate_type == kIQ1_M) && l.up_type == l.gate_type && l.packing == MAYA_PACK_STREAM)) return false;
-    if (l.n_embd % 1024 != 0 || l.n_ff % 16 != 0 || ((l.gate_off | l.up_off | l.down_off) & 15)) return false;
-    const int nw = l.n_embd / 1024;
-    return nw >= 2 && nw <= 8;
+    return pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
 }
 bool down_iq1s_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    return (l.down_type == kIQ1_S || l.down_type == kIQ1_M) && l.packing == MAYA_PACK_STREAM && a.k <= 8 &&
-           (l.n_ff == 1024 || l.n_ff == 1536 || l.n_ff == 2048) && l.n_embd % 16 == 0 && (l.down_off & 15) == 0;
+    return (l.down_type == kIQ1_S || l.down_type == kIQ1_M) && l.packing == MAYA_PACK_STREAM && down_pos_nff_ok(l.n_ff) &&
+           l.n_embd % 16 == 0 && (l.down_off & 15) == 0;
 }
 int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd = nullptr) {
     // (IQ1_S with the head in the launch: one more column, whose first workgroup is the router)
     const dim3 grid((unsigned) (a.layout.n_ff / 16) + (hd ? 1u : 0u), (unsigned) (a.n_tokens * a.k));
     if (a.layout.gate_type == kIQ1_M) {
         if (hd) return fail(MAYA_E_UNSUPPORTED, "gate_up: the IQ1_M rows take no head in their launch");
-        switch (a.layout.n_embd / 1024) {
-            case 2: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<2, 16, 8>), grid, dim3(128), 0, s, a, st.cb); break;
-            case 3: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<3, 16, 8>), grid, dim3(192), 0, s, a, st.cb); break;
-            case 5: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<5, 16, 8>), grid, dim3(320), 0, s, a, st.cb); break;
-            case 4: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<4, 16, 8>), grid, dim3(256), 0, s, a, st.cb); break;
-            case 6: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<6, 16, 8>), grid, dim3(384), 0, s, a, st.cb); break;
-            case 7: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<7, 16, 8>), grid, dim3(448), 0, s, a, st.cb); break;
-            default: hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<8, 16, 8>), grid, dim3(512), 0, s, a, st.cb); break;
+#define MAYA_IQ1M(NWV)                                                                                                                         \
+    if (a.layout.n_embd == 1024 * NWV) hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, a, st.cb);   \
+    else hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<NWV, 16, 7, false>), grid, dim3(64 * NWV), 0, s, a, st.cb);
+        switch (pos_waves(a.layout.n_embd)) {
+            case 2: MAYA_IQ1M(2) break;
+            case 3: MAYA_IQ1M(3) break;
+            case 5: MAYA_IQ1M(5) break;
+            case 4: MAYA_IQ1M(4) break;
+            case 6: MAYA_IQ1M(6) break;
+            case 7: MAYA_IQ1M(7) break;
+            default: MAYA_IQ1M(8) break;
         }
+#undef MAYA_IQ1M
         MAYA_LAUNCHED("gate_up_iq1m_pos_kernel");
         return MAYA_OK;
     }
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
+    const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_IQ1(NWV)                                                                                                          \
-    if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);             \
-    else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);
-    switch (a.layout.n_embd / 1024) {
+    if (hd && fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);  \
+    else if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);   \
+    else if (fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);         \
+    else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, false>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);
+    switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_IQ1(2) break;
         case 3: MAYA_IQ1(3) break;
         case 4: MAYA_IQ1(4) break;
@@ -1824,14 +1843,16 @@ int launch_down_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStrea
     // 32 rows a workgroup for the wide rows (half as many waves rounding h, as in the IQ2_S kernel), else 16
     const bool wide = a.layout.n_embd >= 5120 && a.layout.n_embd % 32 == 0;
     const dim3 grid((unsigned) (a.layout.n_embd / (wide ? 32 : 16)), (unsigned) a.n_tokens);
-#define MAYA_D1(NUV)                                                                                                     \
-    if (wide) {                                                                                                          \
-        if (a.layout.down_type == kIQ1_M) hipLaunchKernelGGL((down_iq1m_pos_kernel<32, 7, NUV>), grid, dim3(512), 0, s, a, st.cb); \
-        else hipLaunchKernelGGL((down_iq1s_pos_kernel<32, 7, NUV>), grid, dim3(512), 0, s, a, st.cb);                    \
-    } else if (a.layout.down_type == kIQ1_M) hipLaunchKernelGGL((down_iq1m_pos_kernel<16, 7, NUV>), grid, dim3(512), 0, s, a, st.cb); \
-    else hipLaunchKernelGGL((down_iq1s_pos_kernel<16, 7, NUV>), grid, dim3(512), 0, s, a, st.cb);
-    if (a.layout.n_ff == 1024) { MAYA_D1(32) } else if (a.layout.n_ff == 1536) { MAYA_D1(48) } else { MAYA_D1(64) }
+#define MAYA_D1T(KERN, R)                                                                                                     \
+    if (a.k <= 8 && a.layout.n_ff == 2048) hipLaunchKernelGGL((KERN<R, 7, 8, 64>), grid, dim3(512), 0, s, a, st.cb);            \
+    else if (a.k <= 8) hipLaunchKernelGGL((KERN<R, 7, 8, 0>), grid, dim3(512), 0, s, a, st.cb);                                 \
+    else hipLaunchKernelGGL((KERN<R, 4, 16, 0>), grid, dim3(1024), 0, s, a, st.cb);
+#define MAYA_D1(R)                                                                     \
+    if (a.layout.down_type == kIQ1_M) { MAYA_D1T(down_iq1m_pos_kernel, R) }              \
+    else { MAYA_D1T(down_iq1s_pos_kernel, R) }
+    if (wide) { MAYA_D1(32) } else { MAYA_D1(16) }
 #undef MAYA_D1
+#undef MAYA_D1T
     MAYA_LAUNCHED("down_iq1s_pos_kernel");
     return MAYA_OK;
 }
@@ -1840,13 +1861,12 @@ int launch_down_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStrea
 bool down_rounds_h(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (down_iq1s_pos_ok(a)) return true;
-    if (l.down_type == kQ4_K) return l.packing == MAYA_PACK_STREAM && a.k <= 8 && down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0 && (l.down_off & 15) == 0;
-    return l.down_type == kIQ2_S && a.k <= 8 && l.packing == MAYA_PACK_STREAM && down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0;
+    if (l.down_type == kQ4_K) return l.packing == MAYA_PACK_STREAM && down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0 && (l.down_off & 15) == 0;
+    return l.down_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0;
 }
 int try_down_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStream_t s, int* rc) {
     const maya_moe_layout& l = a.layout;
-    if (a.k > 8) return 0;
-    if (l.packing != MAYA_PACK_STREAM && !fast_1tok(a)) return 0;
+    if (l.packing != MAYA_PACK_STREAM && (!fast_1tok(a) || a.k > 8)) return 0;
     if (l.packing == MAYA_PACK_STREAM) {
         if (!down_pos_nff_ok(l.n_ff) || l.n_embd % 16 != 0) return 0;
         *rc = launch_down_iq2s_pos(a, st, s);
@@ -1861,13 +1881,11 @@ int try_down_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStream_
 bool gate_up_q4k_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (!(l.gate_type == kQ4_K && l.up_type == kQ4_K && l.packing == MAYA_PACK_STREAM)) return false;
-    if (l.n_embd % 1024 != 0 || l.n_ff % 16 != 0 || ((l.gate_off | l.up_off | l.down_off) & 15)) return false;
-    const int nw = l.n_embd / 1024;
-    return nw >= 2 && nw <= 8;
+    return pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
 }
 bool down_q4k_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    return l.down_type == kQ4_K && l.packing == MAYA_PACK_STREAM && a.k <= 8 && down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0 &&
+    return l.down_type == kQ4_K && l.packing == MAYA_PACK_STREAM && down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0 &&
            (l.down_off & 15) == 0;
 }
 int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHeadIn* hd = nullptr) {
@@ -1877,12 +1895,16 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     // (with the head in the launch: one more column, whose first workgroup is the router)
     const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd ? 1u : 0u), (unsigned) (a.n_tokens * a.k));
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
-#define MAYA_Q4(NWV)                                                                                                       \
-    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, true, true>), grid, dim3(64 * NWV), 0, s, a, h);   \
-    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, false, true>), grid, dim3(64 * NWV), 0, s, a, h);     \
-    else if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, true>), grid, dim3(64 * NWV), 0, s, a, h);          \
-    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8>), grid, dim3(64 * NWV), 0, s, a, h);
-    switch (a.layout.n_embd / 1024) {
+    const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
+#define MAYA_Q4F(NWV, F)                                                                                                    \
+    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, true>), grid, dim3(64 * NWV), 0, s, a, h);   \
+    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, true>), grid, dim3(64 * NWV), 0, s, a, h);     \
+    else if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, a, h);          \
+    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8, F>), grid, dim3(64 * NWV), 0, s, a, h);
+#define MAYA_Q4(NWV)                         \
+    if (fit) { MAYA_Q4F(NWV, true) }        \
+    else { MAYA_Q4F(NWV, false) }
+    switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_Q4(2) break;
         case 3: MAYA_Q4(3) break;
         case 4: MAYA_Q4(4) break;
@@ -1892,29 +1914,26 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
         default: MAYA_Q4(8) break;
     }
 #undef MAYA_Q4
+#undef MAYA_Q4F
     MAYA_LAUNCHED("gate_up_q4k_pos_kernel");
     return MAYA_OK;
 }
 int launch_down_q4k_pos(const maya_moe_args& a, hipStream_t s) {
-    // Rows a workgroup: 32 when that still leaves two workgroups a compute unit (half as many waves rounding h); 8 for
-    // one or two slots on few tokens (more, shorter waves: the rows of one expert alone are latency-bound); else 16.
-    // A workgroup has one wave a slot.
+    // Rows a workgroup: 32 when that still leaves two workgroups a compute unit (half as many waves rounding h); 8, all
+    // requested up front, for one or two slots on few tokens (more, shorter waves: the rows of one expert alone are
+    // latency-bound) and where 16 would leave compute units without a workgroup; else 16.  A workgroup has one wave a slot.
     const int n_embd = a.layout.n_embd;
     const int rows = (long long) (n_embd / 32) * a.n_tokens >= 512 && n_embd % 32 == 0 ? 32
-                     : a.k <= 2 && (long long) (n_embd / 16) * a.n_tokens < 1024 && n_embd % 8 == 0 ? 8 : 16;
+                     : (long long) (n_embd / 16) * a.n_tokens < (a.k <= 2 ? 1024 : 256) && n_embd % 8 == 0 ? 8 : 16;
     const dim3 grid((unsigned) (n_embd / rows), (unsigned) a.n_tokens), block(64u * (unsigned) a.k);
-#define MAYA_ROWS(R)                                                                                              \
-    if (a.layout.n_ff == 1024) hipLaunchKernelGGL((down_q4k_pos_kernel<R, 8, 32>), grid, block, 0, s, a);          \
-    else if (a.layout.n_ff == 1536) hipLaunchKernelGGL((down_q4k_pos_kernel<R, 8, 48>), grid, block, 0, s, a);     \
-    else hipLaunchKernelGGL((down_q4k_pos_kernel<R, 8>), grid, block, 0, s, a);
-    if (rows == 32) { MAYA_ROWS(32) }
-    else if (rows == 8) {
-        // every row of a wave requested up front (128 registers)
-        if (a.layout.n_ff == 1024) hipLaunchKernelGGL((down_q4k_pos_kernel<8, 4, 32, true>), grid, block, 0, s, a);
-        else if (a.layout.n_ff == 1536) hipLaunchKernelGGL((down_q4k_pos_kernel<8, 4, 48, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((down_q4k_pos_kernel<8, 4, 64, true>), grid, block, 0, s, a);
-    }
-    else { MAYA_ROWS(16) }
+    const bool full = a.layout.n_ff == 2048;
+#define MAYA_ROWS(R, MINW, AHEAD)                                                                                              \
+    if (a.k <= 8 && full) hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, 8, 64, AHEAD>), grid, block, 0, s, a);               \
+    else if (a.k <= 8) hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, 8, 0, AHEAD>), grid, block, 0, s, a);                   \
+    else hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, 16, 0, AHEAD>), grid, block, 0, s, a);
+    if (rows == 32) { MAYA_ROWS(32, 8, false) }
+    else if (rows == 8) { MAYA_ROWS(8, 4, true) }   // (128 registers)
+    else { MAYA_ROWS(16, 8, false) }
 #undef MAYA_ROWS
     MAYA_LAUNCHED("down_q4k_pos_kernel");
     return MAYA_OK;
@@ -1923,9 +1942,7 @@ int launch_down_q4k_pos(const maya_moe_args& a, hipStream_t s) {
 bool gate_up_q80_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (!(l.gate_type == kQ8_0 && l.up_type == kQ8_0 && l.packing == MAYA_PACK_STREAM)) return false;
-    if (l.n_embd % 1024 != 0 || l.n_ff % 8 != 0 || ((l.gate_off | l.up_off | l.down_off) & 15)) return false;
-    const int nw = l.n_embd / 1024;
-    return nw >= 2 && nw <= 8;
+    return pos_row_ok(l.n_embd) && l.n_ff % 8 == 0 && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
 }
 bool down_q80_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
@@ -1939,14 +1956,17 @@ inline int q80_group_tokens(const maya_moe_args& a) {
 int launch_gate_up_q80_pos(const maya_moe_args& a, hipStream_t s) {
     const int nt = q80_group_tokens(a);
     const dim3 grid((unsigned) (a.layout.n_ff / 8), (unsigned) (a.n_tokens * a.k));
-#define MAYA_Q8(NWV)                                                                                              \
-    switch (nt) {                                                                                                 \
-        case 8: hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, 8, 8>), grid, dim3(64 * NWV), 0, s, a); break;  \
-        case 4: hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, 4, 8>), grid, dim3(64 * NWV), 0, s, a); break;  \
-        case 2: hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, 2, 8>), grid, dim3(64 * NWV), 0, s, a); break;  \
-        default: hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, 1, 8>), grid, dim3(64 * NWV), 0, s, a); break; \
+#define MAYA_Q8T(NWV, NT)                                                                                                                       \
+    if (a.layout.n_embd == 1024 * NWV) hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, NT, 8, true>), grid, dim3(64 * NWV), 0, s, a);          \
+    else hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, NT, 8, false>), grid, dim3(64 * NWV), 0, s, a);
+#define MAYA_Q8(NWV)                          \
+    switch (nt) {                             \
+        case 8: MAYA_Q8T(NWV, 8) break;       \
+        case 4: MAYA_Q8T(NWV, 4) break;       \
+        case 2: MAYA_Q8T(NWV, 2) break;       \
+        default: MAYA_Q8T(NWV, 1) break;      \
     }
-    switch (a.layout.n_embd / 1024) {
+    switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_Q8(2) break;
         case 3: MAYA_Q8(3) break;
         case 4: MAYA_Q8(4) break;
@@ -1956,6 +1976,7 @@ int launch_gate_up_q80_pos(const maya_moe_args& a, hipStream_t s) {
         default: MAYA_Q8(8) break;
     }
 #undef MAYA_Q8
+#undef MAYA_Q8T
     MAYA_LAUNCHED("gate_up_q80_pos_kernel");
     return MAYA_OK;
 }
@@ -1968,14 +1989,15 @@ int launch_down_q80_pos(const maya_moe_args& a, hipStream_t s) {
     while (per_wave > step && (long long) (a.layout.n_embd / (per_wave * 8)) * a.n_tokens * a.k < 1024) per_wave >>= 1;
     const int wg_rows = per_wave * 8;
     const dim3 grid((unsigned) ((a.layout.n_embd + wg_rows - 1) / wg_rows), (unsigned) (a.n_tokens * a.k));
-#define MAYA_DQ(NUV)                                                                                                    \
-    switch (nt) {                                                                                                       \
-        case 8: hipLaunchKernelGGL((down_q80_pos_kernel<8, NUV>), grid, dim3(512), 0, s, a, wg_rows); break;        \
-        case 4: hipLaunchKernelGGL((down_q80_pos_kernel<4, NUV>), grid, dim3(512), 0, s, a, wg_rows); break;        \
-        case 2: hipLaunchKernelGGL((down_q80_pos_kernel<2, NUV>), grid, dim3(512), 0, s, a, wg_rows); break;        \
-        default: hipLaunchKernelGGL((down_q80_pos_kernel<1, NUV>), grid, dim3(512), 0, s, a, wg_rows); break;       \
+#define MAYA_DQ(NT)                                                                                                             \
+    if (a.layout.n_ff == 2048) hipLaunchKernelGGL((down_q80_pos_kernel<NT, 64>), grid, dim3(512), 0, s, a, wg_rows);            \
+    else hipLaunchKernelGGL((down_q80_pos_kernel<NT, 0>), grid, dim3(512), 0, s, a, wg_rows);
+    switch (nt) {
+        case 8: MAYA_DQ(8) break;
+        case 4: MAYA_DQ(4) break;
+        case 2: MAYA_DQ(2) break;
+        default: MAYA_DQ(1) break;
     }
-    if (a.layout.n_ff == 1024) { MAYA_DQ(32) } else if (a.layout.n_ff == 1536) { MAYA_DQ(48) } else { MAYA_DQ(64) }
 #undef MAYA_DQ
     MAYA_LAUNCHED("down_q80_pos_kernel");
     return MAYA_OK;
@@ -1985,14 +2007,13 @@ int launch_down_q80_pos(const maya_moe_args& a, hipStream_t s) {
 // the shapes the IQ2_S streaming kernels take (what try_gate_up_iq2s_1tok / try_down_iq2s_1tok launch on)
 static bool gate_up_iq2s_fast_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    if (l.packing == MAYA_PACK_STREAM) return l.n_ff % 16 == 0 && l.n_embd % 1024 == 0 && l.n_embd >= 2048 && l.n_embd <= 8192;
+    if (l.packing == MAYA_PACK_STREAM) return l.n_ff % 16 == 0 && pos_row_ok(l.n_embd);
     return fast_1tok(a) && l.n_embd % 1024 == 0 && l.n_embd <= 8192 && l.n_ff % 32 == 0;
 }
 static bool down_iq2s_fast_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    if (a.k > 8) return false;
     if (l.packing == MAYA_PACK_STREAM) return down_pos_nff_ok(l.n_ff) && l.n_embd % 16 == 0;
-    return fast_1tok(a) && l.n_ff % 1024 == 0 && l.n_ff <= 4096 && l.n_embd % 14 == 0;
+    return fast_1tok(a) && a.k <= 8 && l.n_ff % 1024 == 0 && l.n_ff <= 4096 && l.n_embd % 14 == 0;
 }
 // Everything maya_moe_gate_up / maya_moe_down / maya_quant_act refuse (status > 0), asked without launching anything:
 // the calls themselves ask first, and a caller that forks a stream before them (maya_moe_layer_decode_shared) asks before
@@ -2040,9 +2061,7 @@ static int down_refusal(const maya_moe_args* a, const DeviceState& st) {
 bool gate_up_by_entries(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (gate_up_q4k_pos_ok(a) || gate_up_iq1s_pos_ok(a)) return true;
-    if (!(l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM) || l.n_ff % 16 != 0 || l.n_embd % 1024 != 0) return false;
-    const int nw = l.n_embd / 1024;
-    return nw == 4 || nw == 6 || nw == 7 || nw == 8;
+    return l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && gate_up_iq2s_fast_ok(a);
 }
 bool down_by_entries(const maya_moe_args& a) { return down_q4k_pos_ok(a) || down_rounds_h(a); }
 

@@ -95,6 +95,18 @@ CASES = [
     (22, 22, 6144, 2048, 5, 3, 2),
     (22, 22, 7168, 2048, 9, 8, 4),
     (22, 22, 8192, 1536, 4, 4, 3),
+    # rows that end inside a wave of the position-mapped kernels (any multiple of 256; the shortest, one block past a multiple
+    # of 1024, one short of one), down rows likewise, more than 8 slots
+    (12, 12, 256, 256, 4, 2, 3),
+    (22, 22, 1280, 768, 6, 4, 1),
+    (12, 12, 2304, 768, 12, 10, 1),
+    (22, 12, 2816, 1280, 5, 3, 4),
+    (22, 22, 7936, 1792, 13, 11, 2),
+    (19, 22, 1792, 1792, 5, 3, 2),
+    (19, 19, 3328, 512, 12, 9, 1),
+    (29, 29, 3328, 1280, 12, 10, 2),
+    (8, 8, 2560, 1280, 4, 2, 6),
+    (8, 12, 768, 256, 18, 16, 1),
 ]
 
 
@@ -244,7 +256,8 @@ def test_zero_input_and_bf16_input(lib, oracle):
 
 
 @pytest.mark.parametrize("gt,dt,n_embd,n_ff,ne,k,nt", ((22, 12, 1024, 512, 10, 4, 6), (22, 22, 7168, 1024, 6, 4, 3), (22, 12, 4096, 2048, 7, 4, 4), (8, 8, 4096, 2048, 1, 1, 8),
-                                                     (19, 19, 4096, 2048, 5, 4, 4), (29, 29, 4096, 2048, 5, 4, 3)))
+                                                     (19, 19, 4096, 2048, 5, 4, 4), (29, 29, 4096, 2048, 5, 4, 3),
+                                                     (22, 12, 2816, 1280, 12, 10, 4), (19, 29, 1792, 768, 5, 4, 3), (8, 8, 2304, 1280, 5, 4, 4)))
 def test_window_rows_equal_token_rows(lib, gt, dt, n_embd, n_ff, ne, k, nt):
     """A verify window's rows carry the bits its tokens give one at a time (the reference's window contract), in either
     row packing."""
