@@ -62,6 +62,11 @@ CASES = [
     (1024, 512, 4, 2, 4, 4, 8, 0.0),
     (6144, 1536, 6, 2, 10, 8, 4, 0.0),      # the EXL3 configuration's expert shape and window
     (2048, 512, (4, 4, 16), 2, 5, 3, 2, 0.0),   # split gate/up with a general-walk down (16 bits a step)
+    # the layer's row slices: none, slices of unequal length, more slots and tokens than a launch's workgroups leave whole
+    (128, 128, 4, 2, 4, 2, 2, 0.0),
+    (384, 256, 5, 2, 4, 3, 1, 0.0),
+    (640, 384, 6, 2, 6, 3, 3, 0.0),
+    (1408, 896, (7, 7, 3), 2, 12, 10, 16, 0.0),
 ]
 
 
@@ -133,6 +138,23 @@ def test_stages_null_slots_and_window_equals_single_token(ex, oracle):
         h1, out1 = run(None, 1, slice(t, t + 1))
         assert np.array_equal(out1[0], out_win[t])          # the same sums in the same order: the same bits
         assert np.array_equal(h1, h_win[t * k:(t + 1) * k])
+
+
+@pytest.mark.parametrize("n_embd,n_ff,k2,nt", [(640, 384, 6, 4), (2048, 1536, 8, 16), (6144, 1536, 6, 4)])
+def test_a_layers_window_is_its_tokens(ex, n_embd, n_ff, k2, nt):
+    """The layer on a window (several slices a workgroup, two tokens a walk) gives the bits of its tokens one at a time."""
+    from maya_amd import lib
+    n_expert, k = 9, 6
+    l, nbytes = ex.make_layout(n_embd, n_ff, k2, 2)
+    store = lib.ExpertStore([ex.synth_blob(l, nbytes, 40 + e) for e in range(n_expert)])
+    rng = np.random.default_rng(n_embd)
+    logits = torch.from_numpy(rng.standard_normal((nt, n_expert)).astype(np.float32)).cuda()
+    x = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda()
+    win = ex.Exl3Layer(l, n_expert, k, max_tokens=nt).forward(store.table, logits, x).clone()
+    one = ex.Exl3Layer(l, n_expert, k)
+    for t in range(nt):
+        assert torch.equal(one.forward(store.table, logits[t:t + 1], x[t:t + 1])[0], win[t]), t
+    assert float(win.abs().max()) > 0
 
 
 def test_skip_flag_and_bad_shapes(ex):
