@@ -213,7 +213,8 @@ __device__ __forceinline__ void walk_tiles(const uint32_t* __restrict__ trellis,
     }
 }
 
-// ---- the same walk with the bit rate a compile-time constant (K2 <= 10, the mul1 codebook): no LDS staging of the tile.
+// ---- the same walk with the bit rate a compile-time constant (K2 <= 10): no LDS staging of the tile.  (The layer's kernels take it
+// for every codebook: mcg, 6144 x 1536 at 3 bits, one token, 429 us through the general walk, 61 like this.)
 // A lane's 4 windows span 16 + 3 K2 / 2 <= 31 bits, so they sit in the two words around the last window's end - two
 // dword buffer loads at lane-constant offsets, the tile's address in the scalar offset - and one 64-bit shift puts all
 // four into one register, where they are bit-field extracts at compile-time positions.  1024 + the byte sum is an FP16
@@ -229,9 +230,21 @@ __device__ __forceinline__ h2 as_h2(uint32_t v) {
     c.u = v;
     return c.h;
 }
-template <int K2>
+template <int CB, int K2>
 __device__ __forceinline__ void tile_values(uint32_t c, h2& w01, h2& w23) {   // c: the lane's windows
     uint32_t prod[4];
+    if constexpr (CB != 2) {
+        // 3inst / mcg: the sum of the two halves of (state * a [+ b]) & 0x8fff8fff ^ 0x3b603b60; a pair's low halves and its high
+        // halves are gathered into a register each and added two at a time
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t s = __builtin_amdgcn_ubfe(c, Taps<K2>::below(i), 16);
+            prod[i] = ((CB == 1 ? s * 0xCBAC1FEDu : s * 89226354u + 64248484u) & 0x8fff8fffu) ^ 0x3b603b60u;
+        }
+        w01 = as_h2(__builtin_amdgcn_perm(prod[1], prod[0], 0x05040100u)) + as_h2(__builtin_amdgcn_perm(prod[1], prod[0], 0x07060302u));
+        w23 = as_h2(__builtin_amdgcn_perm(prod[3], prod[2], 0x05040100u)) + as_h2(__builtin_amdgcn_perm(prod[3], prod[2], 0x07060302u));
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) prod[i] = __builtin_amdgcn_ubfe(c, Taps<K2>::below(i), 16) * 0x83DCD12Du;
     // 0x6400 + the byte sum (at most 1020: no carry out of the half) = the bits of FP16(1024 + byte sum); the pair's second
@@ -278,7 +291,7 @@ template <int K2> struct TileRing {
     }
 };
 // after_block(b, acc): called with every lane's sums after each 128 rows (8 tiles), b = 0, 1, ...
-template <int K2, int NT, typename F>
+template <int CB, int K2, int NT, typename F>
 __device__ __forceinline__ void walk_tiles_fast(TileRing<K2>& ring, int k, int lane, const __half* xr, int xr_stride, float (&acc)[NT],
                                                 F&& after_block) {
     const int q = (lane >> 1) & 3, nks = k >> 4;
@@ -316,7 +329,7 @@ __device__ __forceinline__ void walk_tiles_fast(TileRing<K2>& ring, int k, int l
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 h2 w01, w23;
-                tile_values<K2>(c[j], w01, w23);
+                tile_values<CB, K2>(c[j], w01, w23);
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     acc[t] = __builtin_amdgcn_fdot2(w01, as_h2(xv[j][t].x), acc[t], false);
@@ -343,7 +356,7 @@ __device__ __forceinline__ void walk(const uint32_t* __restrict__ trellis, int k
     if constexpr (K2 > 0) {
         TileRing<K2> ring;
         ring.request(trellis, k, ld, tc, lane);
-        walk_tiles_fast<K2, NT>(ring, k, lane, xr, xr_stride, acc, [](int, float (&)[NT]) {});
+        walk_tiles_fast<CB, K2, NT>(ring, k, lane, xr, xr_stride, acc, [](int, float (&)[NT]) {});
         column_sums(acc);
     } else walk_tiles<CB, NT>(trellis, k, ld, tc, k2, lane, wt, xr, xr_stride, acc);
 }
@@ -434,7 +447,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_gate_up_kernel(maya_exl3_args
 // the bits they get alone; how many slices a workgroup walks is chosen by how many workgroups the call then has.
 // grid (columns / 128, groups, matrices * S / SP); dynamic LDS: [NT][rows] halves of rotated input, [SP][NT][128] sums.
 __device__ __forceinline__ int slice_block(int s, int nb, int S) { return (s * nb) >> (S >> 1); }   // slice s's first block of nb (S = 1, 2 or 4)
-template <int NT, int K2, bool DOWN>
+template <int CB, int NT, int K2, bool DOWN>
 __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args a, int S, int SP, const __half* __restrict__ hr,
                                                                  float* __restrict__ P) {
     extern __shared__ uint32_t lds[];
@@ -474,7 +487,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
 #pragma unroll
         for (int t = 0; t < NTC; ++t) acc[t] = 0.0f;
         int s = 0, end = slice_block(s0 + 1, nb, S) - b0;
-        walk_tiles_fast<K2, NTC>(ring, kb, lane, xr, kb, acc, [&](int b, float (&v)[NTC]) {
+        walk_tiles_fast<CB, K2, NTC>(ring, kb, lane, xr, kb, acc, [&](int b, float (&v)[NTC]) {
             if (b + 1 == end) {
                 column_sums(v);
                 if (((lane >> 1) & 3) == 0) {
@@ -497,8 +510,11 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
         }
     };
     for (int c0 = 0; c0 < gr.ne;) {
-        if (NT >= 2 && gr.ne - c0 >= 2) {
-            chunk(std::integral_constant<int, 2>{}, c0);
+        if (NT >= 4 && gr.ne - c0 >= 4) {
+            chunk(std::integral_constant<int, NT >= 4 ? 4 : 1>{}, c0);
+            c0 += 4;
+        } else if (NT >= 2 && gr.ne - c0 >= 2) {
+            chunk(std::integral_constant<int, NT >= 2 ? 2 : 1>{}, c0);
             c0 += 2;
         } else {
             chunk(std::integral_constant<int, 1>{}, c0);
@@ -671,21 +687,24 @@ template <int NT, bool DOWN>
 int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, float* P, const DeviceState& st, hipStream_t s) {
     const maya_exl3_layout& l = a.layout;
     const int k = DOWN ? l.n_ff : l.n_embd, n = DOWN ? l.n_embd : l.n_ff, mats = DOWN ? 1 : 2;
-    const int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, st);
+    int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, st);
+    while (SP * NT > 8) SP >>= 1;   // (the closing rotation takes a block of 128 sums a wave)
     const int rows = ((k / 128 + S - 1) / S) * SP * 128;   // the longest workgroup's
     const size_t lds = (size_t) NT * rows * 2 + (size_t) SP * NT * 128 * 4;
     if (lds > (size_t) st.lds_limit) return fail(MAYA_E_SHAPE, "exl3 slices need %zu bytes of LDS, the device gives %d", lds, st.lds_limit);
     const dim3 grid((unsigned) (n / 128), (unsigned) (a.n_tokens * a.k), (unsigned) (mats * (S / SP)));
-#define MAYA_EX(K2V)                                                                                              \
-    case K2V: {                                                                                                   \
-        auto kern = exl3_slices_kernel<NT, K2V, DOWN>;                                                            \
+#define MAYA_EX(CBV, K2V)                                                                                         \
+    case 16 * CBV + K2V: {                                                                                        \
+        auto kern = exl3_slices_kernel<CBV, NT, K2V, DOWN>;                                                       \
         if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); \
         hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, P);                                \
         break;                                                                                                    \
     }
-    switch (l.k2[DOWN ? 2 : 0]) {
-        MAYA_EX(2) MAYA_EX(3) MAYA_EX(4) MAYA_EX(5) MAYA_EX(6) MAYA_EX(7) MAYA_EX(8) MAYA_EX(10)
-        default: return fail(MAYA_E_UNSUPPORTED, "exl3 slices: k2 %d", l.k2[DOWN ? 2 : 0]);
+    switch (16 * l.cb + l.k2[DOWN ? 2 : 0]) {
+        MAYA_EX(2, 2) MAYA_EX(2, 3) MAYA_EX(2, 4) MAYA_EX(2, 5) MAYA_EX(2, 6) MAYA_EX(2, 7) MAYA_EX(2, 8) MAYA_EX(2, 10)
+        MAYA_EX(1, 2) MAYA_EX(1, 4) MAYA_EX(1, 6) MAYA_EX(1, 8) MAYA_EX(1, 10)
+        MAYA_EX(0, 2) MAYA_EX(0, 4) MAYA_EX(0, 6) MAYA_EX(0, 8) MAYA_EX(0, 10)
+        default: return fail(MAYA_E_UNSUPPORTED, "exl3 slices: k2 %d, codebook %d", l.k2[DOWN ? 2 : 0], l.cb);
     }
 #undef MAYA_EX
     MAYA_LAUNCHED("exl3_slices_kernel");
@@ -696,9 +715,9 @@ int launch_exl3_swiglu(const maya_exl3_args& a, int S, const float* P, __half* h
     MAYA_LAUNCHED("exl3_swiglu_kernel");
     return MAYA_OK;
 }
-// the gate/up product in slices when the stage call's `part` holds its partial outputs (mul1, one bit rate <= 5 bits for gate and up):
+// the gate/up product in slices when the stage call's `part` holds its partial outputs (one bit rate <= 5 bits for gate and up):
 // 1 launched, 0 not applicable
-static bool walk_is_fast(const maya_exl3_layout& l, int r) { return l.cb == 2 && l.k2[r] <= 10; }
+static bool walk_is_fast(const maya_exl3_layout& l, int r) { return l.k2[r] <= 10; }
 template <int NT>
 int try_exl3_gu_split(const maya_exl3_args& a, const DeviceState& st, hipStream_t s, int* rc) {
     const maya_exl3_layout& l = a.layout;
@@ -953,9 +972,18 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     if ((rc = exl3_check(&a))) return rc;
     hipStream_t s = as_stream(stream);
     __half* hr = (__half*) w.h;
-    if ((rc = n_tokens > 1 ? launch_exl3_slices<2, false>(a, sl.gu, nullptr, w.part, *st, s) : launch_exl3_slices<1, false>(a, sl.gu, nullptr, w.part, *st, s))) return rc;
+    // tokens that share one decode of the weights: four where an expert has an entry or more on the average
+    // (16 tokens top-8 of 48 experts: 244 us with two before, 186; of 160, 0.8 entries an expert: 451 with two, 468 with four), else two
+    const int nt = n_tokens == 1 ? 1 : n_tokens >= 4 && n_tokens * k >= n_expert ? 4 : 2;
+    auto slices = [&](auto down, int S) {
+        constexpr bool DOWN = decltype(down)::value;
+        return nt == 4   ? launch_exl3_slices<4, DOWN>(a, S, hr, w.part, *st, s)
+               : nt == 2 ? launch_exl3_slices<2, DOWN>(a, S, hr, w.part, *st, s)
+                         : launch_exl3_slices<1, DOWN>(a, S, hr, w.part, *st, s);
+    };
+    if ((rc = slices(std::false_type{}, sl.gu))) return rc;
     if ((rc = launch_exl3_swiglu(a, sl.gu, w.part, hr, s))) return rc;
-    if ((rc = n_tokens > 1 ? launch_exl3_slices<2, true>(a, sl.dn, hr, w.part, *st, s) : launch_exl3_slices<1, true>(a, sl.dn, hr, w.part, *st, s))) return rc;
+    if ((rc = slices(std::true_type{}, sl.dn))) return rc;
     hipLaunchKernelGGL(exl3_combine_kernel, dim3((unsigned) ((l->n_embd + 255) / 256), (unsigned) n_tokens), dim3(256), 0, s, a, (const float*) w.part, sl.dn);
     MAYA_LAUNCHED("exl3_combine_kernel");
     return MAYA_OK;

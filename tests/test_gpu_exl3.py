@@ -67,6 +67,10 @@ CASES = [
     (384, 256, 5, 2, 4, 3, 1, 0.0),
     (640, 384, 6, 2, 6, 3, 3, 0.0),
     (1408, 896, (7, 7, 3), 2, 12, 10, 16, 0.0),
+    # the other codebooks on the compile-time walk; four tokens a walk and what is left of a group
+    (640, 384, 6, 1, 6, 3, 3, 0.0),
+    (512, 256, (10, 10, 2), 0, 6, 3, 2, 0.0),
+    (512, 384, (8, 8, 4), 1, 4, 3, 15, 0.0),
 ]
 
 
@@ -140,12 +144,12 @@ def test_stages_null_slots_and_window_equals_single_token(ex, oracle):
         assert np.array_equal(h1, h_win[t * k:(t + 1) * k])
 
 
-@pytest.mark.parametrize("n_embd,n_ff,k2,nt", [(640, 384, 6, 4), (2048, 1536, 8, 16), (6144, 1536, 6, 4)])
-def test_a_layers_window_is_its_tokens(ex, n_embd, n_ff, k2, nt):
+@pytest.mark.parametrize("n_embd,n_ff,k2,cb,nt", [(640, 384, 6, 2, 4), (2048, 1536, 8, 2, 16), (6144, 1536, 6, 2, 4), (1024, 512, 4, 1, 13)])
+def test_a_layers_window_is_its_tokens(ex, n_embd, n_ff, k2, cb, nt):
     """The layer on a window (several slices a workgroup, two tokens a walk) gives the bits of its tokens one at a time."""
     from maya_amd import lib
     n_expert, k = 9, 6
-    l, nbytes = ex.make_layout(n_embd, n_ff, k2, 2)
+    l, nbytes = ex.make_layout(n_embd, n_ff, k2, cb)
     store = lib.ExpertStore([ex.synth_blob(l, nbytes, 40 + e) for e in range(n_expert)])
     rng = np.random.default_rng(n_embd)
     logits = torch.from_numpy(rng.standard_normal((nt, n_expert)).astype(np.float32)).cuda()
