@@ -439,6 +439,78 @@ __global__ __launch_bounds__(kExThreads) void exl3_gate_up_kernel(maya_exl3_args
     }
 }
 
+// The clamped SwiGLU of an entry's gate/up sums in S slices (slice 0 first) on one wave: the lane's two values of the 128-value block
+// whose first value this lane takes is c (values c and c + 64), P as exl3_slices_kernel left it.
+__device__ __forceinline__ void swiglu_block(const float* __restrict__ P, int S, size_t n, int e, int c, float limit, float& h0, float& h1) {
+    float g[2], u[2];
+    const float* pg = P + ((size_t) e * 2 + 0) * S * n + c;
+    const float* pu = P + ((size_t) e * 2 + 1) * S * n + c;
+    if (S == 4) {   // (the layer's usual form: sixteen loads side by side)
+        float a[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[0][q] = pg[q * n], a[1][q] = pg[q * n + 64], a[2][q] = pu[q * n], a[3][q] = pu[q * n + 64];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            g[i] = __fadd_rn(__fadd_rn(__fadd_rn(a[i][0], a[i][1]), a[i][2]), a[i][3]);
+            u[i] = __fadd_rn(__fadd_rn(__fadd_rn(a[2 + i][0], a[2 + i][1]), a[2 + i][2]), a[2 + i][3]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            g[i] = pg[64 * i], u[i] = pu[64 * i];
+            for (int q = 1; q < S; ++q) {
+                g[i] = __fadd_rn(g[i], pg[q * n + 64 * i]);
+                u[i] = __fadd_rn(u[i], pu[q * n + 64 * i]);
+            }
+        }
+    }
+    h0 = ex_swiglu(g[0], u[0], limit), h1 = ex_swiglu(g[1], u[1], limit);
+}
+
+// ---- the combine at the end of the down launch.  The workgroups of a 128-column block (all groups, all slices) count themselves in
+// done[block], which the gate/up launch before them cleared; the one that comes last adds the block's partial outputs up for
+// every token.  Nobody waits for anybody.  The partial outputs go past the XCD's L2 both ways (agent scope), a workgroup
+// counts itself when its own have arrived; the order of the sums is fixed, so the bits do not depend on who is last.
+// (counters 256 bytes apart: side by side in two cache lines, the 768 workgroups' counts took turns at one memory channel)
+constexpr int kDoneStride = 64;
+__device__ __forceinline__ void store_part(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_part(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void combine_by_last(const maya_exl3_args& a, const float* part, int S, uint32_t* done, uint32_t* lds) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the wave's own partial outputs are where every XCD sees them
+    __syncthreads();
+    if (threadIdx.x == 0) lds[0] = __hip_atomic_fetch_add(done + kDoneStride * blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (lds[0] != gridDim.y * gridDim.z - 1u || (a.skip && *a.skip)) return;
+    const int n = a.layout.n_embd;
+    for (int i = threadIdx.x; i < a.n_tokens * 128; i += kExThreads) {
+        const int t = __builtin_amdgcn_readfirstlane(i >> 7), c = blockIdx.x * 128 + (i & 127), e0 = t * a.k;   // (a wave: half a token's columns)
+        float sum = 0.0f;
+        bool first = true;
+        for (int j0 = 0; j0 < a.k; j0 += 8) {
+            float v[8][2], w[8];
+            uint64_t b[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {   // eight slots' loads side by side (past the last slot: its own again, dropped)
+                const int e = e0 + min(j0 + j, a.k - 1);
+                v[j][0] = load_part(part + (size_t) e * S * n + (uint32_t) c);
+                v[j][1] = load_part(part + ((size_t) e * S + (S - 1)) * n + (uint32_t) c);
+                w[j] = a.plan_w[e];
+                b[j] = a.plan_ptr[e];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (j0 + j >= a.k || b[j] == 0ull) continue;
+                const float p = __fmul_rn(S > 1 ? __fadd_rn(v[j][0], v[j][1]) : v[j][0], w[j]);
+                sum = first ? p : __fadd_rn(sum, p);
+                first = false;
+            }
+        }
+        if (a.add && (!a.add_flag || *a.add_flag)) sum = __fadd_rn(sum, a.add[(size_t) t * n + c]);
+        if (a.add2) sum = __fadd_rn(sum, a.add2[(size_t) t * n + c]);
+        a.out[(size_t) t * n + c] = sum;
+    }
+}
+
 // ---- the products in row slices (the compile-time walk only).  A matrix's rows are cut into S slices of whole 128-row blocks; a
 // workgroup takes 128 columns and SP neighbouring slices of one matrix: it rotates its part of the input (gate/up) or copies the
 // rotated h (down), walks down its rows, and at each slice's end leaves its 128 sums in LDS; these are rotated and scaled at the
@@ -446,13 +518,23 @@ __global__ __launch_bounds__(kExThreads) void exl3_gate_up_kernel(maya_exl3_args
 // holds and the order in which the next kernel adds the slices depend on the expert's shape alone, so a window's tokens get
 // the bits they get alone; how many slices a workgroup walks is chosen by how many workgroups the call then has.
 // grid (columns / 128, groups, matrices * S / SP); dynamic LDS: [NT][rows] halves of rotated input, [SP][NT][128] sums.
+// done: the down launch's counters of column blocks (combine_by_last), cleared by the gate/up launch; NULL: nobody counts.
+// hr NULL (down): the workgroup makes its rows of h itself from the gate/up sums Pgu in Sgu slices.  One token's down launch
+// does - the sums are one trip to memory where the rotated h would be one, against a launch of 4.8 us of its own - windows do
+// not: there every one of a group's 48 workgroups would make them again for each token (4 tokens: 168.5 -> 173.2 us).
 __device__ __forceinline__ int slice_block(int s, int nb, int S) { return (s * nb) >> (S >> 1); }   // slice s's first block of nb (S = 1, 2 or 4)
-template <int CB, int NT, int K2, bool DOWN>
+// COMB (down): the launch adds up as well, over the counters `done`.
+template <int CB, int NT, int K2, bool DOWN, bool COMB>
 __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args a, int S, int SP, const __half* __restrict__ hr,
-                                                                 float* __restrict__ P) {
+                                                                 const float* __restrict__ Pgu, int Sgu, float* P, uint32_t* done) {
     extern __shared__ uint32_t lds[];
+    if (!DOWN && done && blockIdx.y == 0 && blockIdx.z == 0)
+        for (int i = blockIdx.x * kExThreads + threadIdx.x; i < a.layout.n_embd >> 7; i += gridDim.x * kExThreads) done[kDoneStride * i] = 0u;
     ExGroup gr;
-    if (!ex_group_of(a, blockIdx.y, gr)) return;
+    if (!ex_group_of(a, blockIdx.y, gr)) {
+        if constexpr (COMB) combine_by_last(a, P, S, done, lds);
+        return;
+    }
     const int per = S / SP, role = DOWN ? 2 : (int) blockIdx.z / per, s0 = ((int) blockIdx.z % per) * SP;
     const int k = DOWN ? a.layout.n_ff : a.layout.n_embd, n = DOWN ? a.layout.n_embd : a.layout.n_ff, nb = k >> 7;
     const int b0 = slice_block(s0, nb, S), kb = (slice_block(s0 + SP, nb, S) - b0) * 128;   // the workgroup's rows
@@ -471,7 +553,20 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
         TileRing<K2> ring;
         ring.request(trellis, kb, ld, tc, lane);
         __syncthreads();
-        if constexpr (DOWN) {
+        if (DOWN && NT == 1 && hr == nullptr) {
+            const uint16_t* suh = (const uint16_t*) (blob + a.layout.suh[2]) + (size_t) b0 * 128;
+            for (int b = wave; b < kb >> 7; b += kExThreads / 64) {
+                const int i0 = b * 128 + lane;
+                const uint16_t sa = suh[i0], sb = suh[i0 + 64];
+                float h0, h1;
+                swiglu_block(Pgu, Sgu, k, ents[0], b0 * 128 + i0, a.limit, h0, h1);
+                float v0 = __fmul_rn(h0, f16_bits_to_f32(sa)), v1 = __fmul_rn(h1, f16_bits_to_f32(sb));
+                had128_wave(v0, v1, lane);
+                xr[paired_pos(i0)] = __float2half_rn(v0);
+                xr[paired_pos(i0 + 64)] = __float2half_rn(v1);
+            }
+            __syncthreads();
+        } else if constexpr (DOWN) {
 #pragma unroll
             for (int t = 0; t < NTC; ++t)
                 for (int i = threadIdx.x; i < kb >> 3; i += kExThreads)
@@ -506,7 +601,9 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
         for (int i = threadIdx.x; i < SP * NTC * 128; i += kExThreads) {
             const int c = i & 127, j = i >> 7, t = j % NTC, sl = s0 + j / NTC;
             const size_t at = DOWN ? (size_t) ents[t] * S + sl : ((size_t) ents[t] * 2 + role) * S + sl;
-            P[at * n + blockIdx.x * 128 + c] = __fmul_rn(tmp[i], f16_bits_to_f32(sv[c]));
+            const float v = __fmul_rn(tmp[i], f16_bits_to_f32(sv[c]));
+            if constexpr (COMB) store_part(P + at * n + blockIdx.x * 128 + c, v);
+            else P[at * n + blockIdx.x * 128 + c] = v;
         }
     };
     for (int c0 = 0; c0 < gr.ne;) {
@@ -521,6 +618,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
             c0 += 1;
         }
     }
+    if constexpr (COMB) combine_by_last(a, P, S, done, lds);
 }
 // grid (n_ff / 512 rounded up, entries): the clamped SwiGLU of the slices' sums (slice 0 first), a 128-value block a wave: written
 // to h, or - hr given - as the down product's rotated input FP16(H(h * suh)) in the walk's order, once an entry instead
@@ -531,18 +629,8 @@ __global__ __launch_bounds__(256) void exl3_swiglu_kernel(maya_exl3_args a, int 
     if (b * 128 >= n) return;
     const uint64_t blob = a.plan_ptr[e];
     if (blob == 0ull) return;
-    float g[2], u[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const float* pg = P + ((size_t) e * 2 + 0) * S * n + c + 64 * i;
-        const float* pu = P + ((size_t) e * 2 + 1) * S * n + c + 64 * i;
-        g[i] = pg[0], u[i] = pu[0];
-        for (int s = 1; s < S; ++s) {
-            g[i] = __fadd_rn(g[i], pg[(size_t) s * n]);
-            u[i] = __fadd_rn(u[i], pu[(size_t) s * n]);
-        }
-    }
-    const float h0 = ex_swiglu(g[0], u[0], a.limit), h1 = ex_swiglu(g[1], u[1], a.limit);
+    float h0, h1;
+    swiglu_block(P, S, n, e, c, a.limit, h0, h1);
     if (hr == nullptr) {
         a.h[(size_t) e * n + c] = h0;
         a.h[(size_t) e * n + c + 64] = h1;
@@ -683,8 +771,9 @@ static int slices_per_wg(long long wgs, int S, const DeviceState& st) {
     while (sp > 1 && (S % sp != 0 || wgs * (S / sp) < 3ll * st.n_cu)) --sp;
     return sp;
 }
-template <int NT, bool DOWN>
-int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, float* P, const DeviceState& st, hipStream_t s) {
+template <int NT, bool DOWN, bool COMB>
+int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, const float* Pgu, int Sgu, float* P, uint32_t* done, const DeviceState& st,
+                       hipStream_t s) {
     const maya_exl3_layout& l = a.layout;
     const int k = DOWN ? l.n_ff : l.n_embd, n = DOWN ? l.n_embd : l.n_ff, mats = DOWN ? 1 : 2;
     int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, st);
@@ -695,9 +784,9 @@ int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, float* 
     const dim3 grid((unsigned) (n / 128), (unsigned) (a.n_tokens * a.k), (unsigned) (mats * (S / SP)));
 #define MAYA_EX(CBV, K2V)                                                                                         \
     case 16 * CBV + K2V: {                                                                                        \
-        auto kern = exl3_slices_kernel<CBV, NT, K2V, DOWN>;                                                       \
+        auto kern = exl3_slices_kernel<CBV, NT, K2V, DOWN, COMB>;                                                       \
         if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); \
-        hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, P);                                \
+        hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, Pgu, Sgu, P, done);                \
         break;                                                                                                    \
     }
     switch (16 * l.cb + l.k2[DOWN ? 2 : 0]) {
@@ -724,7 +813,7 @@ int try_exl3_gu_split(const maya_exl3_args& a, const DeviceState& st, hipStream_
     if (!walk_is_fast(l, 0) || l.k2[0] != l.k2[1] || !a.part) return 0;
     const int S = (l.n_embd % 256 == 0 && l.n_embd >= 4 * l.n_ff) ? 2 : (l.n_embd >= 2 * l.n_ff ? 1 : 0);
     if (S == 0) return 0;
-    *rc = launch_exl3_slices<NT, false>(a, S, nullptr, a.part, st, s);
+    *rc = launch_exl3_slices<NT, false, false>(a, S, nullptr, nullptr, 0, a.part, nullptr, st, s);
     if (!*rc) *rc = launch_exl3_swiglu(a, S, a.part, nullptr, s);
     return 1;
 }
@@ -896,7 +985,9 @@ static Exl3Slices exl3_slices(const maya_exl3_layout& l) {
 struct Exl3Ws {
     uint64_t *plan_ptr, *grp_ptr;
     int32_t *grp_start, *grp_ent, *n_groups;
-    float *h, *part;   // (slices: h holds the rotated FP16 input of down, part the slices' partial outputs)
+    float *h, *part;   // (slices: h holds the rotated FP16 input of down, part the gate/up slices' sums)
+    float* dn;         // (slices: the down slices' partial outputs - one token's down launch still reads the gate/up sums)
+    uint32_t* done;    // (slices: a counter a 128-column block of the output)
     size_t bytes;
 };
 static Exl3Ws exl3_carve(const maya_exl3_layout& l, int n_tokens, int k, uint8_t* base) {
@@ -915,8 +1006,9 @@ static Exl3Ws exl3_carve(const maya_exl3_layout& l, int n_tokens, int k, uint8_t
     w.n_groups = (int32_t*) take(sizeof(int32_t));
     w.h = (float*) take(sizeof(float) * (size_t) ne * l.n_ff);
     const Exl3Slices sl = exl3_slices(l);
-    const size_t gu = (size_t) 2 * sl.gu * l.n_ff, dn = (size_t) (sl.dn ? sl.dn : 1) * l.n_embd;
-    w.part = (float*) take(sizeof(float) * (size_t) ne * (gu > dn ? gu : dn));
+    w.part = (float*) take(sizeof(float) * (size_t) ne * (sl.gu ? (size_t) 2 * sl.gu * l.n_ff : (size_t) l.n_embd));
+    w.dn = (float*) take(sizeof(float) * (size_t) ne * sl.dn * l.n_embd);
+    w.done = (uint32_t*) take(sl.dn ? sizeof(uint32_t) * kDoneStride * (size_t) (l.n_embd / 128) : 0);
     w.bytes = off;
     return w;
 }
@@ -975,16 +1067,29 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     // tokens that share one decode of the weights: four where an expert has an entry or more on the average
     // (16 tokens top-8 of 48 experts: 244 us with two before, 186; of 160, 0.8 entries an expert: 451 with two, 468 with four), else two
     const int nt = n_tokens == 1 ? 1 : n_tokens >= 4 && n_tokens * k >= n_expert ? 4 : 2;
-    auto slices = [&](auto down, int S) {
-        constexpr bool DOWN = decltype(down)::value;
-        return nt == 4   ? launch_exl3_slices<4, DOWN>(a, S, hr, w.part, *st, s)
-               : nt == 2 ? launch_exl3_slices<2, DOWN>(a, S, hr, w.part, *st, s)
-                         : launch_exl3_slices<1, DOWN>(a, S, hr, w.part, *st, s);
+    const __half* in = n_tokens == 1 ? nullptr : hr;
+    // The combine rides in the down launch up to four tokens: 6144 x 1536 at 3 bits, two tokens 90.3 -> 85.5 us, four 155.5 -> 152;
+    // 4096 x 1280 at 4 bits, one token (with h made there too) 41.5 -> 34.8, four 108.2 -> 103.6.  From eight on nothing was
+    // gained (256.6 -> 259.9): one workgroup a column block then adds up eight tokens, and the launch saved is one in sixty.
+    uint32_t* done = n_tokens <= 4 && nt <= 2 ? w.done : nullptr;
+    auto slices = [&](auto ntc, auto down, auto comb, int S, float* P) {
+        return launch_exl3_slices<decltype(ntc)::value, decltype(down)::value, decltype(comb)::value>(a, S, in, w.part, sl.gu, P, done, *st, s);
     };
-    if ((rc = slices(std::false_type{}, sl.gu))) return rc;
-    if ((rc = launch_exl3_swiglu(a, sl.gu, w.part, hr, s))) return rc;
-    if ((rc = slices(std::true_type{}, sl.dn))) return rc;
-    hipLaunchKernelGGL(exl3_combine_kernel, dim3((unsigned) ((l->n_embd + 255) / 256), (unsigned) n_tokens), dim3(256), 0, s, a, (const float*) w.part, sl.dn);
+    using std::false_type, std::true_type;
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    if ((rc = nt == 4   ? slices(four, false_type{}, false_type{}, sl.gu, w.part)
+              : nt == 2 ? slices(two, false_type{}, false_type{}, sl.gu, w.part)
+                        : slices(one, false_type{}, false_type{}, sl.gu, w.part)))
+        return rc;
+    if (in && (rc = launch_exl3_swiglu(a, sl.gu, w.part, hr, s))) return rc;
+    rc = nt == 4   ? slices(four, true_type{}, false_type{}, sl.dn, w.dn)
+         : nt == 1 ? slices(one, true_type{}, true_type{}, sl.dn, w.dn)
+         : done    ? slices(two, true_type{}, true_type{}, sl.dn, w.dn)
+                   : slices(two, true_type{}, false_type{}, sl.dn, w.dn);
+    if (rc || done) return rc;
+    hipLaunchKernelGGL(exl3_combine_kernel, dim3((unsigned) ((l->n_embd + 255) / 256), (unsigned) n_tokens), dim3(256), 0, s, a, (const float*) w.dn, sl.dn);
     MAYA_LAUNCHED("exl3_combine_kernel");
     return MAYA_OK;
 }

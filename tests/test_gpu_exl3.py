@@ -161,6 +161,44 @@ def test_a_layers_window_is_its_tokens(ex, n_embd, n_ff, k2, cb, nt):
     assert float(win.abs().max()) > 0
 
 
+@pytest.mark.parametrize("n_embd,n_ff,k", [(128, 128, 2), (640, 384, 11), (2048, 1536, 8)])
+def test_a_short_windows_layer_adds_up_in_its_down_launch(ex, n_embd, n_ff, k):
+    """One to four tokens (the column block's last workgroup adds the slots up; one token's down launch makes h itself) against
+    the same tokens of a five-token window (launches of their own): the same bits, with absent experts, a token without any,
+    more slots than one batch of eight, `add`, over repeated calls and replays of a captured one."""
+    from maya_amd import lib
+    n_expert, nt = 14, 5
+    l, nbytes = ex.make_layout(n_embd, n_ff, 6, 2)
+    store = lib.ExpertStore([ex.synth_blob(l, nbytes, 140 + e) for e in range(n_expert)])
+    rng = np.random.default_rng(n_embd)
+    table = store.table.clone()
+    table[[1, 5]] = 0
+    order = np.argsort(-rng.standard_normal((nt, n_expert)), axis=1)
+    ids = torch.from_numpy(order[:, :k].astype(np.int32)).cuda()
+    if k <= 2:
+        ids[2, 0], ids[2, 1] = 1, 5                      # no expert of this token is resident
+    w = torch.from_numpy(rng.random((nt, k)).astype(np.float32)).cuda()
+    x = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda()
+    add = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda()
+    want = ex.Exl3Layer(l, n_expert, k, max_tokens=nt).forward(table, None, x, add=add, routed=(ids, w)).clone()
+    for n in (1, 2, 4):
+        layer = ex.Exl3Layer(l, n_expert, k, max_tokens=n)
+        layer.ws.fill_(0x5a)                             # nothing is expected of the workspace
+        for t in range(0, nt - n + 1):
+            got = layer.forward(table, None, x[t:t + n], add=add[t:t + n], routed=(ids[t:t + n], w[t:t + n]))
+            assert torch.equal(got, want[t:t + n]), (n, t)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            layer.forward(table, None, x[:n], add=add[:n], routed=(ids[:n], w[:n]))
+        for _ in range(3):
+            layer.out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(layer.out[:n], want[:n]), n
+
+
 def test_skip_flag_and_bad_shapes(ex):
     from maya_amd import lib
     l, nbytes = ex.make_layout(256, 128, 4, 2)
