@@ -16,6 +16,7 @@
 
 #include "maya_host.h"
 #include "maya_dev.hpp"
+#include "maya_route.hpp"
 
 namespace maya {
 
@@ -524,14 +525,72 @@ __device__ __forceinline__ void combine_by_last(const maya_exl3_args& a, const f
 // not: there every one of a group's 48 workgroups would make them again for each token (4 tokens: 168.5 -> 173.2 us).
 __device__ __forceinline__ int slice_block(int s, int nb, int S) { return (s * nb) >> (S >> 1); }   // slice s's first block of nb (S = 1, 2 or 4)
 // COMB (down): the launch adds up as well, over the counters `done`.
-template <int CB, int NT, int K2, bool DOWN, bool COMB>
+// HEAD (gate/up, one token, NT = 1): the router rides in the launch.  Every workgroup finds the experts for itself on its last wave by
+// the order of the logits (the exact router there where two are too close to call); the first one routes the token exactly on the
+// wave before and writes ids, weights and plan.  (A workgroup of its own for that took the place of one that walks: 768 fill the
+// chip, and one token of 6144 x 1536 at 4 bits took 52.2 us like that, 50.2 with the router in a launch before.)
+struct Exl3Head {
+    const float* logits;
+    const uint64_t* table;
+    int n_expert;
+    int32_t* ids;
+    float* weights;
+    uint64_t* plan;
+};
+// every thread of a workgroup calls it; lds: kHeadLdsWords.  The blob of slot `slot` (0: none)
+constexpr int kHeadLdsWords = 64 + 256 + 512;
+__device__ __forceinline__ uint64_t exl3_head(const Exl3Head& hd, int k, int slot, bool first, uint32_t* lds) {
+    uint64_t* s_blob = (uint64_t*) lds;
+    float* s_lv = (float*) (lds + 64);
+    uint64_t* s_tab = (uint64_t*) (lds + 64 + 256);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ne = hd.n_expert;
+    const bool picker = wave == kExThreads / 64 - 1;
+    if (picker || (first && wave == kExThreads / 64 - 2)) {
+        float lv[4];
+        uint64_t tab[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = 64 * r + lane;
+            lv[r] = e < ne ? hd.logits[e] : -INFINITY;
+            tab[r] = e < ne ? hd.table[e] : 0ull;
+        }
+        int id;
+        float w;
+        uint64_t ptr;
+        bool exact = true;
+        if (picker) {
+            __builtin_amdgcn_s_setprio(3);   // the workgroup waits for this wave: it goes first on its SIMD
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s_tab[64 * r + lane] = tab[r];
+            exact = !route_wave_order_only(lv, true, ne, k, s_lv, 1e-6f, 60.0f, id);
+            if (!exact) ptr = s_tab[lane < k ? id : 0];
+        }
+        if (exact) route_wave_softmax(lv, tab, ne, k, id, w, ptr);
+        if (lane < k) {
+            if (picker) s_blob[lane] = ptr;
+            else hd.ids[lane] = id, hd.weights[lane] = w, hd.plan[lane] = ptr;
+        }
+        __builtin_amdgcn_s_setprio(0);
+    }
+    __syncthreads();
+    const uint64_t b = s_blob[slot];
+    const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) b), hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (b >> 32));
+    __syncthreads();   // (the rotated input takes this LDS next)
+    return ((uint64_t) hi << 32) | lo;
+}
+template <int CB, int NT, int K2, bool DOWN, bool COMB, bool HEAD = false>
 __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args a, int S, int SP, const __half* __restrict__ hr,
-                                                                 const float* __restrict__ Pgu, int Sgu, float* P, uint32_t* done) {
+                                                                 const float* __restrict__ Pgu, int Sgu, float* P, uint32_t* done, Exl3Head hd) {
     extern __shared__ uint32_t lds[];
     if (!DOWN && done && blockIdx.y == 0 && blockIdx.z == 0)
         for (int i = blockIdx.x * kExThreads + threadIdx.x; i < a.layout.n_embd >> 7; i += gridDim.x * kExThreads) done[kDoneStride * i] = 0u;
     ExGroup gr;
-    if (!ex_group_of(a, blockIdx.y, gr)) {
+    if constexpr (HEAD) {
+        static_assert(NT == 1 && !DOWN, "one token's gate/up launch");
+        gr.e0 = blockIdx.y, gr.ne = 1;
+        gr.blob = exl3_head(hd, a.k, (int) blockIdx.y, blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0, lds);
+        if (gr.blob == 0ull) return;
+    } else if (!ex_group_of(a, blockIdx.y, gr)) {
         if constexpr (COMB) combine_by_last(a, P, S, done, lds);
         return;
     }
@@ -771,22 +830,23 @@ static int slices_per_wg(long long wgs, int S, const DeviceState& st) {
     while (sp > 1 && (S % sp != 0 || wgs * (S / sp) < 3ll * st.n_cu)) --sp;
     return sp;
 }
-template <int NT, bool DOWN, bool COMB>
+template <int NT, bool DOWN, bool COMB, bool HEAD = false>
 int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, const float* Pgu, int Sgu, float* P, uint32_t* done, const DeviceState& st,
-                       hipStream_t s) {
+                       hipStream_t s, const Exl3Head& hd = Exl3Head{}) {
     const maya_exl3_layout& l = a.layout;
     const int k = DOWN ? l.n_ff : l.n_embd, n = DOWN ? l.n_embd : l.n_ff, mats = DOWN ? 1 : 2;
     int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, st);
     while (SP * NT > 8) SP >>= 1;   // (the closing rotation takes a block of 128 sums a wave)
     const int rows = ((k / 128 + S - 1) / S) * SP * 128;   // the longest workgroup's
-    const size_t lds = (size_t) NT * rows * 2 + (size_t) SP * NT * 128 * 4;
+    size_t lds = (size_t) NT * rows * 2 + (size_t) SP * NT * 128 * 4;
+    if (HEAD && lds < 4 * kHeadLdsWords) lds = 4 * kHeadLdsWords;   // (exl3_head's)
     if (lds > (size_t) st.lds_limit) return fail(MAYA_E_SHAPE, "exl3 slices need %zu bytes of LDS, the device gives %d", lds, st.lds_limit);
     const dim3 grid((unsigned) (n / 128), (unsigned) (a.n_tokens * a.k), (unsigned) (mats * (S / SP)));
 #define MAYA_EX(CBV, K2V)                                                                                         \
     case 16 * CBV + K2V: {                                                                                        \
-        auto kern = exl3_slices_kernel<CBV, NT, K2V, DOWN, COMB>;                                                       \
+        auto kern = exl3_slices_kernel<CBV, NT, K2V, DOWN, COMB, HEAD>;                                                       \
         if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); \
-        hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, Pgu, Sgu, P, done);                \
+        hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, Pgu, Sgu, P, done, hd);              \
         break;                                                                                                    \
     }
     switch (16 * l.cb + l.k2[DOWN ? 2 : 0]) {
@@ -1027,7 +1087,12 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     if (workspace_bytes < w.bytes) return fail(MAYA_E_ARG, "exl3 layer: workspace %zu < %zu bytes", workspace_bytes, w.bytes);
     int rc;
     bool grouped = false;
-    if (logits && n_tokens > 1 && n_tokens <= 4 && maya_moe_route_window_ok(nullptr, n_tokens, n_expert, k)) {   // a window of up to four tokens (one pass of the routing workgroup): route, plan and group in one launch
+    const Exl3Slices sl = exl3_slices(*l);
+    // one token on the sliced kernels: the router rides in the gate/up launch (a launch less before it:
+    // 6144 x 1536 at 4 bits 50.2 -> 46.3 us, 4096 x 1280 34.8 -> 31.8, 2048 x 768 23.0 -> 19.1)
+    const bool head = logits && n_tokens == 1 && sl.gu != 0 && n_expert <= 256 && k < n_expert;
+    if (head) {
+    } else if (logits && n_tokens > 1 && n_tokens <= 4 && maya_moe_route_window_ok(nullptr, n_tokens, n_expert, k)) {   // a window of up to four tokens (one pass of the routing workgroup): route, plan and group in one launch
         if ((rc = maya_moe_route_window(nullptr, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start,
                                         w.grp_ent, w.n_groups, stream)))
             return rc;
@@ -1054,7 +1119,6 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     a.part = w.part;
     a.add = add;
     a.out = out;
-    const Exl3Slices sl = exl3_slices(*l);
     if (sl.gu == 0) {
         if ((rc = maya_exl3_gate_up(&a, stream))) return rc;
         return maya_exl3_down(&a, stream);
@@ -1081,6 +1145,8 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     const std::integral_constant<int, 4> four;
     if ((rc = nt == 4   ? slices(four, false_type{}, false_type{}, sl.gu, w.part)
               : nt == 2 ? slices(two, false_type{}, false_type{}, sl.gu, w.part)
+              : head    ? launch_exl3_slices<1, false, false, true>(a, sl.gu, in, w.part, sl.gu, w.part, done, *st, s,
+                                                                    Exl3Head{logits, expert_table, n_expert, ids, weights, w.plan_ptr})
                         : slices(one, false_type{}, false_type{}, sl.gu, w.part)))
         return rc;
     if (in && (rc = launch_exl3_swiglu(a, sl.gu, w.part, hr, s))) return rc;

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "maya_host.h"
+#include "maya_route.hpp"
 #include "maya_iq_grids.h"
 
 namespace maya {
@@ -506,87 +507,6 @@ struct alignas(16) RouterLds {
     unsigned long long lb[256], thr, cand[MAYA_MAX_K * (MAYA_MAX_EXPERTS / 256)];
     int nc;
 };
-// The largest of a wave's values, in every lane's scalar copy: exchanges inside the rows of 16 lanes (lane ^ 1, lane ^ 2,
-// the half-row and row mirrors), then lane 15 of a row to the next row and lane 31 to the upper half; lane 63 has it.
-__device__ __forceinline__ int wave_max_i32(int v) {
-    v = max(v, dpp_i<0xB1>(v));
-    v = max(v, dpp_i<0x4E>(v));
-    v = max(v, dpp_i<0x141>(v));
-    v = max(v, dpp_i<0x140>(v));
-    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-
-// Up to 256 experts, ONE wave, sm.ex filled: lane L keeps experts L, L + 64, L + 128, L + 192 in registers from the sum
-// to the weights, so nothing but the result touches LDS and no workgroup barrier sits on the path.
-//  * the sum: ascending, one add after the other (the reference's order).  The chain of dependent double adds is the
-//    critical path, so every add takes its operand from a lane by v_readlane, eight fetched ahead; all lanes carry the sum.
-//  * the k largest: k rounds of the reference's strict-> arg-max with the lower index on ties
-//    (src/kernels/cuda/router_top10.cu:140-176).  Probabilities are non-negative, so their bit patterns order like the
-//    values as signed integers and -1 marks "taken" or "no such expert"; a round is a 4-way maximum a lane, the wave
-//    maximum, and the first lane (lowest expert: lower register first, then lower lane) that holds it.
-//  * renormalisation: the k weights summed in slot order in double, one division a lane.
-// (the token's exponentials already 4 a lane in ex; the wave's lane i < k returns slot i: its expert and weight.  `tab`:
-// the residency table's entries of the lane's four experts, NULL when no plan is wanted; the slot's blob address then
-// comes back in my_ptr - read from the chosen expert's lane, no second trip to memory.)
-__device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const double (&ex)[4], const uint64_t* tab, int& my_id,
-                                                  float& my_weight, uint64_t& my_ptr) {
-    const int lane = threadIdx.x & 63;
-    int lo[4], hi[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        lo[r] = __double2loint(ex[r]);
-        hi[r] = __double2hiint(ex[r]);
-    }
-    double sum = 0.0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if (64 * r < n_expert) {
-#pragma unroll
-            for (int j0 = 0; j0 < 64; j0 += 8) {
-                int sl[8], sh[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    sl[j] = __builtin_amdgcn_readlane(lo[r], j0 + j);
-                    sh[j] = __builtin_amdgcn_readlane(hi[r], j0 + j);
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) sum += __hiloint2double(sh[j], sl[j]);
-            }
-        }
-    }
-    const float inv = (float) (1.0 / sum);
-    int key[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) key[r] = 64 * r + lane < n_expert ? __float_as_int((float) (ex[r] * (double) inv)) : -1;
-    int id = 0, my_w = 0;
-    uint64_t ptr = 0ull;
-    for (int i = 0; i < k; ++i) {
-        const int top = wave_max_i32(max(max(key[0], key[1]), max(key[2], key[3])));
-        unsigned long long b = __ballot(key[0] == top);
-        int r = 0;
-        if (b == 0ull) b = __ballot(key[1] == top), r = 1;
-        if (b == 0ull) b = __ballot(key[2] == top), r = 2;
-        if (b == 0ull) b = __ballot(key[3] == top), r = 3;
-        const int at = __builtin_amdgcn_readfirstlane(__builtin_ctzll(b));
-#pragma unroll
-        for (int q = 0; q < 4; ++q) key[q] = (q == r && lane == at) ? -1 : key[q];
-        if (lane == i) id = 64 * r + at, my_w = top;
-        if (tab) {
-            const uint64_t tq = r == 0 ? tab[0] : r == 1 ? tab[1] : r == 2 ? tab[2] : tab[3];
-            const uint32_t plo = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) tq, at);
-            const uint32_t phi = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) (tq >> 32), at);
-            if (lane == i) ptr = ((uint64_t) phi << 32) | plo;
-        }
-    }
-    double s = 0.0;
-    for (int i = 0; i < k; ++i) s += (double) __int_as_float(__builtin_amdgcn_readlane(my_w, i));
-    const double sc = fmax(s, 6.103515625e-05);
-    my_id = id;
-    my_weight = (float) ((double) __int_as_float(my_w) / sc);
-    my_ptr = ptr;
-}
 __device__ __forceinline__ void route_narrow(int n_expert, int k, RouterLds& sm) {
     const int lane = threadIdx.x;
     double ex[4];
@@ -735,11 +655,6 @@ struct RouterSpec {
     int kind;            // MAYA_ROUTER_SOFTMAX, MAYA_ROUTER_SIGMOID
     int norm;
 };
-// a float's bits as a signed integer that orders like the float (no -0.0 arises: p > 0 and p + bias = 0 rounds to +0.0)
-__device__ __forceinline__ int float_order_key(float v) {
-    const int b = __float_as_int(v);
-    return b >= 0 ? b : b ^ 0x7fffffff;
-}
 // one wave, up to 256 experts, sm.p and the scores (sm.ex's storage, as floats) filled; on return lane i < k holds slot i
 __device__ __forceinline__ void sigmoid_narrow(int n_expert, int k, const RouterSpec& r, RouterLds& sm) {
     const int lane = threadIdx.x;
@@ -815,74 +730,6 @@ template <int NTH = 256>
 __device__ __forceinline__ void route_any(const float* __restrict__ l, int n_expert, int k, const RouterSpec& r, RouterLds& sm) {
     if (r.kind == MAYA_ROUTER_SIGMOID) route_token_sigmoid<NTH>(l, n_expert, k, r, sm);
     else route_token<NTH>(l, n_expert, k, sm);
-}
-
-// The softmax router on ONE wave, nothing but registers (up to 256 experts, 4 a lane: lane L holds experts L, L + 64, ...;
-// lv = -inf and tab = 0 past the end): the maximum, the exponentials, then route_narrow_regs.  Lane i < k returns slot i.
-__device__ __forceinline__ void route_wave_softmax(const float (&lv)[4], const uint64_t (&tab)[4], int n_expert, int k, int& id,
-                                                   float& w, uint64_t& ptr) {
-    const int lane = threadIdx.x & 63;
-    float mx = fmaxf(fmaxf(lv[0], lv[1]), fmaxf(lv[2], lv[3]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
-    double ex[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ex[r] = 64 * r + lane < n_expert ? exp((double) lv[r] - (double) mx) : 0.0;
-    route_narrow_regs(n_expert, k, ex, tab, id, w, ptr);
-}
-
-// Which k experts the softmax router picks, and in which order, WITHOUT the probabilities: p = exp(l - max) / sum grows
-// with the logit, so the k largest logits in descending order are the k largest probabilities in descending order as long
-// as rounding cannot merge or reorder two of them.  Two logits more than 1e-6 apart give probabilities whose ratio
-// exceeds 1 + 1e-6, far beyond the 2^-24 relative rounding of a float, and a probability within e^-60 of the largest
-// is a normal float.  So: every logit finite, each pick more than 1e-6 above the next, the k-th more than 1e-6 above
-// everything not picked, and all of that within 60 of the first - then the picks and their order are the exact router's.
-// Anything else (ties, near ties, the sub-normal range, NaN / Inf) returns false and the caller runs the exact router.
-//
-// A round must be short (k + 1 of them run one after the other on one wave while its workgroup waits), so a key is one
-// word that names its expert: the logit's ordered bits with the low byte replaced by 255 - index.  The largest key of
-// the wave IS the pick, with no search for the lane that holds it.  The 8 bits given up make picks inside one
-// 256-ulp bucket come out in index order: the check below therefore compares the picks' TRUE logits (a wrong order
-// shows as a negative gap), and holds the k-th pick against the upper end of the (k + 1)-th pick's bucket, above which
-// nothing unpicked can lie.  One wave, k < n_expert <= 256, k + 1 <= 64; s_lv [256] floats of LDS scratch; lane i < k
-// gets slot i's expert.
-// (The sigmoid router picks by the score p + bias itself, so its keys ARE the exact router's: margin 0 - any strictly
-// descending order is the router's - and no range to keep; `fin` then says that no logit and no score is non-finite.)
-__device__ __forceinline__ bool route_wave_order_only(const float (&lv)[4], bool fin, int n_expert, int k, float* s_lv, float margin,
-                                                      float range, int& my_id) {
-    const int lane = threadIdx.x & 63;
-    constexpr int kNone = (int) 0x80000000;
-    int k0, k1, k2, k3;
-    {
-        int key[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = 64 * r + lane;
-            const bool have = e < n_expert;
-            key[r] = have ? (int) (((uint32_t) float_order_key(lv[r]) & 0xffffff00u) | (uint32_t) (255 - e)) : kNone;
-            fin = fin && (!have || isfinite(lv[r]));
-            s_lv[e] = lv[r];
-        }
-        k0 = key[0], k1 = key[1], k2 = key[2], k3 = key[3];
-    }
-    int my_key = kNone;
-    for (int i = 0; i <= k; ++i) {
-        const int top = wave_max_i32(max(max(k0, k1), max(k2, k3)));
-        k0 = k0 == top ? kNone : k0;
-        k1 = k1 == top ? kNone : k1;
-        k2 = k2 == top ? kNone : k2;
-        k3 = k3 == top ? kNone : k3;
-        my_key = lane == i ? top : my_key;
-    }
-    const int id = 255 - (my_key & 255);
-    const float val = lane <= k ? s_lv[id] : 0.0f;
-    const int ub_key = my_key | 255;
-    const float ub = __int_as_float(ub_key >= 0 ? ub_key : ub_key ^ 0x7fffffff);   // the bucket's upper end
-    const float nxt = __shfl_down(lane == k ? ub : val, 1, kWave);
-    const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), 0));
-    const bool apart = lane >= k || (val - nxt > margin && first - nxt <= range);
-    my_id = id;
-    return __all(fin && apart) != 0;
 }
 
 // The sigmoid router on ONE wave, nothing but registers (route_token_sigmoid's arithmetic; up to 256 experts, 4 a lane:

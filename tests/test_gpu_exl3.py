@@ -199,6 +199,40 @@ def test_a_short_windows_layer_adds_up_in_its_down_launch(ex, n_embd, n_ff, k):
             assert torch.equal(layer.out[:n], want[:n]), n
 
 
+@pytest.mark.parametrize("n_embd,n_ff,n_expert,k", [(128, 128, 3, 2), (640, 384, 256, 8), (1024, 512, 70, 16), (640, 384, 8, 8), (640, 384, 300, 4)])
+def test_one_tokens_router_in_the_gate_up_launch(ex, n_embd, n_ff, n_expert, k):
+    """One token routed inside the gate/up launch (more experts than slots, up to 256; else its own launch) against the router's
+    call and the layer on its results, bit for bit: ties at the top and at the cut, equal rows, logits a last place apart,
+    far below the first, NaN and infinities, absent experts."""
+    from maya_amd import lib
+    l, nbytes = ex.make_layout(n_embd, n_ff, 6, 2)
+    distinct = 7
+    store = lib.ExpertStore([ex.synth_blob(l, nbytes, 240 + e) for e in range(distinct)])
+    rng = np.random.default_rng(n_expert + k)
+    table = store.table[torch.from_numpy(rng.integers(0, distinct, n_expert)).cuda()].contiguous()
+    table[n_expert // 2] = 0
+    base = rng.standard_normal((9, n_expert)).astype(np.float32)
+    base[1] = 0.25
+    base[2, ::2] = 4.0
+    order = np.argsort(-base[3])
+    base[3, order[k - 1]] = np.nextafter(base[3, order[min(k, n_expert - 1)]], np.float32(10))   # the cut, a last place apart
+    base[4] = -1e30
+    base[4, n_expert - 1] = 0.0
+    base[5] *= 40
+    base[6, 1] = np.nan
+    base[7, 2] = np.inf
+    base[8, :] = np.round(base[8] * 2) / 2
+    x = torch.from_numpy(rng.standard_normal((1, n_embd)).astype(np.float32)).cuda()
+    layer = ex.Exl3Layer(l, n_expert, k)
+    for r in range(base.shape[0]):
+        logits = torch.from_numpy(base[r:r + 1]).cuda()
+        ids, w, _ = lib.route_plan(logits, k, table)
+        out = layer.forward(table, logits, x).clone()
+        assert torch.equal(layer.ids[:1], ids) and torch.equal(layer.weights[:1].view(torch.int32), w.view(torch.int32)), r
+        want = layer.forward(table, None, x, routed=(ids, w))
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32)), r
+
+
 def test_skip_flag_and_bad_shapes(ex):
     from maya_amd import lib
     l, nbytes = ex.make_layout(256, 128, 4, 2)
