@@ -425,38 +425,6 @@ typedef float pf_v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 pf_v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 
-// A tile's outputs: lane (ln, kh) holds weight row ln for the tile's rows 32 m + 8 b + 4 kh + r (i = 4 b + r).  Gate/up: the up row
-// of a feature sits 16 lanes above its gate row; of two rows' values the lower lane takes the first row and the upper lane
-// the second (one exchange gives each what it lacks), so every lane makes an output - with the lower lanes alone at work the
-// SwiGLU's 47 instructions an output were a sixth of the kernel's at n_embd = 4096.  A 4096-token chunk on 288 experts of
-// 4096 x 2048: 3030 -> 2975 us.
-template <bool GU, int NM>
-__device__ __forceinline__ void pf_store(const PfGemm& a, const pf_v16f (&acc)[NM], float scale, int64_t n0, int row0, int nrows, int ln, int kh) {
-    const bool lower = ln < 16;
-    float* const o = a.out + (size_t) row0 * a.n + n0 + (GU ? (ln & 15) : ln);
-    const int n = (int) a.n;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            if (32 * m + 8 * b >= nrows) continue;   // (uniform)
-#pragma unroll
-            for (int r = 0; r < 4; r += GU ? 2 : 1) {
-                const int i = 4 * b + r;
-                if constexpr (GU) {
-                    const float got = xor_lane<16>(lower ? acc[m][i + 1] : acc[m][i]);
-                    const float g = lower ? acc[m][i] : got, u = lower ? got : acc[m][i + 1];
-                    const int row = 32 * m + 8 * b + 4 * kh + r + (lower ? 0 : 1);
-                    if (row < nrows) o[(size_t) (unsigned) (row * n)] = pf_swiglu(__fmul_rn(g, scale), __fmul_rn(u, scale), a.limit);
-                } else {
-                    const int row = 32 * m + 8 * b + 4 * kh + r;
-                    if (row < nrows) o[(size_t) (unsigned) (row * n)] = __fmul_rn(acc[m][i], scale);
-                }
-            }
-        }
-    }
-}
-
 // One tile of NM x 32 rows against the wave's 32 weight rows (gate/up: the gate rows of 16 features, then their up rows;
 // down: 32 output rows), on the 32x32 matrix instructions: lane (ln = lane & 31, kh = lane >> 5) holds 16 of a
 // sub-block's 32 values of activation row ln (A operand, from LDS) and of weight row ln (B operand, decoded in
@@ -637,7 +605,21 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* b0, uint8_t* b
     }
     if (!wave_on) return;
 
-    pf_store<GU, NM>(a, acc, 1.0f, n0, row0, nrows, ln, kh);
+    // outputs: lane (ln, kh) holds weight row ln for the tile's rows 32 m + 8 b + 4 kh + r (i = 4 b + r)
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = 32 * m + 8 * (i >> 2) + 4 * kh + (i & 3);
+            if constexpr (GU) {
+                // the up row of a feature sits 16 lanes above its gate row
+                const float up = __shfl(acc[m][i], (lane + 16) & 63, kWave);
+                if (ln < 16 && r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = pf_swiglu(acc[m][i], up, a.limit);
+            } else {
+                if (r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = acc[m][i];
+            }
+        }
+    }
 }
 
 #include "maya_prefill_iq2s.hpp"

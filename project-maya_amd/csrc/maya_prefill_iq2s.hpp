@@ -189,7 +189,21 @@ __device__ __forceinline__ void pf_tile_iq2s(const PfGemm& a, uint8_t* b0, uint8
     }
     if (!wave_on) return;
 
-    pf_store<GU, NM>(a, acc, 0.125f, n0, row0, nrows, ln, kh);
+    // outputs: lane (ln, kh) holds weight row ln for the tile's rows 32 m + 8 b + 4 kh + r (i = 4 b + r)
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = 32 * m + 8 * (i >> 2) + 4 * kh + (i & 3);
+            const float val = __fmul_rn(acc[m][i], 0.125f);
+            if constexpr (GU) {
+                const float up = __shfl(val, (lane + 16) & 63, kWave);   // the up row of a feature sits 16 lanes above its gate row
+                if (ln < 16 && r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = pf_swiglu(val, up, a.limit);
+            } else {
+                if (r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = val;
+            }
+        }
+    }
 }
 
 // grid (bands of weight rows, tiles at most)
