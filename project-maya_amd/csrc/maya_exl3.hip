@@ -16,6 +16,7 @@
 
 #include "maya_host.h"
 #include "maya_dev.hpp"
+#include "maya_groups.hpp"
 #include "maya_route.hpp"
 
 namespace maya {
@@ -100,31 +101,6 @@ __device__ __forceinline__ void had128_wave(float& v0, float& v1, int lane) {
     const float s = 1.0f / sqrtf(128.0f);
     v0 = __fmul_rn(v0, s);
     v1 = __fmul_rn(v1, s);
-}
-
-struct ExGroup {
-    uint64_t blob;
-    int e0, ne;
-};
-__device__ __forceinline__ bool ex_group_of(const maya_exl3_args& a, int g, ExGroup& r) {
-    if (a.skip && *a.skip) return false;
-    if (a.grp_ptr) {
-        // (all asked for at once: past the last group these are words of the arrays that nobody wrote, and dropped)
-        const int ng = *a.n_groups, end = a.grp_start[g + 1];
-        r.blob = a.grp_ptr[g];
-        r.e0 = a.grp_start[g];
-        r.ne = end - r.e0;
-        if (g >= ng) return false;
-    } else {
-        if (g >= a.n_tokens * a.k) return false;
-        r.blob = a.plan_ptr[g];
-        r.e0 = g;
-        r.ne = 1;
-    }
-    return r.blob != 0ull && r.ne > 0;
-}
-__device__ __forceinline__ int ex_entry_of(const maya_exl3_args& a, const ExGroup& r, int i) {
-    return a.grp_ptr ? a.grp_ent[r.e0 + i] : r.e0;
 }
 
 // xr = FP16(H(x * suh)) of one activation into LDS; every wave of the workgroup takes blocks of 128 values (`tmp` is not
@@ -375,8 +351,8 @@ __device__ __forceinline__ float ex_swiglu(float g, float u, float limit) {
 template <int CB, int NT, int K2>
 __global__ __launch_bounds__(kExThreads) void exl3_gate_up_kernel(maya_exl3_args a) {
     extern __shared__ uint32_t lds[];
-    ExGroup gr;
-    if (!ex_group_of(a, blockIdx.y, gr)) return;
+    GroupRef gr;
+    if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int k = a.layout.n_embd, n = a.layout.n_ff;
     uint32_t* wt = lds + (threadIdx.x >> 6) * 64;
     __half* xr = (__half*) (lds + 8 * 64);                       // [NT][2][k]
@@ -390,7 +366,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_gate_up_kernel(maya_exl3_args
         constexpr int NTC = decltype(ntc)::value;
         int ents[NTC];
 #pragma unroll
-        for (int t = 0; t < NTC; ++t) ents[t] = ex_entry_of(a, gr, c0 + t);
+        for (int t = 0; t < NTC; ++t) ents[t] = entry_of(a, gr, c0 + t);
         __syncthreads();
         for (int t = 0; t < NTC; ++t) {
             const float* x = a.x + (size_t) (ents[t] / a.k) * xs;
@@ -525,6 +501,7 @@ __device__ __forceinline__ void combine_by_last(const maya_exl3_args& a, const f
 // not: there every one of a group's 48 workgroups would make them again for each token (4 tokens: 168.5 -> 173.2 us).
 __device__ __forceinline__ int slice_block(int s, int nb, int S) { return (s * nb) >> (S >> 1); }   // slice s's first block of nb (S = 1, 2 or 4)
 // COMB (down): the launch adds up as well, over the counters `done`.
+// whole_groups: the group arrays are a layer's workspace, a word for every entry (group_of); 0: a stage call's, which may end sooner.
 // HEAD (gate/up, one token, NT = 1): the router rides in the launch.  Every workgroup finds the experts for itself on its last wave by
 // the order of the logits (the exact router there where two are too close to call); the first one routes the token exactly on the
 // wave before and writes ids, weights and plan.  (A workgroup of its own for that took the place of one that walks: 768 fill the
@@ -580,17 +557,17 @@ __device__ __forceinline__ uint64_t exl3_head(const Exl3Head& hd, int k, int slo
 }
 template <int CB, int NT, int K2, bool DOWN, bool COMB, bool HEAD = false>
 __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args a, int S, int SP, const __half* __restrict__ hr,
-                                                                 const float* __restrict__ Pgu, int Sgu, float* P, uint32_t* done, Exl3Head hd) {
+                                                                 const float* __restrict__ Pgu, int Sgu, float* P, uint32_t* done, Exl3Head hd, int whole_groups) {
     extern __shared__ uint32_t lds[];
     if (!DOWN && done && blockIdx.y == 0 && blockIdx.z == 0)
         for (int i = blockIdx.x * kExThreads + threadIdx.x; i < a.layout.n_embd >> 7; i += gridDim.x * kExThreads) done[kDoneStride * i] = 0u;
-    ExGroup gr;
+    GroupRef gr;
     if constexpr (HEAD) {
         static_assert(NT == 1 && !DOWN, "one token's gate/up launch");
         gr.e0 = blockIdx.y, gr.ne = 1;
         gr.blob = exl3_head(hd, a.k, (int) blockIdx.y, blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0, lds);
         if (gr.blob == 0ull) return;
-    } else if (!ex_group_of(a, blockIdx.y, gr)) {
+    } else if (!(whole_groups ? group_of<true>(a, blockIdx.y, gr) : group_of<false>(a, blockIdx.y, gr))) {
         if constexpr (COMB) combine_by_last(a, P, S, done, lds);
         return;
     }
@@ -608,7 +585,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
         constexpr int NTC = decltype(ntc)::value;
         int ents[NTC];
 #pragma unroll
-        for (int t = 0; t < NTC; ++t) ents[t] = ex_entry_of(a, gr, c0 + t);
+        for (int t = 0; t < NTC; ++t) ents[t] = entry_of(a, gr, c0 + t);
         TileRing<K2> ring;
         ring.request(trellis, kb, ld, tc, lane);
         __syncthreads();
@@ -706,8 +683,8 @@ __global__ __launch_bounds__(256) void exl3_swiglu_kernel(maya_exl3_args a, int 
 template <int CB, int NT, int K2>
 __global__ __launch_bounds__(kExThreads) void exl3_down_kernel(maya_exl3_args a) {
     extern __shared__ uint32_t lds[];
-    ExGroup gr;
-    if (!ex_group_of(a, blockIdx.y, gr)) return;
+    GroupRef gr;
+    if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int k = a.layout.n_ff, n = a.layout.n_embd;
     uint32_t* wt = lds + (threadIdx.x >> 6) * 64;
     __half* xr = (__half*) (lds + 8 * 64);             // [NT][k]
@@ -719,7 +696,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_down_kernel(maya_exl3_args a)
         constexpr int NTC = decltype(ntc)::value;
         int ents[NTC];
 #pragma unroll
-        for (int t = 0; t < NTC; ++t) ents[t] = ex_entry_of(a, gr, c0 + t);
+        for (int t = 0; t < NTC; ++t) ents[t] = entry_of(a, gr, c0 + t);
         __syncthreads();
         for (int t = 0; t < NTC; ++t)
             rotate_in<(K2 > 0)>(a.h + (size_t) ents[t] * k, (const uint16_t*) (blob + a.layout.suh[2]), k, tmp, xr + (size_t) t * k);
@@ -831,8 +808,8 @@ static int slices_per_wg(long long wgs, int S, const DeviceState& st) {
     return sp;
 }
 template <int NT, bool DOWN, bool COMB, bool HEAD = false>
-int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, const float* Pgu, int Sgu, float* P, uint32_t* done, const DeviceState& st,
-                       hipStream_t s, const Exl3Head& hd = Exl3Head{}) {
+int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, const float* Pgu, int Sgu, float* P, uint32_t* done, bool whole_groups,
+                       const DeviceState& st, hipStream_t s, const Exl3Head& hd = Exl3Head{}) {
     const maya_exl3_layout& l = a.layout;
     const int k = DOWN ? l.n_ff : l.n_embd, n = DOWN ? l.n_embd : l.n_ff, mats = DOWN ? 1 : 2;
     int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, st);
@@ -846,7 +823,7 @@ int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, const f
     case 16 * CBV + K2V: {                                                                                        \
         auto kern = exl3_slices_kernel<CBV, NT, K2V, DOWN, COMB, HEAD>;                                                       \
         if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); \
-        hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, Pgu, Sgu, P, done, hd);              \
+        hipLaunchKernelGGL(kern, grid, dim3(kExThreads), lds, s, a, S, SP, hr, Pgu, Sgu, P, done, hd, whole_groups ? 1 : 0);              \
         break;                                                                                                    \
     }
     switch (16 * l.cb + l.k2[DOWN ? 2 : 0]) {
@@ -873,7 +850,7 @@ int try_exl3_gu_split(const maya_exl3_args& a, const DeviceState& st, hipStream_
     if (!walk_is_fast(l, 0) || l.k2[0] != l.k2[1] || !a.part) return 0;
     const int S = (l.n_embd % 256 == 0 && l.n_embd >= 4 * l.n_ff) ? 2 : (l.n_embd >= 2 * l.n_ff ? 1 : 0);
     if (S == 0) return 0;
-    *rc = launch_exl3_slices<NT, false, false>(a, S, nullptr, nullptr, 0, a.part, nullptr, st, s);
+    *rc = launch_exl3_slices<NT, false, false>(a, S, nullptr, nullptr, 0, a.part, nullptr, false, st, s);
     if (!*rc) *rc = launch_exl3_swiglu(a, S, a.part, nullptr, s);
     return 1;
 }
@@ -1137,7 +1114,7 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     // gained (256.6 -> 259.9): one workgroup a column block then adds up eight tokens, and the launch saved is one in sixty.
     uint32_t* done = n_tokens <= 4 && nt <= 2 ? w.done : nullptr;
     auto slices = [&](auto ntc, auto down, auto comb, int S, float* P) {
-        return launch_exl3_slices<decltype(ntc)::value, decltype(down)::value, decltype(comb)::value>(a, S, in, w.part, sl.gu, P, done, *st, s);
+        return launch_exl3_slices<decltype(ntc)::value, decltype(down)::value, decltype(comb)::value>(a, S, in, w.part, sl.gu, P, done, true, *st, s);
     };
     using std::false_type, std::true_type;
     const std::integral_constant<int, 1> one;
@@ -1145,7 +1122,7 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     const std::integral_constant<int, 4> four;
     if ((rc = nt == 4   ? slices(four, false_type{}, false_type{}, sl.gu, w.part)
               : nt == 2 ? slices(two, false_type{}, false_type{}, sl.gu, w.part)
-              : head    ? launch_exl3_slices<1, false, false, true>(a, sl.gu, in, w.part, sl.gu, w.part, done, *st, s,
+              : head    ? launch_exl3_slices<1, false, false, true>(a, sl.gu, in, w.part, sl.gu, w.part, done, true, *st, s,
                                                                     Exl3Head{logits, expert_table, n_expert, ids, weights, w.plan_ptr})
                         : slices(one, false_type{}, false_type{}, sl.gu, w.part)))
         return rc;

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(64 * NW) void gate_up_q80_pos_kernel(maya_moe_args 
     static_assert(ROWS % R == 0, "whole steps");
     __shared__ float part[2][2 * NW][8];
     GroupRef gr;
-    if (!group_of(a, blockIdx.y, gr)) return;
+    if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
     const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // blocks a row; the lane's position among 32 NW
@@ -106,7 +106,7 @@ template <int NT, int NU>
 __global__ __launch_bounds__(512) void down_q80_pos_kernel(maya_moe_args a, int wg_rows) {
     constexpr int R = 8 / NT;
     GroupRef gr;
-    if (!group_of(a, blockIdx.y, gr)) return;
+    if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int wave = threadIdx.x >> 6, lane0 = threadIdx.x & 63;
     // (an idle lane reads the last position's weights again and meets them with zero activations)
     const int nu = NU ? NU : a.layout.n_ff >> 5;

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "maya_host.h"
+#include "maya_groups.hpp"
 #include "maya_route.hpp"
 #include "maya_iq_grids.h"
 
@@ -1160,30 +1161,6 @@ __device__ __forceinline__ void stage_act(int* lds_act, int k, const maya_act& s
     }
 }
 
-struct GroupRef {
-    uint64_t blob;
-    int e0, ne;          // entries [e0, e0 + ne) of grp_ent (or the single entry e0 when grp_ent is null)
-};
-__device__ __forceinline__ bool group_of(const maya_moe_args& a, int g, GroupRef& r) {
-    if (a.skip && *a.skip) return false;
-    const int total = a.n_tokens * a.k;
-    if (a.grp_ptr) {
-        if (g >= *a.n_groups) return false;
-        r.blob = a.grp_ptr[g];
-        r.e0 = a.grp_start[g];
-        r.ne = a.grp_start[g + 1] - r.e0;
-    } else {
-        if (g >= total) return false;
-        r.blob = a.plan_ptr[g];
-        r.e0 = g;
-        r.ne = 1;
-    }
-    return r.blob != 0ull && r.ne > 0;
-}
-__device__ __forceinline__ int entry_of(const maya_moe_args& a, const GroupRef& r, int i) {
-    return a.grp_ptr ? a.grp_ent[r.e0 + i] : r.e0;
-}
-
 __device__ __forceinline__ float swiglu(float g, float u, float limit) {
     if (limit > 0.0f && limit < INFINITY) {
         g = fminf(g, limit);
@@ -1207,7 +1184,7 @@ template <int TG, int TU, int NT>
 __global__ __launch_bounds__(kGuThreads) void gate_up_kernel(maya_moe_args a, Codebooks cb, int wg_rows) {
     extern __shared__ __align__(16) int lds[];
     GroupRef gr;
-    if (!group_of(a, blockIdx.y, gr)) return;
+    if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int k = a.layout.n_embd, n_ff = a.layout.n_ff;
     // the codebooks of the gate and of the up type (one copy when they share it)
     constexpr int cbg = Fmt<TG>::kLdsWords, cbu = Fmt<TG>::kLdsWords == Fmt<TU>::kLdsWords ? 0 : Fmt<TU>::kLdsWords;
@@ -1267,7 +1244,7 @@ template <int TD, int NT>
 __global__ __launch_bounds__(kDnThreads) void down_kernel(maya_moe_args a, Codebooks cb, int wg_rows) {
     extern __shared__ __align__(16) int lds[];
     GroupRef gr;
-    if (!group_of(a, blockIdx.y, gr)) return;
+    if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int k = a.layout.n_ff, n_embd = a.layout.n_embd;
     constexpr int cbw = Fmt<TD>::kLdsWords;
     stage_codebook<TD, kDnThreads>(lds, cb);

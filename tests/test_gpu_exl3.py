@@ -144,6 +144,37 @@ def test_stages_null_slots_and_window_equals_single_token(ex, oracle):
         assert np.array_equal(h1, h_win[t * k:(t + 1) * k])
 
 
+@pytest.mark.parametrize("k2", [(4, 4, 4), (16, 16, 16)])
+def test_stage_calls_take_group_arrays_that_end_with_the_groups(ex, k2):
+    """grp_ptr [groups], grp_start [groups + 1], in front of words that would be other groups: the bits of the whole arrays, on the
+    compile-time walk (gate/up in slices) and on the general one (test_groups_on_the_host.py holds the indices themselves)."""
+    from maya_amd import lib
+    n_embd, n_ff, k, nt, n_expert = 512, 256, 4, 4, 5
+    l, nbytes = ex.make_layout(n_embd, n_ff, k2, 2)
+    store = lib.ExpertStore([ex.synth_blob(l, nbytes, 640 + e) for e in range(n_expert)])
+    rng = np.random.default_rng(640)
+    ids = torch.from_numpy(np.stack([rng.permutation(n_expert)[:k] for _ in range(nt)]).astype(np.int32)).cuda()
+    plan = lib.plan(ids.reshape(-1), store.table)
+    w = torch.from_numpy(rng.uniform(0.1, 1.0, (nt, k)).astype(np.float32)).cuda()
+    x = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda()
+    gp, gs, ge, ng = lib.group(plan)
+    n = int(ng.item())
+    assert n < nt * k
+    ptrs = torch.cat([gp[:n], gp[:1].expand(nt * k - n)]).contiguous()          # the groups end here; then the first expert again,
+    starts = torch.cat([gs[:n + 1], gs[:2].repeat(nt * k)[:nt * k - n]]).contiguous()   # with its entries
+    got = []
+    for groups in ((gp, gs, ge, ng), (ptrs, starts, ge, ng)):
+        h = torch.zeros((nt * k, n_ff), dtype=torch.float32, device="cuda")
+        part = torch.zeros((nt * k, n_embd), dtype=torch.float32, device="cuda")
+        out = torch.zeros((nt, n_embd), dtype=torch.float32, device="cuda")
+        a = ex.make_args(l, nt, k, plan, w, x, h, part, out, groups=groups)
+        ex.gate_up(a)
+        ex.down(a)
+        torch.cuda.synchronize()
+        got.append((h, out))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and float(got[0][1].abs().max()) > 0
+
+
 @pytest.mark.parametrize("n_embd,n_ff,k2,cb,nt", [(640, 384, 6, 2, 4), (2048, 1536, 8, 2, 16), (6144, 1536, 6, 2, 4), (1024, 512, 4, 1, 13)])
 def test_a_layers_window_is_its_tokens(ex, n_embd, n_ff, k2, cb, nt):
     """The layer on a window (several slices a workgroup, two tokens a walk) gives the bits of its tokens one at a time."""
