@@ -11,6 +11,7 @@
 // row), activations are staged through LDS a 256-value super-block at a time, double-buffered.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <math.h>
 #include <stdint.h>
 
@@ -794,6 +795,11 @@ static int prefill_check(const char* what, const maya_moe_layout* l, const uint6
         return fail(MAYA_E_SHAPE, "%s: n_embd %d / n_ff %d: multiples of 256 wanted", what, l->n_embd, l->n_ff);
     // (IQ2_S: the 16-byte copies of a quad's index words want quads of a multiple of 16 bytes: 328 bytes a block)
     if (type_a == kIQ2_S && k % 512) return fail(MAYA_E_SHAPE, "%s: IQ2_S rows of %lld values: a multiple of 512 wanted", what, (long long) k);
+    if (type_a == kIQ2_S) {
+        int rc = prefill_iq2s_lds_ok<true>(what);
+        if (!rc) rc = prefill_iq2s_lds_ok<false>(what);
+        if (rc) return rc;
+    }
     if ((l->gate_off | l->up_off | l->down_off) & 15) return fail(MAYA_E_ARG, "%s: matrix offsets not 16-byte aligned", what);
     // (an entry is a row of the second grid dimension in the quantizers' launches)
     if (n_entries <= 0 || n_entries > 65535 || n_expert <= 0) return fail(MAYA_E_SHAPE, "%s: entries %d (1..65535) experts %d", what, n_entries, n_expert);

@@ -15,6 +15,7 @@
 // output every 32 values, 79 % of the cycles in vector issue.  A 75-token chunk on
 // 160 experts of 6144 x 1536 735 -> 535 us; gate/up IQ2_S with Q4_K down, 1187 tokens on 256 of 7168 x 2048, 2830 -> 2190 us.
 constexpr int kIqMags = 0, kIqSigns = 8192, kIqScales = kIqSigns + 2048, kIqTables = kIqScales + 256;   // byte offsets in LDS
+constexpr int kIqLdsBytes = kIqTables + 3 * kPfBufBytesNoS;
 
 struct IqLook {   // the LDS look-ups of one sub-block: selectors and signs of the lane's two grid entries, its group's digits
     pf_i2 m0, m1, s0, s1;
@@ -209,10 +210,10 @@ __device__ __forceinline__ void pf_tile_iq2s(const PfGemm& a, uint8_t* b0, uint8
 // grid (bands of weight rows, tiles at most)
 template <bool GU>
 __global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebooks cb) {
-    // ONE array, so that it starts at LDS address 0 and the tables' addresses need no base added (five additions a sub-block)
-    __shared__ __attribute__((aligned(256))) uint8_t lds[kIqTables + 3 * kPfBufBytesNoS];
+    // ONE array, so that it starts at LDS address 0 and the tables' addresses need no base added (five additions a sub-block):
+    // prefill_iq2s_lds_ok holds the built kernel against that before a launch
+    __shared__ __attribute__((aligned(256))) uint8_t lds[kIqLdsBytes];
     uint8_t *tables = lds, *b0 = lds + kIqTables, *b1 = b0 + kPfBufBytesNoS, *b2 = b1 + kPfBufBytesNoS;
-    if (pf_lds_addr(lds) != 0) return;   // (never: the kernel has no other LDS)
     const int tile = blockIdx.y;
     if (tile >= *a.plan.n_tiles) return;
     const int tid = threadIdx.x;
@@ -242,4 +243,18 @@ __global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebook
     const int nrows = min(kPfRows, a.plan.bounds[ex + 1] - row0);
     if (nrows <= 32) pf_tile_iq2s<GU, 1>(a, b0, b1, b2, ex, row0, nrows);
     else pf_tile_iq2s<GU, 2>(a, b0, b1, b2, ex, row0, nrows);
+}
+// Refuses a built kernel that has other LDS than its array (a second __shared__ object may be placed in front of it, and the
+// tables would be read from the wrong addresses).  Asked of the runtime once a kernel.
+template <bool GU>
+static int prefill_iq2s_lds_ok(const char* what) {
+    static std::atomic<size_t> bytes{0};
+    if (bytes.load(std::memory_order_relaxed) == 0) {
+        hipFuncAttributes at{};
+        MAYA_HIP(hipFuncGetAttributes(&at, (const void*) prefill_iq2s_kernel<GU>));
+        bytes.store(at.sharedSizeBytes, std::memory_order_relaxed);
+    }
+    const size_t got = bytes.load(std::memory_order_relaxed);
+    if (got != (size_t) kIqLdsBytes) return fail(MAYA_E_UNSUPPORTED, "%s: the IQ2_S kernel was built with %zu bytes of LDS, its array has %d", what, got, kIqLdsBytes);
+    return MAYA_OK;
 }

@@ -1,0 +1,59 @@
+"""What the built library says about its kernels (the gfx950 code objects' own metadata), where a kernel's code counts on it."""
+import os
+import re
+import struct
+
+import pytest
+
+msgpack = pytest.importorskip("msgpack")
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "project-maya_amd", "csrc")
+
+
+def kernels(path):
+    """name -> metadata of every gfx950 kernel in a library's offload bundles."""
+    d, found, at = open(path, "rb").read(), {}, 0
+    while (b := d.find(b"__CLANG_OFFLOAD_BUNDLE__", at)) >= 0:
+        n, = struct.unpack_from("<Q", d, b + 24)
+        at = b + 32
+        for _ in range(n):
+            off, size, name_len = struct.unpack_from("<QQQ", d, at)
+            name = d[at + 24:at + 24 + name_len]
+            at += 24 + name_len
+            if b"gfx950" in name:
+                found.update(code_object_kernels(d[b + off:b + off + size]))
+    return found
+
+
+def code_object_kernels(e):
+    sections, = struct.unpack_from("<Q", e, 40)
+    entry, count = struct.unpack_from("<HH", e, 58)
+    for i in range(count):
+        _, kind, _, _, at, size = struct.unpack_from("<IIQQQQ", e, sections + i * entry)
+        end = at + size
+        while kind == 7 and at < end:   # SHT_NOTE
+            name_size, desc_size, note = struct.unpack_from("<III", e, at)
+            desc = at + 12 + (name_size + 3) // 4 * 4
+            at = desc + (desc_size + 3) // 4 * 4
+            if note == 32:              # NT_AMDGPU_METADATA
+                yield from ((k[".name"], k) for k in msgpack.unpackb(e[desc:desc + desc_size], strict_map_key=False)["amdhsa.kernels"])
+
+
+def constant(text, name, known):
+    return int(eval(re.search(r"\b%s = ([^,;]+)[,;]" % name, text).group(1), {}, known))
+
+
+def test_the_iq2s_prompt_kernels_have_no_lds_but_their_array():
+    """Their tables' look-ups count LDS addresses from 0: a second object there is refused at the first call, and seen here first."""
+    lib = os.path.join(ROOT, "project-maya_amd", "libmaya_moe.so")
+    if not os.path.exists(lib):
+        from maya_amd import build
+        build.build()
+    text = open(os.path.join(CSRC, "maya_prefill.hip")).read() + open(os.path.join(CSRC, "maya_prefill_iq2s.hpp")).read()
+    known = {}
+    for name in ("kPfRows", "kPfPlane", "kPfDOffNoS", "kPfBufBytesNoS", "kIqSigns", "kIqScales", "kIqTables", "kIqLdsBytes"):
+        known[name] = constant(text, name, known)
+    got = {n: k for n, k in kernels(lib).items() if "prefill_iq2s_kernel" in n}
+    assert len(got) == 2
+    for n, k in got.items():
+        assert k[".group_segment_fixed_size"] == known["kIqLdsBytes"], n
