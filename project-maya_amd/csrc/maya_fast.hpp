@@ -310,9 +310,11 @@ struct QuadIQ2S {
 struct QuadOffs {  // byte offsets of the lane's fields inside a quad; quads advance through the scalar offset
     uint32_t is, hs, d;
 };
-// (nu: sub-blocks a row)
-__device__ __forceinline__ QuadOffs quad_offs(uint32_t mat_off, int nu, int u) {
-    return QuadOffs{mat_off + 32u * u, mat_off + 32u * nu + 8u * u, mat_off + 40u * nu + 8u * (u >> 3)};
+// (nu: sub-blocks a row.  A lane past the row's last position, `on` false, asks behind the resource's `past` bytes: its weights,
+// scale among them, read as zero and touch no memory.  It had the last position's, met with a zero scale, and a row whose last
+// block's scale is infinite came out as NaN instead of an infinity: Inf * 0.)
+__device__ __forceinline__ QuadOffs quad_offs(uint32_t mat_off, int nu, int u, bool on, uint32_t past) {
+    return QuadOffs{on ? mat_off + 32u * u : past, on ? mat_off + 32u * nu + 8u * u : past, on ? mat_off + 40u * nu + 8u * (u >> 3) : past};
 }
 // A raw buffer resource over `bytes` of weights at `base`: loads take a per-lane 32-bit offset plus a scalar offset
 // (no vector address arithmetic in the row loop), and a load past `bytes` returns zero instead of faulting.
@@ -393,9 +395,9 @@ __device__ __forceinline__ void quad_values(const QuadIQ2S& q, const uint2* grid
 // ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the sub-block positions of a (gate row, up row) pair; grid
 // (n_ff / ROWS, entries).  DEPTH rows are in flight per lane.
 // Rows of any multiple of 256 values: NW = n_embd / 1024 rounded up, at least 2 (pos_waves), and a lane past the row's last
-// position reads that position's weights again - a line its neighbours ask for anyway - and meets them with zero codes and
-// a zero scale, so the sums are the same lane by lane.  The kernels took whole multiples of 1024 before; rows in
-// between, and down rows of other than 1024, 1536 and 2048 values, went to the general kernels at two to five times the time.
+// position gets weights that read as zero (quad_offs), zero codes and a zero scale, so the sums are the same lane by lane.
+// The kernels took whole multiples of 1024 before; rows in between, and down rows of other than 1024, 1536 and 2048 values,
+// went to the general kernels at two to five times the time.
 // FIT: n_embd = 1024 NW, every lane has a position (known to the compiler, 0.3 to 1 us less a launch).
 template <int NW, int ROWS, int DEPTH, int MINW, bool FIT>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq2s_pos_kernel(maya_moe_args a, Codebooks cb) {
@@ -432,8 +434,9 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq2s_pos_kernel(maya_mo
     const uint32_t qb = (uint32_t) nu * 41u;  // bytes of a quad of rows: 4 x 82 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
     // one resource over the expert's gate and up rows; the up rows ride in the lane offset
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
-    const QuadOffs qo = quad_offs(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
+    const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, gu_bytes);
+    const QuadOffs qo = quad_offs(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u, on, gu_bytes);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     QuadIQ2S ring[DEPTH];
@@ -805,7 +808,7 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
     const int n_ff = a.layout.n_ff;
     const int tiles_per_entry = n_ff >> 3, n_tiles = n_ent * tiles_per_entry;
     const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
-    const QuadOffs qo = quad_offs(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
+    const QuadOffs qo = quad_offs(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u, on, gu_bytes);
     // the resource of a tile's expert (an absent expert: an empty resource, whose loads read as zero and touch nothing);
     // the entry is the same for the whole workgroup: its blob address is a scalar load (HEAD: read from LDS and moved to
     // scalar registers)
@@ -915,7 +918,7 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq2s_pos_kernel(const u
     const uint64_t c_ptr = plan_ptr[ci];
     const float c_w = plan_w[ci];
     const int nu = NU ? NU : n_pos;
-    const bool on = NU == 64 || lane < nu;   // (an idle lane reads the last position's data and uses zeros)
+    const bool on = NU == 64 || lane < nu;   // (an idle lane reads the last position's h and uses zeros; its weights read as zero)
     const int pos = on ? lane : nu - 1;
     const bool rounded = hq_q != nullptr;
     int y[8];
@@ -943,7 +946,7 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq2s_pos_kernel(const u
     const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
     const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (mat_lo | mat_hi) != 0u ? (uint32_t) (n_embd >> 2) * qb : 0u);
-    const QuadOffs qo = quad_offs(0u, nu, pos);
+    const QuadOffs qo = quad_offs(0u, nu, pos, on, (uint32_t) (n_embd >> 2) * qb);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     // the first rows' weights are requested before the tables are stored and h is rounded: one trip to memory for the

@@ -38,8 +38,8 @@ struct QuadIQ1S {
 struct QuadOffs1 {
     uint32_t i4, qh, d;
 };
-__device__ __forceinline__ QuadOffs1 quad_offs1(uint32_t mat_off, int nu, int u) {
-    return QuadOffs1{mat_off + 16u * u, mat_off + 16u * nu + 8u * u, mat_off + 24u * nu + 8u * (u >> 3)};
+__device__ __forceinline__ QuadOffs1 quad_offs1(uint32_t mat_off, int nu, int u, bool on, uint32_t past) {   // (as quad_offs)
+    return QuadOffs1{on ? mat_off + 16u * u : past, on ? mat_off + 16u * nu + 8u * u : past, on ? mat_off + 24u * nu + 8u * (u >> 3) : past};
 }
 __device__ __forceinline__ QuadIQ1S load_quad1(__amdgpu_buffer_rsrc_t rs, const QuadOffs1& o, uint32_t quad_off) {
     QuadIQ1S q;
@@ -120,8 +120,9 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(maya_mo
     const int sy = sum32_codes(y);
     const uint32_t qb = (uint32_t) nu * 25u;  // bytes of a quad of rows: 4 x 50 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
-    const QuadOffs1 qo = quad_offs1(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
+    const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, gu_bytes);
+    const QuadOffs1 qo = quad_offs1(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u, on, gu_bytes);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     QuadIQ1S nxt = load_quad1(rs, qo, quad0);
@@ -179,11 +180,10 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1s_pos_kernel(maya_mo
         const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
         const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
         const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) (n_embd >> 2) * qb);
-        // (an idle lane - past the row's nu positions - reads the last position's weights again and meets them with zero
-        // activations)
+        // (an idle lane - past the row's nu positions - has weights that read as zero and zero activations)
         const bool on = NU == 64 || lane < nu;
         const int pos = on ? lane : nu - 1;
-        const QuadOffs1 qo = quad_offs1(0u, nu, pos);
+        const QuadOffs1 qo = quad_offs1(0u, nu, pos, on, (uint32_t) (n_embd >> 2) * qb);
         const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
         constexpr int NQ = ROWS / 4;
         QuadIQ1S nxt = load_quad1(rs, qo, quad0);
@@ -262,8 +262,8 @@ struct QuadIQ1M {
 struct QuadOffsM {
     uint32_t i4, qh, d;
 };
-__device__ __forceinline__ QuadOffsM quad_offsm(uint32_t mat_off, int nu, int u) {
-    return QuadOffsM{mat_off + 16u * u, mat_off + 16u * nu + 8u * u, mat_off + 24u * nu + 32u * (u >> 3)};
+__device__ __forceinline__ QuadOffsM quad_offsm(uint32_t mat_off, int nu, int u, bool on, uint32_t past) {   // (as quad_offs)
+    return QuadOffsM{on ? mat_off + 16u * u : past, on ? mat_off + 16u * nu + 8u * u : past, on ? mat_off + 24u * nu + 32u * (u >> 3) : past};
 }
 __device__ __forceinline__ QuadIQ1M load_quadm(__amdgpu_buffer_rsrc_t rs, const QuadOffsM& o, uint32_t quad_off) {
     QuadIQ1M q;
@@ -345,8 +345,9 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1m_pos_kernel(maya_mo
     const int sh = 16 + 6 * (u & 7);
     const uint32_t qb = (uint32_t) nu * 28u;  // bytes of a quad of rows: 4 x 56 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
-    const QuadOffsM qo = quad_offsm(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u);
+    const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, gu_bytes);
+    const QuadOffsM qo = quad_offsm(is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, nu, u, on, gu_bytes);
     const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
     constexpr int NQ = ROWS / 4;
     QuadIQ1M nxt = load_quadm(rs, qo, quad0);
@@ -404,11 +405,10 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1m_pos_kernel(maya_mo
         const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
         const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
         const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) (n_embd >> 2) * qb);
-        // (an idle lane - past the row's nu positions - reads the last position's weights again and meets them with zero
-        // activations)
+        // (an idle lane - past the row's nu positions - has weights that read as zero and zero activations)
         const bool on = NU == 64 || lane < nu;
         const int pos = on ? lane : nu - 1;
-        const QuadOffsM qo = quad_offsm(0u, nu, pos);
+        const QuadOffsM qo = quad_offsm(0u, nu, pos, on, (uint32_t) (n_embd >> 2) * qb);
         const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
         constexpr int NQ = ROWS / 4;
         QuadIQ1M nxt = load_quadm(rs, qo, quad0);

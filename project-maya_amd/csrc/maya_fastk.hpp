@@ -17,11 +17,12 @@ struct PosQ4K {
     int sh;                // bit offset of the lane's two sub-blocks' scale bytes in their packed word
     int wsel;              // which packed word (sub-blocks 0-3 or 4-7)
 };
-// position u of a row: block u >> 3, piece u & 7 (sub-block pair j = piece >> 1, half = piece & 1)
-__device__ __forceinline__ void pos_q4k_init(PosQ4K& p, int u, uint32_t mat_off) {
+// position u of a row: block u >> 3, piece u & 7 (sub-block pair j = piece >> 1, half = piece & 1); an idle lane (`on` false)
+// asks behind the resource's `past` bytes, as in quad_offs
+__device__ __forceinline__ void pos_q4k_init(PosQ4K& p, int u, uint32_t mat_off, bool on = true, uint32_t past = 0u) {
     const int b = u >> 3, piece = u & 7, j = piece >> 1;
-    p.o_hdr = mat_off + 144u * b;
-    p.o_q = p.o_hdr + 16u + 16u * piece;
+    p.o_hdr = on ? mat_off + 144u * b : past;
+    p.o_q = on ? mat_off + 144u * b + 16u + 16u * piece : past;
     p.wsel = j >> 1;
     p.sh = 16 * (j & 1);
 }
@@ -83,7 +84,8 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
     const bool on = FIT || lu < nu;
     const int u = on ? lu : nu - 1;
     PosQ4K p;
-    pos_q4k_init(p, u, is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u);
+    const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
+    pos_q4k_init(p, u, is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u, on, gu_bytes);
     int e;
     uint64_t blob;
     if constexpr (HEAD) {
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
     }
     const uint32_t rb = (uint32_t) nu * 18u;   // bytes of a row: 144 a block
     const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(blob + a.layout.gate_off, gu_bytes);
     u32x4 hn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, (uint32_t) r0 * rb, 0);
     u32x4 qn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_q, (uint32_t) r0 * rb, 0);
     u32x4 ha[AHEAD ? ROWS : 1], qa[AHEAD ? ROWS : 1];
@@ -175,13 +177,13 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(maya_moe
     const int e0 = by * a.k, ent = e0 + wave;
     const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
     if (blob != 0ull) {
-        // (an idle lane reads the last position's weights again and meets them with zero activations)
+        // (an idle lane's weights read as zero, and so do its activations)
         const bool on = NU == 64 || lane < nu;
         const int pos = on ? lane : nu - 1;
         PosQ4K p;
-        pos_q4k_init(p, pos, 0u);
-        // the first row's weights are requested before h is rounded: their latency hides behind that arithmetic
         const uint32_t rb = (uint32_t) nu * 18u;   // bytes of a row: 144 a block
+        pos_q4k_init(p, pos, 0u, on, (uint32_t) n_embd * rb);
+        // the first row's weights are requested before h is rounded: their latency hides behind that arithmetic
         const uint64_t mat = blob + a.layout.down_off;
         const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
         const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));

@@ -61,9 +61,10 @@ __global__ __launch_bounds__(64 * NW) void gate_up_q80_pos_kernel(maya_moe_args 
     const int u = on ? lu : nu - 1;
     const int k = 32 * nu, n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
     const uint32_t rb = (uint32_t) nu * 34u;   // bytes of a row
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(gr.blob + a.layout.gate_off, (uint32_t) (a.layout.down_off - a.layout.gate_off));
+    const uint32_t gu_bytes = (uint32_t) (a.layout.down_off - a.layout.gate_off);
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(gr.blob + a.layout.gate_off, gu_bytes);
     const uint32_t mat = is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u;
-    const uint32_t oq = mat + 32u * u, od = mat + 32u * nu + 2u * u;
+    const uint32_t oq = mat + 32u * u, od = on ? mat + 32u * nu + 2u * u : gu_bytes;   // (an idle lane's scale: as in quad_offs)
     int step = 0;
     for (int c0 = 0; c0 < gr.ne; c0 += NT) {
         int ents[NT], y[NT][8];
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(512) void down_q80_pos_kernel(maya_moe_args a, int 
     GroupRef gr;
     if (!group_of<false>(a, blockIdx.y, gr)) return;
     const int wave = threadIdx.x >> 6, lane0 = threadIdx.x & 63;
-    // (an idle lane reads the last position's weights again and meets them with zero activations)
+    // (an idle lane reads the last position's codes again and meets them with zero activations; its scale reads as zero)
     const int nu = NU ? NU : a.layout.n_ff >> 5;
     const bool on = NU == 64 || lane0 < nu;
     const int lane = on ? lane0 : nu - 1;
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(512) void down_q80_pos_kernel(maya_moe_args a, int 
     const uint32_t rb = (uint32_t) nu * 34u;
     const uint64_t mat = gr.blob + a.layout.down_off;
     const __amdgpu_buffer_rsrc_t rs = weight_rsrc(mat, (uint32_t) n_embd * rb);
-    const uint32_t oq = 32u * lane, od = 32u * nu + 2u * lane;
+    const uint32_t oq = 32u * lane, od = on ? 32u * nu + 2u * lane : (uint32_t) n_embd * rb;
     for (int c0 = 0; c0 < gr.ne; c0 += NT) {
         int ents[NT], y[NT][8];
         float dx[NT];

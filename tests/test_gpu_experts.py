@@ -229,6 +229,57 @@ def test_two_byte_aligned_blobs_clamp_and_add(lib, oracle):
     assert rel_l2(out, wout + add) <= TOL
 
 
+def one_sign_rows(t, n_rows, k, rng, d=None):
+    """Rows of equal positive values: the format's smallest sub-scales, one code, block scales of a usual size or d."""
+    nb = n_rows * (k // synth.BLOCK_VALUES[t])
+    b = np.zeros((nb, synth.BLOCK_BYTES[t]), dtype=np.uint8)
+    bits = (rng.uniform(2e-4, 4e-4, nb) if d is None else np.full(nb, d)).astype(np.float16).view(np.uint16)
+    if t == synth.IQ1_M:   # the grid's last entry, +1 eight times
+        b[:, 0:32], b[:, 32:48] = 0xff, 0x77
+        for i in range(4):
+            b[:, 49 + 2 * i] = ((bits >> (4 * i)) & 15) << 4
+        return b
+    b[:, 0:2] = bits.view(np.uint8).reshape(nb, 2)
+    if t == synth.Q8_0:
+        b[:, 2:] = 64
+    elif t == synth.Q4_K:
+        b[:, 4:8], b[:, 12:16], b[:, 16:] = 1, 1, 0xff
+    elif t == synth.IQ1_S:
+        b[:, 2:34], b[:, 34::2], b[:, 35::2] = 0xff, 0xff, 0x0f
+    return b
+
+
+@pytest.mark.parametrize("where", ("up", "down"))
+@pytest.mark.parametrize("nt", (1, 3))
+@pytest.mark.parametrize("t", (8, 12, 22, 19, 29))
+def test_an_infinite_scale_in_a_rows_last_block(lib, oracle, t, nt, where):
+    """Rows that end inside a wave, every third with an infinite scale in its last block, all products positive: an up row gives
+    +limit, a down row +Inf, in either packing - no lane past the row's end may make a NaN of it (which clamps to -limit)."""
+    n_embd, n_ff, ne, k = 1280, 768, 4, 2
+    limit = 1.0 if where == "up" else float("inf")
+    rng = np.random.default_rng(t + nt)
+    blobs = []
+    for _ in range(ne):
+        mats = []
+        for role, rows, n in (("gate", n_ff, n_embd), ("up", n_ff, n_embd), ("down", n_embd, n_ff)):
+            m = one_sign_rows(t, rows, n, rng).reshape(rows, -1)
+            if role == where:
+                m[::3, -synth.BLOCK_BYTES[t]:] = one_sign_rows(t, 1, synth.BLOCK_VALUES[t], rng, np.inf)
+            mats.append(m.reshape(-1))
+        blobs.append(np.concatenate(mats))
+    logits = rng.standard_normal((nt, ne)).astype(np.float32)
+    x = rng.uniform(0.5, 1.5, (nt, n_embd)).astype(np.float32)
+    with np.errstate(all="ignore"):
+        wi, ww, want = oracle_layer(oracle, t, t, blobs, k, n_embd, n_ff, logits, x, limit=limit)
+    assert not np.isnan(want).any() and np.isinf(want).any() == (where == "down")
+    for packing in (0, 1):
+        ids, w, out, _ = run_layer(lib, t, t, blobs, k, n_embd, n_ff, logits, x, limit=limit, packing=packing)
+        assert np.array_equal(ids, wi)
+        assert np.array_equal(np.isinf(out), np.isinf(want)) and np.array_equal(np.sign(out), np.sign(want)), packing
+        finite = np.isfinite(want)
+        assert rel_l2(out[finite], want[finite]) <= TOL, packing
+
+
 def test_null_plan_slots_are_left_out(lib, oracle):
     gt, dt, n_embd, n_ff, ne, k, nt = 22, 22, 512, 256, 8, 4, 3
     blobs = make_experts(gt, dt, n_embd, n_ff, ne, 55)
