@@ -266,9 +266,13 @@ def test_sigmoid_router_in_the_gate_up_launch(lib, norm, with_bias):
 
 
 @pytest.mark.parametrize("ty,n_embd,n_ff,ne,k", ((12, 2048, 512, 40, 8), (12, 2048, 2048, 12, 8), (12, 3072, 512, 9, 4), (12, 7168, 256, 6, 1),
-                                                   (19, 2048, 512, 40, 8), (19, 3072, 256, 9, 4), (19, 5120, 256, 7, 2)))
+                                                   (19, 2048, 512, 40, 8), (19, 3072, 256, 9, 4), (19, 5120, 256, 7, 2),
+                                                   (12, 768, 256, 40, 8), (12, 1792, 1280, 20, 12), (12, 7936, 256, 6, 1),
+                                                   (19, 768, 512, 9, 4), (19, 2816, 768, 24, 11), (22, 1280, 768, 40, 8),
+                                                   (22, 3328, 256, 24, 10), (22, 7936, 1792, 5, 2)))
 def test_other_types_head_in_the_gate_up_launch(lib, oracle, ty, n_embd, n_ff, ne, k):
-    """The same for Q4_K and IQ1_S experts (their position-mapped gate/up kernels with the head in them): for Q4_K
+    """The same for Q4_K and IQ1_S experts (their position-mapped gate/up kernels with the head in them), and for all three
+    on rows that are no whole multiple of 1024 (lanes past the row's end) and with more than 8 slots: for Q4_K
     the 8-row launch of few entries and the 16-row one; row lengths whose middle wave holds gate and up lanes (3072,
     5120); one slot (k = 1); F32, BF16 and F16 x; edge logits; the sigmoid router.  ids, weights and output bit for bit
     those of the three-launch layer, and the CPU path's within 1e-3."""

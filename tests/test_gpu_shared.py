@@ -61,6 +61,8 @@ def two_calls(w, logits, x, add, limit):
     (IQ2_S, Q4_K, Q8_0, 7168, 2048, 32, 8, 8),    # configs[2]'s types and shape (fewer experts resident)
     (IQ2_S, IQ2_S, Q8_0, 7168, 2048, 16, 8, 1),   # one token: the down kernel that rounds h itself waits for the join
     (Q4_K, Q4_K, Q4_K, 4096, 1024, 8, 2, 3),
+    (IQ2_S, Q4_K, Q8_0, 2816, 1280, 16, 4, 3),    # rows that end inside a wave
+    (Q4_K, Q4_K, IQ2_S, 1792, 768, 12, 10, 2),    # and more than 8 slots
 ])
 def test_layer_with_shared_expert_is_the_two_calls(lib, gt, dt, st, E, FF, NE, TK, T):
     w = build(lib, gt, dt, st, E, FF, NE, TK, T, 500 + T)
