@@ -103,8 +103,7 @@ __device__ __forceinline__ void had128_wave(float& v0, float& v1, int lane) {
     v1 = __fmul_rn(v1, s);
 }
 
-// xr = FP16(H(x * suh)) of one activation into LDS; every wave of the workgroup takes blocks of 128 values (`tmp` is not
-// used: the transform runs in registers)
+// xr = FP16(H(x * suh)) of one activation into LDS; every wave of the workgroup takes blocks of 128 values, transformed in registers
 // PAIRED (the compile-time walk): inside every 16 rows the word of rows 2q, 2q + 1 and the word of rows 2q + 8, 2q + 9 -
 // a lane's four rows - sit side by side (words 2q, 2q + 1), so the walk reads them in one 8-byte LDS read
 __device__ __forceinline__ int paired_pos(int i) {
@@ -112,9 +111,7 @@ __device__ __forceinline__ int paired_pos(int i) {
     return (i & ~15) | ((w < 4 ? 2 * w : 2 * (w - 4) + 1) << 1) | (i & 1);
 }
 template <bool PAIRED>
-__device__ __forceinline__ void rotate_in(const float* __restrict__ x, const uint16_t* __restrict__ suh, int k, float* tmp,
-                                          __half* xr) {
-    (void) tmp;
+__device__ __forceinline__ void rotate_in(const float* __restrict__ x, const uint16_t* __restrict__ suh, int k, __half* xr) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int nb = k >> 7;
     // a wave's blocks three at a time: their loads go out together (one block a pass of the loop is one trip to memory a
@@ -371,7 +368,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_gate_up_kernel(maya_exl3_args
         for (int t = 0; t < NTC; ++t) {
             const float* x = a.x + (size_t) (ents[t] / a.k) * xs;
             for (int role = 0; role < 2; ++role)
-                rotate_in<(K2 > 0)>(x, (const uint16_t*) (blob + a.layout.suh[role]), k, tmp, xr + ((size_t) t * 2 + role) * k);
+                rotate_in<(K2 > 0)>(x, (const uint16_t*) (blob + a.layout.suh[role]), k, xr + ((size_t) t * 2 + role) * k);
         }
         float raw[2][NTC];
 #pragma unroll
@@ -612,7 +609,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_slices_kernel(maya_exl3_args 
             const int64_t xs = a.x_stride ? a.x_stride : k;
             const uint16_t* suh = (const uint16_t*) (blob + a.layout.suh[role]) + (size_t) b0 * 128;
             for (int t = 0; t < NTC; ++t)
-                rotate_in<true>(a.x + (size_t) (ents[t] / a.k) * xs + (size_t) b0 * 128, suh, kb, tmp, xr + (size_t) t * kb);
+                rotate_in<true>(a.x + (size_t) (ents[t] / a.k) * xs + (size_t) b0 * 128, suh, kb, xr + (size_t) t * kb);
         }
         float acc[NTC];
 #pragma unroll
@@ -699,7 +696,7 @@ __global__ __launch_bounds__(kExThreads) void exl3_down_kernel(maya_exl3_args a)
         for (int t = 0; t < NTC; ++t) ents[t] = entry_of(a, gr, c0 + t);
         __syncthreads();
         for (int t = 0; t < NTC; ++t)
-            rotate_in<(K2 > 0)>(a.h + (size_t) ents[t] * k, (const uint16_t*) (blob + a.layout.suh[2]), k, tmp, xr + (size_t) t * k);
+            rotate_in<(K2 > 0)>(a.h + (size_t) ents[t] * k, (const uint16_t*) (blob + a.layout.suh[2]), k, xr + (size_t) t * k);
         float acc[NTC];
 #pragma unroll
         for (int t = 0; t < NTC; ++t) acc[t] = 0.0f;
@@ -800,8 +797,9 @@ int launch_exl3_gate_up(const maya_exl3_args& a, const DeviceState& st, hipStrea
     MAYA_LAUNCHED("exl3_gate_up_kernel");
     return MAYA_OK;
 }
-// Slices a workgroup walks: as many as leave the call three workgroups a compute unit (what its registers and LDS let a compute
-// unit hold at once), at least one.
+// Slices a workgroup walks: as many as leave the call three workgroups a compute unit, at least one.  Three is what the registers of
+// the two-token kernels (70) let a compute unit hold at once; one token's hold four (58) or three (70, the down launch that makes h),
+// the four-token ones two (96 to 100): a call of theirs that is cut for three runs its last third as a second round.
 static int slices_per_wg(long long wgs, int S, const DeviceState& st) {
     int sp = S;
     while (sp > 1 && (S % sp != 0 || wgs * (S / sp) < 3ll * st.n_cu)) --sp;

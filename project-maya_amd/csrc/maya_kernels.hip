@@ -1443,6 +1443,10 @@ int launch_down_t(const maya_moe_args& a, const DeviceState& st, hipStream_t s) 
 // between whole multiples of 1024 (n_ff: outside 1024, 1536, 2048), and more than 8 slots, went to the general kernels before:
 // Q4_K 2048 x 768 top-8, one token, 25.2 us a layer, 16.6 like this; IQ2_S 2816 x 768 29.7 -> 15.7; Q4_K 6912 x 1280 top-10, five
 // tokens, 733 -> 143; IQ2_S gate/up with Q4_K down 4864 x 1280, eight tokens, 430 -> 89; Q8_0 2560 x 1280, six tokens, 148 -> 81.
+// The general kernels share a decode among an expert's tokens, these (but for Q8_0) decode for every entry, so the lead narrows with
+// the entries an expert, without turning over: 16 tokens on one expert of 2816 x 1280, Q4_K 158 -> 29, IQ2_S 111 -> 45; top-10 of 16
+// experts 498 -> 125 and 337 -> 172; all of 16 experts, IQ2_S 4096 x 2048, 451 -> 406; the least, IQ2_XXS gate/up (general) with
+// IQ2_S down 2816 x 1280, all of 10 experts, 251 and 253.
 static bool pos_row_ok(int n_embd) { return n_embd % 256 == 0 && n_embd >= 256 && n_embd <= 8192; }
 static int pos_waves(int n_embd) { return n_embd <= 2048 ? 2 : (n_embd + 1023) / 1024; }
 static bool down_pos_nff_ok(int n_ff) { return n_ff % 256 == 0 && n_ff >= 256 && n_ff <= 2048; }
@@ -1460,8 +1464,10 @@ int launch_gate_up_iq2s_gguf(const maya_moe_args& a, const DeviceState& st, hipS
     MAYA_LAUNCHED("gate_up_iq2s_1tok_kernel");
     return MAYA_OK;
 }
-// the position-mapped kernels: gate/up 16 rows a workgroup at the 6 waves a SIMD its registers allow; down 16 rows at 7
-// waves a SIMD (8 spill), or n_embd / 256 rows for the wide rows
+// the position-mapped kernels: gate/up 16 rows a workgroup, compiled for 8 waves a SIMD (62 registers; 65, seven waves, with NW = 7);
+// down 16 rows for 7 (70 to 72 registers; held to 64 they spill 32 to 52 bytes a lane and 4096 x 2048, four tokens, takes 75 us
+// instead of 56), or n_embd / 256 rows for the wide rows.  n_ff = 1024 and 1536 known to the compiler as 2048 is made no
+// difference: 4096 x 1024, four tokens, 41.4 and 41.5 us, 5120 x 1536 59.3 and 58.5.
 template <int NW>
 int launch_gate_up_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
     constexpr int kRows = 16;
@@ -1626,6 +1632,9 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     // (IQ1_S with the head in the launch: one more column, whose first workgroup is the router)
     const dim3 grid((unsigned) (a.layout.n_ff / 16) + (hd ? 1u : 0u), (unsigned) (a.n_tokens * a.k));
     if (a.layout.gate_type == kIQ1_M) {
+        // Compiled for 8 waves a SIMD where rows fill their lanes, 7 where they do not.  At 8 some of either spill two registers; at
+        // 64 experts top-8 the former lose nothing by it (7168 x 2048, 16 tokens, 315 us against 320 at 7; 4096 x 2048, four tokens,
+        // 56.6 against 55.4), the latter do (3840 x 2048, four and 16 tokens, 54.7 and 176 us at 7, 55.7 and 182 at 8).
         if (hd) return fail(MAYA_E_UNSUPPORTED, "gate_up: the IQ1_M rows take no head in their launch");
 #define MAYA_IQ1M(NWV)                                                                                                                         \
     if (a.layout.n_embd == 1024 * NWV) hipLaunchKernelGGL((gate_up_iq1m_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, a, st.cb);   \
@@ -1664,7 +1673,8 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     return MAYA_OK;
 }
 int launch_down_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
-    // 32 rows a workgroup for the wide rows (half as many waves rounding h, as in the IQ2_S kernel), else 16
+    // 32 rows a workgroup for the wide rows (half as many waves rounding h, as in the IQ2_S kernel), else 16.
+    // (7 waves a SIMD leave the 53 and 64 registers the kernels take; of 16 slots one workgroup is 4 waves a SIMD already)
     const bool wide = a.layout.n_embd >= 5120 && a.layout.n_embd % 32 == 0;
     const dim3 grid((unsigned) (a.layout.n_embd / (wide ? 32 : 16)), (unsigned) a.n_tokens);
 #define MAYA_D1T(KERN, R)                                                                                                     \

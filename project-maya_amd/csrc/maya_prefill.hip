@@ -1,14 +1,13 @@
 // maya_prefill.hip - a prompt chunk's routed experts on gfx950: the device-side plan (count, scan, stable scatter, tile
-// list), the per-32 int8 activation quantizer over the plan's rows, and the grouped GEMM of Q4_K weights with those
-// activations on the int8 matrix cores.
+// list), the Q8_K activation quantizers over the plan's rows, and the grouped GEMM of Q4_K weights with those
+// activations on the int8 matrix cores (IQ2_S weights: maya_prefill_iq2s.hpp).
 //
-// The GEMM: a workgroup takes one tile (up to 64 rows of one expert) and a band of weight rows; its 4 waves take 4
-// tiles of 16 weight rows each (gate/up: 2 tiles of gate rows and the same features' 2 tiles of up rows, so the SwiGLU
-// and the requantization of H per 32 features stay inside the wave).  Per 32 values of the inner dimension one
-// v_mfma_i32_16x16x32_i8 gives the exact integer dots of 16 tokens' codes with 16 weight rows' 4-bit codes; the F32
-// scales (d * sc of the weight sub-block, the activation block's d) and the minimum's term (dmin * m times the
-// activation block's s) are applied per output.  Weights stream from HBM straight into registers (each lane reads its own
-// row), activations are staged through LDS a 256-value super-block at a time, double-buffered.
+// The GEMM: a workgroup takes one tile (up to 64 rows of one expert) and a band of weight rows; each of its 4 waves takes 32
+// weight rows (gate/up: the gate rows of 16 features and their up rows, so the SwiGLU stays inside the wave).  A Q4_K weight is
+// two int8 planes (its code times the low and the high 3 bits of its sub-block's scale), and v_mfma_i32_32x32x32_i8 sums a whole
+// 256-value super-block of either exactly; the two F32 scales and the minimums' term are applied once an output a super-block.
+// Weights stream from HBM straight into registers one super-block ahead (each lane reads its own row), activations go to LDS
+// without registers two super-blocks ahead, through three buffers.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -362,7 +361,7 @@ __device__ __forceinline__ uint32_t pf_scale_codes(uint32_t w, uint32_t f) {
 
 // LDS reads of the GEMM loop are written out by hand.  The compiler cannot tell which LDS buffer a direct-to-LDS copy
 // fills, so before any LDS read of its own it waits for every copy in flight - here that would be the copy of the
-// super-block two ahead, issued moments earlier.  These reads it does not see; each group is followed by pf_lds_wait
+// super-block two ahead, issued moments earlier.  These reads it does not see; each group is followed by a wait
 // on the registers it filled (the values pass through the wait, so nothing that uses them can move above it).
 __device__ __forceinline__ uint32_t pf_lds_addr(const void* p) {
     return (uint32_t) (uintptr_t) (const __attribute__((address_space(3))) void*) p;
@@ -371,16 +370,6 @@ typedef int pf_i2 __attribute__((ext_vector_type(2)));
 template <int OFF> __device__ __forceinline__ pf_i2 pf_lds_b64(uint32_t addr) {
     pf_i2 v;
     asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
-    return v;
-}
-template <int OFF> __device__ __forceinline__ uint32_t pf_lds_u16(uint32_t addr) {
-    uint32_t v;
-    asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
-    return v;
-}
-template <int OFF> __device__ __forceinline__ float pf_lds_f32(uint32_t addr) {
-    float v;
-    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
     return v;
 }
 template <int OFF> __device__ __forceinline__ v4f pf_lds_f32x4(uint32_t addr) {
@@ -392,17 +381,6 @@ template <int OFF> __device__ __forceinline__ v4i pf_lds_i32x4(uint32_t addr) {
     v4i v;
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
     return v;
-}
-template <int N, typename T> __device__ __forceinline__ void pf_lds_wait(T (&r)[N]) {
-    if constexpr (N == 1) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]));
-    else if constexpr (N == 2) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]));
-    else if constexpr (N == 3) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]));
-    else if constexpr (N == 4) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
-    else if constexpr (N == 6) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]));
-    else {
-        static_assert(N == 8, "1, 2, 3, 4, 6 or 8 registers");
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7]));
-    }
 }
 // the registers r have landed once at most BUT later LDS reads are outstanding (LDS operations complete in order)
 template <int BUT, int N> __device__ __forceinline__ void pf_lds_wait_but(v4i (&r)[N]) {
@@ -793,7 +771,8 @@ static int prefill_check(const char* what, const maya_moe_layout* l, const uint6
         return fail(MAYA_E_UNSUPPORTED, "%s: IQ2_S rows are taken in the stream packing (maya_moe_repack)", what);
     if (l->n_embd <= 0 || l->n_ff <= 0 || l->n_embd % 256 || l->n_ff % 256)
         return fail(MAYA_E_SHAPE, "%s: n_embd %d / n_ff %d: multiples of 256 wanted", what, l->n_embd, l->n_ff);
-    // (IQ2_S: the 16-byte copies of a quad's index words want quads of a multiple of 16 bytes: 328 bytes a block)
+    // (IQ2_S: refused since the kernel's first form, whose 16-byte copies wanted quads - 328 bytes a block - of a multiple of 16 bytes.
+    // The present one reads 8 bytes at a time; a last block of its own has not been tried on it.)
     if (type_a == kIQ2_S && k % 512) return fail(MAYA_E_SHAPE, "%s: IQ2_S rows of %lld values: a multiple of 512 wanted", what, (long long) k);
     if (type_a == kIQ2_S) {
         int rc = prefill_iq2s_lds_ok<true>(what);
