@@ -122,8 +122,8 @@ def event_time(fn, reps, stream, rounds=ROUNDS):
 # HBM bytes a step (a launch of the named kernel for the prefill chunks) read from rocprofv3's FETCH_SIZE and WRITE_SIZE
 # counters, scaled by a plain copy of known size (profiles/other_configs_hbm_traffic_pmc.txt); they belong to the
 # synthetic inputs these workloads make (fixed seeds), so they are constants here
-TRAFFIC_BYTES = {"single_q4k": 25286343, "batch8_mixed": 1097088000, "exl3_verify": 336937077,
-                 "prefill_q4k": 2122985062, "prefill_iq2s": 1253165670, "prefill_mixed": 1253165670}
+TRAFFIC_BYTES = {"single_q4k": 25455616, "batch8_mixed": 1097086054, "exl3_verify": 339187098,
+                 "prefill_q4k": 2032205107, "prefill_iq2s": 1224389018, "prefill_mixed": 1224389018}
 
 
 def hbm_roofline(kernel, bytes_launch, seconds, traffic=None):
@@ -412,7 +412,7 @@ def exl3_verify(K, W, k2=6):
                                    ": EXL3 %g-bit trellis experts (k2 %d, mul1), 160 experts top-8, hidden 6144, " % (k2 / 2, k2) +
                                    "intermediate 1536, 4-token verify window; 8 logit sets rotate",
                        "distinct_experts_per_step": d_avg, "algorithmic_bytes_per_step": int(nbytes)},
-            "roofline": hbm_roofline("layer (exl3_gu_split_kernel + exl3_swiglu_kernel + exl3_down_kernel + exl3_combine_kernel)", nbytes, sec,
+            "roofline": hbm_roofline("layer (window_head_kernel + exl3_slices_kernel gate/up + exl3_swiglu_kernel + exl3_slices_kernel down)", nbytes, sec,
                                      TRAFFIC_BYTES["exl3_verify"] if k2 == 6 else None)}
 
 
