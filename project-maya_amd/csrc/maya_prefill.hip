@@ -2,12 +2,11 @@
 // list), the Q8_K activation quantizers over the plan's rows, and the grouped GEMM of Q4_K weights with those
 // activations on the int8 matrix cores (IQ2_S weights: maya_prefill_iq2s.hpp).
 //
-// The GEMM: a workgroup takes one tile (up to 64 rows of one expert) and a band of weight rows; each of its 4 waves takes 32
-// weight rows (gate/up: the gate rows of 16 features and their up rows, so the SwiGLU stays inside the wave).  A Q4_K weight is
-// two int8 planes (its code times the low and the high 3 bits of its sub-block's scale), and v_mfma_i32_32x32x32_i8 sums a whole
-// 256-value super-block of either exactly; the two F32 scales and the minimums' term are applied once an output a super-block.
-// Weights stream from HBM straight into registers one super-block ahead (each lane reads its own row), activations go to LDS
-// without registers two super-blocks ahead, through three buffers.
+// The GEMM: a workgroup takes up to 128 rows of one expert (two tiles of the plan) and a band of weight rows; each of its 4 waves
+// takes 32 weight rows (gate/up: the gate rows of 16 features and their up rows, so the SwiGLU stays inside the wave).  A Q4_K
+// weight is two int8 planes (its code times the low and the high 3 bits of its sub-block's scale), and v_mfma_i32_32x32x32_i8 sums
+// a whole 256-value super-block of either exactly; the two F32 scales and the minimums' term are applied once an output a
+// super-block.  Weights and activations go from HBM to LDS without registers, two super-blocks and three row groups ahead.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -293,48 +292,9 @@ struct PfGemm {
     float limit;
 };
 
-// LDS of one buffer: the codes [kPfRows][256] (16-byte chunk c of row r at position c ^ (r & 15): the 16 rows x 4
-// k-groups of a matrix-core operand read then hit distinct banks), s [kPfRows][8], d [kPfRows]
-constexpr int kPfPlane = kPfRows * 256;
-constexpr int kPfSOff = kPfPlane, kPfDOff = kPfSOff + kPfRows * 32;
-constexpr int kPfBufBytes = kPfDOff + kPfRows * 4;
-constexpr int kPfDOffNoS = kPfPlane, kPfBufBytesNoS = kPfDOffNoS + kPfRows * 4;   // (a buffer without s: types without minimums)
-
+// The codes of a group of rows in LDS: 256 bytes a row, 16-byte chunk c of row r at position c ^ (r & 15): the 16 rows x 4
+// k-groups of a matrix-core operand read then hit distinct banks.
 typedef __attribute__((address_space(3))) void* pf_lptr;
-// The tile's activations go from global memory to LDS without passing registers (each lane's 16 bytes land at the
-// wave's base + 16 lane): buffer loads whose per-lane offsets are fixed for the tile - the super-block rides in the
-// scalar offset - so a copy costs no vector arithmetic.  Rows past the tile's end repeat its last row (their results
-// are never stored).
-template <int NMT, bool WITH_S = true>
-struct PfDma {
-    __amdgpu_buffer_rsrc_t rq, rs, rd;
-    uint32_t oq[NMT], os, od;
-    int wave;
-    __device__ __forceinline__ void init(const PfGemm& a, int row0, int nrows, int wave_, int lane) {
-        wave = wave_;
-        const int last = nrows - 1;
-        rq = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.q + (size_t) row0 * a.k), 0, (int) (nrows * a.k), 0x00020000);
-        rs = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.s + (size_t) row0 * (a.k >> 4)), 0, (int) (nrows * (a.k >> 5) * 4), 0x00020000);
-        rd = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.d + (size_t) row0 * (a.k >> 8)), 0, (int) (nrows * (a.k >> 8) * 4), 0x00020000);
-#pragma unroll
-        for (int n = 0; n < NMT; ++n) {
-            const int r = 4 * (wave + 4 * n) + (lane >> 4), cp = lane & 15;   // rows 4 i .. 4 i + 3, i = wave + 4 n
-            oq[n] = (uint32_t) (min(r, last) * (int) a.k + ((cp ^ (r & 15)) * 16));
-        }
-        os = (uint32_t) (min(32 * wave + (lane >> 1), last) * (int) (a.k >> 5) * 4 + (lane & 1) * 16);
-        od = (uint32_t) (min(lane, last) * (int) (a.k >> 8) * 4);
-    }
-    // super-block sb into the buffer at `buf`
-    __device__ __forceinline__ void copy(uint8_t* buf, int sb) const {
-#pragma unroll
-        for (int n = 0; n < NMT; ++n)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (pf_lptr) (buf + (wave + 4 * n) * 1024), 16, oq[n], sb * 256, 0, 0);
-        if (WITH_S && wave < 2 && 32 * wave < 16 * NMT)   // s: 32 rows an instruction, 32 bytes a row
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (pf_lptr) (buf + kPfSOff + wave * 1024), 16, os, sb * 32, 0, 0);
-        if (wave == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (pf_lptr) (buf + (WITH_S ? kPfDOff : kPfDOffNoS)), 4, od, sb * 4, 0, 0);
-    }
-};
-
 // the 8 six-bit scales and 8 six-bit minimums of a Q4_K block's 12 bytes, as bytes of two words each
 // (get_scale_min_k4, include/strata/artifact/dequant.hpp:162-172)
 __device__ __forceinline__ void q4k_unpack_scales(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t (&sc)[2], uint32_t (&mn)[2]) {
@@ -404,34 +364,123 @@ typedef float pf_v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 pf_v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 
-// One tile of NM x 32 rows against the wave's 32 weight rows (gate/up: the gate rows of 16 features, then their up rows;
+// A tile of up to 4 x 32 rows against the wave's 32 weight rows (gate/up: the gate rows of 16 features, then their up rows;
 // down: 32 output rows), on the 32x32 matrix instructions: lane (ln = lane & 31, kh = lane >> 5) holds 16 of a
 // sub-block's 32 values of activation row ln (A operand, from LDS) and of weight row ln (B operand, decoded in
-// registers), and 16 outputs: weight row ln against the rows 8 b + 4 kh + r (b, r = 0..3) of the 32.  These
-// instructions take 32 cycles, and the vector ALU issues about four instructions under each of them; the 16-cycle
-// 16x16 forms leave it no slot (measured with a microbenchmark of matrix instructions followed by vector instructions), which is what bounds a
-// kernel that has as many vector instructions as this one.
-template <bool GU, int NM>
-__device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* b0, uint8_t* b1, uint8_t* b2, int ex, int row0, int nrows) {
-    // (global address space: a generic pointer's loads would count as LDS operations too, and every wait for them
-    // would also wait for the copies into LDS behind them)
-    typedef const __attribute__((address_space(1))) uint8_t* wptr;
-    constexpr int NMT = 2 * NM;   // groups of 16 rows: what the copies into LDS count in
-    wptr blob = (wptr) a.table[ex];
+// registers), and 16 outputs: weight row ln against the rows 8 b + 4 kh + r (b, r = 0..3) of the 32.  The 32-cycle
+// instructions leave the vector ALU about six slots each; the 16-cycle 16x16 forms leave it none.
+//
+// The work goes by passes: a pass is one group of 32 rows against one super-block.  A super-block's weights are decoded in its
+// first pass and stay in 64 registers for the others, so a tile of 128 rows pays a quarter of the decode a row group:
+// 12 vector instructions a matrix instruction at 64 rows with a decode each, 7 now.
+//
+// Weights and activations both go to LDS without registers, and a lane reads its pieces from there.  A lane that loads its
+// own weight row from memory makes each lane of the instruction a cache access of its own: 64 clocks a compute unit for
+// 1 KB out of L2, five such loads a wave a super-block, and the data path of the cache busy 85 % of the kernel.  A copy takes a
+// row's 144 bytes by nine lanes in a run (19 clocks).  A row in LDS is 36 banks on from the one before, so the 16-byte reads of
+// 16 rows meet every bank once.
+//
+// Tiles of up to 24 rows (NB blocks of 8) take the codes themselves to the matrix cores, one instruction a sub-block instead of
+// two planes': the sub-block sums of their few rows times the scales cost less on the vector ALU (4 multiply-adds a lane for 8
+// rows) than the planes' 64 multiplies and 8 matrix instructions, up to 24 rows; at 32 the two forms take the same.
+//
+// Measured, one box: 4096 tokens top-8 of 288 experts of 4096 x 2048, gate/up 1817 -> 1420 us, down 891 -> 745; 512 tokens
+// top-8 of 256 experts of 7168 x 2048 under a skewed routing (70 of its 93 experts with 24 rows or fewer), 627 -> 520 and 336 ->
+// 291.  What bounds it: on full tiles vector issue (59 % of the cycles) and matrix time (50 %), at the 1.75 GHz that this
+// load leaves of 2.4; few rows an expert stream their weights at 3.2 TB/s, of 5.2 without arithmetic.
+constexpr int kPfGroups = 4;                         // row groups of a workgroup at most: two of the plan's tiles
+constexpr int kPfRing = 4;                           // activations of a pass in LDS, three passes ahead
+constexpr int kPfSlotS = 8192, kPfSlotD = kPfSlotS + 1024, kPfSlot = kPfSlotD + 256;   // codes [32][256], sums [32][16], scales [32]
+constexpr int kPfWave = 32 * 144, kPfWStep = 4 * kPfWave, kPfWAt = kPfRing * kPfSlot;   // weights [2][4 waves][32 rows][144]
+constexpr int kPfLdsBytes = kPfWAt + 2 * kPfWStep;
+
+// a wave's weight rows of a super-block into LDS: 16 bytes a lane, the nine pieces of a row in a run
+template <bool GU> struct PfWeights {
+    static constexpr int kMats = GU ? 2 : 1, kRows = 32 / kMats, kWhole = kRows * 9 / 64, kTail = kRows * 9 % 64;
+    static constexpr int kCopies = kMats * (kWhole + 1);
+    __amdgpu_buffer_rsrc_t r[kMats];
+    uint32_t at[kWhole + 1];
+    int lane;
+    __device__ __forceinline__ void init(const PfGemm& a, const uint8_t* blob, int64_t n0, int lane_) {
+        lane = lane_;
+#pragma unroll
+        for (int m = 0; m < kMats; ++m)
+            r[m] = __builtin_amdgcn_make_buffer_rsrc((void*) (blob + a.off[m] + (size_t) n0 * a.row_bytes), 0, (int) (kRows * a.row_bytes), 0x00020000);
+#pragma unroll
+        for (int i = 0; i <= kWhole; ++i) {
+            const int u = 64 * i + lane;
+            at[i] = (uint32_t) ((u / 9) * (int) a.row_bytes + (u % 9) * 16);
+        }
+    }
+    __device__ __forceinline__ void copy(uint8_t* to, int sb) const {
+#pragma unroll
+        for (int m = 0; m < kMats; ++m)
+#pragma unroll
+            for (int i = 0; i < kWhole; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + i * 1024), 16, at[i], sb * 144, 0, 0);
+        // (the lane number is hidden from the compiler: it would follow one `if` into the next, merge copies of different places and
+        // pick their LDS address by lane, which has to be the same for the wave)
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        if (l < kTail) {
+#pragma unroll
+            for (int m = 0; m < kMats; ++m)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + kWhole * 1024), 16, at[kWhole], sb * 144, 0, 0);
+        }
+    }
+};
+
+// The tile's activations, a row group of a super-block at a time.  Every group but the last is whole: its copies are the first
+// one's at another scalar offset.  Rows past the tile's end repeat its last row (their results are never stored).
+struct PfRowsDma {
+    __amdgpu_buffer_rsrc_t rq, rs, rd;
+    uint32_t oq[2], os, od, lq[2], ls, ld;   // the first group's offsets, the last one's
+    int wave, k;
+    __device__ __forceinline__ void init(const PfGemm& a, int row0, int nrows, int groups, int wave_, int lane) {
+        wave = wave_;
+        k = (int) a.k;
+        const int last = nrows - 1;
+        rq = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.q + (size_t) row0 * a.k), 0, (int) (nrows * a.k), 0x00020000);
+        rs = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.s + (size_t) row0 * (a.k >> 4)), 0, (int) (nrows * (a.k >> 5) * 4), 0x00020000);
+        rd = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.d + (size_t) row0 * (a.k >> 8)), 0, (int) (nrows * (a.k >> 8) * 4), 0x00020000);
+        const int l0 = 32 * (groups - 1);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int r = 4 * (wave + 4 * n) + (lane >> 4), c = ((lane & 15) ^ (r & 15)) * 16;   // rows 4 i .. 4 i + 3, i = wave + 4 n
+            oq[n] = (uint32_t) (r * k + c);
+            lq[n] = (uint32_t) (min(l0 + r, last) * k + c);
+        }
+        os = (uint32_t) ((lane >> 1) * (k >> 5) * 4 + (lane & 1) * 16);
+        ls = (uint32_t) (min(l0 + (lane >> 1), last) * (k >> 5) * 4 + (lane & 1) * 16);
+        od = (uint32_t) ((lane & 31) * (k >> 8) * 4);
+        ld = (uint32_t) (min(l0 + (lane & 31), last) * (k >> 8) * 4);
+    }
+    template <bool LAST> __device__ __forceinline__ void copy(uint8_t* buf, int sb, int m) const {
+        const int at = LAST ? 0 : 32 * m;
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (pf_lptr) (buf + (wave + 4 * n) * 1024), 16, LAST ? lq[n] : oq[n], sb * 256 + at * k, 0, 0);
+        if (wave == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (pf_lptr) (buf + kPfSlotS), 16, LAST ? ls : os, sb * 32 + at * (k >> 3), 0, 0);
+        if (wave == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (pf_lptr) (buf + kPfSlotD), 4, LAST ? ld : od, sb * 4 + at * (k >> 6), 0, 0);
+    }
+};
+
+template <int BUT> __device__ __forceinline__ void pf_lds_wait_row(v4i& h, v4i (&q)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(h), "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]) : "n"(BUT));
+}
+template <int BUT> __device__ __forceinline__ void pf_lds_wait1(v4i& r) { asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(BUT)); }
+// FP16 1024 + c of two bytes c of w, as a pair
+__device__ __forceinline__ pf_v2h pf_bytes_1024(uint32_t w, uint32_t sel) {
+    return __builtin_bit_cast(pf_v2h, __builtin_amdgcn_perm(0x64646464u, w, sel));
+}
+
+template <bool GU, int NM, int NB = 0>
+__device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, int row0, int nrows) {
+    const uint8_t* blob = (const uint8_t*) a.table[ex];
     const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    wptr wrow;
-    int64_t n0;   // the wave's first feature (gate/up) or output row (down)
-    if constexpr (GU) {
-        n0 = (int64_t) blockIdx.x * 64 + wave * 16;
-        wrow = blob + a.off[ln >> 4] + (size_t) (n0 + (ln & 15)) * a.row_bytes;
-    } else {
-        n0 = (int64_t) blockIdx.x * 128 + wave * 32;
-        wrow = blob + a.off[0] + (size_t) (n0 + ln) * a.row_bytes;
-    }
-    const bool wave_on = n0 < a.n;   // (a.n is a multiple of the wave's rows: checked on the host)
-
+    // the wave's first feature (gate/up) or output row (down): n is a multiple of 256, every workgroup has all its rows
+    const int64_t n0 = GU ? (int64_t) blockIdx.x * 64 + wave * 16 : (int64_t) blockIdx.x * 128 + wave * 32;
     pf_v16f acc[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m)
@@ -439,166 +488,192 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* b0, uint8_t* b
         for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
 
     const int nsb = (int) (a.k >> 8);
-    // The activations run two super-blocks ahead through three LDS buffers, the weights one ahead in registers.  The
-    // buffers are three separate arrays and the loop below is unrolled over them, so that the compiler can tell a read
-    // of one from a copy into another (it would otherwise wait for every copy in flight before each LDS read).
-    PfDma<NMT> dma;
-    dma.init(a, row0, nrows, wave, lane);
-    dma.copy(b0, 0);
-    if (nsb > 1) dma.copy(b1, 1);
-    // the weights of a super-block: the 16-byte header of the lane's row and four 16-byte pieces of its codes, bytes
-    // 32 c + 16 kh of the row's 128 (c = 0..3): the low nibbles are 16 values of sub-block 2 c, the high ones of 2 c + 1
-    typedef uint32_t w4 __attribute__((ext_vector_type(4)));
-    w4 q[4], qn[4], hdr, hdrn;
-    auto load_block = [&](int sb, w4 (&dq)[4], w4& dh) {
-        wptr blk = wrow + (size_t) sb * 144;
-        dh = *(const __attribute__((address_space(1))) w4*) blk;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) dq[c] = *(const __attribute__((address_space(1))) w4*) (blk + 16 + 32 * c + 16 * kh);
+    PfRowsDma dma;
+    dma.init(a, row0, nrows, NM, wave, lane);
+    PfWeights<GU> wts;
+    uint8_t* const wlds = lds + kPfWAt + wave * kPfWave;
+    // the copies of pass (sb, m) + 3 go into the slot of the pass before (sb, m); in the prologue, of passes 0..2
+    auto copy_pass = [&](auto mc, int sb, int slot) {   // (M in 0 .. NM + 2: pass M of super-block sb on)
+        constexpr int M = decltype(mc)::value, m = M % NM;
+        const int b = sb + M / NM;
+        if (b < nsb) dma.template copy<m == NM - 1>(lds + slot * kPfSlot, b, m);
     };
-    if (wave_on) load_block(0, q, hdr);
+    pf_for_m<0, 3>([&](auto mc) { copy_pass(mc, 0, decltype(mc)::value); });
+    int slot = 0;
+    wts.init(a, blob, n0, lane);
+    wts.copy(wlds, 0);
+    if (nsb > 1) wts.copy(wlds + kPfWStep, 1);
     // a lane's 16 codes of sub-block j: the row's 16-byte chunk 2 j + kh, which sits at that index ^ (the row & 15)
-    const int a_base = ln * 256, a_swz = ((ln & 15) ^ kh) << 4;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    auto step = [&](int sb, const uint8_t* buf, uint8_t* buf2) {   // super-block sb from buf; sb + 2 is copied into buf2
+    const uint32_t a_base = ln * 256 + (((ln & 15) ^ kh) << 4);
+    const uint32_t m_shift = 2 * kh;
+    const pf_v2h m_mul = kh ? pf_v2h{(_Float16) 16.0f, (_Float16) 16.0f} : pf_v2h{(_Float16) 1.0f, (_Float16) 1.0f};
+    const pf_v2h m_add = kh ? pf_v2h{(_Float16) -16384.0f, (_Float16) -16384.0f} : pf_v2h{(_Float16) -1024.0f, (_Float16) -1024.0f};
+    const uint32_t lbase = pf_lds_addr(lds), wbase = pf_lds_addr(wlds) + ln * 144;
+    for (int sb = 0; sb < nsb; ++sb) {
+        const bool steady = sb + 2 < nsb;
+        v4i P[8][2];   // the block's planes: sub-block, low and high digit
         float d = 0.0f, ndmin = 0.0f;
-        uint32_t sc[2], mn[2];
-        if (wave_on) {
-            d = f16_bits_to_f32((uint16_t) (hdr.x & 0xffffu));
-            ndmin = -f16_bits_to_f32((uint16_t) (hdr.x >> 16));
-            q4k_unpack_scales(hdr.y, hdr.z, hdr.w, sc, mn);
-            if (sb + 1 < nsb) load_block(sb + 1, qn, hdrn);
-        }
-        // (after the weights' loads, so that waiting for everything but these copies covers the weights too)
-        if (sb + 2 < nsb) dma.copy(buf2, sb + 2);
-        if (wave_on) {
-            const uint32_t lbuf = pf_lds_addr(buf);
-            // The two plane products of the block, int32: [m][0] = (q lo) . c, [1] = (q hi) . c, a matrix instruction a
-            // sub-block and plane, accumulated over the 8 sub-blocks.  The activation operand of sub-block jj + 1 is
-            // requested from LDS before the arithmetic of sub-block jj, and the operands of the block's closing stage
-            // (the code sums, the block scales) before the last sub-block: a read issued just ahead of its use leaves
-            // the wave waiting for LDS eight times a step.
-            pf_v16i dot[NM][2];
-            v4i xr[2][NM];
-            auto read_x = [&](int jj, v4i (&dst)[NM]) {
-                const uint32_t at = lbuf + a_base + (a_swz ^ ((2 * jj) << 4));
-                pf_for_m<0, NM>([&](auto mc) {
-                    constexpr int m = decltype(mc)::value;
-                    dst[m] = pf_lds_i32x4<m * 8192>(at);
-                });
-            };
-            v4i sa[NM];
-            v4f dxr[NM][4];
-            auto read_tail = [&](auto mc) {   // the closing stage's operands of row group m: its code sums and block scales
-                constexpr int m = decltype(mc)::value;
-                sa[m] = pf_lds_i32x4<kPfSOff + m * 1024>(lbuf + ln * 32 + kh * 16);
-                const uint32_t at = lbuf + 16 * kh;
-                dxr[m][0] = pf_lds_f32x4<kPfDOff + m * 128>(at);
-                dxr[m][1] = pf_lds_f32x4<kPfDOff + m * 128 + 32>(at);
-                dxr[m][2] = pf_lds_f32x4<kPfDOff + m * 128 + 64>(at);
-                dxr[m][3] = pf_lds_f32x4<kPfDOff + m * 128 + 96>(at);
-            };
-            read_x(0, xr[0]);
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const int c = jj >> 1, j = jj & 1;
-                if (jj < 7) read_x(jj + 1, xr[(jj + 1) & 1]);
-                if (jj == 7) read_tail(std::integral_constant<int, 0>{});
-                const uint32_t f = (sc[c >> 1] >> (16 * (c & 1) + 8 * j)) & 0x3fu, flo = f & 7u, fhi = f >> 3;
-                v4i wl, wh;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t w = (q[c][i] >> (4 * j)) & 0x0f0f0f0fu;
-                    wl[i] = (int) pf_scale_codes(w, flo);
-                    wh[i] = (int) pf_scale_codes(w, fhi);
-                }
-                // this sub-block's operand has landed once only the reads issued after it are outstanding (LDS answers in order)
-                if (jj < 7) pf_lds_wait_but<NM>(xr[jj & 1]);
-                else pf_lds_wait_but<5>(xr[jj & 1]);
-#pragma unroll
-                for (int m = 0; m < NM; ++m) {
-                    const pf_v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-                    dot[m][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj & 1][m], wl, jj ? dot[m][0] : z, 0, 0, 0);
-                    dot[m][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj & 1][m], wh, jj ? dot[m][1] : z, 0, 0, 0);
-                }
+        pf_v8h mb;
+        pf_for_m<0, NM>([&](auto mc) {
+            constexpr int m = decltype(mc)::value;
+            // What this pass reads has landed once only what was issued after it is in flight: the activations of the two passes
+            // behind it (at least two copies a wave each) and the weights issued in the three passes before this one; the weights
+            // of a tile of one group were issued two passes ago, behind the next pass's activations.
+            constexpr int kW = PfWeights<GU>::kCopies;
+            constexpr int kIssued = ((m + 4 * NM - 1) % NM == 0) + ((m + 4 * NM - 2) % NM == 0) + ((m + 4 * NM - 3) % NM == 0);
+            constexpr int kBut = NM == 1 ? 2 + kW : 4 + kW * kIssued;
+            if (!steady || (m == 0 && sb == 0)) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBut) : "memory");
+            const uint32_t lbuf = lbase + slot * kPfSlot;
+            v4i hdr, q[4];
+            if constexpr (m == 0) {
+                const uint32_t at = wbase + (sb & 1) * kPfWStep;
+                hdr = pf_lds_i32x4<0>(at);
+                // four 16-byte pieces of the row's codes, bytes 32 c + 16 kh of its 128: the low nibbles are 16 values of
+                // sub-block 2 c, the high ones of 2 c + 1
+                q[0] = pf_lds_i32x4<16>(at + 16 * kh);
+                q[1] = pf_lds_i32x4<48>(at + 16 * kh);
+                q[2] = pf_lds_i32x4<80>(at + 16 * kh);
+                q[3] = pf_lds_i32x4<112>(at + 16 * kh);
             }
-            // The minimums' integer term sum_j m_j (sum of sub-block j's codes), exactly, from one FP16 matrix instruction:
-            // k = 0..7 pairs m_j with the sums' low digits, k = 8..15 pairs 64 m_j with their high digits (every operand
-            // and every partial sum an integer below 2^24).
-            pf_v8h mb;
-            {
-                const float mul = kh ? 64.0f : 1.0f;
+            copy_pass(std::integral_constant<int, m + 3>{}, sb, (slot + 3) & 3);
+            slot = (slot + 1) & 3;
+            // The two plane products of the block, int32, a matrix instruction a sub-block and plane, accumulated over the 8
+            // sub-blocks.  The activation operand is requested from LDS two sub-blocks ahead.
+            pf_v16i dot[2];
+            v4i xr[3];
+            const uint32_t xa = lbuf + a_base;
+            xr[0] = pf_lds_i32x4<0>(xa);
+            xr[1] = pf_lds_i32x4<0>(xa ^ 32);
+            int sum[NB ? 4 * NB : 1];
+            pf_v16i part[NB ? 3 : 1];   // (sub-block sums, worked off two sub-blocks on: a matrix instruction's results take a while)
+            auto add_part = [&](int jj, const uint32_t (&sc)[2]) {
+                const int scale = (int) ((sc[jj >> 2] >> (8 * (jj & 3))) & 0x3fu);
+#pragma unroll
+                for (int i = 0; i < 4 * NB; ++i) {
+                    sum[i] = __mul24(part[NB ? jj % 3 : 0][i], scale) + (jj ? sum[i] : 0);
+                    asm("" : "+v"(sum[i]));   // (keeps multiply and add one instruction)
+                }
+                // (the registers of rows that are not there stay taken until now: given away behind the matrix instruction, they made
+                // the next instruction wait until it had written them)
+                asm volatile("" ::"v"(part[NB ? jj % 3 : 0]));
+            };
+            uint32_t sc[2], mn[2];
+            pf_u16x2 flo[2][2], fhi[2][2];
+            if constexpr (m == 0) {
+                pf_lds_wait_row<2>(hdr, q);
+                // (the wave's weights are in registers: their LDS takes the super-block after the next one's)
+                if (steady) wts.copy(wlds + (sb & 1) * kPfWStep, sb + 2);
+                d = f16_bits_to_f32((uint16_t) (hdr[0] & 0xffff));
+                ndmin = -f16_bits_to_f32((uint16_t) ((uint32_t) hdr[0] >> 16));
+                q4k_unpack_scales((uint32_t) hdr[1], (uint32_t) hdr[2], (uint32_t) hdr[3], sc, mn);
+                // the scales' low and high digits as 16-bit pairs: [w][p] those of sub-blocks 4 w + p and 4 w + 2 + p
 #pragma unroll
                 for (int w = 0; w < 2; ++w)
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        const pf_v2h t = __builtin_bit_cast(pf_v2h, __builtin_amdgcn_cvt_pkrtz(__fmul_rn((float) ((mn[w] >> (16 * i)) & 0xffu), mul),
-                                                                                              __fmul_rn((float) ((mn[w] >> (16 * i + 8)) & 0xffu), mul)));
-                        mb[4 * w + 2 * i] = t[0], mb[4 * w + 2 * i + 1] = t[1];
+                    for (int p = 0; p < 2; ++p) {
+                        flo[w][p] = __builtin_bit_cast(pf_u16x2, (sc[w] >> (8 * p)) & 0x00070007u);
+                        fhi[w][p] = __builtin_bit_cast(pf_u16x2, (sc[w] >> (8 * p + 3)) & 0x00070007u);
                     }
-            }
-            // once a block: lo + 8 hi = the block's integer sum (< 2^25), then d_x (d_w sum - dmin_w minimums)
-            pf_for_m<0, NM>([&](auto mc) {
-                constexpr int m = decltype(mc)::value;
-                if constexpr (m + 1 < NM) {
-                    read_tail(std::integral_constant<int, m + 1>{});
-                    pf_lds_wait_tail<5>(sa[m], dxr[m]);
-                } else {
-                    pf_lds_wait_tail<0>(sa[m], dxr[m]);
+                // The minimums' operand: k = 0..7 pairs m_j with the sums' low digits, k = 8..15 pairs 64 m_j with their
+                // high digits.  A byte b behind 0x64 is FP16 1024 + b: m, or 4 m and 16 times that.
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    const uint32_t mw = mn[w] << m_shift;
+                    const pf_v2h t0 = __builtin_elementwise_fma(pf_bytes_1024(mw, 0x04010400u), m_mul, m_add);
+                    const pf_v2h t1 = __builtin_elementwise_fma(pf_bytes_1024(mw, 0x04030402u), m_mul, m_add);
+                    mb[4 * w] = t0[0], mb[4 * w + 1] = t0[1], mb[4 * w + 2] = t1[0], mb[4 * w + 3] = t1[1];
                 }
-                const pf_v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-                const pf_v16f mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_v8h, sa[m]), mb, z, 0, 0, 0);
-                // (a lane's outputs 4 b .. 4 b + 3 are the tile's rows 32 m + 8 b + 4 kh + 0..3: blocks of 8 rows past the
-                // tile's last row are skipped - most tiles of a skewed routing hold 8 rows or fewer)
-                const int nb = (nrows - 32 * m + 7) >> 3;
+            }
+            v4i sa;
+            v4f dxr[4];
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    if (b < nb) {
+            for (int jj = 0; jj < 8; ++jj) {
+                if (jj < 6) xr[(jj + 2) % 3] = pf_lds_i32x4<0>(xa ^ (32 * (jj + 2)));
+                if (jj == 6) {   // the closing stage's operands: the code sums, the block scales
+                    sa = pf_lds_i32x4<kPfSlotS>(lbuf + ln * 32 + kh * 16);
+                    const uint32_t at = lbuf + 16 * kh;
+                    dxr[0] = pf_lds_f32x4<kPfSlotD>(at);
+                    dxr[1] = pf_lds_f32x4<kPfSlotD + 32>(at);
+                    dxr[2] = pf_lds_f32x4<kPfSlotD + 64>(at);
+                    dxr[3] = pf_lds_f32x4<kPfSlotD + 96>(at);
+                }
+                if constexpr (m == 0 && NB == 0) {
+                    const int c = jj >> 1, j = jj & 1;
+                    const pf_u16x2 lo = flo[jj >> 2][j], hi = fhi[jj >> 2][j];
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int i = 4 * b + r;
-                            const float t = fmaf(ndmin, mins[i], __fmul_rn(d, (float) (dot[m][0][i] + 8 * dot[m][1][i])));
-                            acc[m][i] = fmaf(dxr[m][b][r], t, acc[m][i]);
-                        }
+                    for (int i = 0; i < 4; ++i) {
+                        // four 4-bit codes (one a byte) times a factor <= 7: no byte overflows, so one packed 16-bit multiply does it
+                        const pf_u16x2 w = __builtin_bit_cast(pf_u16x2, ((uint32_t) q[c][i] >> (4 * j)) & 0x0f0f0f0fu);
+                        P[jj][0][i] = __builtin_bit_cast(int, c & 1 ? w * lo.yy : w * lo.xx);
+                        P[jj][1][i] = __builtin_bit_cast(int, c & 1 ? w * hi.yy : w * hi.xx);
                     }
                 }
-            });
-            if (sb + 1 < nsb) {
-                hdr = hdrn;
+                // this sub-block's operand has landed once only the reads issued after it are outstanding (LDS answers in order)
+                if (jj < 6) pf_lds_wait1<2>(xr[jj % 3]);
+                else if (jj == 6) pf_lds_wait1<6>(xr[jj % 3]);
+                else pf_lds_wait1<5>(xr[jj % 3]);
+                const pf_v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                if constexpr (NB != 0) {
+                    v4i w;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) q[c] = qn[c];
+                    for (int i = 0; i < 4; ++i) w[i] = (int) (((uint32_t) q[jj >> 1][i] >> (4 * (jj & 1))) & 0x0f0f0f0fu);
+                    part[jj % 3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], w, z, 0, 0, 0);
+                    if (jj > 1) add_part(jj - 2, sc);
+                    continue;
+                }
+                dot[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], P[jj][0], jj ? dot[0] : z, 0, 0, 0);
+                dot[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], P[jj][1], jj ? dot[1] : z, 0, 0, 0);
             }
-        }
-        // super-block sb + 1 has landed once only the wave's youngest NMT operations may still be in flight: this
-        // iteration's copies (of sb + 2), or - in the last steps, which copy nothing - some of the five weight loads
-        // issued above; a wave that holds no weight rows has nothing younger than its last copies then and waits for all
-        // (a bare barrier: __syncthreads() would first wait for every memory operation of the wave, these copies included)
-        if (sb + 2 < nsb || wave_on) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NMT) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-    for (int sb = 0; sb < nsb; sb += 3) {
-        step(sb, b0, b2);
-        if (sb + 1 < nsb) step(sb + 1, b1, b0);
-        if (sb + 2 < nsb) step(sb + 2, b2, b1);
+            // The minimums' integer term sum_j m_j (sum of sub-block j's codes), exactly, from one FP16 matrix instruction
+            // (every operand and every partial sum an integer below 2^24); then once a block lo + 8 hi = the block's
+            // integer sum (< 2^25) and d_x (d_w sum - dmin_w minimums)
+            pf_lds_wait_tail<0>(sa, dxr);
+            const pf_v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            const pf_v16f mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_v8h, sa), mb, z, 0, 0, 0);
+            if constexpr (NB != 0) add_part(6, sc), add_part(7, sc);
+            // (a lane's outputs 4 b .. 4 b + 3 are the tile's rows 32 m + 8 b + 4 kh + 0..3: blocks of 8 rows past the
+            // tile's last row are skipped - most tiles of a skewed routing hold 8 rows or fewer)
+            const int nb = m == NM - 1 ? (nrows - 32 * m + 7) >> 3 : 4;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                if (NB ? b < NB : m < NM - 1 || b < nb) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int i = 4 * b + r;
+                        const float t = fmaf(ndmin, mins[i], __fmul_rn(d, (float) (NB ? sum[NB ? i : 0] : dot[0][i] + 8 * dot[1][i])));
+                        acc[m][i] = fmaf(dxr[b][r], t, acc[m][i]);
+                    }
+                }
+            }
+            asm volatile("" : "+v"(acc[m]));   // (here, not when the block's other passes are done: that would keep every pass's sums)
+        });
     }
-    if (!wave_on) return;
-
     // outputs: lane (ln, kh) holds weight row ln for the tile's rows 32 m + 8 b + 4 kh + r (i = 4 b + r)
+    pf_for_m<0, NM>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = 32 * m + 8 * (i >> 2) + 4 * kh + (i & 3);
+        for (int b = 0; b < 4; ++b) {
+            const int r0 = 32 * m + 8 * b;
+            if (NB ? b >= NB : m == NM - 1 && r0 >= nrows) continue;
             if constexpr (GU) {
-                // the up row of a feature sits 16 lanes above its gate row
-                const float up = __shfl(acc[m][i], (lane + 16) & 63, kWave);
-                if (ln < 16 && r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = pf_swiglu(acc[m][i], up, a.limit);
+                // The up row of a feature sits 16 lanes above its gate row.  One swap of every second 16 lanes between two rows'
+                // values leaves the lanes of the gate rows with gate and up of the first, the others with those of the second.
+                float* o = a.out + (size_t) (row0 + r0 + 4 * kh) * a.n + n0 + (ln & 15) + (ln < 16 ? 0 : a.n);
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    const auto gu = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[m][4 * b + r]), __float_as_uint(acc[m][4 * b + r + 1]), false, false);
+                    const float h = pf_swiglu(__uint_as_float(gu[0]), __uint_as_float(gu[1]), a.limit);
+                    if (m < NM - 1 || r0 + 4 * kh + r + (ln >> 4) < nrows) o[(size_t) r * a.n] = h;
+                }
             } else {
-                if (r < nrows) a.out[(size_t) (row0 + r) * a.n + n0 + ln] = acc[m][i];
+                float* o = a.out + (size_t) (row0 + r0 + 4 * kh) * a.n + n0 + ln;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (m < NM - 1 || r0 + 4 * kh + r < nrows) o[(size_t) r * a.n] = acc[m][4 * b + r];
             }
         }
-    }
+    });
 }
 
 #include "maya_prefill_iq2s.hpp"
@@ -606,13 +681,19 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* b0, uint8_t* b
 // grid (bands of weight rows, tiles at most)
 template <bool GU>
 __global__ __launch_bounds__(256, 2) void prefill_q4k_kernel(PfGemm a) {
-    __shared__ __attribute__((aligned(16))) uint8_t b0[kPfBufBytes], b1[kPfBufBytes], b2[kPfBufBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kPfLdsBytes];
     const int tile = blockIdx.y;
     if (tile >= *a.plan.n_tiles) return;
-    const int ex = a.plan.tile_expert[tile], row0 = a.plan.tile_row0[tile];
-    const int nrows = min(kPfRows, a.plan.bounds[ex + 1] - row0);
-    if (nrows <= 32) pf_tile<GU, 1>(a, b0, b1, b2, ex, row0, nrows);
-    else pf_tile<GU, 2>(a, b0, b1, b2, ex, row0, nrows);
+    const int ex = a.plan.tile_expert[tile], row0 = a.plan.tile_row0[tile], first = a.plan.bounds[ex];
+    if ((row0 - first) % (32 * kPfGroups) != 0) return;   // (the workgroup of the tile before takes this one too)
+    const int nrows = min(32 * kPfGroups, a.plan.bounds[ex + 1] - row0);
+    if (nrows <= 8) pf_tile<GU, 1, 1>(a, lds, ex, row0, nrows);
+    else if (nrows <= 16) pf_tile<GU, 1, 2>(a, lds, ex, row0, nrows);
+    else if (nrows <= 24) pf_tile<GU, 1, 3>(a, lds, ex, row0, nrows);
+    else if (nrows <= 32) pf_tile<GU, 1>(a, lds, ex, row0, nrows);
+    else if (nrows <= 64) pf_tile<GU, 2>(a, lds, ex, row0, nrows);
+    else if (nrows <= 96) pf_tile<GU, 3>(a, lds, ex, row0, nrows);
+    else pf_tile<GU, 4>(a, lds, ex, row0, nrows);
 }
 
 template <int ODT>

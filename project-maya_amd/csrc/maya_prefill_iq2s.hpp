@@ -14,6 +14,39 @@
 // added (2 ls + 1) x its sums on the vector ALU: 41 vector instructions to decode 512 weights and two multiply-adds an
 // output every 32 values, 79 % of the cycles in vector issue.  A 75-token chunk on
 // 160 experts of 6144 x 1536 735 -> 535 us; gate/up IQ2_S with Q4_K down, 1187 tokens on 256 of 7168 x 2048, 2830 -> 2190 us.
+// LDS of one buffer of activations: the codes [kPfRows][256], d [kPfRows]
+constexpr int kPfPlane = kPfRows * 256;
+constexpr int kPfDOffNoS = kPfPlane, kPfBufBytesNoS = kPfDOffNoS + kPfRows * 4;
+// The tile's activations go from global memory to LDS without passing registers (each lane's 16 bytes land at the
+// wave's base + 16 lane): buffer loads whose per-lane offsets are fixed for the tile - the super-block rides in the
+// scalar offset - so a copy costs no vector arithmetic.  Rows past the tile's end repeat its last row (their results
+// are never stored).
+template <int NMT>
+struct PfDma {
+    __amdgpu_buffer_rsrc_t rq, rd;
+    uint32_t oq[NMT], od;
+    int wave;
+    __device__ __forceinline__ void init(const PfGemm& a, int row0, int nrows, int wave_, int lane) {
+        wave = wave_;
+        const int last = nrows - 1;
+        rq = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.q + (size_t) row0 * a.k), 0, (int) (nrows * a.k), 0x00020000);
+        rd = __builtin_amdgcn_make_buffer_rsrc((void*) (a.x.d + (size_t) row0 * (a.k >> 8)), 0, (int) (nrows * (a.k >> 8) * 4), 0x00020000);
+#pragma unroll
+        for (int n = 0; n < NMT; ++n) {
+            const int r = 4 * (wave + 4 * n) + (lane >> 4), cp = lane & 15;   // rows 4 i .. 4 i + 3, i = wave + 4 n
+            oq[n] = (uint32_t) (min(r, last) * (int) a.k + ((cp ^ (r & 15)) * 16));
+        }
+        od = (uint32_t) (min(lane, last) * (int) (a.k >> 8) * 4);
+    }
+    // super-block sb into the buffer at `buf`
+    __device__ __forceinline__ void copy(uint8_t* buf, int sb) const {
+#pragma unroll
+        for (int n = 0; n < NMT; ++n)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (pf_lptr) (buf + (wave + 4 * n) * 1024), 16, oq[n], sb * 256, 0, 0);
+        if (wave == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (pf_lptr) (buf + kPfDOffNoS), 4, od, sb * 4, 0, 0);
+    }
+};
+
 constexpr int kIqMags = 0, kIqSigns = 8192, kIqScales = kIqSigns + 2048, kIqTables = kIqScales + 256;   // byte offsets in LDS
 constexpr int kIqLdsBytes = kIqTables + 3 * kPfBufBytesNoS;
 
@@ -60,7 +93,7 @@ __device__ __forceinline__ void pf_tile_iq2s(const PfGemm& a, uint8_t* b0, uint8
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
 
-    PfDma<NMT, false> dma;
+    PfDma<NMT> dma;
     dma.init(a, row0, nrows, wave, lane);
     dma.copy(b0, 0);
     if (nsb > 1) dma.copy(b1, 1);

@@ -191,6 +191,46 @@ def test_stages_and_layer_match_checker(pf, oracle, case):
     assert torch.equal(got2, out)
 
 
+EDGE_ROWS = [1, 7, 8, 9, 16, 17, 24, 25, 32, 33, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257]
+
+
+@pytest.mark.parametrize("n_embd, n_ff", [(256, 512), (512, 256), (768, 768), (1536, 256)], ids=str)
+def test_experts_of_every_number_of_row_groups(pf, oracle, n_embd, n_ff):
+    """Experts of EDGE_ROWS rows each in one chunk - both sides of a block of 8 rows, of a row group, of a workgroup's rows - with 1, 2,
+    3 and 6 super-blocks a row, fewer and more than run ahead: h and the down rows against the CPU path's row dots.  The integer sums
+    are the same and the F32 ones of at most 6 blocks differ by order: 1e-5."""
+    from maya_amd import lib
+    import synth
+    ne = len(EDGE_ROWS)
+    blobs = make_blobs(oracle, ne, n_embd, n_ff, 3 * n_embd + n_ff)
+    up_off, down_off, _ = synth.blob_offsets(Q4_K, Q4_K, n_embd, n_ff)
+    rng = np.random.default_rng(n_embd)
+    ids = np.repeat(np.arange(ne, dtype=np.int32), EDGE_ROWS)
+    rng.shuffle(ids)
+    x = rng.standard_normal((ids.size, n_embd)).astype(np.float32)
+    layout, _ = lib.layout(Q4_K, Q4_K, n_embd, n_ff)
+    table = lib.ExpertStore(blobs)
+    p = pf.plan(dev(ids), table.table)
+    hq = pf.gate_up(layout, table.table, p, pf.quant(dev(x), p, 1))
+    part = pf.down(layout, table.table, p, hq)
+    torch.cuda.synchronize()
+    h, part, row_entry = hq.f32.cpu().numpy(), part.cpu().numpy(), p.row_entry.cpu().numpy()
+    assert np.array_equal(np.bincount(ids, minlength=ne), EDGE_ROWS)
+    first = np.concatenate([[0], np.cumsum(EDGE_ROWS)])
+    for e in range(ne):
+        at = range(EDGE_ROWS[e])
+        for r in sorted({i for i in at if i % 32 in (0, 1, 6, 12, 19, 31)} | {EDGE_ROWS[e] - 1}):   # (a row of every 8, of every group)
+            row = int(first[e]) + r
+            tok = int(row_entry[row])
+            assert ids[tok] == e
+            a = oracle.quant_act(Q4_K, x[tok])
+            g, u = oracle.rows(Q4_K, blobs[e], n_embd, n_ff, a), oracle.rows(Q4_K, blobs[e][up_off:], n_embd, n_ff, a)
+            want = [oracle.lib().mo_swiglu(float(gv), float(uv), float("inf")) for gv, uv in zip(g, u)]
+            assert rel_l2(h[row], np.array(want, dtype=np.float32)) <= 1e-5, (EDGE_ROWS[e], r)
+            want = oracle.rows(Q4_K, blobs[e][down_off:], n_ff, n_embd, oracle.quant_act(Q4_K, h[row]))
+            assert rel_l2(part[row], want) <= 1e-5, (EDGE_ROWS[e], r)
+
+
 IQ_CASES = [
     # gate/up type, down type, n_embd, n_ff, n_expert, k, n_tokens, limit, experts that are not resident
     (22, 22, 512, 512, 6, 2, 41, 0.0, ()),
