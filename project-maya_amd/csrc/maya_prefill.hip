@@ -342,11 +342,9 @@ template <int OFF> __device__ __forceinline__ v4i pf_lds_i32x4(uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
     return v;
 }
-// the registers r have landed once at most BUT later LDS reads are outstanding (LDS operations complete in order)
-template <int BUT, int N> __device__ __forceinline__ void pf_lds_wait_but(v4i (&r)[N]) {
-    static_assert(N == 1 || N == 2, "1 or 2 registers");
-    if constexpr (N == 1) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r[0]) : "n"(BUT));
-    else asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r[0]), "+v"(r[1]) : "n"(BUT));
+// (... have landed once at most BUT later LDS reads are outstanding: LDS operations complete in order)
+template <int BUT> __device__ __forceinline__ void pf_lds_wait_tail(v4f (&d)[4]) {
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]) : "n"(BUT));
 }
 template <int BUT> __device__ __forceinline__ void pf_lds_wait_tail(v4i& a, v4f (&d)[4]) {
     asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(a), "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]) : "n"(BUT));
@@ -391,48 +389,10 @@ typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 constexpr int kPfGroups = 4;                         // row groups of a workgroup at most: two of the plan's tiles
 constexpr int kPfRing = 4;                           // activations of a pass in LDS, three passes ahead
 constexpr int kPfSlotS = 8192, kPfSlotD = kPfSlotS + 1024, kPfSlot = kPfSlotD + 256;   // codes [32][256], sums [32][16], scales [32]
-constexpr int kPfWave = 32 * 144, kPfWStep = 4 * kPfWave, kPfWAt = kPfRing * kPfSlot;   // weights [2][4 waves][32 rows][144]
-constexpr int kPfLdsBytes = kPfWAt + 2 * kPfWStep;
-
-// a wave's weight rows of a super-block into LDS: 16 bytes a lane, the nine pieces of a row in a run
-template <bool GU> struct PfWeights {
-    static constexpr int kMats = GU ? 2 : 1, kRows = 32 / kMats, kWhole = kRows * 9 / 64, kTail = kRows * 9 % 64;
-    static constexpr int kCopies = kMats * (kWhole + 1);
-    __amdgpu_buffer_rsrc_t r[kMats];
-    uint32_t at[kWhole + 1];
-    int lane;
-    __device__ __forceinline__ void init(const PfGemm& a, const uint8_t* blob, int64_t n0, int lane_) {
-        lane = lane_;
-#pragma unroll
-        for (int m = 0; m < kMats; ++m)
-            r[m] = __builtin_amdgcn_make_buffer_rsrc((void*) (blob + a.off[m] + (size_t) n0 * a.row_bytes), 0, (int) (kRows * a.row_bytes), 0x00020000);
-#pragma unroll
-        for (int i = 0; i <= kWhole; ++i) {
-            const int u = 64 * i + lane;
-            at[i] = (uint32_t) ((u / 9) * (int) a.row_bytes + (u % 9) * 16);
-        }
-    }
-    __device__ __forceinline__ void copy(uint8_t* to, int sb) const {
-#pragma unroll
-        for (int m = 0; m < kMats; ++m)
-#pragma unroll
-            for (int i = 0; i < kWhole; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + i * 1024), 16, at[i], sb * 144, 0, 0);
-        // (the lane number is hidden from the compiler: it would follow one `if` into the next, merge copies of different places and
-        // pick their LDS address by lane, which has to be the same for the wave)
-        int l = lane;
-        asm volatile("" : "+v"(l));
-        if (l < kTail) {
-#pragma unroll
-            for (int m = 0; m < kMats; ++m)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + kWhole * 1024), 16, at[kWhole], sb * 144, 0, 0);
-        }
-    }
-};
 
 // The tile's activations, a row group of a super-block at a time.  Every group but the last is whole: its copies are the first
 // one's at another scalar offset.  Rows past the tile's end repeat its last row (their results are never stored).
-struct PfRowsDma {
+template <bool SUMS> struct PfRowsDma {   // SUMS: with the code sums that a type with minimums wants
     __amdgpu_buffer_rsrc_t rq, rs, rd;
     uint32_t oq[2], os, od, lq[2], ls, ld;   // the first group's offsets, the last one's
     int wave, k;
@@ -460,22 +420,131 @@ struct PfRowsDma {
 #pragma unroll
         for (int n = 0; n < 2; ++n)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (pf_lptr) (buf + (wave + 4 * n) * 1024), 16, LAST ? lq[n] : oq[n], sb * 256 + at * k, 0, 0);
-        if (wave == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (pf_lptr) (buf + kPfSlotS), 16, LAST ? ls : os, sb * 32 + at * (k >> 3), 0, 0);
+        if (SUMS && wave == 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (pf_lptr) (buf + kPfSlotS), 16, LAST ? ls : os, sb * 32 + at * (k >> 3), 0, 0);
         if (wave == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (pf_lptr) (buf + kPfSlotD), 4, LAST ? ld : od, sb * 4 + at * (k >> 6), 0, 0);
     }
 };
 
-template <int BUT> __device__ __forceinline__ void pf_lds_wait_row(v4i& h, v4i (&q)[4]) {
-    asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(h), "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]) : "n"(BUT));
-}
 template <int BUT> __device__ __forceinline__ void pf_lds_wait1(v4i& r) { asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(BUT)); }
 // FP16 1024 + c of two bytes c of w, as a pair
 __device__ __forceinline__ pf_v2h pf_bytes_1024(uint32_t w, uint32_t sel) {
     return __builtin_bit_cast(pf_v2h, __builtin_amdgcn_perm(0x64646464u, w, sel));
 }
 
-template <bool GU, int NM, int NB = 0>
+// What the tile wants of a weight type: the copies of a wave's 32 rows of a super-block into LDS (kCopies instructions, kWave
+// bytes), a lane's reads of its row's part of them, and the two planes of a sub-block out of the registers these filled.
+template <bool GU> struct PfQ4K {
+    static constexpr bool kSums = true;
+    static constexpr int kLdsAt = 0, kWave = 32 * 144;
+    static constexpr int kMats = GU ? 2 : 1, kRows = 32 / kMats, kWhole = kRows * 9 / 64, kTail = kRows * 9 % 64;
+    static constexpr int kCopies = kMats * (kWhole + 1);
+    static constexpr int kHiFactor = 8, kLook = 0;   // (a sum is lo + 8 hi; LDS look-ups of a sub-block's planes)
+    __amdgpu_buffer_rsrc_t r[kMats];
+    uint32_t at[kWhole + 1], row_at, m_shift;
+    int lane;
+    pf_v2h m_mul, m_add;
+    __device__ __forceinline__ void init(const PfGemm& a, const uint8_t* blob, int64_t n0, int lane_) {
+        lane = lane_;
+#pragma unroll
+        for (int m = 0; m < kMats; ++m)
+            r[m] = __builtin_amdgcn_make_buffer_rsrc((void*) (blob + a.off[m] + (size_t) n0 * a.row_bytes), 0, (int) (kRows * a.row_bytes), 0x00020000);
+#pragma unroll
+        for (int i = 0; i <= kWhole; ++i) {   // 16 bytes a lane, the nine pieces of a row in a run
+            const int u = 64 * i + lane;
+            at[i] = (uint32_t) ((u / 9) * (int) a.row_bytes + (u % 9) * 16);
+        }
+        const int kh = lane >> 5;
+        row_at = (lane & 31) * 144 + 16 * kh;
+        m_shift = 2 * kh;
+        m_mul = kh ? pf_v2h{(_Float16) 16.0f, (_Float16) 16.0f} : pf_v2h{(_Float16) 1.0f, (_Float16) 1.0f};
+        m_add = kh ? pf_v2h{(_Float16) -16384.0f, (_Float16) -16384.0f} : pf_v2h{(_Float16) -1024.0f, (_Float16) -1024.0f};
+    }
+    __device__ __forceinline__ void copy(uint8_t* to, int sb) const {
+#pragma unroll
+        for (int m = 0; m < kMats; ++m)
+#pragma unroll
+            for (int i = 0; i < kWhole; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + i * 1024), 16, at[i], sb * 144, 0, 0);
+        // (the lane number is hidden from the compiler: it would follow one `if` into the next, merge copies of different places and
+        // pick their LDS address by lane, which has to be the same for the wave)
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        if (l < kTail) {
+#pragma unroll
+            for (int m = 0; m < kMats; ++m)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + kWhole * 1024), 16, at[kWhole], sb * 144, 0, 0);
+        }
+    }
+    struct Row {   // a lane's part of its row: the header, four 16-byte pieces of the codes (bytes 32 c + 16 kh of their 128: the low
+                   // nibbles are 16 values of sub-block 2 c, the high ones of 2 c + 1), and what `open` makes of them
+        v4i hdr, q[4];
+        float d, ndmin;
+        uint32_t sc[2];
+        pf_u16x2 flo[2][2], fhi[2][2];
+        pf_v8h mb;
+    };
+    __device__ __forceinline__ void read(Row& w, uint32_t base) const {
+        const uint32_t at = base + row_at;
+        w.hdr = pf_lds_i32x4<0>(base + (lane & 31) * 144);
+        w.q[0] = pf_lds_i32x4<16>(at);
+        w.q[1] = pf_lds_i32x4<48>(at);
+        w.q[2] = pf_lds_i32x4<80>(at);
+        w.q[3] = pf_lds_i32x4<112>(at);
+    }
+    template <int BUT> __device__ __forceinline__ void wait(Row& w) const {
+        asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(w.hdr), "+v"(w.q[0]), "+v"(w.q[1]), "+v"(w.q[2]), "+v"(w.q[3]) : "n"(BUT));
+    }
+    __device__ __forceinline__ void open(Row& w) const {
+        uint32_t mn[2];
+        w.d = f16_bits_to_f32((uint16_t) (w.hdr[0] & 0xffff));
+        w.ndmin = -f16_bits_to_f32((uint16_t) ((uint32_t) w.hdr[0] >> 16));
+        q4k_unpack_scales((uint32_t) w.hdr[1], (uint32_t) w.hdr[2], (uint32_t) w.hdr[3], w.sc, mn);
+        // the scales' low and high digits as 16-bit pairs: [i][p] those of sub-blocks 4 i + p and 4 i + 2 + p
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                w.flo[i][p] = __builtin_bit_cast(pf_u16x2, (w.sc[i] >> (8 * p)) & 0x00070007u);
+                w.fhi[i][p] = __builtin_bit_cast(pf_u16x2, (w.sc[i] >> (8 * p + 3)) & 0x00070007u);
+            }
+        // The minimums' operand: k = 0..7 pairs m_j with the sums' low digits, k = 8..15 pairs 64 m_j with their high digits.
+        // A byte b behind 0x64 is FP16 1024 + b: m, or 4 m and 16 times that.
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t mw = mn[i] << m_shift;
+            const pf_v2h t0 = __builtin_elementwise_fma(pf_bytes_1024(mw, 0x04010400u), m_mul, m_add);
+            const pf_v2h t1 = __builtin_elementwise_fma(pf_bytes_1024(mw, 0x04030402u), m_mul, m_add);
+            w.mb[4 * i] = t0[0], w.mb[4 * i + 1] = t0[1], w.mb[4 * i + 2] = t1[0], w.mb[4 * i + 3] = t1[1];
+        }
+    }
+    template <int J> __device__ __forceinline__ void look(Row&) const {}
+    template <int BUT> __device__ __forceinline__ void wait_look(int, Row&, v4i& x) const { pf_lds_wait1<BUT>(x); }
+    __device__ __forceinline__ void planes(const Row& w, int j, v4i& wl, v4i& wh) const {
+        const pf_u16x2 lo = w.flo[j >> 2][j & 1], hi = w.fhi[j >> 2][j & 1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // four 4-bit codes (one a byte) times a factor <= 7: no byte overflows, so one packed 16-bit multiply does it
+            const pf_u16x2 c = __builtin_bit_cast(pf_u16x2, ((uint32_t) w.q[j >> 1][i] >> (4 * (j & 1))) & 0x0f0f0f0fu);
+            wl[i] = __builtin_bit_cast(int, j & 2 ? c * lo.yy : c * lo.xx);
+            wh[i] = __builtin_bit_cast(int, j & 2 ? c * hi.yy : c * hi.xx);
+        }
+    }
+    __device__ __forceinline__ v4i codes(const Row& w, int j) const {
+        v4i c;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] = (int) (((uint32_t) w.q[j >> 1][i] >> (4 * (j & 1))) & 0x0f0f0f0fu);
+        return c;
+    }
+};
+
+template <typename W> struct PfLds {   // the weight type's tables, the activations' ring, the weights [2][4 waves]
+    static constexpr int ring = W::kLdsAt, w = ring + kPfRing * kPfSlot, w_step = 4 * W::kWave, bytes = w + 2 * w_step;
+};
+
+// NB: 0, or the blocks of 8 rows of a tile that takes the codes themselves to the matrix cores
+template <typename W, bool GU, int NM, int NB = 0>
 __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, int row0, int nrows) {
+    typedef PfLds<W> S;
     const uint8_t* blob = (const uint8_t*) a.table[ex];
     const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -488,54 +557,39 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
         for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
 
     const int nsb = (int) (a.k >> 8);
-    PfRowsDma dma;
+    PfRowsDma<W::kSums> dma;
     dma.init(a, row0, nrows, NM, wave, lane);
-    PfWeights<GU> wts;
-    uint8_t* const wlds = lds + kPfWAt + wave * kPfWave;
+    W wts;
+    uint8_t* const wlds = lds + S::w + wave * W::kWave;
     // the copies of pass (sb, m) + 3 go into the slot of the pass before (sb, m); in the prologue, of passes 0..2
     auto copy_pass = [&](auto mc, int sb, int slot) {   // (M in 0 .. NM + 2: pass M of super-block sb on)
         constexpr int M = decltype(mc)::value, m = M % NM;
         const int b = sb + M / NM;
-        if (b < nsb) dma.template copy<m == NM - 1>(lds + slot * kPfSlot, b, m);
+        if (b < nsb) dma.template copy<m == NM - 1>(lds + S::ring + slot * kPfSlot, b, m);
     };
     pf_for_m<0, 3>([&](auto mc) { copy_pass(mc, 0, decltype(mc)::value); });
     int slot = 0;
     wts.init(a, blob, n0, lane);
     wts.copy(wlds, 0);
-    if (nsb > 1) wts.copy(wlds + kPfWStep, 1);
+    if (nsb > 1) wts.copy(wlds + S::w_step, 1);
     // a lane's 16 codes of sub-block j: the row's 16-byte chunk 2 j + kh, which sits at that index ^ (the row & 15)
     const uint32_t a_base = ln * 256 + (((ln & 15) ^ kh) << 4);
-    const uint32_t m_shift = 2 * kh;
-    const pf_v2h m_mul = kh ? pf_v2h{(_Float16) 16.0f, (_Float16) 16.0f} : pf_v2h{(_Float16) 1.0f, (_Float16) 1.0f};
-    const pf_v2h m_add = kh ? pf_v2h{(_Float16) -16384.0f, (_Float16) -16384.0f} : pf_v2h{(_Float16) -1024.0f, (_Float16) -1024.0f};
-    const uint32_t lbase = pf_lds_addr(lds), wbase = pf_lds_addr(wlds) + ln * 144;
+    const uint32_t lbase = pf_lds_addr(lds) + S::ring, wbase = pf_lds_addr(wlds);
     for (int sb = 0; sb < nsb; ++sb) {
         const bool steady = sb + 2 < nsb;
         v4i P[8][2];   // the block's planes: sub-block, low and high digit
-        float d = 0.0f, ndmin = 0.0f;
-        pf_v8h mb;
+        typename W::Row w;
         pf_for_m<0, NM>([&](auto mc) {
             constexpr int m = decltype(mc)::value;
             // What this pass reads has landed once only what was issued after it is in flight: the activations of the two passes
             // behind it (at least two copies a wave each) and the weights issued in the three passes before this one; the weights
             // of a tile of one group were issued two passes ago, behind the next pass's activations.
-            constexpr int kW = PfWeights<GU>::kCopies;
             constexpr int kIssued = ((m + 4 * NM - 1) % NM == 0) + ((m + 4 * NM - 2) % NM == 0) + ((m + 4 * NM - 3) % NM == 0);
-            constexpr int kBut = NM == 1 ? 2 + kW : 4 + kW * kIssued;
+            constexpr int kBut = NM == 1 ? 2 + W::kCopies : 4 + W::kCopies * kIssued;
             if (!steady || (m == 0 && sb == 0)) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
             else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBut) : "memory");
             const uint32_t lbuf = lbase + slot * kPfSlot;
-            v4i hdr, q[4];
-            if constexpr (m == 0) {
-                const uint32_t at = wbase + (sb & 1) * kPfWStep;
-                hdr = pf_lds_i32x4<0>(at);
-                // four 16-byte pieces of the row's codes, bytes 32 c + 16 kh of its 128: the low nibbles are 16 values of
-                // sub-block 2 c, the high ones of 2 c + 1
-                q[0] = pf_lds_i32x4<16>(at + 16 * kh);
-                q[1] = pf_lds_i32x4<48>(at + 16 * kh);
-                q[2] = pf_lds_i32x4<80>(at + 16 * kh);
-                q[3] = pf_lds_i32x4<112>(at + 16 * kh);
-            }
+            if constexpr (m == 0) wts.read(w, wbase + (sb & 1) * S::w_step);
             copy_pass(std::integral_constant<int, m + 3>{}, sb, (slot + 3) & 3);
             slot = (slot + 1) & 3;
             // The two plane products of the block, int32, a matrix instruction a sub-block and plane, accumulated over the 8
@@ -547,107 +601,99 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
             xr[1] = pf_lds_i32x4<0>(xa ^ 32);
             int sum[NB ? 4 * NB : 1];
             pf_v16i part[NB ? 3 : 1];   // (sub-block sums, worked off two sub-blocks on: a matrix instruction's results take a while)
-            auto add_part = [&](int jj, const uint32_t (&sc)[2]) {
-                const int scale = (int) ((sc[jj >> 2] >> (8 * (jj & 3))) & 0x3fu);
+            auto add_part = [&](int jj) {
+                if constexpr (NB != 0) {
+                    const int scale = (int) ((w.sc[jj >> 2] >> (8 * (jj & 3))) & 0x3fu);
 #pragma unroll
-                for (int i = 0; i < 4 * NB; ++i) {
-                    sum[i] = __mul24(part[NB ? jj % 3 : 0][i], scale) + (jj ? sum[i] : 0);
-                    asm("" : "+v"(sum[i]));   // (keeps multiply and add one instruction)
-                }
-                // (the registers of rows that are not there stay taken until now: given away behind the matrix instruction, they made
-                // the next instruction wait until it had written them)
-                asm volatile("" ::"v"(part[NB ? jj % 3 : 0]));
-            };
-            uint32_t sc[2], mn[2];
-            pf_u16x2 flo[2][2], fhi[2][2];
-            if constexpr (m == 0) {
-                pf_lds_wait_row<2>(hdr, q);
-                // (the wave's weights are in registers: their LDS takes the super-block after the next one's)
-                if (steady) wts.copy(wlds + (sb & 1) * kPfWStep, sb + 2);
-                d = f16_bits_to_f32((uint16_t) (hdr[0] & 0xffff));
-                ndmin = -f16_bits_to_f32((uint16_t) ((uint32_t) hdr[0] >> 16));
-                q4k_unpack_scales((uint32_t) hdr[1], (uint32_t) hdr[2], (uint32_t) hdr[3], sc, mn);
-                // the scales' low and high digits as 16-bit pairs: [w][p] those of sub-blocks 4 w + p and 4 w + 2 + p
-#pragma unroll
-                for (int w = 0; w < 2; ++w)
-#pragma unroll
-                    for (int p = 0; p < 2; ++p) {
-                        flo[w][p] = __builtin_bit_cast(pf_u16x2, (sc[w] >> (8 * p)) & 0x00070007u);
-                        fhi[w][p] = __builtin_bit_cast(pf_u16x2, (sc[w] >> (8 * p + 3)) & 0x00070007u);
+                    for (int i = 0; i < 4 * NB; ++i) {
+                        sum[i] = __mul24(part[jj % 3][i], scale) + (jj ? sum[i] : 0);
+                        asm("" : "+v"(sum[i]));   // (keeps multiply and add one instruction)
                     }
-                // The minimums' operand: k = 0..7 pairs m_j with the sums' low digits, k = 8..15 pairs 64 m_j with their
-                // high digits.  A byte b behind 0x64 is FP16 1024 + b: m, or 4 m and 16 times that.
-#pragma unroll
-                for (int w = 0; w < 2; ++w) {
-                    const uint32_t mw = mn[w] << m_shift;
-                    const pf_v2h t0 = __builtin_elementwise_fma(pf_bytes_1024(mw, 0x04010400u), m_mul, m_add);
-                    const pf_v2h t1 = __builtin_elementwise_fma(pf_bytes_1024(mw, 0x04030402u), m_mul, m_add);
-                    mb[4 * w] = t0[0], mb[4 * w + 1] = t0[1], mb[4 * w + 2] = t1[0], mb[4 * w + 3] = t1[1];
+                    // (the registers of rows that are not there stay taken until now: given away behind the matrix instruction, they
+                    // made the next instruction wait until it had written them)
+                    asm volatile("" ::"v"(part[jj % 3]));
                 }
+            };
+            if constexpr (m == 0) {
+                wts.template wait<2>(w);
+                // (the wave's weights are in registers: their LDS takes the super-block after the next one's)
+                if (steady) wts.copy(wlds + (sb & 1) * S::w_step, sb + 2);
+                wts.open(w);
+                wts.template look<0>(w);
             }
             v4i sa;
             v4f dxr[4];
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                if (jj < 6) xr[(jj + 2) % 3] = pf_lds_i32x4<0>(xa ^ (32 * (jj + 2)));
-                if (jj == 6) {   // the closing stage's operands: the code sums, the block scales
-                    sa = pf_lds_i32x4<kPfSlotS>(lbuf + ln * 32 + kh * 16);
+            pf_for_m<0, 8>([&](auto jc) {
+                constexpr int jj = decltype(jc)::value;
+                if constexpr (m == 0 && jj < 7) wts.template look<jj + 1>(w);
+                if constexpr (jj < 6) xr[(jj + 2) % 3] = pf_lds_i32x4<0>(xa ^ (32 * (jj + 2)));
+                if constexpr (jj == 6) {   // the closing stage's operands: the code sums, the block scales
+                    if constexpr (W::kSums) sa = pf_lds_i32x4<kPfSlotS>(lbuf + ln * 32 + kh * 16);
                     const uint32_t at = lbuf + 16 * kh;
                     dxr[0] = pf_lds_f32x4<kPfSlotD>(at);
                     dxr[1] = pf_lds_f32x4<kPfSlotD + 32>(at);
                     dxr[2] = pf_lds_f32x4<kPfSlotD + 64>(at);
                     dxr[3] = pf_lds_f32x4<kPfSlotD + 96>(at);
                 }
-                if constexpr (m == 0 && NB == 0) {
-                    const int c = jj >> 1, j = jj & 1;
-                    const pf_u16x2 lo = flo[jj >> 2][j], hi = fhi[jj >> 2][j];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        // four 4-bit codes (one a byte) times a factor <= 7: no byte overflows, so one packed 16-bit multiply does it
-                        const pf_u16x2 w = __builtin_bit_cast(pf_u16x2, ((uint32_t) q[c][i] >> (4 * j)) & 0x0f0f0f0fu);
-                        P[jj][0][i] = __builtin_bit_cast(int, c & 1 ? w * lo.yy : w * lo.xx);
-                        P[jj][1][i] = __builtin_bit_cast(int, c & 1 ? w * hi.yy : w * hi.xx);
-                    }
-                }
-                // this sub-block's operand has landed once only the reads issued after it are outstanding (LDS answers in order)
-                if (jj < 6) pf_lds_wait1<2>(xr[jj % 3]);
-                else if (jj == 6) pf_lds_wait1<6>(xr[jj % 3]);
-                else pf_lds_wait1<5>(xr[jj % 3]);
+                // this sub-block's operands have landed once only the reads issued after them are outstanding (LDS answers in
+                // order): the activations of the two sub-blocks behind it, the next one's look-ups, the closing stage's
+                constexpr int kTail = 4 + (W::kSums ? 1 : 0), kNext = m == 0 && jj < 7 ? W::kLook : 0;
+                constexpr int kAfter = (jj < 6 ? 2 : jj == 6 ? 1 + kTail : kTail) + kNext - (kNext && jj == 0 ? 1 : 0);
+                if constexpr (m == 0) wts.template wait_look<kAfter>(jj, w, xr[jj % 3]);
+                else pf_lds_wait1<kAfter>(xr[jj % 3]);
                 const pf_v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
                 if constexpr (NB != 0) {
-                    v4i w;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) w[i] = (int) (((uint32_t) q[jj >> 1][i] >> (4 * (jj & 1))) & 0x0f0f0f0fu);
-                    part[jj % 3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], w, z, 0, 0, 0);
-                    if (jj > 1) add_part(jj - 2, sc);
-                    continue;
+                    part[jj % 3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], wts.codes(w, jj), z, 0, 0, 0);
+                    if (jj > 1) add_part(jj - 2);
+                } else {
+                    if constexpr (m == 0) wts.planes(w, jj, P[jj][0], P[jj][1]);
+                    dot[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], P[jj][0], jj ? dot[0] : z, 0, 0, 0);
+                    dot[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], P[jj][1], jj ? dot[1] : z, 0, 0, 0);
                 }
-                dot[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], P[jj][0], jj ? dot[0] : z, 0, 0, 0);
-                dot[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xr[jj % 3], P[jj][1], jj ? dot[1] : z, 0, 0, 0);
-            }
-            // The minimums' integer term sum_j m_j (sum of sub-block j's codes), exactly, from one FP16 matrix instruction
-            // (every operand and every partial sum an integer below 2^24); then once a block lo + 8 hi = the block's
-            // integer sum (< 2^25) and d_x (d_w sum - dmin_w minimums)
-            pf_lds_wait_tail<0>(sa, dxr);
-            const pf_v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            const pf_v16f mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_v8h, sa), mb, z, 0, 0, 0);
-            if constexpr (NB != 0) add_part(6, sc), add_part(7, sc);
+            });
+            // Once a block lo + 8 hi = the block's integer sum (< 2^25) and d_x (d_w sum - dmin_w minimums); the minimums' integer term
+            // sum_j m_j (sum of sub-block j's codes) comes, exactly, from one FP16 matrix instruction (every operand and every
+            // partial sum an integer below 2^24).
             // (a lane's outputs 4 b .. 4 b + 3 are the tile's rows 32 m + 8 b + 4 kh + 0..3: blocks of 8 rows past the
             // tile's last row are skipped - most tiles of a skewed routing hold 8 rows or fewer)
             const int nb = m == NM - 1 ? (nrows - 32 * m + 7) >> 3 : 4;
+            if constexpr (W::kSums) {
+                pf_lds_wait_tail<0>(sa, dxr);
+                const pf_v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                const pf_v16f mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_v8h, sa), w.mb, z, 0, 0, 0);
+                if constexpr (NB != 0) add_part(6), add_part(7);
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                if (NB ? b < NB : m < NM - 1 || b < nb) {
+                for (int b = 0; b < 4; ++b) {
+                    if (NB ? b < NB : m < NM - 1 || b < nb) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int i = 4 * b + r;
-                        const float t = fmaf(ndmin, mins[i], __fmul_rn(d, (float) (NB ? sum[NB ? i : 0] : dot[0][i] + 8 * dot[1][i])));
-                        acc[m][i] = fmaf(dxr[b][r], t, acc[m][i]);
+                        for (int r = 0; r < 4; ++r) {
+                            const int i = 4 * b + r;
+                            const float t = fmaf(w.ndmin, mins[i], __fmul_rn(w.d, (float) (NB ? sum[NB ? i : 0] : dot[0][i] + W::kHiFactor * dot[1][i])));
+                            acc[m][i] = fmaf(dxr[b][r], t, acc[m][i]);
+                        }
+                    }
+                }
+            } else {
+                pf_lds_wait_tail<0>(dxr);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    if (m < NM - 1 || b < nb) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int i = 4 * b + r;
+                            acc[m][i] = fmaf(__fmul_rn(dxr[b][r], w.d), (float) (dot[0][i] + W::kHiFactor * dot[1][i]), acc[m][i]);
+                        }
                     }
                 }
             }
             asm volatile("" : "+v"(acc[m]));   // (here, not when the block's other passes are done: that would keep every pass's sums)
         });
+    }
+    if constexpr (!W::kSums) {
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[m][i] = __fmul_rn(acc[m][i], W::kOutFactor);
     }
     // outputs: lane (ln, kh) holds weight row ln for the tile's rows 32 m + 8 b + 4 kh + r (i = 4 b + r)
     pf_for_m<0, NM>([&](auto mc) {
@@ -676,24 +722,34 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
     });
 }
 
+// The workgroup's rows: the tile and, of the same expert, the next one.  False where there are none: past the last tile, or the
+// workgroup of the tile before takes them.
+struct PfTile { int ex, row0, nrows; };
+__device__ __forceinline__ bool pf_my_tile(const PfGemm& a, PfTile& t) {
+    const int tile = blockIdx.y;
+    if (tile >= *a.plan.n_tiles) return false;
+    t.ex = a.plan.tile_expert[tile], t.row0 = a.plan.tile_row0[tile];
+    if ((t.row0 - a.plan.bounds[t.ex]) % (32 * kPfGroups) != 0) return false;
+    t.nrows = min(32 * kPfGroups, a.plan.bounds[t.ex + 1] - t.row0);
+    return true;
+}
+
 #include "maya_prefill_iq2s.hpp"
 
 // grid (bands of weight rows, tiles at most)
 template <bool GU>
 __global__ __launch_bounds__(256, 2) void prefill_q4k_kernel(PfGemm a) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kPfLdsBytes];
-    const int tile = blockIdx.y;
-    if (tile >= *a.plan.n_tiles) return;
-    const int ex = a.plan.tile_expert[tile], row0 = a.plan.tile_row0[tile], first = a.plan.bounds[ex];
-    if ((row0 - first) % (32 * kPfGroups) != 0) return;   // (the workgroup of the tile before takes this one too)
-    const int nrows = min(32 * kPfGroups, a.plan.bounds[ex + 1] - row0);
-    if (nrows <= 8) pf_tile<GU, 1, 1>(a, lds, ex, row0, nrows);
-    else if (nrows <= 16) pf_tile<GU, 1, 2>(a, lds, ex, row0, nrows);
-    else if (nrows <= 24) pf_tile<GU, 1, 3>(a, lds, ex, row0, nrows);
-    else if (nrows <= 32) pf_tile<GU, 1>(a, lds, ex, row0, nrows);
-    else if (nrows <= 64) pf_tile<GU, 2>(a, lds, ex, row0, nrows);
-    else if (nrows <= 96) pf_tile<GU, 3>(a, lds, ex, row0, nrows);
-    else pf_tile<GU, 4>(a, lds, ex, row0, nrows);
+    typedef PfQ4K<GU> W;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[PfLds<W>::bytes];
+    PfTile t;
+    if (!pf_my_tile(a, t)) return;
+    if (t.nrows <= 8) pf_tile<W, GU, 1, 1>(a, lds, t.ex, t.row0, t.nrows);
+    else if (t.nrows <= 16) pf_tile<W, GU, 1, 2>(a, lds, t.ex, t.row0, t.nrows);
+    else if (t.nrows <= 24) pf_tile<W, GU, 1, 3>(a, lds, t.ex, t.row0, t.nrows);
+    else if (t.nrows <= 32) pf_tile<W, GU, 1>(a, lds, t.ex, t.row0, t.nrows);
+    else if (t.nrows <= 64) pf_tile<W, GU, 2>(a, lds, t.ex, t.row0, t.nrows);
+    else if (t.nrows <= 96) pf_tile<W, GU, 3>(a, lds, t.ex, t.row0, t.nrows);
+    else pf_tile<W, GU, 4>(a, lds, t.ex, t.row0, t.nrows);
 }
 
 template <int ODT>

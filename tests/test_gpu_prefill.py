@@ -194,22 +194,25 @@ def test_stages_and_layer_match_checker(pf, oracle, case):
 EDGE_ROWS = [1, 7, 8, 9, 16, 17, 24, 25, 32, 33, 64, 65, 96, 97, 127, 128, 129, 160, 256, 257]
 
 
-@pytest.mark.parametrize("n_embd, n_ff", [(256, 512), (512, 256), (768, 768), (1536, 256)], ids=str)
-def test_experts_of_every_number_of_row_groups(pf, oracle, n_embd, n_ff):
-    """Experts of EDGE_ROWS rows each in one chunk - both sides of a block of 8 rows, of a row group, of a workgroup's rows - with 1, 2,
-    3 and 6 super-blocks a row, fewer and more than run ahead: h and the down rows against the CPU path's row dots.  The integer sums
+@pytest.mark.parametrize("t, n_embd, n_ff", [(Q4_K, 256, 512), (Q4_K, 512, 256), (Q4_K, 768, 768), (Q4_K, 1536, 256),
+                                             (22, 512, 1024), (22, 1536, 512)], ids=str)
+def test_experts_of_every_number_of_row_groups(pf, oracle, t, n_embd, n_ff):
+    """Experts of EDGE_ROWS rows each in one chunk - both sides of a block of 8 rows, of a row group, of a workgroup's rows - with 1 to 6
+    super-blocks a row, fewer and more than run ahead: h and the down rows against the CPU path's row dots.  The integer sums
     are the same and the F32 ones of at most 6 blocks differ by order: 1e-5."""
     from maya_amd import lib
     import synth
     ne = len(EDGE_ROWS)
-    blobs = make_blobs(oracle, ne, n_embd, n_ff, 3 * n_embd + n_ff)
-    up_off, down_off, _ = synth.blob_offsets(Q4_K, Q4_K, n_embd, n_ff)
+    gen = np.random.default_rng(3 * n_embd + n_ff)
+    blobs = make_blobs(oracle, ne, n_embd, n_ff, 3 * n_embd + n_ff) if t == Q4_K else [synth.expert_blob(t, t, n_embd, n_ff, gen) for _ in range(ne)]
+    up_off, down_off, _ = synth.blob_offsets(t, t, n_embd, n_ff)
     rng = np.random.default_rng(n_embd)
     ids = np.repeat(np.arange(ne, dtype=np.int32), EDGE_ROWS)
     rng.shuffle(ids)
     x = rng.standard_normal((ids.size, n_embd)).astype(np.float32)
-    layout, _ = lib.layout(Q4_K, Q4_K, n_embd, n_ff)
-    table = lib.ExpertStore(blobs)
+    layout, _ = lib.layout(t, t, n_embd, n_ff)
+    table = lib.ExpertStore(blobs, pack_layout=layout)
+    layout = lib.copy_layout(layout, lib.PACK_STREAM)
     p = pf.plan(dev(ids), table.table)
     hq = pf.gate_up(layout, table.table, p, pf.quant(dev(x), p, 1))
     part = pf.down(layout, table.table, p, hq)
@@ -223,11 +226,11 @@ def test_experts_of_every_number_of_row_groups(pf, oracle, n_embd, n_ff):
             row = int(first[e]) + r
             tok = int(row_entry[row])
             assert ids[tok] == e
-            a = oracle.quant_act(Q4_K, x[tok])
-            g, u = oracle.rows(Q4_K, blobs[e], n_embd, n_ff, a), oracle.rows(Q4_K, blobs[e][up_off:], n_embd, n_ff, a)
+            a = oracle.quant_act(t, x[tok])
+            g, u = oracle.rows(t, blobs[e], n_embd, n_ff, a), oracle.rows(t, blobs[e][up_off:], n_embd, n_ff, a)
             want = [oracle.lib().mo_swiglu(float(gv), float(uv), float("inf")) for gv, uv in zip(g, u)]
             assert rel_l2(h[row], np.array(want, dtype=np.float32)) <= 1e-5, (EDGE_ROWS[e], r)
-            want = oracle.rows(Q4_K, blobs[e][down_off:], n_ff, n_embd, oracle.quant_act(Q4_K, h[row]))
+            want = oracle.rows(t, blobs[e][down_off:], n_ff, n_embd, oracle.quant_act(t, h[row]))
             assert rel_l2(part[row], want) <= 1e-5, (EDGE_ROWS[e], r)
 
 
