@@ -158,61 +158,99 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
     }
 }
 
-// ---- down + combine, n_ff = 32 nu <= 2048 (nu positions a row on the first nu lanes of one wave, the lanes past them idle):
-// wave w = slot w of token blockIdx.y, of at most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a
-// rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.
+// The sums over a 32-lane half of four values a lane: row (lane >> 3) & 3's in every lane, by the pairs of lanes reduce8_half takes.
+__device__ __forceinline__ float reduce4_half(const float (&acc)[4], int lane) {
+    const bool b4 = lane & 16, b3 = lane & 8;
+    float v2[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float send = b4 ? acc[i] : acc[i + 2], keep = b4 ? acc[i + 2] : acc[i];
+        v2[i] = keep + xor_lane<16>(send);
+    }
+    const float send = b3 ? v2[0] : v2[1], keep = b3 ? v2[1] : v2[0];
+    float v = keep + xor_lane<8>(send);
+    v += xor_lane<4>(v);
+    v += xor_lane<2>(v);
+    v += xor_lane<1>(v);
+    return v;
+}
+
+// ---- down + combine, n_ff = 32 nu <= 2048 (nu positions a row, lanes past them idle): wave w = slot w of token blockIdx.y, of at
+// most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h
+// to Q8_K itself.
+// PAIR (nu <= 32): a wave takes two rows at a time, one on either half of its lanes - rows r .. r + 3 of a batch below, r + 4 ..
+// r + 7 above - instead of leaving half of them without a position.
 // AHEAD: all ROWS rows of the wave are requested before anything else is done (one or two slots on one token: a few
 // hundred waves on the whole chip, each with one row in flight, run at the memory's latency a row).
-template <int ROWS, int MINW, int SLOTS, int NU, bool AHEAD = false>
-__global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(maya_moe_args a) {
+// The leading arguments repeat fields of `a`: they arrive in scalar registers with the dispatch (down_iq2s_pos_kernel).  What
+// the kernel asks of memory first - the plan, the combine's weights, h - goes out side by side; it used to wait for the plan
+// before h, and the combine read plan and weights slot by slot at the end.
+// Measured: 2048 x 768 top-8, one token, 8.1 -> 4.6 us a launch (sixteen layers in a graph 249 -> 196 us); 7168 x 2048 top-1 5.5 -> 5.0.
+template <int ROWS, int MINW, int SLOTS, int NU, bool AHEAD = false, bool PAIR = false>
+__global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(const uint64_t* __restrict__ plan_ptr, const float* __restrict__ plan_w,
+                                                                  const float* __restrict__ h, const int32_t* __restrict__ skip,
+                                                                  const int8_t* __restrict__ hq_q, int k, int n_embd, int n_pos, maya_moe_args a) {
     static_assert(ROWS % 8 == 0, "rows come in batches of 8");
     static_assert(!AHEAD || ROWS == 8, "every row up front: one batch");
+    static_assert(!PAIR || NU == 0, "two rows a wave: at most 32 positions");
+    constexpr int NB = PAIR ? 4 : 8;   // row steps of a batch
     __shared__ float part[SLOTS][ROWS];
-    if (a.skip && *a.skip) return;
-    const int n_embd = a.layout.n_embd, nu = NU ? NU : a.layout.n_ff >> 5;
+    __shared__ float s_w[SLOTS];
+    __shared__ int s_on[SLOTS];
+    const int nu = NU ? NU : n_pos;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int bx, by;
     down_block_of_grid(bx, by);
     const int r0 = bx * ROWS;
-    const int e0 = by * a.k, ent = e0 + wave;
-    const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
-    if (blob != 0ull) {
-        // (an idle lane's weights read as zero, and so do its activations)
-        const bool on = NU == 64 || lane < nu;
-        const int pos = on ? lane : nu - 1;
-        PosQ4K p;
-        const uint32_t rb = (uint32_t) nu * 18u;   // bytes of a row: 144 a block
-        pos_q4k_init(p, pos, 0u, on, (uint32_t) n_embd * rb);
-        // the first row's weights are requested before h is rounded: their latency hides behind that arithmetic
-        const uint64_t mat = blob + a.layout.down_off;
-        const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
-        const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
-        const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) n_embd * rb);
-        u32x4 hn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, (uint32_t) r0 * rb, 0);
-        u32x4 qn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_q, (uint32_t) r0 * rb, 0);
-        u32x4 ha[AHEAD ? ROWS : 1], qa[AHEAD ? ROWS : 1];
-        if constexpr (AHEAD) {
+    const int e0 = by * k, ent = e0 + wave;   // (64 k threads: every wave has a slot)
+    const int skipv = skip ? *skip : 0;
+    const uint64_t blob = plan_ptr[ent];      // (asked for first: the weights' request waits for this one)
+    const int ci = e0 + min((int) threadIdx.x & (SLOTS - 1), k - 1);
+    const uint64_t c_ptr = plan_ptr[ci];
+    const float c_w = plan_w[ci];
+    // (an idle lane's weights read as zero, and so do its activations)
+    const int at = PAIR ? lane & 31 : lane;
+    const bool on = NU == 64 || at < nu;
+    const int pos = on ? at : nu - 1;
+    PosQ4K p;
+    // Q8_K of h in registers (quant_q8k_block's arithmetic): the lane's 32 values are two runs of 16, a block is 8 lanes; the
+    // block's signed maximum is the value at the FIRST largest magnitude, so candidates carry their index
+    const int piece = pos & 7, j = piece >> 1, half = piece & 1;
+    const bool rounded = hq_q != nullptr;
+    float v[32];
+    if (rounded) {
+        pos_q4k_codes(p, pos, hq_q + (size_t) ent * (32 * nu), a.hq.d + (size_t) ent * nu, a.hq.bsums + (size_t) ent * (2 * nu));
+    } else {
+        const float* hrow = h + (size_t) ent * (32 * nu) + 256 * (pos >> 3) + 64 * j + 16 * half;
 #pragma unroll
-            for (int i = 1; i < ROWS; ++i) {
-                ha[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, (uint32_t) (r0 + i) * rb, 0);
-                qa[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_q, (uint32_t) (r0 + i) * rb, 0);
-            }
+        for (int i = 0; i < 4; ++i) {
+            const float4 lo = *(const float4*) (hrow + 4 * i), hi = *(const float4*) (hrow + 32 + 4 * i);
+            v[4 * i] = lo.x, v[4 * i + 1] = lo.y, v[4 * i + 2] = lo.z, v[4 * i + 3] = lo.w;
+            v[16 + 4 * i] = hi.x, v[16 + 4 * i + 1] = hi.y, v[16 + 4 * i + 2] = hi.z, v[16 + 4 * i + 3] = hi.w;
         }
-        if (a.hq.q) {
-            pos_q4k_codes(p, pos, a.hq.q + (size_t) ent * (32 * nu), a.hq.d + (size_t) ent * nu, a.hq.bsums + (size_t) ent * (2 * nu));
-        } else {
-            // Q8_K of h in registers (quant_q8k_block's arithmetic): the lane's 32 values are two runs of 16, a block is
-            // 8 lanes; the block's signed maximum is the value at the FIRST largest magnitude, so candidates carry their index
-            const int piece = pos & 7, j = piece >> 1, half = piece & 1;
-            const int v0 = 256 * (pos >> 3) + 64 * j + 16 * half;
-            const float* hrow = a.h + (size_t) ent * (32 * nu);
-            float v[32];
+    }
+    if (skipv) return;
+    const uint32_t rb = (uint32_t) nu * 18u, past = (uint32_t) n_embd * rb;   // bytes of a row: 144 a block
+    pos_q4k_init(p, pos, PAIR ? (uint32_t) (lane >> 5) * 4u * rb : 0u, on, past);
+    // the first rows' weights are requested before h is rounded: their latency hides behind that arithmetic
+    // (no blob: an empty resource, whose loads read as zero and touch nothing)
+    const uint64_t mat = blob ? blob + a.layout.down_off : 0ull;
+    const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
+    const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (mat_lo | mat_hi) != 0u ? past : 0u);
+    constexpr int DEPTH = AHEAD ? NB : 1;
+    u32x4 hd[DEPTH], qd[DEPTH];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 lo = *(const float4*) (hrow + v0 + 4 * i), hi = *(const float4*) (hrow + v0 + 32 + 4 * i);
-                v[4 * i] = lo.x, v[4 * i + 1] = lo.y, v[4 * i + 2] = lo.z, v[4 * i + 3] = lo.w;
-                v[16 + 4 * i] = hi.x, v[16 + 4 * i + 1] = hi.y, v[16 + 4 * i + 2] = hi.z, v[16 + 4 * i + 3] = hi.w;
-            }
+    for (int i = 0; i < DEPTH; ++i) {
+        hd[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, (uint32_t) (r0 + i) * rb, 0);
+        qd[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_q, (uint32_t) (r0 + i) * rb, 0);
+    }
+    if (threadIdx.x < SLOTS) {
+        s_on[threadIdx.x] = (int) threadIdx.x < k && c_ptr != 0ull;
+        s_w[threadIdx.x] = c_w;
+    }
+    if (blob != 0ull) {
+        if (!rounded) {
             if (!on) {
 #pragma unroll
                 for (int i = 0; i < 32; ++i) v[i] = 0.0f;
@@ -227,33 +265,27 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(maya_moe
             p.shi = dot4(0x01010101, p.yhi[0], dot4(0x01010101, p.yhi[1], dot4(0x01010101, p.yhi[2], dot4(0x01010101, p.yhi[3], 0))));
         }
         pos_q4k_idle(p, on);
-        float acc[8];
-        if constexpr (AHEAD) {
-            ha[0] = hn, qa[0] = qn;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                acc[i] = pos_q4k_value(p, ha[i], qa[i]);
-                asm volatile("" : "+v"(acc[i]));
-            }
-            float v = reduce8_half(acc, lane);
-            v = add_other_half(v);
-            if ((lane & 35) == 0) part[wave][(lane >> 2) & 7] = v;
-        } else
 #pragma unroll 1
         for (int r = 0; r < ROWS; r += 8) {
+            float acc[NB];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const u32x4 hc = hn, qc = qn;
-                if (r + i + 1 < ROWS) {
-                    hn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, (uint32_t) (r0 + r + i + 1) * rb, 0);
-                    qn = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_q, (uint32_t) (r0 + r + i + 1) * rb, 0);
+            for (int i = 0; i < NB; ++i) {
+                const u32x4 hc = hd[i % DEPTH], qc = qd[i % DEPTH];
+                if (!AHEAD && (i + 1 < NB || r + 8 < ROWS)) {   // (the next step's rows, or the next batch's first)
+                    const uint32_t next = (uint32_t) (r0 + r + (i + 1 < NB ? i + 1 : 8)) * rb;
+                    hd[0] = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_hdr, next, 0);
+                    qd[0] = __builtin_amdgcn_raw_buffer_load_b128(rs, p.o_q, next, 0);
                 }
                 acc[i] = pos_q4k_value(p, hc, qc);
                 asm volatile("" : "+v"(acc[i]));
             }
-            float v = reduce8_half(acc, lane);
-            v = add_other_half(v);
-            if ((lane & 35) == 0) part[wave][r + ((lane >> 2) & 7)] = v;
+            if constexpr (PAIR) {
+                const float s = reduce4_half(acc, lane);
+                if ((lane & 7) == 0) part[wave][r + 4 * (lane >> 5) + ((lane >> 3) & 3)] = s;
+            } else {
+                const float s = add_other_half(reduce8_half(acc, lane));
+                if ((lane & 35) == 0) part[wave][r + ((lane >> 2) & 7)] = s;
+            }
         }
     }
     __syncthreads();
@@ -261,19 +293,21 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(maya_moe
         const int c = threadIdx.x;
         float sum = 0.0f;
         bool first = true;
-        for (int i = 0; i < a.k; ++i) {
-            if (a.plan_ptr[e0 + i] == 0ull) continue;
-            const float pv = __fmul_rn(part[i][c], a.plan_w[e0 + i]);
-            sum = first ? pv : __fadd_rn(sum, pv);
-            first = false;
+#pragma unroll
+        for (int i = 0; i < SLOTS; ++i) {   // the present slots in slot order; the first product starts the sum
+            const bool have = s_on[i] != 0;
+            const float pv = __fmul_rn(part[i][c], s_w[i]);
+            const float t = first ? pv : __fadd_rn(sum, pv);
+            sum = have ? t : sum;
+            first = first && !have;
         }
         const size_t o = (size_t) by * n_embd + r0 + c;
         if (a.add && (!a.add_flag || *a.add_flag)) sum = __fadd_rn(sum, a.add[o]);
         if (a.add2) sum = __fadd_rn(sum, a.add2[o]);
         a.out[o] = sum;
         if (a.part)
-            for (int i = 0; i < a.k; ++i)
-                if (a.plan_ptr[e0 + i] != 0ull) a.part[(size_t) (e0 + i) * n_embd + r0 + c] = part[i][c];
+            for (int i = 0; i < k; ++i)
+                if (s_on[i]) a.part[(size_t) (e0 + i) * n_embd + r0 + c] = part[i][c];
     }
 }
 

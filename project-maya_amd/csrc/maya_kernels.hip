@@ -1761,14 +1761,20 @@ int launch_down_q4k_pos(const maya_moe_args& a, hipStream_t s) {
                      : (long long) (n_embd / 16) * a.n_tokens < (a.k <= 2 ? 1024 : 256) && n_embd % 8 == 0 ? 8 : 16;
     const dim3 grid((unsigned) (n_embd / rows), (unsigned) a.n_tokens), block(64u * (unsigned) a.k);
     const bool full = a.layout.n_ff == 2048;
-#define MAYA_ROWS(R, MINW, AHEAD)                                                                                              \
-    if (a.k <= 8 && full) hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, 8, 64, AHEAD>), grid, block, 0, s, a);               \
-    else if (a.k <= 8) hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, 8, 0, AHEAD>), grid, block, 0, s, a);                   \
-    else hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, 16, 0, AHEAD>), grid, block, 0, s, a);
+    const bool pair = a.layout.n_ff <= 1024;
+#define MAYA_DOWN(R, MINW, SLOTS, NU, AHEAD, PAIR) \
+    hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, SLOTS, NU, AHEAD, PAIR>), grid, block, 0, s, a.plan_ptr, a.plan_w, a.h, a.skip, a.hq.q, a.k, n_embd, a.layout.n_ff >> 5, a);
+#define MAYA_ROWS(R, MINW, AHEAD)                                    \
+    if (a.k <= 8 && full) { MAYA_DOWN(R, MINW, 8, 64, AHEAD, false) } \
+    else if (a.k <= 8 && pair) { MAYA_DOWN(R, MINW, 8, 0, AHEAD, true) } \
+    else if (a.k <= 8) { MAYA_DOWN(R, MINW, 8, 0, AHEAD, false) }     \
+    else if (pair) { MAYA_DOWN(R, MINW, 16, 0, AHEAD, true) }         \
+    else { MAYA_DOWN(R, MINW, 16, 0, AHEAD, false) }
     if (rows == 32) { MAYA_ROWS(32, 8, false) }
     else if (rows == 8) { MAYA_ROWS(8, 4, true) }   // (128 registers)
     else { MAYA_ROWS(16, 8, false) }
 #undef MAYA_ROWS
+#undef MAYA_DOWN
     MAYA_LAUNCHED("down_q4k_pos_kernel");
     return MAYA_OK;
 }
