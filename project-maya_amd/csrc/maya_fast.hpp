@@ -502,6 +502,14 @@ struct LayerHeadIn {
     int n_expert, x_dtype, sigmoid;
     LayerHead out;
 };
+// What such a launch asks of memory first, as plain pointers and integers at the head of its arguments (they arrive in scalar
+// registers with the dispatch; a structure passed by value is read from memory first): the fields of LayerHeadIn, a.skip, a.k
+// and, in `mode`, x's dtype, the sigmoid router's bit 8 and n_embd / 32 from bit 16 on.
+#define MAYA_HEAD_PARAMS                                                                                                              \
+    const float *__restrict__ logits, const uint64_t *__restrict__ table, const void *__restrict__ x, const float *__restrict__ bias, \
+        const int32_t *__restrict__ skip, int n_expert, int mode, int n_ent
+#define MAYA_HEAD_ARGS(hd, a)                                                                                   \
+    hd.logits, hd.table, hd.x, hd.bias, a.skip, hd.n_expert, hd.x_dtype | (hd.sigmoid ? 256 : 0) | (a.layout.n_embd >> 5) << 16, a.k
 // The head of a one-token layer inside a gate/up launch whose workgroups are a (gate row, up row) pair's 2 * 32 NW
 // positions, grid (row blocks + 1, k): called by every thread once.  The workgroup (last column, 0) is the exact router
 // (ids, weights, plan: hd.out); the rest of that column leaves.  Every other workgroup picks the experts on its last

@@ -86,14 +86,14 @@ __device__ __forceinline__ int sum32_codes(const int (&y)[8]) {
 // grid (n_ff / ROWS, entries); entry e = token e / k, slot e % k.  Rows in batches of 8 (two quads), a quad ahead.
 // HEAD (one token): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k).
 template <int NW, int ROWS, int MINW, bool FIT, bool HEAD = false>
-__global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(maya_moe_args a, Codebooks cb, LayerHeadIn hd) {
+__global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(MAYA_HEAD_PARAMS, maya_moe_args a, Codebooks cb, LayerHead out) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
     constexpr int NU = 32 * NW;
     __shared__ __align__(16) int lds[kFast1LdsWords];
     __shared__ float part[2][2 * NW][8];
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
+    const int nu = FIT ? NU : mode >> 16, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
     const bool on = FIT || lu < nu;
     const int u = on ? lu : nu - 1;
     const int e = blockIdx.y;
@@ -102,10 +102,11 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(maya_mo
     float dy8;
     if constexpr (HEAD) {
         float d;
-        if (!head_in_gate_up<NW>(hd, a.k, a.skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob)) return;
+        const LayerHeadIn hd = {logits, table, x, bias, n_expert, mode & 255, (mode >> 8) & 1, out};
+        if (!head_in_gate_up<NW>(hd, n_ent, skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob)) return;
         dy8 = d * 0.125f;
     } else {
-        if (a.skip && *a.skip) return;
+        if (skip && *skip) return;
         blob = a.plan_ptr[e];
         if (blob == 0ull) return;
         const int tok = e / a.k;

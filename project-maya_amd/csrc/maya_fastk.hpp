@@ -72,15 +72,16 @@ __device__ __forceinline__ float pos_q4k_value(const PosQ4K& p, const u32x4 hdr,
 // AHEAD (8 rows): all of a lane's rows are requested up front - the launches of a few entries, whose workgroups do not fill
 // the chip and would otherwise run at the memory's latency a row.
 // HEAD (one token): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k).
+// The leading arguments (MAYA_HEAD_ARGS) are what it asks of memory first, in scalar registers with the dispatch.
 template <int NW, int ROWS, int MINW, bool FIT, bool AHEAD = false, bool HEAD = false>
-__global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe_args a, LayerHeadIn hd) {
+__global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(MAYA_HEAD_PARAMS, maya_moe_args a, LayerHead out) {
     static_assert(ROWS % 8 == 0, "rows come in batches of 8");
     static_assert(!AHEAD || ROWS == 8, "every row up front: one batch");
     constexpr int NU = 32 * NW;
     __shared__ float part[2][2 * NW][8];
     const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
     const bool is_up = t >= NU;
-    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // positions a row; the lane's among 32 NW
+    const int nu = FIT ? NU : mode >> 16, lu = is_up ? t - NU : t;   // positions a row; the lane's among 32 NW
     const bool on = FIT || lu < nu;
     const int u = on ? lu : nu - 1;
     PosQ4K p;
@@ -94,14 +95,15 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(maya_moe
         int y[8];
         float d;
         e = (int) blockIdx.y;
-        if (!head_in_gate_up<NW>(hd, a.k, a.skip, is_up, on, lu, v0, v0 + 32, y, d, blob)) return;
+        const LayerHeadIn hd = {logits, table, x, bias, n_expert, mode & 255, (mode >> 8) & 1, out};
+        if (!head_in_gate_up<NW>(hd, n_ent, skip, is_up, on, lu, v0, v0 + 32, y, d, blob)) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i) p.ylo[i] = y[i], p.yhi[i] = y[4 + i];
         p.dx = d;
         p.slo = dot4(0x01010101, p.ylo[0], dot4(0x01010101, p.ylo[1], dot4(0x01010101, p.ylo[2], dot4(0x01010101, p.ylo[3], 0))));
         p.shi = dot4(0x01010101, p.yhi[0], dot4(0x01010101, p.yhi[1], dot4(0x01010101, p.yhi[2], dot4(0x01010101, p.yhi[3], 0))));
     } else {
-        if (a.skip && *a.skip) return;
+        if (skip && *skip) return;
         // (a window's entries in the order of grp_ent where one is given: the entries of an expert side by side; -1 ends it)
         e = (a.grp_ent && !a.grp_ptr) ? a.grp_ent[blockIdx.y] : (int) blockIdx.y;
         if (e < 0) return;

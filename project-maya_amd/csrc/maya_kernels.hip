@@ -1655,10 +1655,10 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_IQ1(NWV)                                                                                                          \
-    if (hd && fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);  \
-    else if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);   \
-    else if (fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);         \
-    else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, false>), grid, dim3(64 * NWV), 0, s, a, st.cb, h);
+    if (hd && fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
+    else if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);   \
+    else if (fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);         \
+    else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, false>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);
     switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_IQ1(2) break;
         case 3: MAYA_IQ1(3) break;
@@ -1731,10 +1731,10 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_Q4F(NWV, F)                                                                                                    \
-    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, true>), grid, dim3(64 * NWV), 0, s, a, h);   \
-    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, true>), grid, dim3(64 * NWV), 0, s, a, h);     \
-    else if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, a, h);          \
-    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8, F>), grid, dim3(64 * NWV), 0, s, a, h);
+    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);   \
+    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);     \
+    else if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);          \
+    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8, F>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
 #define MAYA_Q4(NWV)                         \
     if (fit) { MAYA_Q4F(NWV, true) }        \
     else { MAYA_Q4F(NWV, false) }
