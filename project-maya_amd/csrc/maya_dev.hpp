@@ -174,6 +174,53 @@ __device__ __forceinline__ void q8k_round_lane32(const float (&v)[32], IndexOf i
     }
 }
 
+// One activation, and 32 of them in a row (16 bytes a load where they are aligned; `on` false: zeros), as floats
+template <int DT> __device__ __forceinline__ float act_load(const void* x, int64_t i) {
+    if constexpr (DT == MAYA_DT_F32) return ((const float*) x)[i];
+    else if constexpr (DT == MAYA_DT_BF16) return __uint_as_float((uint32_t) ((const uint16_t*) x)[i] << 16);
+    else return f16_bits_to_f32(((const uint16_t*) x)[i]);
+}
+template <int DT>
+__device__ __forceinline__ void act_load32(const void* x, int64_t i0, bool on, float (&v)[32]) {
+    if (!on) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) v[i] = 0.0f;
+        return;
+    }
+    if constexpr (DT == MAYA_DT_F32) {
+        const float* p = (const float*) x + i0;
+        if (((uintptr_t) p & 15) == 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float4 t = ((const float4*) p)[i];
+                v[4 * i] = t.x, v[4 * i + 1] = t.y, v[4 * i + 2] = t.z, v[4 * i + 3] = t.w;
+            }
+            return;
+        }
+    } else {
+        const uint16_t* p = (const uint16_t*) x + i0;
+        if (((uintptr_t) p & 15) == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint4 t = ((const uint4*) p)[i];
+                const uint32_t w[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (DT == MAYA_DT_BF16) {
+                        v[8 * i + 2 * j] = __uint_as_float(w[j] << 16);
+                        v[8 * i + 2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+                    } else {
+                        v[8 * i + 2 * j] = f16_bits_to_f32(w[j] & 0xffffu);
+                        v[8 * i + 2 * j + 1] = f16_bits_to_f32(w[j] >> 16);
+                    }
+                }
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i] = act_load<DT>(x, i0 + i);
+}
 // A table of NWORDS 32-bit words from global memory into LDS by a workgroup of NT threads, in 16-byte pieces: every
 // piece a thread moves is REQUESTED before the first one is stored, so the table costs one trip to memory.  (Written as
 // a loop "lds[i] = src[i]; i += NT" the compiler waits for each load before it issues the next: one trip a pass, five

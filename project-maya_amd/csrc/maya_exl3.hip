@@ -1067,7 +1067,7 @@ int maya_exl3_layer_decode(const maya_exl3_layout* l, const uint64_t* expert_tab
     // 6144 x 1536 at 4 bits 50.2 -> 46.3 us, 4096 x 1280 34.8 -> 31.8, 2048 x 768 23.0 -> 19.1)
     const bool head = logits && n_tokens == 1 && sl.gu != 0 && n_expert <= 256 && k < n_expert;
     if (head) {
-    } else if (logits && n_tokens > 1 && n_tokens <= 4 && maya_moe_route_window_ok(nullptr, n_tokens, n_expert, k)) {   // a window of up to four tokens (one pass of the routing workgroup): route, plan and group in one launch
+    } else if (logits && n_tokens > 1 && maya_moe_route_window_ok(nullptr, n_tokens, n_expert, k)) {   // route, plan and group in one launch
         if ((rc = maya_moe_route_window(nullptr, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start,
                                         w.grp_ent, w.n_groups, stream)))
             return rc;

@@ -873,9 +873,14 @@ __device__ __forceinline__ void group_entries(GroupLds& g, int n, uint64_t* __re
         const uint64_t ptr = e < n ? g.ptr[e] : 0ull;
         const uint32_t plo = (uint32_t) ptr, phi = (uint32_t) (ptr >> 32);
         unsigned long long same = 0ull;
-        for (int f = 0; f < n; ++f) {
-            const uint32_t flo = (uint32_t) __builtin_amdgcn_readlane((int) plo, f), fhi = (uint32_t) __builtin_amdgcn_readlane((int) phi, f);
-            if (flo == plo && fhi == phi) same |= 1ull << f;
+        for (int f0 = 0; f0 < n; f0 += 8) {   // (lanes past the entries hold no blob: they are alike among themselves alone)
+            uint32_t flo[8], fhi[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) flo[j] = (uint32_t) __builtin_amdgcn_readlane((int) plo, f0 + j), fhi[j] = (uint32_t) __builtin_amdgcn_readlane((int) phi, f0 + j);
+            uint32_t m = 0u;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m |= flo[j] == plo && fhi[j] == phi ? 1u << j : 0u;
+            same |= (unsigned long long) m << f0;
         }
         const bool valid = ptr != 0ull;
         if (!valid) same = 0ull;
@@ -885,11 +890,16 @@ __device__ __forceinline__ void group_entries(GroupLds& g, int n, uint64_t* __re
         const unsigned long long leaders = __ballot(leader == e);
         const int gi = valid ? __popcll(leaders & ((1ull << leader) - 1ull)) : -1;
         const int ng = __popcll(leaders);
-        int start = 0;
-        for (int f = 0; f < n; ++f) {
-            const int lf = __builtin_amdgcn_readlane(leader, f);
-            start += (lf >= 0 && lf < leader) ? 1 : 0;
-        }
+        // the entries of the groups before a lane's own: the leaders' group sizes, summed over the lanes up to its leader
+        int sum = leader == e ? __popcll(same) : 0;
+        const int size = sum;
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x111, 0xf, 0xf, false);   // (from 1, 2, 4, 8 lanes below inside the rows of 16,
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x112, 0xf, 0xf, false);   // then from the rows before)
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x114, 0xf, 0xf, false);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x118, 0xf, 0xf, false);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x142, 0xa, 0xf, false);
+        sum += __builtin_amdgcn_update_dpp(0, sum, 0x143, 0xc, 0xf, false);
+        const int start = __shfl(sum - size, valid ? leader : 0, kWave);
         const int total = __popcll(__ballot(valid));
         if (leader == e) {
             grp_ptr[gi] = ptr;
@@ -968,53 +978,113 @@ __global__ __launch_bounds__(256) void group_kernel(const uint64_t* __restrict__
     group_entries(g, n, grp_ptr, grp_start, grp_ent, n_groups);
 }
 
-// A window's head in ONE launch (2 ... 16 tokens, the softmax router, up to 256 experts), grid (1 + n_embd / 256, tokens):
-// workgroup (0, 0) routes every token - a wave a token, the token's experts 4 a lane, nothing but registers: the
-// maximum, the exponentials, then route_narrow_regs - writes ids / weights / plan and groups the plan itself
-// (group_kernel's arithmetic), so a window needs no grouping launch; the workgroups (b >= 1, t) round x like
-// layer_head_kernel's.  x NULL: routing only, grid (1, 1).
+// The head of several tokens in ONE launch (up to 16, either router, up to 256 experts, 256 entries): route, plan, group, Q8_K of x.
+// Workgroup 0 has a wave a token: it picks the token's experts from the ORDER of the logits (route_wave_order_only; the exact
+// router on the same wave where that does not settle it), writes the plan and groups it itself (group_kernel's arithmetic).  The
+// workgroups 1 ... ceil(tokens / 4) route four tokens each exactly, a wave each, for ids and weights, which nothing in the launch
+// waits for; the rest round x, 32 values a lane (q8k_round_lane32).  x NULL: no such workgroups.
+// It takes 6.9 us for 4 tokens of 160 experts with the sigmoid router, where a routing launch and a grouping launch behind it took
+// 10.0; without x and with the softmax router 5.4, where exact routing in workgroup 0 with the grouping behind it took 10.4.  Layers:
+// IQ1_S 6144 x 2048, 2 tokens, 44.4 -> 41.7 us, 4 tokens 77.0 -> 75.4; IQ2_S 7168 x 2048 with Q4_K down, 8 tokens, 220 -> 214.5;
+// Q4_K 2048 x 768, 3 tokens, 30.1 -> 27.5; EXL3 6144 x 1536 at 3 bits, 4 tokens, 152.3 -> 148.6.
+constexpr int kHeadRoute = 4, kHeadRound = 32768;   // tokens of a routing workgroup, values of a rounding one
 template <int DT>
-__global__ __launch_bounds__(256) void window_head_kernel(const float* __restrict__ logits, int n_expert, int k, int n_tokens,
-                                                          const uint64_t* __restrict__ table, int32_t* __restrict__ ids,
-                                                          float* __restrict__ weights, uint64_t* __restrict__ plan,
-                                                          uint64_t* __restrict__ grp_ptr, int32_t* __restrict__ grp_start,
-                                                          int32_t* __restrict__ grp_ent, int32_t* __restrict__ n_groups,
-                                                          const void* __restrict__ x, int64_t n_embd, maya_act xq) {
+__global__ __launch_bounds__(1024) void window_head_kernel(const float* __restrict__ logits, const uint64_t* __restrict__ table,
+                                                           const void* __restrict__ x, int n_expert, int k, int n_tokens, int n_embd, RouterSpec rs,
+                                                           int32_t* __restrict__ ids, float* __restrict__ weights, uint64_t* __restrict__ plan,
+                                                           uint64_t* __restrict__ grp_ptr, int32_t* __restrict__ grp_start,
+                                                           int32_t* __restrict__ grp_ent, int32_t* __restrict__ n_groups, maya_act xq) {
     __shared__ GroupLds g;
-    __shared__ int qs[264];
-    if (blockIdx.x == 0) {
-        if (blockIdx.y != 0) return;
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        for (int t = wave; t < n_tokens; t += 4) {
-            const float* l = logits + (size_t) t * n_expert;
-            float lv[4];
-            uint64_t tab[4];
+    __shared__ float s_lv[MAYA_MAX_TOKENS][256];
+    __shared__ uint64_t s_tab[256];
+    const int tid = threadIdx.x, lane = tid & 63, n_route = (n_tokens + kHeadRoute - 1) / kHeadRoute;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int) blockIdx.x > n_route) {
+        const int64_t v0 = (int64_t) ((int) blockIdx.x - 1 - n_route) * kHeadRound + (int64_t) tid * 32;
+        const bool on = v0 < (int64_t) n_tokens * n_embd;   // (rows of whole 256-value blocks: the 8 lanes of a block are on or off together)
+        float v[32];
+        act_load32<DT>(x, v0, on, v);
+        int y[8];
+        float d;
+        q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
+        if (!on) return;
+        int4* q = (int4*) (xq.q + v0);
+        q[0] = make_int4(y[0], y[1], y[2], y[3]);
+        q[1] = make_int4(y[4], y[5], y[6], y[7]);
+        int s[2] = {0, 0};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int e = 64 * r + lane;
-                lv[r] = e < n_expert ? l[e] : -INFINITY;
-                tab[r] = e < n_expert ? table[e] : 0ull;
-            }
-            int id;
-            float w;
-            uint64_t ptr;
-            route_wave_softmax(lv, tab, n_expert, k, id, w, ptr);
-            if (lane < k) {
-                ids[(size_t) t * k + lane] = id;
-                weights[(size_t) t * k + lane] = w;
+        for (int i = 0; i < 8; ++i) s[i >> 2] = dot4(0x01010101, y[i], s[i >> 2]);
+        *(uint32_t*) (xq.bsums + (v0 >> 4)) = ((uint32_t) s[0] & 0xffffu) | ((uint32_t) s[1] << 16);
+        xq.d[v0 >> 5] = d;
+        return;
+    }
+    const bool pick = blockIdx.x == 0, sigm = rs.kind == MAYA_ROUTER_SIGMOID;
+    const int t = pick ? wave : wave < kHeadRoute ? ((int) blockIdx.x - 1) * kHeadRoute + wave : n_tokens;
+    if (t < n_tokens) {
+        const float* l = logits + (size_t) t * n_expert;
+        float lv[4], bv[4], pr[4], sc[4];
+        uint64_t tab[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = 64 * r + lane;
+            lv[r] = e < n_expert ? l[e] : -INFINITY;
+            tab[r] = e < n_expert ? table[e] : 0ull;
+            bv[r] = rs.bias && e < n_expert ? rs.bias[e] : 0.0f;
+        }
+        bool fin = true;
+        if (sigm) fin = sigmoid_scores(lv, bv, rs.bias != nullptr, n_expert, pr, sc);
+        int id = 0;
+        float w = 0.0f;
+        uint64_t ptr = 0ull;
+        bool exact = !pick || k >= n_expert;
+        if (pick) {   // (every wave writes the whole table and reads it behind its own writes)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s_tab[64 * r + lane] = tab[r];
+        }
+        if (!exact) {
+            exact = !(sigm ? route_wave_order_only(sc, fin, n_expert, k, s_lv[t], 0.0f, INFINITY, id)
+                           : route_wave_order_only(lv, true, n_expert, k, s_lv[t], 1e-6f, 60.0f, id));
+            ptr = s_tab[!exact && lane < k ? id : 0];
+        }
+        if (exact) {
+            if (sigm) route_wave_sigmoid(pr, sc, fin, tab, n_expert, k, rs.norm, rs.w_scale, id, w, ptr);
+            else route_wave_softmax(lv, tab, n_expert, k, id, w, ptr);
+        }
+        if (lane < k) {
+            if (pick) {
                 plan[(size_t) t * k + lane] = ptr;
                 g.ptr[t * k + lane] = ptr;
+            } else {
+                ids[(size_t) t * k + lane] = id;
+                weights[(size_t) t * k + lane] = w;
             }
         }
-        const int n = n_tokens * k;
-        if ((int) threadIdx.x >= n) g.ptr[threadIdx.x] = 0ull;
-        __syncthreads();
-        group_entries(g, n, grp_ptr, grp_start, grp_ent, n_groups);
-    } else {
-        const int t = blockIdx.y, b = blockIdx.x - 1, j = threadIdx.x;
-        const float xv = load_x<DT>(x, (int64_t) t * n_embd + (int64_t) b * 256 + j);
-        quant_q8k_block(xv, j, true, qs, xq, (size_t) t * n_embd + (size_t) b * 256);
     }
+    if (!pick) return;
+    const int n = n_tokens * k;
+    if (tid >= n && tid < 256) g.ptr[tid] = 0ull;
+    __syncthreads();
+    if (tid >= 256) return;   // (a barrier counts the waves that have not ended)
+    group_entries(g, n, grp_ptr, grp_start, grp_ent, n_groups);
+}
+// what it covers
+inline bool window_head_ok(int n_tokens, int n_expert, int k) {
+    return n_tokens >= 1 && n_tokens <= MAYA_MAX_TOKENS && n_expert >= 1 && n_expert <= 256 && k >= 1 && k <= MAYA_MAX_K && k <= n_expert && n_tokens * k <= 256;
+}
+static int launch_window_head(const RouterSpec& rs, const float* logits, int n_tokens, int n_expert, int k, const uint64_t* table, int32_t* ids,
+                              float* weights, uint64_t* plan, uint64_t* grp_ptr, int32_t* grp_start, int32_t* grp_ent, int32_t* n_groups,
+                              const void* x, int x_dtype, int n_embd, maya_act xq, hipStream_t s) {
+    const int64_t rounding = x ? ((int64_t) n_tokens * n_embd + kHeadRound - 1) / kHeadRound : 0;
+    const dim3 grid((unsigned) (1 + (n_tokens + kHeadRoute - 1) / kHeadRoute + rounding)), block(1024);
+#define MAYA_WH(DT) hipLaunchKernelGGL(window_head_kernel<DT>, grid, block, 0, s, logits, table, x, n_expert, k, n_tokens, n_embd, rs, ids, weights, plan, grp_ptr, grp_start, grp_ent, n_groups, xq)
+    switch (x ? x_dtype : MAYA_DT_F32) {
+        case MAYA_DT_BF16: MAYA_WH(MAYA_DT_BF16); break;
+        case MAYA_DT_F16: MAYA_WH(MAYA_DT_F16); break;
+        default: MAYA_WH(MAYA_DT_F32); break;
+    }
+#undef MAYA_WH
+    MAYA_LAUNCHED("window_head_kernel");
+    return MAYA_OK;
 }
 
 // ------------------------------------------------------------------------------------------------ expert rows
@@ -2174,10 +2244,10 @@ int maya_moe_route_window(const maya_router* router, const float* logits, int n_
         return fail(MAYA_E_ARG, "route_window: null pointer");
     if (!maya_moe_route_window_ok(router, n_tokens, n_expert, k))
         return fail(MAYA_E_UNSUPPORTED, "route_window: the softmax router, up to 256 experts and 256 entries (tokens %d experts %d k %d)", n_tokens, n_expert, k);
-    hipLaunchKernelGGL(window_head_kernel<MAYA_DT_F32>, dim3(1, 1), dim3(256), 0, as_stream(stream), logits, n_expert, k, n_tokens, expert_table, ids,
-                       weights, plan_ptr, grp_ptr, grp_start, grp_ent, n_groups, nullptr, (int64_t) 0, maya_act{nullptr, nullptr, nullptr});
-    MAYA_LAUNCHED("window_head_kernel");
-    return MAYA_OK;
+    RouterSpec rs;
+    router_spec(nullptr, rs);
+    return launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, plan_ptr, grp_ptr, grp_start, grp_ent, n_groups, nullptr, 0, 0,
+                              maya_act{nullptr, nullptr, nullptr}, as_stream(stream));
 }
 
 int maya_moe_route_tiered(const maya_router* router, const float* logits, int n_tokens, int layer, int n_expert, int k,
@@ -2445,11 +2515,6 @@ int maya_mv(const maya_mv_job* jobs, int n_jobs, void* stream) {
     return MAYA_OK;
 }
 
-// Windows of up to this many tokens take window_head_kernel: its one workgroup routes four tokens at a time, so four tokens
-// cost one router's time and save the grouping launch (configs[4], 4 tokens: 172.9 -> 171.3 us), eight cost two and lose
-// more than the launch saves (configs[2], 8 tokens: 256.0 -> 261.8 us, A/B on one box).
-constexpr int kWindowHeadTokens = 4;
-
 // workspace carve-up of maya_moe_layer_decode (every region 256-byte aligned)
 struct LayerWs {
     uint64_t *plan_ptr, *grp_ptr;
@@ -2569,17 +2634,15 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
                                            : launch_gate_up_iq1s_pos(a, *st, s, &hd)))
             return rc;
         gate_up_done = true;
-    } else if (logits && q8k_act(l->gate_type) && n_expert <= MAYA_MAX_EXPERTS && x_dtype >= 0 && x_dtype <= 2 && n_tokens > 1 &&
-        n_tokens <= kWindowHeadTokens && maya_moe_route_window_ok(router, n_tokens, n_expert, k)) {
-        // a window, one launch: route every token, plan, group, Q8_K of x
-        const dim3 grid((unsigned) (1 + l->n_embd / 256), (unsigned) n_tokens);
-        hipStream_t s = as_stream(stream);
-        switch (x_dtype) {
-            case MAYA_DT_F32: hipLaunchKernelGGL(window_head_kernel<MAYA_DT_F32>, grid, dim3(256), 0, s, logits, n_expert, k, n_tokens, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups, x, (int64_t) l->n_embd, w.x); break;
-            case MAYA_DT_BF16: hipLaunchKernelGGL(window_head_kernel<MAYA_DT_BF16>, grid, dim3(256), 0, s, logits, n_expert, k, n_tokens, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups, x, (int64_t) l->n_embd, w.x); break;
-            default: hipLaunchKernelGGL(window_head_kernel<MAYA_DT_F16>, grid, dim3(256), 0, s, logits, n_expert, k, n_tokens, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups, x, (int64_t) l->n_embd, w.x); break;
-        }
-        MAYA_LAUNCHED("window_head_kernel");
+    } else if (logits && n_tokens > 1 && !join && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 && x_dtype <= 2) {
+        // several tokens, one launch: route, plan, group and - where the gate rows meet Q8_K codes - round x.  (Not beside a shared
+        // expert: its launches run in the head's time, and what is left of them when the routed gate/up starts costs more
+        // than the head gains: 8 tokens 235 us with two launches and 237 with one, 16 tokens 424 and 433.)
+        const bool q8k = q8k_act(l->gate_type);
+        if ((rc = launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups,
+                                     q8k ? x : nullptr, x_dtype, l->n_embd, w.x, as_stream(stream))))
+            return rc;
+        if (!q8k && (rc = maya_quant_act(l->gate_type, x, x_dtype, 0, n_tokens, l->n_embd, w.x, stream))) return rc;
         grouped = true;
     } else if (logits && q8k_act(l->gate_type) && n_expert <= MAYA_MAX_EXPERTS && x_dtype >= 0 && x_dtype <= 2) {
         // one launch: route, plan, Q8_K of x

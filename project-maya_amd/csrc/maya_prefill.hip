@@ -164,12 +164,6 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
 }
 
 // ------------------------------------------------------------------------------------------ activation quantizer
-template <int DT> __device__ __forceinline__ float pf_load(const void* x, int64_t i) {
-    if constexpr (DT == MAYA_DT_F32) return ((const float*) x)[i];
-    else if constexpr (DT == MAYA_DT_BF16) return __uint_as_float((uint32_t) ((const uint16_t*) x)[i] << 16);
-    else return f16_bits_to_f32(((const uint16_t*) x)[i]);
-}
-__device__ __forceinline__ int pf_rint(float f) { return (int) rintf(f); }
 
 // Q8_K rows - the activation format of the reference's CPU expert path for the K-quants
 // (src/kernels/cuda/quantize_act.cu:161-207) - rounded 32 values a lane, 8 lanes a 256-value block (q8k_round_lane32: no
@@ -183,47 +177,6 @@ struct PfLane {
     float d;
     int sum;
 };
-template <int DT>
-__device__ __forceinline__ void pf_load32(const void* x, int64_t i0, bool on, float (&v)[32]) {
-    if (!on) {
-#pragma unroll
-        for (int i = 0; i < 32; ++i) v[i] = 0.0f;
-        return;
-    }
-    if constexpr (DT == MAYA_DT_F32) {
-        const float* p = (const float*) x + i0;
-        if (((uintptr_t) p & 15) == 0) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float4 t = ((const float4*) p)[i];
-                v[4 * i] = t.x, v[4 * i + 1] = t.y, v[4 * i + 2] = t.z, v[4 * i + 3] = t.w;
-            }
-            return;
-        }
-    } else {
-        const uint16_t* p = (const uint16_t*) x + i0;
-        if (((uintptr_t) p & 15) == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint4 t = ((const uint4*) p)[i];
-                const uint32_t w[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if constexpr (DT == MAYA_DT_BF16) {
-                        v[8 * i + 2 * j] = __uint_as_float(w[j] << 16);
-                        v[8 * i + 2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-                    } else {
-                        v[8 * i + 2 * j] = f16_bits_to_f32(w[j] & 0xffffu);
-                        v[8 * i + 2 * j + 1] = f16_bits_to_f32(w[j] >> 16);
-                    }
-                }
-            }
-            return;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 32; ++i) v[i] = pf_load<DT>(x, i0 + i);
-}
 __device__ __forceinline__ PfLane pf_round_lane(const float (&v)[32], int lane) {
     PfLane o;
     q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, o.y, o.d);
@@ -253,7 +206,7 @@ __global__ __launch_bounds__(256) void prefill_quant_kernel(const void* __restri
     const int64_t v0 = ((int64_t) blockIdx.x * 256 + threadIdx.x) * 32;
     const bool on = v0 < k;   // (k is a multiple of 256: the 8 lanes of a block are on or off together)
     float v[32];
-    pf_load32<DT>(x, (int64_t) t * x_stride + v0, on, v);
+    act_load32<DT>(x, (int64_t) t * x_stride + v0, on, v);
     const PfLane c = pf_round_lane(v, lane);
     if (!on) return;
     for (int j = 0; j < top_k; ++j) {
@@ -270,7 +223,7 @@ __global__ __launch_bounds__(256) void prefill_quant_rows_kernel(const float* __
     const int64_t v0 = ((int64_t) blockIdx.x * 256 + threadIdx.x) * 32;
     const bool on = v0 < k;
     float v[32];
-    pf_load32<MAYA_DT_F32>(x, (int64_t) row * k + v0, on, v);
+    act_load32<MAYA_DT_F32>(x, (int64_t) row * k + v0, on, v);
     const PfLane c = pf_round_lane(v, lane);
     if (on) pf_store_lane(o, (size_t) row, k, v0, lane, c);
 }

@@ -99,6 +99,37 @@ def test_head_in_the_gate_up_launch_is_the_exact_router(lib, oracle, layer, dtyp
     assert np.array_equal(fused.ids.cpu().numpy(), wi) and rel_l2(out[0], wout[0]) <= 1e-3
 
 
+@pytest.mark.parametrize("sigmoid", (False, True))
+@pytest.mark.parametrize("nt", (2, 5, 11))
+def test_head_of_several_tokens_is_the_exact_router(lib, layer, nt, sigmoid):
+    """Several tokens in one call, every row one of the edge cases: ids and weights bit for bit the routing launch's, x rounded the same
+    from an address that is not 16-byte aligned, and a token's output - which hangs on what the head's first workgroup picked from the
+    order of the logits - bit for bit what the token gives alone."""
+    blobs, store, _, alone = layer
+    rng = np.random.default_rng(31 + nt)
+    rows = list(logit_cases().values())
+    bias = dev((rng.standard_normal(NE) * 0.1).astype(np.float32))
+    router = lib.Router(lib.ROUTER_SIGMOID, 1, bias.data_ptr(), 2.5) if sigmoid else None
+    many, off_by = lib.MoeLayer(22, 22, N_EMBD, N_FF, NE, K, max_tokens=nt, packing=1), 2
+    xa = torch.zeros(nt * N_EMBD + 4, dtype=torch.float32, device="cuda")
+    x = torch.from_numpy(rng.standard_normal((nt, N_EMBD)).astype(np.float32)).cuda()
+    x[0, 256:512] = 0.0
+    x_un = xa[off_by:off_by + nt * N_EMBD].view(nt, N_EMBD)
+    x_un.copy_(x)
+    for first in range(0, len(rows), nt):
+        lg = dev(np.stack([rows[(first + i) % len(rows)] for i in range(nt)]))
+        out = many.forward(store.table, lg, x, router=router).clone()
+        ids, w = many.ids.clone(), many.weights.clone()
+        out_un = many.forward(store.table, lg, x_un, router=router).clone()
+        ids2, w2, _ = lib.route_plan(lg, K, store.table, router)
+        torch.cuda.synchronize()
+        assert torch.equal(ids, ids2) and torch.equal(w.view(torch.int32), w2.view(torch.int32)), first
+        assert torch.equal(out.view(torch.int32), out_un.view(torch.int32)), first
+        for t in range(nt):
+            one = alone.forward(store.table, lg[t:t + 1].contiguous(), x[t:t + 1].contiguous(), router=router)
+            assert torch.equal(out[t].view(torch.int32), one[0].view(torch.int32)), (first, t)
+
+
 def test_absent_experts_and_k_next_to_the_expert_count(lib, oracle):
     """k = n_expert - 1 (the order-only pick needs one expert beyond the slots) and k = n_expert (the head then stays a
     launch of its own); experts missing from the table give no contribution on either path."""
