@@ -342,9 +342,11 @@ int maya_moe_layer_decode_end(const maya_moe_layout* l, const uint64_t* expert_t
  *   out[t] = shared->add[t] + shared_expert(x[t]) + sum_j weights[t][j] * expert_{ids[t][j]}(x[t]).
  * The reference runs the shared expert's down rows as extra blocks of the routed experts' gate/up launch
  * (include/strata/kernels/glm_fast.hpp:496-501, src/kernels/cuda/glm_fast.cu:4841-4849) so that they cost no time of
- * their own; here the shared expert's launches (quantize x, gate/up, quantize h, down + add) go to a second stream that
- * the library keeps a device (default priority), forked from `stream` by an event when the call starts and joined back
- * before the routed down launch, which adds the routed experts to the shared expert's output.  Every result is the bits
+ * their own.  Here a shared expert of stream-packed Q8_0 rows (the position-mapped kernels' sizes) is two launches on `stream`
+ * in front of the routed gate/up: the layer's head rounds x for it too, its down launch rounds h and adds.  One of other
+ * types has four launches (quantize x, gate/up, quantize h, down + add), which go to a second stream that the library keeps
+ * a device (default priority), forked from `stream` by an event when the call starts and joined back before the routed
+ * down launch, which adds the routed experts to the shared expert's output.  Every result is the bits
  * of maya_moe_gate_up / maya_moe_down on `shared` followed by maya_moe_layer_decode_routed with add = shared->out.
  *   shared: the stage arguments of the shared expert as maya_moe_gate_up / maya_moe_down take them - k = 1, n_tokens
  *   entries, plan_ptr all its blob, plan_w all 1, its groups (one group of n_tokens entries), its own x / h / hq (NULL
@@ -353,7 +355,7 @@ int maya_moe_layer_decode_end(const maya_moe_layout* l, const uint64_t* expert_t
  * The fork and the join are event records and waits, so the call may be captured in a HIP graph (maya_init() first).
  * Every refusal of the stages (status > 0) is found before the fork: such a call has launched nothing on either stream.
  * Calls on one device are serialised on the host by a lock.  The device has ONE such second stream: while `stream` is being
- * captured that second stream belongs to the capture until hipStreamEndCapture, and a call from any other stream (eager,
+ * captured that second stream belongs to the capture until hipStreamEndCapture (whatever the shared expert's type), and a call from any other stream (eager,
  * or inside another capture) in between is refused with MAYA_E_BUSY and launches nothing - the open capture is not
  * disturbed and may call again.  After a HIP error (status < 0) `stream` has joined the second stream again when the
  * call returns. */

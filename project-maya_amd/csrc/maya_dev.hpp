@@ -173,6 +173,23 @@ __device__ __forceinline__ void q8k_round_lane32(const float (&v)[32], IndexOf i
         y[i] = (int) __builtin_amdgcn_perm(hi, lo, 0x05040100u);
     }
 }
+// one lane's 32 values as one Q8_0 block: quant_q80_kernel's rounding, the block's amax inside the lane
+__device__ __forceinline__ void q80_round_lane32(const float (&v)[32], int (&y)[8], float& d) {
+    float am = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) am = i ? fmaxf(am, fabsf(v[i])) : fabsf(v[0]);
+    const float d0 = __fdiv_rn(am, 127.0f);
+    const bool big = d0 > 65504.0f;
+    const float inv = am == 0.0f ? 0.0f : big ? __fdiv_rn(1.0f, 65504.0f) : __fdiv_rn(127.0f, am);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w |= ((uint32_t) max(-128, min(127, (int) rintf(__fmul_rn(v[4 * i + j], inv)))) & 0xffu) << (8 * j);
+        y[i] = (int) w;
+    }
+    d = __half2float(__float2half_rn(big ? 65504.0f : d0));
+}
 
 // One activation, and 32 of them in a row (16 bytes a load where they are aligned; `on` false: zeros), as floats
 template <int DT> __device__ __forceinline__ float act_load(const void* x, int64_t i) {

@@ -982,7 +982,8 @@ __global__ __launch_bounds__(256) void group_kernel(const uint64_t* __restrict__
 // Workgroup 0 has a wave a token: it picks the token's experts from the ORDER of the logits (route_wave_order_only; the exact
 // router on the same wave where that does not settle it), writes the plan and groups it itself (group_kernel's arithmetic).  The
 // workgroups 1 ... ceil(tokens / 4) route four tokens each exactly, a wave each, for ids and weights, which nothing in the launch
-// waits for; the rest round x, 32 values a lane (q8k_round_lane32).  x NULL: no such workgroups.
+// waits for; the rest round x, 32 values a lane: to Q8_K (xq; q8k_round_lane32), then to Q8_0 (xs; q80_round_lane32), each where its
+// codes have a place.
 // It takes 6.9 us for 4 tokens of 160 experts with the sigmoid router, where a routing launch and a grouping launch behind it took
 // 10.0; without x and with the softmax router 5.4, where exact routing in workgroup 0 with the grouping behind it took 10.4.  Layers:
 // IQ1_S 6144 x 2048, 2 tokens, 44.4 -> 41.7 us, 4 tokens 77.0 -> 75.4; IQ2_S 7168 x 2048 with Q4_K down, 8 tokens, 220 -> 214.5;
@@ -993,29 +994,36 @@ __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restri
                                                            const void* __restrict__ x, int n_expert, int k, int n_tokens, int n_embd, RouterSpec rs,
                                                            int32_t* __restrict__ ids, float* __restrict__ weights, uint64_t* __restrict__ plan,
                                                            uint64_t* __restrict__ grp_ptr, int32_t* __restrict__ grp_start,
-                                                           int32_t* __restrict__ grp_ent, int32_t* __restrict__ n_groups, maya_act xq) {
+                                                           int32_t* __restrict__ grp_ent, int32_t* __restrict__ n_groups, maya_act xq, maya_act xs) {
     __shared__ GroupLds g;
     __shared__ float s_lv[MAYA_MAX_TOKENS][256];
     __shared__ uint64_t s_tab[256];
     const int tid = threadIdx.x, lane = tid & 63, n_route = (n_tokens + kHeadRoute - 1) / kHeadRoute;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if ((int) blockIdx.x > n_route) {
-        const int64_t v0 = (int64_t) ((int) blockIdx.x - 1 - n_route) * kHeadRound + (int64_t) tid * 32;
-        const bool on = v0 < (int64_t) n_tokens * n_embd;   // (rows of whole 256-value blocks: the 8 lanes of a block are on or off together)
+        const int64_t values = (int64_t) n_tokens * n_embd;
+        int b = (int) blockIdx.x - 1 - n_route;
+        const int nb = (int) ((values + kHeadRound - 1) / kHeadRound);
+        const bool q80 = !xq.q || b >= nb;
+        if (xq.q && q80) b -= nb;
+        const int64_t v0 = (int64_t) b * kHeadRound + (int64_t) tid * 32;
+        const bool on = v0 < values;   // (rows of whole 256-value blocks: the 8 lanes of a block are on or off together)
         float v[32];
         act_load32<DT>(x, v0, on, v);
         int y[8];
         float d;
-        q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
+        if (q80) q80_round_lane32(v, y, d);
+        else q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
         if (!on) return;
-        int4* q = (int4*) (xq.q + v0);
+        const maya_act to = q80 ? xs : xq;
+        int4* q = (int4*) (to.q + v0);
         q[0] = make_int4(y[0], y[1], y[2], y[3]);
         q[1] = make_int4(y[4], y[5], y[6], y[7]);
         int s[2] = {0, 0};
 #pragma unroll
         for (int i = 0; i < 8; ++i) s[i >> 2] = dot4(0x01010101, y[i], s[i >> 2]);
-        *(uint32_t*) (xq.bsums + (v0 >> 4)) = ((uint32_t) s[0] & 0xffffu) | ((uint32_t) s[1] << 16);
-        xq.d[v0 >> 5] = d;
+        *(uint32_t*) (to.bsums + (v0 >> 4)) = ((uint32_t) s[0] & 0xffffu) | ((uint32_t) s[1] << 16);
+        to.d[v0 >> 5] = d;
         return;
     }
     const bool pick = blockIdx.x == 0, sigm = rs.kind == MAYA_ROUTER_SIGMOID;
@@ -1073,11 +1081,11 @@ inline bool window_head_ok(int n_tokens, int n_expert, int k) {
 }
 static int launch_window_head(const RouterSpec& rs, const float* logits, int n_tokens, int n_expert, int k, const uint64_t* table, int32_t* ids,
                               float* weights, uint64_t* plan, uint64_t* grp_ptr, int32_t* grp_start, int32_t* grp_ent, int32_t* n_groups,
-                              const void* x, int x_dtype, int n_embd, maya_act xq, hipStream_t s) {
-    const int64_t rounding = x ? ((int64_t) n_tokens * n_embd + kHeadRound - 1) / kHeadRound : 0;
+                              const void* x, int x_dtype, int n_embd, maya_act xq, maya_act xs, hipStream_t s) {
+    const int64_t rounding = ((int64_t) n_tokens * n_embd + kHeadRound - 1) / kHeadRound * ((xq.q != nullptr) + (xs.q != nullptr));
     const dim3 grid((unsigned) (1 + (n_tokens + kHeadRoute - 1) / kHeadRoute + rounding)), block(1024);
-#define MAYA_WH(DT) hipLaunchKernelGGL(window_head_kernel<DT>, grid, block, 0, s, logits, table, x, n_expert, k, n_tokens, n_embd, rs, ids, weights, plan, grp_ptr, grp_start, grp_ent, n_groups, xq)
-    switch (x ? x_dtype : MAYA_DT_F32) {
+#define MAYA_WH(DT) hipLaunchKernelGGL(window_head_kernel<DT>, grid, block, 0, s, logits, table, x, n_expert, k, n_tokens, n_embd, rs, ids, weights, plan, grp_ptr, grp_start, grp_ent, n_groups, xq, xs)
+    switch (rounding ? x_dtype : MAYA_DT_F32) {
         case MAYA_DT_BF16: MAYA_WH(MAYA_DT_BF16); break;
         case MAYA_DT_F16: MAYA_WH(MAYA_DT_F16); break;
         default: MAYA_WH(MAYA_DT_F32); break;
@@ -1863,18 +1871,21 @@ inline int q80_group_tokens(const maya_moe_args& a) {
     if (!a.grp_ptr) return 1;
     return a.n_tokens >= 5 ? 8 : a.n_tokens >= 3 ? 4 : a.n_tokens >= 2 ? 2 : 1;
 }
-int launch_gate_up_q80_pos(const maya_moe_args& a, hipStream_t s) {
+// xf: one token's activations, which the workgroups round themselves (a.x is not read)
+int launch_gate_up_q80_pos(const maya_moe_args& a, hipStream_t s, const void* xf = nullptr, int x_dtype = 0) {
     const int nt = q80_group_tokens(a);
     const dim3 grid((unsigned) (a.layout.n_ff / 8), (unsigned) (a.n_tokens * a.k));
-#define MAYA_Q8T(NWV, NT)                                                                                                                       \
-    if (a.layout.n_embd == 1024 * NWV) hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, NT, 8, true>), grid, dim3(64 * NWV), 0, s, a);          \
-    else hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, NT, 8, false>), grid, dim3(64 * NWV), 0, s, a);
-#define MAYA_Q8(NWV)                          \
-    switch (nt) {                             \
-        case 8: MAYA_Q8T(NWV, 8) break;       \
-        case 4: MAYA_Q8T(NWV, 4) break;       \
-        case 2: MAYA_Q8T(NWV, 2) break;       \
-        default: MAYA_Q8T(NWV, 1) break;      \
+#define MAYA_Q8L(NWV, NT, FIT, SELF) hipLaunchKernelGGL((gate_up_q80_pos_kernel<NWV, NT, 8, FIT, SELF>), grid, dim3(64 * NWV), 0, s, a, xf, x_dtype)
+#define MAYA_Q8T(NWV, NT, SELF)                                           \
+    if (a.layout.n_embd == 1024 * NWV) MAYA_Q8L(NWV, NT, true, SELF);     \
+    else MAYA_Q8L(NWV, NT, false, SELF);
+#define MAYA_Q8(NWV)                                    \
+    switch (xf ? 0 : nt) {                              \
+        case 8: MAYA_Q8T(NWV, 8, false) break;          \
+        case 4: MAYA_Q8T(NWV, 4, false) break;          \
+        case 2: MAYA_Q8T(NWV, 2, false) break;          \
+        case 1: MAYA_Q8T(NWV, 1, false) break;          \
+        default: MAYA_Q8T(NWV, 1, true) break;          \
     }
     switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_Q8(2) break;
@@ -1887,16 +1898,18 @@ int launch_gate_up_q80_pos(const maya_moe_args& a, hipStream_t s) {
     }
 #undef MAYA_Q8
 #undef MAYA_Q8T
+#undef MAYA_Q8L
     MAYA_LAUNCHED("gate_up_q80_pos_kernel");
     return MAYA_OK;
 }
-int launch_down_q80_pos(const maya_moe_args& a, hipStream_t s) {
+int launch_down_q80_pos(const maya_moe_args& a, hipStream_t s, bool one_group = false) {
     const int nt = q80_group_tokens(a);
     // a wave takes per_wave rows, a multiple of the 8 / nt rows of a step: 8 (64 rows a workgroup) unless the call has so
-    // few entries that the grid would not cover the chip
-    const int step = 8 / nt;
+    // few entries that the grid would not cover the chip.  All tokens on one blob: 4, under which the rounding of h, once a
+    // workgroup, costs more than the waves gain (7168 x 2048: 8 tokens 15.3 / 11.8 / 13.2 us with 8 / 4 / 2 rows, 16 tokens 24.6 / 18.8 / 21.3).
+    const int step = 8 / nt, least = one_group && step < 4 ? 4 : step, groups = one_group ? 1 : a.n_tokens * a.k;
     int per_wave = 8;
-    while (per_wave > step && (long long) (a.layout.n_embd / (per_wave * 8)) * a.n_tokens * a.k < 1024) per_wave >>= 1;
+    while (per_wave > least && (long long) (a.layout.n_embd / (per_wave * 8)) * groups < 1024) per_wave >>= 1;
     const int wg_rows = per_wave * 8;
     const dim3 grid((unsigned) ((a.layout.n_embd + wg_rows - 1) / wg_rows), (unsigned) (a.n_tokens * a.k));
 #define MAYA_DQ(NT)                                                                                                             \
@@ -1910,6 +1923,13 @@ int launch_down_q80_pos(const maya_moe_args& a, hipStream_t s) {
     }
 #undef MAYA_DQ
     MAYA_LAUNCHED("down_q80_pos_kernel");
+    return MAYA_OK;
+}
+int down_q80(const maya_moe_args& a, hipStream_t s) {
+    if (const int rc = launch_down_q80_pos(a, s)) return rc;
+    if (a.k == 1) return MAYA_OK;   // (the rows were combined there)
+    hipLaunchKernelGGL(combine_kernel, dim3((unsigned) ((a.layout.n_embd + 255) / 256), (unsigned) a.n_tokens), dim3(256), 0, s, a);
+    MAYA_LAUNCHED("combine_kernel");
     return MAYA_OK;
 }
 
@@ -2246,8 +2266,9 @@ int maya_moe_route_window(const maya_router* router, const float* logits, int n_
         return fail(MAYA_E_UNSUPPORTED, "route_window: the softmax router, up to 256 experts and 256 entries (tokens %d experts %d k %d)", n_tokens, n_expert, k);
     RouterSpec rs;
     router_spec(nullptr, rs);
+    const maya_act none{nullptr, nullptr, nullptr};
     return launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, plan_ptr, grp_ptr, grp_start, grp_ent, n_groups, nullptr, 0, 0,
-                              maya_act{nullptr, nullptr, nullptr}, as_stream(stream));
+                              none, none, as_stream(stream));
 }
 
 int maya_moe_route_tiered(const maya_router* router, const float* logits, int n_tokens, int layer, int n_expert, int k,
@@ -2389,13 +2410,7 @@ int maya_moe_down(const maya_moe_args* a, void* stream) {
     }
     if (down_q4k_pos_ok(*a)) return launch_down_q4k_pos(*a, s);
     if (down_iq1s_pos_ok(*a)) return launch_down_iq1s_pos(*a, *st, s);
-    if (down_q80_pos_ok(*a)) {
-        if (const int rc = launch_down_q80_pos(*a, s)) return rc;
-        const dim3 cgrid((unsigned) ((a->layout.n_embd + 255) / 256), (unsigned) a->n_tokens);
-        hipLaunchKernelGGL(combine_kernel, cgrid, dim3(256), 0, s, *a);
-        MAYA_LAUNCHED("combine_kernel");
-        return MAYA_OK;
-    }
+    if (down_q80_pos_ok(*a)) return down_q80(*a, s);
     int rc;
     switch (a->layout.down_type) {
         case kIQ2_S: rc = launch_down_t<kIQ2_S>(*a, *st, s); break;
@@ -2562,7 +2577,7 @@ int maya_moe_layer_decode(const maya_moe_layout* l, const uint64_t* expert_table
 }
 }  // extern "C"
 
-// The layer's launches.  `join`: an event the down launch waits for (the shared expert's output, which `add` then points
+// The layer's launches.  `q80`: a shared expert of Q8_0 rows, run between the layer's own launches on the same stream.  `join`: an event the down launch waits for (the shared expert's output, which `add` then points
 // at), *joined set once the stream waits for it.
 // The routed layer's refusals (status > 0) and its stage arguments over the carved workspace, without launching anything.
 static int layer_setup(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, int k, const maya_router* router,
@@ -2610,7 +2625,7 @@ enum { kLayerWhole = 0, kLayerBegin = 1, kLayerEnd = 2 };
 static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, int k, const maya_router* router,
                              const float* logits, const void* x, int x_dtype, int n_tokens, float limit, const float* add,
                              int32_t* ids, float* weights, float* out, void* workspace, size_t workspace_bytes, void* stream,
-                             hipEvent_t join, bool* joined, int phase = kLayerWhole) {
+                             hipEvent_t join, bool* joined, int phase = kLayerWhole, const maya_moe_args* q80 = nullptr) {
     DeviceState* st;
     if (const int rc = current_state(&st)) return rc;
     RouterSpec rs;
@@ -2622,6 +2637,14 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
         return rc0;
     int rc;
     bool grouped = !head, gate_up_done = !head;
+    const maya_act none{nullptr, nullptr, nullptr};
+    const bool q80_down = down_q80_pos_ok(a);   // (that launch rounds h itself)
+    maya_moe_args sh;
+    if (q80) {
+        sh = *q80;
+        sh.hq = none, sh.part = nullptr;
+        if (n_tokens == 1 && ((rc = launch_gate_up_q80_pos(sh, as_stream(stream), x, x_dtype)) || (rc = launch_down_q80_pos(sh, as_stream(stream), true)))) return rc;
+    }
     if (!head) {
         // (the second half of a call made in two: the plan, the groups and h are in the workspace)
     } else if (layer_head_in_gate_up_ok(a, rs, logits, n_expert, x, x_dtype)) {
@@ -2635,14 +2658,15 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
             return rc;
         gate_up_done = true;
     } else if (logits && n_tokens > 1 && !join && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 && x_dtype <= 2) {
-        // several tokens, one launch: route, plan, group and - where the gate rows meet Q8_K codes - round x.  (Not beside a shared
-        // expert: its launches run in the head's time, and what is left of them when the routed gate/up starts costs more
-        // than the head gains: 8 tokens 235 us with two launches and 237 with one, 16 tokens 424 and 433.)
+        // several tokens, one launch: route, plan, group and round x, for the routed experts' rows and a shared Q8_0 expert's.  (Not
+        // beside a shared expert on the second stream: its launches run in the head's time, and what is left of them when the
+        // routed gate/up starts costs more than the head gains: 8 tokens 235 us with two launches and 237 with one, 16 tokens
+        // 424 and 433.)
         const bool q8k = q8k_act(l->gate_type);
+        if (q80 && !q8k) sh.x = w.x;
         if ((rc = launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups,
-                                     q8k ? x : nullptr, x_dtype, l->n_embd, w.x, as_stream(stream))))
+                                     x, x_dtype, l->n_embd, q8k ? w.x : none, !q8k ? w.x : q80 ? sh.x : none, as_stream(stream))))
             return rc;
-        if (!q8k && (rc = maya_quant_act(l->gate_type, x, x_dtype, 0, n_tokens, l->n_embd, w.x, stream))) return rc;
         grouped = true;
     } else if (logits && q8k_act(l->gate_type) && n_expert <= MAYA_MAX_EXPERTS && x_dtype >= 0 && x_dtype <= 2) {
         // one launch: route, plan, Q8_K of x
@@ -2663,6 +2687,10 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
         }
         if ((rc = maya_quant_act(l->gate_type, x, x_dtype, 0, n_tokens, l->n_embd, w.x, stream))) return rc;
     }
+    if (q80 && n_tokens > 1) {
+        if (!grouped && (rc = maya_quant_act(kQ8_0, x, x_dtype, 0, n_tokens, l->n_embd, sh.x, stream))) return rc;
+        if ((rc = launch_gate_up_q80_pos(sh, as_stream(stream))) || (rc = launch_down_q80_pos(sh, as_stream(stream), true))) return rc;
+    }
     if (n_tokens > 1) {
         if (!grouped && (rc = maya_moe_group(w.plan_ptr, n_tokens * k, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups, stream))) return rc;
         if (gate_up_by_entries(a) && down_by_entries(a)) {
@@ -2679,7 +2707,9 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
     }
     if (!gate_up_done && (rc = maya_moe_gate_up(&a, stream))) return rc;
     if (!tail) return MAYA_OK;
-    if (down_rounds_h(a)) {
+    if (q80_down) {
+        a.hq = none;
+    } else if (down_rounds_h(a)) {
         a.hq = maya_act{nullptr, nullptr, nullptr};
         a.part = nullptr;
     } else {
@@ -2688,6 +2718,10 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
     if (join) {
         MAYA_HIP(hipStreamWaitEvent(as_stream(stream), join, 0));
         *joined = true;
+    }
+    if (q80_down) {
+        if (k == 1) a.part = nullptr;
+        return down_q80(a, as_stream(stream));
     }
     return maya_moe_down(&a, stream);
 }
@@ -2745,18 +2779,30 @@ int maya_moe_layer_decode_shared(const maya_moe_layout* l, const uint64_t* exper
     // one call at a time a device: the side stream and its two events are the device's
     std::lock_guard<std::mutex> lock(st->side_mu);
     hipStream_t s = as_stream(stream);
+    const bool q80 = gate_up_q80_pos_ok(*shared) && down_q80_pos_ok(*shared);
+    hipStreamCaptureStatus mine_st = hipStreamCaptureStatusNone;
     {   // A side stream that an earlier call left inside a capture that has not ended belongs to that capture's graph until
         // hipStreamEndCapture: work forked onto it from another stream (eager, or another capture) would land in the wrong
         // graph or break the open capture.  The same capture calling again (a graph of several layers) is fine.
-        hipStreamCaptureStatus side_st = hipStreamCaptureStatusNone, mine_st = hipStreamCaptureStatusNone;
+        hipStreamCaptureStatus side_st = hipStreamCaptureStatusNone;
         unsigned long long side_id = 0, mine_id = 0;
         MAYA_HIP(hipStreamGetCaptureInfo(st->side, &side_st, &side_id));
         MAYA_HIP(hipStreamGetCaptureInfo(s, &mine_st, &mine_id));
         if (side_st != hipStreamCaptureStatusNone && !(mine_st == hipStreamCaptureStatusActive && mine_id == side_id))
             return fail(MAYA_E_BUSY, "layer_decode_shared: the device's side stream is inside another stream's capture; end that capture first");
     }
+    if (q80 && mine_st != hipStreamCaptureStatusActive)
+        return layer_decode_core(l, expert_table, n_expert, k, router, logits, x, x_dtype, n_tokens, limit, shared->out, ids, weights, out, workspace,
+                                 workspace_bytes, stream, nullptr, nullptr, kLayerWhole, shared);
     MAYA_HIP(hipEventRecord(st->side_fork, s));
     MAYA_HIP(hipStreamWaitEvent(st->side, st->side_fork, 0));
+    if (q80) {   // (a capture holds the second stream until it ends, whichever types it meets; nothing is launched there)
+        const int rc = layer_decode_core(l, expert_table, n_expert, k, router, logits, x, x_dtype, n_tokens, limit, shared->out, ids, weights, out, workspace,
+                                         workspace_bytes, stream, nullptr, nullptr, kLayerWhole, shared);
+        hipError_t e = hipEventRecord(st->side_join, st->side);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s, st->side_join, 0);
+        return e != hipSuccess && !rc ? hip_fail(e, "layer_decode_shared: joining the shared expert's stream") : rc;
+    }
     // the shared expert beside the routed experts' head and gate/up launches: quantize x, gate/up, quantize h, down + add
     int rc = maya_quant_act(shared->layout.gate_type, x, x_dtype, 0, n_tokens, shared->layout.n_embd, shared->x, st->side);
     if (!rc) rc = maya_moe_gate_up(shared, st->side);

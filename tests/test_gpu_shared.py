@@ -188,3 +188,68 @@ def test_another_stream_is_refused_while_the_side_stream_is_inside_a_capture(lib
         got2 = w["layer"].forward(w["table"], logits, x, shared=w["dense"], stream=s2).clone()
     s2.synchronize()
     assert torch.equal(got2, want)
+
+
+@pytest.mark.parametrize("gt,E,FF,NE,TK,T,dtype", [
+    (IQ2_S, 7168, 2048, 24, 8, 1, torch.bfloat16),    # one token: the shared expert's gate/up rounds x itself
+    (Q4_K, 2304, 768, 40, 3, 1, torch.float16),       # rows that end inside a wave
+    (Q4_K, 2048, 512, 300, 2, 5, torch.float32),      # more experts than the head of several tokens takes: x rounded by its own launch
+    (Q8_0, 2816, 1280, 20, 4, 9, torch.bfloat16),     # the head rounds x once for both; two chunks of tokens
+    (Q4_K, 4096, 2048, 32, 1, 16, torch.float32),     # one slot a token
+])
+def test_shared_q8_0_in_one_stream(lib, gt, E, FF, NE, TK, T, dtype):
+    """A Q8_0 shared expert's two launches round x and h and combine themselves: the bits of its stage calls with their own
+    launches for that, then the routed layer on top; x also from an address that is not 16-byte aligned."""
+    w = build(lib, gt, gt, Q8_0, E, FF, NE, TK, T, 600 + T)
+    for rep in range(2):
+        logits, x, add = inputs(E, NE, T, 610 + rep)
+        x = x.to(dtype)
+        x[0, 32:64] = 0.0
+        buf = torch.zeros(T * E + 2, dtype=dtype, device="cuda")
+        xs = buf[2:].view(T, E).copy_(x) if rep else x
+        use_add = None if rep else add
+        got = w["layer"].forward(w["table"], logits, xs, add=use_add, shared=w["dense"], shared_limit=5.0).clone()
+        shared = w["dense"].out.clone()
+        want = two_calls(w, logits, x, use_add, 5.0)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(shared, w["dense"].out), rep
+
+
+def test_down_of_one_slot_combines_as_of_two(lib):
+    """down_q80_pos_kernel writes a one-slot call's combined rows itself: the bits of the two-slot call whose second slot is left
+    out (which combines in a launch), with a token whose only slot is left out, weights, both residuals, a flagged one and skip."""
+    import ctypes as C
+    E, FF, T = 2304, 768, 3
+    gguf, bb = lib.layout(Q8_0, Q8_0, E, FF)
+    raw = workloads.random_blocks(bb, *FIELDS[Q8_0], 77)
+    blob = torch.empty_like(raw)
+    lib.repack(gguf, raw, blob)
+    rng = np.random.default_rng(78)
+    t = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()  # noqa: E731
+    h, add, add2, wts = t(T, FF), t(T, E), t(T, E), t(T)
+    ptr1 = torch.tensor([blob.data_ptr(), 0, blob.data_ptr()], dtype=torch.int64, device="cuda")
+    ptr2 = torch.stack([ptr1, torch.zeros_like(ptr1)], 1).reshape(-1).contiguous()
+    h2 = torch.stack([h, h], 1).reshape(2 * T, FF).contiguous()
+    w2 = torch.stack([wts, wts], 1).reshape(-1).contiguous()
+    flag, skip = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+
+    def down(k, ptr, wt, hh):
+        grp = lib.group(ptr)
+        hq = lib.quant_act(Q8_0, hh)
+        out, part = torch.full((T, E), 3.0, device="cuda"), torch.zeros((T * k, E), device="cuda")
+        a = lib.Args()
+        a.layout = lib.copy_layout(gguf, lib.PACK_STREAM)
+        a.n_tokens, a.k = T, k
+        a.plan_ptr, a.plan_w = ptr.data_ptr(), wt.data_ptr()
+        a.grp_ptr, a.grp_start, a.grp_ent, a.n_groups = (g.data_ptr() for g in grp)
+        a.x, a.h, a.hq, a.part, a.out = hq.c(), hh.data_ptr(), hq.c(), part.data_ptr(), out.data_ptr()
+        a.add, a.add2, a.add_flag, a.skip = add.data_ptr(), add2.data_ptr(), flag.data_ptr(), skip.data_ptr()
+        lib.check(lib.load().maya_moe_down(C.byref(a), lib._stream(None)))
+        torch.cuda.synchronize()
+        return out, part
+    for f, s in ((0, 0), (1, 0), (1, 1)):
+        flag.fill_(f)
+        skip.fill_(s)
+        (one, p1), (two, p2) = down(1, ptr1, wts, h), down(2, ptr2, w2, h2)
+        assert torch.equal(one, two), (f, s)
+        assert s or torch.equal(p1[::2], p2.view(T, 2, E)[::2, 0])
