@@ -1440,6 +1440,7 @@ __global__ __launch_bounds__(kDnThreads) void mv_kernel(MvBatch b, Codebooks cb,
 #include "maya_fast1.hpp"
 #include "maya_fastk.hpp"
 #include "maya_fastq.hpp"
+#include "maya_fastx.hpp"
 #include "maya_fastmv.hpp"
 #include "maya_tiers.hpp"
 
@@ -1523,8 +1524,7 @@ int launch_down_t(const maya_moe_args& a, const DeviceState& st, hipStream_t s) 
 // tokens, 733 -> 143; IQ2_S gate/up with Q4_K down 4864 x 1280, eight tokens, 430 -> 89; Q8_0 2560 x 1280, six tokens, 148 -> 81.
 // The general kernels share a decode among an expert's tokens, these (but for Q8_0) decode for every entry, so the lead narrows with
 // the entries an expert, without turning over: 16 tokens on one expert of 2816 x 1280, Q4_K 158 -> 29, IQ2_S 111 -> 45; top-10 of 16
-// experts 498 -> 125 and 337 -> 172; all of 16 experts, IQ2_S 4096 x 2048, 451 -> 406; the least, IQ2_XXS gate/up (general) with
-// IQ2_S down 2816 x 1280, all of 10 experts, 251 and 253.
+// experts 498 -> 125 and 337 -> 172, IQ2_XXS gate/up with IQ2_S down 206 -> 94; all of 16 experts, IQ2_S 4096 x 2048, 451 -> 406.
 static bool pos_row_ok(int n_embd) { return n_embd % 256 == 0 && n_embd >= 256 && n_embd <= 8192; }
 static int pos_waves(int n_embd) { return n_embd <= 2048 ? 2 : (n_embd + 1023) / 1024; }
 static bool down_pos_nff_ok(int n_ff) { return n_ff % 256 == 0 && n_ff >= 256 && n_ff <= 2048; }
@@ -1750,6 +1750,30 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     MAYA_LAUNCHED("gate_up_iq1s_pos_kernel");
     return MAYA_OK;
 }
+// ---- IQ2_XXS (either packing: the type's rows stay in GGUF order)
+bool gate_up_iq2xxs_pos_ok(const maya_moe_args& a) {
+    const maya_moe_layout& l = a.layout;
+    return l.gate_type == kIQ2_XXS && l.up_type == kIQ2_XXS && pos_row_ok(l.n_embd) && l.n_ff % 16 == 0;
+}
+int launch_gate_up_iq2xxs_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
+    const dim3 grid((unsigned) (a.layout.n_ff / 16), (unsigned) (a.n_tokens * a.k));
+    // (compiled for 7 waves a SIMD: at 8 four registers are spilled, 51.9 -> 56.0 us for four tokens of 4096 x 2048, 275 -> 285 for 16 of 6144 x 2048)
+#define MAYA_XXS(NWV)                                                                                                                            \
+    if (a.layout.n_embd == 1024 * NWV) hipLaunchKernelGGL((gate_up_iq2xxs_pos_kernel<NWV, 16, 7, true>), grid, dim3(64 * NWV), 0, s, a, st.cb);   \
+    else hipLaunchKernelGGL((gate_up_iq2xxs_pos_kernel<NWV, 16, 7, false>), grid, dim3(64 * NWV), 0, s, a, st.cb);
+    switch (pos_waves(a.layout.n_embd)) {
+        case 2: MAYA_XXS(2) break;
+        case 3: MAYA_XXS(3) break;
+        case 4: MAYA_XXS(4) break;
+        case 5: MAYA_XXS(5) break;
+        case 6: MAYA_XXS(6) break;
+        case 7: MAYA_XXS(7) break;
+        default: MAYA_XXS(8) break;
+    }
+#undef MAYA_XXS
+    MAYA_LAUNCHED("gate_up_iq2xxs_pos_kernel");
+    return MAYA_OK;
+}
 int launch_down_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
     // 32 rows a workgroup for the wide rows (half as many waves rounding h, as in the IQ2_S kernel), else 16.
     // (7 waves a SIMD leave the 53 and 64 registers the kernels take; of 16 slots one workgroup is 4 waves a SIMD already)
@@ -1956,7 +1980,7 @@ static int gate_up_refusal(const maya_moe_args* a, const DeviceState& st) {
                       (tg == kIQ1_S && tu == kIQ1_M) || (tg == kIQ1_M && tu == kIQ1_S);
     if (!pair) return fail(MAYA_E_UNSUPPORTED, "gate_up: no kernel for gate type %d with up type %d", tg, tu);
     const bool pos = (tg == kIQ2_S && tu == kIQ2_S && gate_up_iq2s_fast_ok(*a)) || gate_up_q4k_pos_ok(*a) || gate_up_iq1s_pos_ok(*a) ||
-                     gate_up_q80_pos_ok(*a);
+                     gate_up_q80_pos_ok(*a) || gate_up_iq2xxs_pos_ok(*a);
     if (!pos) {   // the general kernel: its activation tile and codebooks must fit the device's LDS
         const int nt = a->grp_ptr ? (a->n_tokens >= 4 ? 4 : a->n_tokens >= 2 ? 2 : 1) : 1;
         const int cbw = codebook_words(tg) + (codebook_words(tg) == codebook_words(tu) ? 0 : codebook_words(tu));
@@ -1990,7 +2014,7 @@ static int down_refusal(const maya_moe_args* a, const DeviceState& st) {
 
 bool gate_up_by_entries(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    if (gate_up_q4k_pos_ok(a) || gate_up_iq1s_pos_ok(a)) return true;
+    if (gate_up_q4k_pos_ok(a) || gate_up_iq1s_pos_ok(a) || gate_up_iq2xxs_pos_ok(a)) return true;
     return l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && gate_up_iq2s_fast_ok(a);
 }
 bool down_by_entries(const maya_moe_args& a) { return down_q4k_pos_ok(a) || down_rounds_h(a); }
@@ -2374,6 +2398,7 @@ int maya_moe_gate_up(const maya_moe_args* a, void* stream) {
     if (gate_up_q4k_pos_ok(*a)) return launch_gate_up_q4k_pos(*a, s);
     if (gate_up_iq1s_pos_ok(*a)) return launch_gate_up_iq1s_pos(*a, *st, s);
     if (gate_up_q80_pos_ok(*a)) return launch_gate_up_q80_pos(*a, s);
+    if (gate_up_iq2xxs_pos_ok(*a)) return launch_gate_up_iq2xxs_pos(*a, *st, s);
 #define MAYA_GU(TG, TU) if (tg == TG && tu == TU) return launch_gate_up_t<TG, TU>(*a, *st, s);
     MAYA_GU(kIQ2_S, kIQ2_S)
     MAYA_GU(kQ4_K, kQ4_K)

@@ -73,7 +73,7 @@ CASES = [
     (29, 29, 7168, 2048, 9, 8, 3),
     (29, 19, 6144, 2048, 4, 2, 2),
     (12, 29, 8192, 2048, 4, 3, 2),
-    # IQ2_XXS (the general kernels): one token, a window, mixed with IQ2_S either side
+    # IQ2_XXS: one token, a window, mixed with IQ2_S either side
     (16, 16, 1024, 512, 8, 4, 1),
     (16, 16, 7168, 2048, 9, 8, 3),
     (16, 22, 4096, 2048, 6, 4, 2),
@@ -124,6 +124,31 @@ def test_layer_matches_cpu_path(lib, oracle, gt, dt, n_embd, n_ff, ne, k, nt, pa
     assert np.array_equal(ids, wi)
     for t in range(nt):
         assert rel_l2(out[t], wout[t]) <= TOL, (t, rel_l2(out[t], wout[t]))
+
+
+@pytest.mark.parametrize("n_embd,n_ff,ne,k,nt,misalign", (
+    (256, 256, 4, 2, 3, 2),       # one block a row: 8 lanes of 64 have a position
+    (2048, 512, 8, 4, 1, 0),      # rows that fill their lanes, one token
+    (2304, 768, 12, 10, 2, 6),    # rows that end inside a wave, more than 8 slots
+    (7936, 1280, 5, 3, 5, 0),     # one block short of the widest but one
+    (8192, 256, 3, 2, 16, 2),     # the widest, 16 tokens
+))
+def test_iq2_xxs_gate_rows_at_any_two_byte_address(lib, oracle, n_embd, n_ff, ne, k, nt, misalign):
+    """gate_up_iq2xxs_pos_kernel at the ends of its range: GGUF rows from addresses that are only even, against the CPU path
+    (the tolerance of every layer test: the same integer products, summed in another order), and a token of a window bit for bit
+    the token alone."""
+    blobs = make_experts(16, 22, n_embd, n_ff, ne, 1600 + nt)
+    rng = np.random.default_rng(1601 + nt)
+    logits = rng.standard_normal((nt, ne)).astype(np.float32)
+    x = rng.standard_normal((nt, n_embd)).astype(np.float32)
+    ids, _, out, _ = run_layer(lib, 16, 22, blobs, k, n_embd, n_ff, logits, x, misalign=misalign)
+    wi, _, wout = oracle_layer(oracle, 16, 22, blobs, k, n_embd, n_ff, logits, x)
+    assert np.array_equal(ids, wi)
+    packed = run_layer(lib, 16, 22, blobs, k, n_embd, n_ff, logits, x, packing=1)[2]
+    for t in range(nt):
+        assert rel_l2(out[t], wout[t]) <= TOL and rel_l2(packed[t], wout[t]) <= TOL, t
+    alone = run_layer(lib, 16, 22, blobs, k, n_embd, n_ff, logits[nt - 1:], x[nt - 1:], packing=1)[2]
+    assert np.array_equal(alone[0].view(np.int32), packed[nt - 1].view(np.int32))
 
 
 def encoded_q4k_expert(oracle, n_embd, n_ff, seed):
