@@ -19,14 +19,18 @@
 namespace maya {
 
 template <int NT>
-__device__ __forceinline__ void stage_iq1s_table(int* lds, const Codebooks& cb) {
-    TablePieces<4096, NT> t;
-    table_request(cb.iq1s, t);
+__device__ __forceinline__ void store_iq1s_table(int* lds, const TablePieces<4096, NT>& t) {
     table_store(lds, t, [](int w) {
         const uint32_t g = (uint32_t) w;
         const uint32_t neg = (g >> 1) & 0x01010101u, pos = g & ~(g >> 1) & 0x01010101u;
         return (int) (0x09090909u + (pos << 3) - (neg << 3));
     });
+}
+template <int NT>
+__device__ __forceinline__ void stage_iq1s_table(int* lds, const Codebooks& cb) {
+    TablePieces<4096, NT> t;
+    table_request(cb.iq1s, t);
+    store_iq1s_table(lds, t);
 }
 constexpr int kFast1LdsWords = 4096;
 
@@ -155,101 +159,6 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(MAYA_HE
             }
             if (r0 + r + t < n_ff) a.h[(size_t) e * n_ff + r0 + r + t] = swiglu(g, up, a.limit);
         }
-    }
-}
-
-// ---- down + combine, n_ff = 32 nu <= 2048 (a row on the first nu lanes of one wave): wave w = slot w of token blockIdx.y, of at
-// most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.  The
-// slots' rows meet in LDS and are summed in slot order.
-template <int ROWS, int MINW, int SLOTS, int NU>
-__global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1s_pos_kernel(maya_moe_args a, Codebooks cb) {
-    static_assert(ROWS % 8 == 0, "a batch is two quads");
-    __shared__ __align__(16) int lds[kFast1LdsWords];
-    __shared__ float part[SLOTS][ROWS];
-    if (a.skip && *a.skip) return;
-    stage_iq1s_table<64 * SLOTS>(lds, cb);
-    const uint2* grid = (const uint2*) lds;
-    const int n_embd = a.layout.n_embd, nu = NU ? NU : a.layout.n_ff >> 5;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r0 = blockIdx.x * ROWS;
-    const int e0 = blockIdx.y * a.k, ent = e0 + wave;
-    const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
-    __syncthreads();
-    if (blob != 0ull) {
-        const uint32_t qb = (uint32_t) nu * 25u;   // bytes of a quad of rows
-        const uint64_t mat = blob + a.layout.down_off;
-        const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
-        const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
-        const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) (n_embd >> 2) * qb);
-        // (an idle lane - past the row's nu positions - has weights that read as zero and zero activations)
-        const bool on = NU == 64 || lane < nu;
-        const int pos = on ? lane : nu - 1;
-        const QuadOffs1 qo = quad_offs1(0u, nu, pos, on, (uint32_t) (n_embd >> 2) * qb);
-        const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
-        constexpr int NQ = ROWS / 4;
-        QuadIQ1S nxt = load_quad1(rs, qo, quad0);
-        int y[8];
-        float dy8;
-        if (a.hq.q) {
-            const int4* q = (const int4*) (a.hq.q + (size_t) ent * (32 * nu));
-            const int4 ya = q[2 * pos], yb = q[2 * pos + 1];
-            y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-            dy8 = a.hq.d[(size_t) ent * nu + pos] * 0.125f;
-        } else {
-            const float4* hv = (const float4*) (a.h + (size_t) ent * (32 * nu) + 32 * pos);
-            float v[32];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float4 t = hv[i];
-                v[4 * i] = t.x, v[4 * i + 1] = t.y, v[4 * i + 2] = t.z, v[4 * i + 3] = t.w;
-            }
-            if (!on) {
-#pragma unroll
-                for (int i = 0; i < 32; ++i) v[i] = 0.0f;
-            }
-            float d;
-            q8k_round_lane32(v, [&](int i) { return 32 * (lane & 7) + i; }, y, d);
-            dy8 = d * 0.125f;
-        }
-        idle_lane_zero(on, y, dy8);
-        const int sy = sum32_codes(y);
-        float acc[8];
-#pragma unroll 1
-        for (int r = 0; r < ROWS; r += 8) {
-            const int q = r >> 2;
-            {
-                const QuadIQ1S cur = nxt;
-                nxt = load_quad1(rs, qo, quad0 + (uint32_t) (q + 1) * qb);
-                quad1_values<0>(cur, grid, y, sy, dy8, acc);
-            }
-            {
-                const QuadIQ1S cur = nxt;
-                if (q + 2 < NQ) nxt = load_quad1(rs, qo, quad0 + (uint32_t) (q + 2) * qb);
-                quad1_values<4>(cur, grid, y, sy, dy8, acc);
-            }
-            float v = reduce8_half(acc, lane);
-            v = add_other_half(v);
-            if ((lane & 35) == 0) part[wave][r + ((lane >> 2) & 7)] = v;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < ROWS) {
-        const int c = threadIdx.x;
-        float sum = 0.0f;
-        bool first = true;
-        for (int i = 0; i < a.k; ++i) {
-            if (a.plan_ptr[e0 + i] == 0ull) continue;
-            const float p = __fmul_rn(part[i][c], a.plan_w[e0 + i]);
-            sum = first ? p : __fadd_rn(sum, p);
-            first = false;
-        }
-        const size_t o = (size_t) blockIdx.y * n_embd + r0 + c;
-        if (a.add && (!a.add_flag || *a.add_flag)) sum = __fadd_rn(sum, a.add[o]);
-        if (a.add2) sum = __fadd_rn(sum, a.add2[o]);
-        a.out[o] = sum;
-        if (a.part)
-            for (int i = 0; i < a.k; ++i)
-                if (a.plan_ptr[e0 + i] != 0ull) a.part[(size_t) (e0 + i) * n_embd + r0 + c] = part[i][c];
     }
 }
 
@@ -383,51 +292,79 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1m_pos_kernel(maya_mo
     }
 }
 
-// ---- down + combine, n_ff = 32 nu <= 2048 (a row on the first nu lanes of one wave): wave w = slot w of token blockIdx.y, of at
-// most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.  The
-// slots' rows meet in LDS and are summed in slot order.
-template <int ROWS, int MINW, int SLOTS, int NU>
-__global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1m_pos_kernel(maya_moe_args a, Codebooks cb) {
+// ---- down + combine, n_ff = 32 nu <= 2048 (a row on the first nu lanes of one wave): wave w = slot w of a token, of at most SLOTS,
+// rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h to Q8_K itself.
+// The slots' rows meet in LDS and are summed in slot order.
+// PAIR (nu <= 32): a quad of rows on either half of the wave's lanes, instead of leaving half of them without a position.
+// The leading arguments, and what is asked for side by side before the weights - plan, table, h -: down_iq2s_pos_kernel.  The table
+// used to be read and stored before the plan was asked for: one token, IQ1_S 6144 x 2048 26.6 -> 25.3 us a layer, with PAIR
+// IQ1_S 4096 x 768 15.2 -> 13.3, IQ1_M 19.9 -> 17.7, IQ1_S 4096 x 512 four tokens 28.2 -> 22.9, IQ1_M 6144 x 1024 top-8 twelve
+// tokens 130 -> 112.
+template <typename F, int ROWS, int MINW, int SLOTS, int NU, bool PAIR>
+__global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1_pos_kernel(const uint64_t* __restrict__ plan_ptr, const float* __restrict__ plan_w,
+                                                                 const float* __restrict__ h, const uint64_t* __restrict__ iq1s_grid,
+                                                                 const int32_t* __restrict__ skip, const int8_t* __restrict__ hq_q, int k,
+                                                                 int n_embd, int n_pos, maya_moe_args a) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
+    static_assert(!PAIR || NU == 0, "two quads a wave: at most 32 positions");
     __shared__ __align__(16) int lds[kFast1LdsWords];
     __shared__ float part[SLOTS][ROWS];
-    if (a.skip && *a.skip) return;
-    stage_iq1s_table<64 * SLOTS>(lds, cb);
+    __shared__ float s_w[SLOTS];
+    __shared__ int s_on[SLOTS];
     const uint2* grid = (const uint2*) lds;
-    const int n_embd = a.layout.n_embd, nu = NU ? NU : a.layout.n_ff >> 5;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r0 = blockIdx.x * ROWS;
-    const int e0 = blockIdx.y * a.k, ent = e0 + wave;
-    const uint64_t blob = wave < a.k ? a.plan_ptr[ent] : 0ull;
+    int bx, by;
+    down_block_of_grid(bx, by);
+    const int r0 = bx * ROWS, e0 = by * k;
+    const int skipv = skip ? *skip : 0;
+    const int ent = e0 + min(wave, k - 1);   // (a wave past slot k - 1 has no rows: it helps with the table)
+    uint64_t blob = plan_ptr[ent];
+    TablePieces<4096, 64 * SLOTS> tp;
+    table_request(iq1s_grid, tp);
+    const int ci = e0 + min((int) threadIdx.x & (SLOTS - 1), k - 1);
+    const uint64_t c_ptr = plan_ptr[ci];
+    const float c_w = plan_w[ci];
+    // (an idle lane - past the row's nu positions - has weights that read as zero and zero activations)
+    const int nu = NU ? NU : n_pos, at = PAIR ? lane & 31 : lane;
+    const bool on = NU == 64 || at < nu;
+    const int pos = on ? at : nu - 1;
+    const bool rounded = hq_q != nullptr;
+    int y[8];
+    float dy8 = 0.0f;
+    float v[32];
+    if (__builtin_amdgcn_readfirstlane(wave) >= k) {   // (of one slot, seven of eight waves; their loads cost 1 us of 18)
+    } else if (rounded) {
+        const int4* q = (const int4*) (hq_q + (size_t) ent * (32 * nu));
+        const int4 ya = q[2 * pos], yb = q[2 * pos + 1];
+        y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
+        dy8 = a.hq.d[(size_t) ent * nu + pos] * 0.125f;
+    } else {
+        const float4* hv = (const float4*) (h + (size_t) ent * (32 * nu) + 32 * pos);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float4 t = hv[i];
+            v[4 * i] = t.x, v[4 * i + 1] = t.y, v[4 * i + 2] = t.z, v[4 * i + 3] = t.w;
+        }
+    }
+    if (skipv) return;
+    if (wave >= k) blob = 0ull;
+    const uint32_t qb = (uint32_t) nu * F::kQuadBytes, past = (uint32_t) (n_embd >> 2) * qb;   // bytes of a quad of rows, of the matrix
+    // (no blob: an empty resource, whose loads read as zero and touch nothing)
+    const uint64_t mat = blob ? blob + a.layout.down_off : 0ull;
+    const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
+    const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (mat_lo | mat_hi) != 0u ? past : 0u);
+    const auto qo = F::offs(PAIR ? (uint32_t) (lane >> 5) * qb : 0u, nu, pos, on, past);
+    const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
+    typename F::Quad nxt = F::load(rs, qo, quad0);
+    store_iq1s_table<64 * SLOTS>(lds, tp);
+    if (threadIdx.x < SLOTS) {
+        s_on[threadIdx.x] = (int) threadIdx.x < k && c_ptr != 0ull;
+        s_w[threadIdx.x] = c_w;
+    }
     __syncthreads();
     if (blob != 0ull) {
-        const uint32_t qb = (uint32_t) nu * 28u;   // bytes of a quad of rows
-        const uint64_t mat = blob + a.layout.down_off;
-        const uint32_t mat_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) mat);
-        const uint32_t mat_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (mat >> 32));
-        const __amdgpu_buffer_rsrc_t rs = weight_rsrc(((uint64_t) mat_hi << 32) | (uint64_t) mat_lo, (uint32_t) (n_embd >> 2) * qb);
-        // (an idle lane - past the row's nu positions - has weights that read as zero and zero activations)
-        const bool on = NU == 64 || lane < nu;
-        const int pos = on ? lane : nu - 1;
-        const QuadOffsM qo = quad_offsm(0u, nu, pos, on, (uint32_t) (n_embd >> 2) * qb);
-        const uint32_t quad0 = (uint32_t) (r0 >> 2) * qb;
-        constexpr int NQ = ROWS / 4;
-        QuadIQ1M nxt = load_quadm(rs, qo, quad0);
-        int y[8];
-        float dy8;
-        if (a.hq.q) {
-            const int4* q = (const int4*) (a.hq.q + (size_t) ent * (32 * nu));
-            const int4 ya = q[2 * pos], yb = q[2 * pos + 1];
-            y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-            dy8 = a.hq.d[(size_t) ent * nu + pos] * 0.125f;
-        } else {
-            const float4* hv = (const float4*) (a.h + (size_t) ent * (32 * nu) + 32 * pos);
-            float v[32];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float4 t = hv[i];
-                v[4 * i] = t.x, v[4 * i + 1] = t.y, v[4 * i + 2] = t.z, v[4 * i + 3] = t.w;
-            }
+        if (!rounded) {
             if (!on) {
 #pragma unroll
                 for (int i = 0; i < 32; ++i) v[i] = 0.0f;
@@ -437,26 +374,32 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1m_pos_kernel(maya_mo
             dy8 = d * 0.125f;
         }
         idle_lane_zero(on, y, dy8);
-        int sy8[4];
-        sums8_codes(y, sy8);
-        const int sh = 16 + 6 * (lane & 7);
+        const F f(y, lane);
         float acc[8];
 #pragma unroll 1
         for (int r = 0; r < ROWS; r += 8) {
             const int q = r >> 2;
-            {
-                const QuadIQ1M cur = nxt;
-                nxt = load_quadm(rs, qo, quad0 + (uint32_t) (q + 1) * qb);
-                quadm_values<0>(cur, grid, y, sy8, sh, dy8, acc);
+            if constexpr (PAIR) {
+                const typename F::Quad cur = nxt;
+                if (r + 8 < ROWS) nxt = F::load(rs, qo, quad0 + (uint32_t) (q + 2) * qb);
+                f.template values<0>(cur, grid, y, dy8, acc);
+                const float four[4] = {acc[0], acc[1], acc[2], acc[3]};
+                const float s = reduce4_half(four, lane);
+                if ((lane & 7) == 0) part[wave][r + 4 * (lane >> 5) + ((lane >> 3) & 3)] = s;
+            } else {
+                {
+                    const typename F::Quad cur = nxt;
+                    nxt = F::load(rs, qo, quad0 + (uint32_t) (q + 1) * qb);
+                    f.template values<0>(cur, grid, y, dy8, acc);
+                }
+                {
+                    const typename F::Quad cur = nxt;
+                    if (r + 8 < ROWS) nxt = F::load(rs, qo, quad0 + (uint32_t) (q + 2) * qb);
+                    f.template values<4>(cur, grid, y, dy8, acc);
+                }
+                const float s = add_other_half(reduce8_half(acc, lane));
+                if ((lane & 35) == 0) part[wave][r + ((lane >> 2) & 7)] = s;
             }
-            {
-                const QuadIQ1M cur = nxt;
-                if (q + 2 < NQ) nxt = load_quadm(rs, qo, quad0 + (uint32_t) (q + 2) * qb);
-                quadm_values<4>(cur, grid, y, sy8, sh, dy8, acc);
-            }
-            float v = reduce8_half(acc, lane);
-            v = add_other_half(v);
-            if ((lane & 35) == 0) part[wave][r + ((lane >> 2) & 7)] = v;
         }
     }
     __syncthreads();
@@ -464,20 +407,46 @@ __global__ __launch_bounds__(64 * SLOTS, MINW) void down_iq1m_pos_kernel(maya_mo
         const int c = threadIdx.x;
         float sum = 0.0f;
         bool first = true;
-        for (int i = 0; i < a.k; ++i) {
-            if (a.plan_ptr[e0 + i] == 0ull) continue;
-            const float p = __fmul_rn(part[i][c], a.plan_w[e0 + i]);
-            sum = first ? p : __fadd_rn(sum, p);
-            first = false;
+#pragma unroll
+        for (int i = 0; i < SLOTS; ++i) {   // the present slots in slot order; the first product starts the sum
+            const bool have = s_on[i] != 0;
+            const float p = __fmul_rn(part[i][c], s_w[i]);
+            const float t = first ? p : __fadd_rn(sum, p);
+            sum = have ? t : sum;
+            first = first && !have;
         }
-        const size_t o = (size_t) blockIdx.y * n_embd + r0 + c;
+        const size_t o = (size_t) by * n_embd + r0 + c;
         if (a.add && (!a.add_flag || *a.add_flag)) sum = __fadd_rn(sum, a.add[o]);
         if (a.add2) sum = __fadd_rn(sum, a.add2[o]);
         a.out[o] = sum;
         if (a.part)
-            for (int i = 0; i < a.k; ++i)
-                if (a.plan_ptr[e0 + i] != 0ull) a.part[(size_t) (e0 + i) * n_embd + r0 + c] = part[i][c];
+            for (int i = 0; i < k; ++i)
+                if (s_on[i]) a.part[(size_t) (e0 + i) * n_embd + r0 + c] = part[i][c];
     }
 }
+struct DownIq1S {
+    typedef QuadIQ1S Quad;
+    static constexpr uint32_t kQuadBytes = 25u;   // a sub-block position: 4 rows x 50 a block of 8
+    int sy;
+    __device__ __forceinline__ DownIq1S(const int (&y)[8], int) : sy(sum32_codes(y)) {}
+    __device__ static __forceinline__ QuadOffs1 offs(uint32_t mat, int nu, int u, bool on, uint32_t past) { return quad_offs1(mat, nu, u, on, past); }
+    __device__ static __forceinline__ Quad load(__amdgpu_buffer_rsrc_t rs, const QuadOffs1& o, uint32_t at) { return load_quad1(rs, o, at); }
+    template <int B>
+    __device__ __forceinline__ void values(const Quad& q, const uint2* grid, const int (&y)[8], float dy8, float (&acc)[8]) const {
+        quad1_values<B>(q, grid, y, sy, dy8, acc);
+    }
+};
+struct DownIq1M {
+    typedef QuadIQ1M Quad;
+    static constexpr uint32_t kQuadBytes = 28u;
+    int sy8[4], sh;
+    __device__ __forceinline__ DownIq1M(const int (&y)[8], int lane) : sh(16 + 6 * (lane & 7)) { sums8_codes(y, sy8); }
+    __device__ static __forceinline__ QuadOffsM offs(uint32_t mat, int nu, int u, bool on, uint32_t past) { return quad_offsm(mat, nu, u, on, past); }
+    __device__ static __forceinline__ Quad load(__amdgpu_buffer_rsrc_t rs, const QuadOffsM& o, uint32_t at) { return load_quadm(rs, o, at); }
+    template <int B>
+    __device__ __forceinline__ void values(const Quad& q, const uint2* grid, const int (&y)[8], float dy8, float (&acc)[8]) const {
+        quadm_values<B>(q, grid, y, sy8, sh, dy8, acc);
+    }
+};
 
 }  // namespace maya

@@ -160,23 +160,6 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(MAYA_HEA
     }
 }
 
-// The sums over a 32-lane half of four values a lane: row (lane >> 3) & 3's in every lane, by the pairs of lanes reduce8_half takes.
-__device__ __forceinline__ float reduce4_half(const float (&acc)[4], int lane) {
-    const bool b4 = lane & 16, b3 = lane & 8;
-    float v2[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const float send = b4 ? acc[i] : acc[i + 2], keep = b4 ? acc[i + 2] : acc[i];
-        v2[i] = keep + xor_lane<16>(send);
-    }
-    const float send = b3 ? v2[0] : v2[1], keep = b3 ? v2[1] : v2[0];
-    float v = keep + xor_lane<8>(send);
-    v += xor_lane<4>(v);
-    v += xor_lane<2>(v);
-    v += xor_lane<1>(v);
-    return v;
-}
-
 // ---- down + combine, n_ff = 32 nu <= 2048 (nu positions a row, lanes past them idle): wave w = slot w of token blockIdx.y, of at
 // most SLOTS, rows in batches of 8; grid (n_embd / ROWS, tokens).  Without a rounded h (hq.q == NULL) a wave rounds its slot's h
 // to Q8_K itself.

@@ -1626,6 +1626,9 @@ int launch_down_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStrea
     // SIMD the same number of rows, and half as many waves rounding h as with 16), else 16.
     const int n_embd = a.layout.n_embd;
     const int wide = n_embd % 1024 == 0 && n_embd >= 5120 && n_embd <= 8192 ? n_embd / 256 : 16;
+    // Rows of up to 1024 values: two quads at a time; 32 rows a workgroup where that still gives every compute unit one (4096 x 768, one
+    // token, 14.7 -> 15.3 us a layer with 32 and 13.6 with 16).
+    const bool pair = a.layout.n_ff <= 1024;
 #define MAYA_ROWS(R, MINW)                                                                                                    \
     {                                                                                                                         \
         const dim3 grid((unsigned) (n_embd / R), (unsigned) a.n_tokens);                                                      \
@@ -1636,7 +1639,15 @@ int launch_down_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStrea
         else hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, 4, 16, 0>), grid, dim3(1024), 0, s, MAYA_DN_HEAD, a, st.cb);       \
     }
 #define MAYA_DN_HEAD a.plan_ptr, a.plan_w, a.h, st.cb.iq2s, a.skip, a.hq.q, a.k, n_embd, a.layout.n_ff >> 5
-    switch (wide) {
+#define MAYA_PAIR(R)                                                                                                          \
+    {                                                                                                                         \
+        const dim3 grid((unsigned) (n_embd / R), (unsigned) a.n_tokens);                                                      \
+        if (a.k <= 8) hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, 6, 8, 0, true>), grid, dim3(512), 0, s, MAYA_DN_HEAD, a, st.cb);   \
+        else hipLaunchKernelGGL((down_iq2s_pos_kernel<R, 1, 4, 16, 0, true>), grid, dim3(1024), 0, s, MAYA_DN_HEAD, a, st.cb);  \
+    }
+    if (pair && n_embd % 32 == 0 && n_embd / 32 * a.n_tokens >= 256) MAYA_PAIR(32)
+    else if (pair) MAYA_PAIR(16)
+    else switch (wide) {
         case 20: MAYA_ROWS(20, 4) break;
         case 24: MAYA_ROWS(24, 4) break;
         case 28: MAYA_ROWS(28, 4) break;
@@ -1645,6 +1656,7 @@ int launch_down_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipStrea
     }
 #undef MAYA_DN_HEAD
 #undef MAYA_ROWS
+#undef MAYA_PAIR
     MAYA_LAUNCHED("down_iq2s_pos_kernel");
     return MAYA_OK;
 }
@@ -1776,20 +1788,27 @@ int launch_gate_up_iq2xxs_pos(const maya_moe_args& a, const DeviceState& st, hip
 }
 int launch_down_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
     // 32 rows a workgroup for the wide rows (half as many waves rounding h, as in the IQ2_S kernel), else 16.
-    // (7 waves a SIMD leave the 53 and 64 registers the kernels take; of 16 slots one workgroup is 4 waves a SIMD already)
-    const bool wide = a.layout.n_embd >= 5120 && a.layout.n_embd % 32 == 0;
+    // (workgroups of 8 waves: three of them are 6 waves a SIMD, 84 registers; of 16 slots one workgroup is 4 waves a SIMD already)
+    const bool pair = a.layout.n_ff <= 1024;   // (as launch_down_iq2s_pos)
+    const bool wide = (pair ? a.layout.n_embd / 32 * a.n_tokens >= 256 : a.layout.n_embd >= 5120) && a.layout.n_embd % 32 == 0;
     const dim3 grid((unsigned) (a.layout.n_embd / (wide ? 32 : 16)), (unsigned) a.n_tokens);
-#define MAYA_D1T(KERN, R)                                                                                                     \
-    if (a.k <= 8 && a.layout.n_ff == 2048) hipLaunchKernelGGL((KERN<R, 7, 8, 64>), grid, dim3(512), 0, s, a, st.cb);            \
-    else if (a.k <= 8) hipLaunchKernelGGL((KERN<R, 7, 8, 0>), grid, dim3(512), 0, s, a, st.cb);                                 \
-    else hipLaunchKernelGGL((KERN<R, 4, 16, 0>), grid, dim3(1024), 0, s, a, st.cb);
-#define MAYA_D1(R)                                                                     \
-    if (a.layout.down_type == kIQ1_M) { MAYA_D1T(down_iq1m_pos_kernel, R) }              \
-    else { MAYA_D1T(down_iq1s_pos_kernel, R) }
+#define MAYA_D1L(F, R, MINW, SLOTS, NU, PAIR)                                                                                          \
+    hipLaunchKernelGGL((down_iq1_pos_kernel<F, R, MINW, SLOTS, NU, PAIR>), grid, dim3(64 * SLOTS), 0, s, a.plan_ptr, a.plan_w, a.h, st.cb.iq1s, \
+                       a.skip, a.hq.q, a.k, (int) a.layout.n_embd, a.layout.n_ff >> 5, a);
+#define MAYA_D1T(F, R)                                             \
+    if (a.k <= 8 && pair) MAYA_D1L(F, R, 6, 8, 0, true)             \
+    else if (pair) MAYA_D1L(F, R, 4, 16, 0, true)                   \
+    else if (a.k <= 8 && a.layout.n_ff == 2048) MAYA_D1L(F, R, 6, 8, 64, false) \
+    else if (a.k <= 8) MAYA_D1L(F, R, 6, 8, 0, false)               \
+    else MAYA_D1L(F, R, 4, 16, 0, false)
+#define MAYA_D1(R)                                                      \
+    if (a.layout.down_type == kIQ1_M) { MAYA_D1T(DownIq1M, R) }          \
+    else { MAYA_D1T(DownIq1S, R) }
     if (wide) { MAYA_D1(32) } else { MAYA_D1(16) }
 #undef MAYA_D1
 #undef MAYA_D1T
-    MAYA_LAUNCHED("down_iq1s_pos_kernel");
+#undef MAYA_D1L
+    MAYA_LAUNCHED("down_iq1_pos_kernel");
     return MAYA_OK;
 }
 

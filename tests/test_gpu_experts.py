@@ -151,6 +151,31 @@ def test_iq2_xxs_gate_rows_at_any_two_byte_address(lib, oracle, n_embd, n_ff, ne
     assert np.array_equal(alone[0].view(np.int32), packed[nt - 1].view(np.int32))
 
 
+@pytest.mark.parametrize("gt,dt,n_embd,n_ff,ne,k,nt", (
+    (22, 22, 2048, 256, 6, 1, 5),      # 8 positions a half wave, one slot; a grid of 16 rows a workgroup either way
+    (19, 19, 4096, 1024, 12, 9, 2),    # full halves, more than 8 slots; 32 rows a workgroup for two tokens, 16 for one
+    (29, 29, 8192, 768, 6, 3, 3),      # idle lanes in either half; 32 rows both
+    (19, 22, 2816, 1024, 8, 8, 3),
+    (22, 29, 2304, 512, 4, 2, 4),
+))
+def test_down_rows_of_up_to_1024_values(lib, oracle, gt, dt, n_embd, n_ff, ne, k, nt):
+    """Two quads of rows a wave: against the CPU path, and bit for bit what each token gives alone, with an expert that is not resident."""
+    blobs = make_experts(gt, dt, n_embd, n_ff, ne, 1700 + nt)
+    rng = np.random.default_rng(1701 + nt)
+    logits = rng.standard_normal((nt, ne)).astype(np.float32)
+    x = rng.standard_normal((nt, n_embd)).astype(np.float32)
+    ids, _, out, _ = run_layer(lib, gt, dt, blobs, k, n_embd, n_ff, logits, x, packing=1)
+    wi, _, wout = oracle_layer(oracle, gt, dt, blobs, k, n_embd, n_ff, logits, x)
+    assert np.array_equal(ids, wi)
+    for t in range(nt):
+        assert rel_l2(out[t], wout[t]) <= TOL, t
+    here = set(range(ne)) - {int(wi[0, 0])}
+    many = run_layer(lib, gt, dt, blobs, k, n_embd, n_ff, logits, x, packing=1, resident=here)[2]
+    for t in range(nt):
+        one = run_layer(lib, gt, dt, blobs, k, n_embd, n_ff, logits[t:t + 1], x[t:t + 1], packing=1, resident=here)[2]
+        assert np.array_equal(one[0].view(np.int32), many[t].view(np.int32)), t
+
+
 def encoded_q4k_expert(oracle, n_embd, n_ff, seed):
     """One expert as BASELINE's single-expert configuration states it: gate / up [n_ff x n_embd] and down [n_embd x n_ff]
     drawn from N(0, 0.02) in F32 and quantized to Q4_K (the checker's own encoder: the reference never quantizes weights)."""
