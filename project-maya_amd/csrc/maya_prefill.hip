@@ -341,7 +341,8 @@ typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 // load leaves of 2.4; few rows an expert stream their weights at 3.2 TB/s, of 5.2 without arithmetic.
 constexpr int kPfGroups = 4;                         // row groups of a workgroup at most: two of the plan's tiles
 constexpr int kPfRing = 4;                           // activations of a pass in LDS, three passes ahead
-constexpr int kPfSlotS = 8192, kPfSlotD = kPfSlotS + 1024, kPfSlot = kPfSlotD + 256;   // codes [32][256], sums [32][16], scales [32]
+constexpr int kPfPlane = 32 * 256;                   // codes of a pass
+constexpr int kPfSlotS = kPfPlane, kPfSlotD = kPfSlotS + 1024, kPfSlot = kPfSlotD + 256;   // codes [32][256], sums [32][16], scales [32]
 
 // The tile's activations, a row group of a super-block at a time.  Every group but the last is whole: its copies are the first
 // one's at another scalar offset.  Rows past the tile's end repeat its last row (their results are never stored).
