@@ -1526,6 +1526,15 @@ int launch_down_t(const maya_moe_args& a, const DeviceState& st, hipStream_t s) 
 // the entries an expert, without turning over: 16 tokens on one expert of 2816 x 1280, Q4_K 158 -> 29, IQ2_S 111 -> 45; top-10 of 16
 // experts 498 -> 125 and 337 -> 172, IQ2_XXS gate/up with IQ2_S down 206 -> 94; all of 16 experts, IQ2_S 4096 x 2048, 451 -> 406.
 static bool pos_row_ok(int n_embd) { return n_embd % 256 == 0 && n_embd >= 256 && n_embd <= 8192; }
+// A blob's matrices may lie in any order, but the position-mapped gate/up kernels hold the way from the gate rows to the up rows in 32
+// bits, and those of the stream packing read both inside down_off - gate_off bytes from the gate rows on (32 bits too, so down rows in
+// front of the gate rows only make that longer).  Other orders are the general kernels'.
+static bool gate_up_rows_ok(const maya_moe_layout& l) {
+    const uint64_t gate = (uint64_t) (l.n_embd / block_values(l.gate_type)) * block_bytes(l.gate_type) * l.n_ff;
+    const uint64_t up = (uint64_t) (l.n_embd / block_values(l.up_type)) * block_bytes(l.up_type) * l.n_ff;
+    const uint64_t lim = l.packing == MAYA_PACK_STREAM ? (uint64_t) (uint32_t) (l.down_off - l.gate_off) : 0xffffffffull;
+    return l.up_off >= l.gate_off && l.up_off - l.gate_off <= lim && up <= lim - (l.up_off - l.gate_off) && gate <= lim;
+}
 static int pos_waves(int n_embd) { return n_embd <= 2048 ? 2 : (n_embd + 1023) / 1024; }
 static bool down_pos_nff_ok(int n_ff) { return n_ff % 256 == 0 && n_ff >= 256 && n_ff <= 2048; }
 
@@ -1606,7 +1615,7 @@ static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& r
         return false;
     if (l.gate_type == kQ4_K) return gate_up_q4k_pos_ok(a);
     if (l.gate_type == kIQ1_S) return gate_up_iq1s_pos_ok(a);
-    return l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && l.n_ff % 16 == 0 && pos_row_ok(l.n_embd);
+    return l.gate_type == kIQ2_S && l.up_type == kIQ2_S && l.packing == MAYA_PACK_STREAM && l.n_ff % 16 == 0 && pos_row_ok(l.n_embd) && gate_up_rows_ok(l);
 }
 static int launch_layer_gate_up_iq2s(const maya_moe_args& a, const LayerHeadIn& hd, const DeviceState& st, hipStream_t s) {
     switch (pos_waves(a.layout.n_embd)) {
@@ -1679,7 +1688,7 @@ int try_gate_up_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStre
     // (the position-mapped kernels take the entries of several tokens one by one, whether grouped or not: every entry
     // is computed as its token alone would compute it)
     if (l.packing == MAYA_PACK_STREAM) {
-        if (l.n_ff % 16 != 0) return 0;
+        if (l.n_ff % 16 != 0 || !gate_up_rows_ok(l)) return 0;
         if (a.n_tokens == 1) {
             switch (pos_row_ok(l.n_embd) ? pos_waves(l.n_embd) : 0) {
                 case 2: *rc = launch_gate_up_iq2s_tiles<2>(a, st, s); return 1;
@@ -1711,7 +1720,7 @@ int try_gate_up_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStre
 bool gate_up_iq1s_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (!((l.gate_type == kIQ1_S || l.gate_type == kIQ1_M) && l.up_type == l.gate_type && l.packing == MAYA_PACK_STREAM)) return false;
-    return pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
+    return pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && gate_up_rows_ok(l) && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
 }
 bool down_iq1s_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
@@ -1765,7 +1774,7 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
 // ---- IQ2_XXS (either packing: the type's rows stay in GGUF order)
 bool gate_up_iq2xxs_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    return l.gate_type == kIQ2_XXS && l.up_type == kIQ2_XXS && pos_row_ok(l.n_embd) && l.n_ff % 16 == 0;
+    return l.gate_type == kIQ2_XXS && l.up_type == kIQ2_XXS && pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && gate_up_rows_ok(l);
 }
 int launch_gate_up_iq2xxs_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
     const dim3 grid((unsigned) (a.layout.n_ff / 16), (unsigned) (a.n_tokens * a.k));
@@ -1836,7 +1845,7 @@ int try_down_iq2s_1tok(const maya_moe_args& a, const DeviceState& st, hipStream_
 bool gate_up_q4k_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (!(l.gate_type == kQ4_K && l.up_type == kQ4_K && l.packing == MAYA_PACK_STREAM)) return false;
-    return pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
+    return pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && gate_up_rows_ok(l) && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
 }
 bool down_q4k_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
@@ -1903,7 +1912,7 @@ int launch_down_q4k_pos(const maya_moe_args& a, hipStream_t s) {
 bool gate_up_q80_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
     if (!(l.gate_type == kQ8_0 && l.up_type == kQ8_0 && l.packing == MAYA_PACK_STREAM)) return false;
-    return pos_row_ok(l.n_embd) && l.n_ff % 8 == 0 && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
+    return pos_row_ok(l.n_embd) && l.n_ff % 8 == 0 && gate_up_rows_ok(l) && ((l.gate_off | l.up_off | l.down_off) & 15) == 0;
 }
 bool down_q80_pos_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
@@ -1980,7 +1989,7 @@ int down_q80(const maya_moe_args& a, hipStream_t s) {
 // the shapes the IQ2_S streaming kernels take (what try_gate_up_iq2s_1tok / try_down_iq2s_1tok launch on)
 static bool gate_up_iq2s_fast_ok(const maya_moe_args& a) {
     const maya_moe_layout& l = a.layout;
-    if (l.packing == MAYA_PACK_STREAM) return l.n_ff % 16 == 0 && pos_row_ok(l.n_embd);
+    if (l.packing == MAYA_PACK_STREAM) return l.n_ff % 16 == 0 && pos_row_ok(l.n_embd) && gate_up_rows_ok(l);
     return fast_1tok(a) && l.n_embd % 1024 == 0 && l.n_embd <= 8192 && l.n_ff % 32 == 0;
 }
 static bool down_iq2s_fast_ok(const maya_moe_args& a) {

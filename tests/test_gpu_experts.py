@@ -126,6 +126,34 @@ def test_layer_matches_cpu_path(lib, oracle, gt, dt, n_embd, n_ff, ne, k, nt, pa
         assert rel_l2(out[t], wout[t]) <= TOL, (t, rel_l2(out[t], wout[t]))
 
 
+@pytest.mark.parametrize("nt", (1, 3))
+@pytest.mark.parametrize("order", ("ugd", "gdu", "dgu"))
+@pytest.mark.parametrize("t,packing", ((16, 0), (22, 1), (12, 1), (8, 1), (19, 1), (29, 1)))
+def test_matrices_of_a_blob_in_any_order(lib, oracle, t, packing, order, nt):
+    """The offsets of a layout say where a blob's matrices lie: up rows in front of the gate rows, down rows between or first."""
+    n_embd, n_ff, ne, k = 1024, 512, 5, 3
+    blobs = make_experts(t, t, n_embd, n_ff, ne, 900 + t)
+    plain, nbytes = lib.layout(t, t, n_embd, n_ff)
+    part = {"g": (0, plain.up_off), "u": (plain.up_off, plain.down_off), "d": (plain.down_off, nbytes)}
+    moved, _ = lib.layout(t, t, n_embd, n_ff)
+    at = 0
+    for m in order:
+        setattr(moved, {"g": "gate_off", "u": "up_off", "d": "down_off"}[m], at)
+        at += part[m][1] - part[m][0]
+    store = lib.ExpertStore([np.concatenate([b[slice(*part[m])] for m in order]) for b in blobs], pack_layout=moved if packing else None)
+    rng = np.random.default_rng(901 + t)
+    logits = rng.standard_normal((nt, ne)).astype(np.float32)
+    x = rng.standard_normal((nt, n_embd)).astype(np.float32)
+    layer = lib.MoeLayer(t, t, n_embd, n_ff, ne, k, max_tokens=nt, packing=packing)
+    layer.layout = lib.copy_layout(moved, packing)
+    print("case", t, packing, order, nt, flush=True)
+    out = layer.forward(store.table, dev(logits), dev(x))
+    torch.cuda.synchronize()
+    wout = oracle_layer(oracle, t, t, blobs, k, n_embd, n_ff, logits, x)[2]
+    for i in range(nt):
+        assert rel_l2(out[i].cpu().numpy(), wout[i]) <= TOL, i
+
+
 @pytest.mark.parametrize("n_embd,n_ff,ne,k,nt,misalign", (
     (256, 256, 4, 2, 3, 2),       # one block a row: 8 lanes of 64 have a position
     (2048, 512, 8, 4, 1, 0),      # rows that fill their lanes, one token
