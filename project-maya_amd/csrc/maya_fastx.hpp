@@ -47,8 +47,9 @@ __device__ __forceinline__ RowsIQ2XXS load_xxs(uint64_t mat, uint32_t row0, uint
     }
     return q;
 }
-// one sub-block against the lane's codes y and their negation yn (unit_value's way with the signs); dy8 = activation scale / 8
-__device__ __forceinline__ float xxs_value(const u32x2 w, uint32_t d, const char* lds, const int (&y)[8], const int (&yn)[8], float dy8) {
+// one sub-block against the lane's codes y and their negation yn (unit_value's way with the signs), added to the lane's chain as
+// row_dot adds it: d = activation scale
+__device__ __forceinline__ float xxs_add(const u32x2 w, uint32_t db, const char* lds, const int (&y)[8], const int (&yn)[8], float d, float acc) {
     int s = 0;
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
@@ -58,91 +59,89 @@ __device__ __forceinline__ float xxs_value(const u32x2 w, uint32_t d, const char
         s = dot4((int) g.y, (int) __builtin_amdgcn_perm((uint32_t) yn[2 * l + 1], (uint32_t) y[2 * l + 1], sl.y), s);
     }
     const int isum = __mul24(2 * (int) (w.y >> 28) + 1, s);
-    return __fmul_rn(__fmul_rn(f16_bits_to_f32((uint16_t) d), dy8), (float) isum);
+    return fmaf(__fmul_rn(__fmul_rn(f16_bits_to_f32((uint16_t) db), 0.125f), d), (float) isum, acc);
 }
-template <int B>
-__device__ __forceinline__ void xxs_values(const RowsIQ2XXS& q, const int* lds, const int (&y)[8], const int (&yn)[8], float dy8, float (&acc)[8]) {
-#define MAYA_ROW(R)                                                              \
-    acc[B + R] = xxs_value(q.w[R], q.d[R], (const char*) lds, y, yn, dy8);       \
-    asm volatile("" : "+v"(acc[B + R]));                                         \
-    __builtin_amdgcn_sched_barrier(0);
-    MAYA_ROW(0) MAYA_ROW(1) MAYA_ROW(2) MAYA_ROW(3)
-#undef MAYA_ROW
+// four rows' sub-blocks onto acc[B] ... acc[B + 3]; a lane past the row's last position (`on` false) adds nothing
+template <int B, int ROWS>
+__device__ __forceinline__ void xxs_rows(const RowsIQ2XXS& q, const int* lds, const int (&y)[8], const int (&yn)[8], float d, bool on, float (&acc)[ROWS]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float t = xxs_add(q.w[r], q.d[r], (const char*) lds, y, yn, d, acc[B + r]);
+        acc[B + r] = on ? t : acc[B + r];
+        asm volatile("" : "+v"(acc[B + r]));
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
-// ---- gate/up: gate_up_iq2s_pos_kernel's split - a workgroup of NW waves = 2 * 32 NW lanes for the sub-block positions of a (gate
-// row, up row) pair, ROWS pairs, four rows ahead; grid (n_ff / ROWS, entries).  A lane past the row's last position reads the last
-// one's words and has zero codes and scales.
-// Bound by the LDS look-ups (8 of 8 bytes a sub-block of 8 bytes).  The general kernel gave 8 waves a row pair at a time with the
-// activations read back from LDS for every row, and took 241 us where this one takes 51 (four tokens of 160 experts top-8, 6144 x 2048,
-// 188 MB); the layer with IQ2_S down 268 -> 77.6, one token 37.5 -> 27.7, 16 tokens 683 -> 275, 2816 x 1280 four tokens 107.7 -> 34.6.
-template <int NW, int ROWS, int MINW, bool FIT>
-__global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq2xxs_pos_kernel(maya_moe_args a, Codebooks cb) {
-    static_assert(ROWS % 8 == 0, "a batch is eight rows");
-    constexpr int NU = 32 * NW;
+// ---- gate/up: a wave takes ROWS (gate row, up row) pairs, the gate rows on its lanes 0 .. 31, the up rows on 32 .. 63: lane l adds the
+// sub-blocks l, l + 32, ... of a row up one behind the other, and 32 lanes meet at the end - gate_up_kernel's order, so that h is
+// its h bit for bit.  Four waves a workgroup; grid (n_ff / (4 ROWS), entries).  The walk is 32 sub-blocks at a time over all ROWS
+// pairs, so that a lane's activations of these are read and negated once, four rows' weights ahead.
+// Bound by the LDS look-ups (8 of 8 bytes a sub-block of 8 bytes) and the vector instructions between them.  The general kernel gives
+// 8 waves a row pair at a time with the activations read back from LDS for every row.  Layers with IQ2_S down, general / this: 6144 x
+// 2048 top-8 of 160, one token 38.7 / 29.5 us, four 298 / 79.6, 16 875 / 278; 2816 x 1280 top-4, four tokens 61.9 / 25.6.  A form
+// that gave a workgroup one row pair's positions side by side took 28.7, 86.0, 308 and 25.0, and summed in another order.
+template <int ROWS, int MINW>
+__global__ __launch_bounds__(256, MINW) void gate_up_iq2xxs_pos_kernel(maya_moe_args a, Codebooks cb) {
+    static_assert(ROWS == 4 || ROWS == 8, "batches of four rows");
     __shared__ __align__(16) int lds[kFastXLdsWords];
-    __shared__ float part[2][2 * NW][8];
     if (a.skip && *a.skip) return;
     const int e = (a.grp_ent && !a.grp_ptr) ? a.grp_ent[blockIdx.y] : (int) blockIdx.y;   // (the order of grp_ent: gate_up_iq2s_pos_kernel)
     if (e < 0) return;
     const uint64_t blob = a.plan_ptr[e];
     if (blob == 0ull) return;
-    const int t = threadIdx.x, lane = t & 63, hw = t >> 5;
-    const bool is_up = t >= NU;
-    const int nu = FIT ? NU : a.layout.n_embd >> 5, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
-    const bool on = FIT || lu < nu;
-    const int u = on ? lu : nu - 1;
-    const int n_ff = a.layout.n_ff, r0 = blockIdx.x * ROWS;
+    const int lane = threadIdx.x & 63, l = lane & 31, wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+    const bool is_up = lane >= 32;
+    const int nu = a.layout.n_embd >> 5, nc = (nu + 31) >> 5;   // sub-blocks a row, steps of 32
+    const int n_ff = a.layout.n_ff;
+    const uint32_t r0 = (uint32_t) ((int) blockIdx.x * 4 + wave) * ROWS;
     const uint32_t rb = (uint32_t) (nu >> 3) * 66u;   // bytes of a row
     const uint64_t mat = blob + a.layout.gate_off;
-    const uint32_t od = (is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u) + (uint32_t) (u >> 3) * 66u;
-    const uint32_t ow = od + 2u + 8u * (uint32_t) (u & 7);
-    RowsIQ2XXS nxt = load_xxs(mat, (uint32_t) r0, rb, ow, od);
-    stage_iq2xxs_tables<64 * NW>(lds, cb);
+    const uint32_t om = is_up ? (uint32_t) (a.layout.up_off - a.layout.gate_off) : 0u;
+    // (a lane past the row's last position reads the last one's words)
+    auto load = [&](int c, int b) {
+        const uint32_t u = (uint32_t) min(32 * c + l, nu - 1), od = om + (u >> 3) * 66u;
+        return load_xxs(mat, r0 + 4 * b, rb, od + 2u + 8u * (u & 7u), od);
+    };
     const int tok = e / a.k;
-    int y[8];
-    {
-        const int4* q = (const int4*) (a.x.q + (size_t) tok * (32 * nu));
-        const int4 ya = q[2 * u], yb = q[2 * u + 1];
-        y[0] = ya.x, y[1] = ya.y, y[2] = ya.z, y[3] = ya.w, y[4] = yb.x, y[5] = yb.y, y[6] = yb.z, y[7] = yb.w;
-    }
-    float dy8 = a.x.d[(size_t) tok * nu + u] * 0.125f;
-    idle_lane_zero(on, y, dy8);
-    int yn[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) yn[i] = neg4(y[i]);
+    const int4* xq = (const int4*) (a.x.q + (size_t) tok * (32 * nu));
+    const float* xd = a.x.d + (size_t) tok * nu;
+    RowsIQ2XXS nxt = load(0, 0);
+    int4 ya = xq[2 * min(l, nu - 1)], yb = xq[2 * min(l, nu - 1) + 1];
+    float dn = xd[min(l, nu - 1)];
+    stage_iq2xxs_tables<256>(lds, cb);
     __syncthreads();
-    float acc[8];
+    float acc[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) acc[i] = 0.0f;
 #pragma unroll 1
-    for (int r = 0; r < ROWS; r += 8) {
-        {
-            const RowsIQ2XXS cur = nxt;
-            nxt = load_xxs(mat, (uint32_t) (r0 + r + 4), rb, ow, od);
-            xxs_values<0>(cur, lds, y, yn, dy8, acc);
+    for (int c = 0; c < nc; ++c) {
+        const bool on = 32 * c + l < nu, more = c + 1 < nc;
+        const int y[8] = {ya.x, ya.y, ya.z, ya.w, yb.x, yb.y, yb.z, yb.w};
+        const float d = dn;
+        if (more) {
+            const int u = min(32 * (c + 1) + l, nu - 1);
+            ya = xq[2 * u], yb = xq[2 * u + 1];
+            dn = xd[u];
         }
-        {
-            const RowsIQ2XXS cur = nxt;
-            if (r + 8 < ROWS) nxt = load_xxs(mat, (uint32_t) (r0 + r + 8), rb, ow, od);
-            xxs_values<4>(cur, lds, y, yn, dy8, acc);
-        }
-        if constexpr (!FIT) {   // (an idle lane's weights are another's: a scale that is not a number stays out)
+        int yn[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] = on ? acc[i] : 0.0f;
+        for (int i = 0; i < 8; ++i) yn[i] = neg4(y[i]);
+        if constexpr (ROWS == 8) {
+            const RowsIQ2XXS cur = nxt;
+            nxt = load(c, 1);
+            xxs_rows<0>(cur, lds, y, yn, d, on, acc);
         }
-        const float v = reduce8_half(acc, lane);
-        const int buf = (r >> 3) & 1;
-        if ((lane & 3) == 0) part[buf][hw][(lane >> 2) & 7] = v;
-        __syncthreads();
-        if (t < 8) {
-            float g = part[buf][0][t], up = part[buf][NW][t];
-#pragma unroll
-            for (int w = 1; w < NW; ++w) {
-                g += part[buf][w][t];
-                up += part[buf][NW + w][t];
-            }
-            if (r0 + r + t < n_ff) a.h[(size_t) e * n_ff + r0 + r + t] = swiglu(g, up, a.limit);
-        }
+        const RowsIQ2XXS cur = nxt;
+        if (more) nxt = load(c + 1, 0);
+        xxs_rows<ROWS - 4>(cur, lds, y, yn, d, on, acc);
     }
+    float g;
+    if constexpr (ROWS == 8) g = reduce8_half(acc, lane);
+    else g = reduce4_half(acc, lane);
+    const float up = xor_lane<32>(g);
+    constexpr int each = 32 / ROWS;   // lanes that hold a row's sum
+    if (lane < 32 && lane % each == 0) a.h[(size_t) e * n_ff + r0 + lane / each] = swiglu(g, up, a.limit);
 }
 
 }  // namespace maya

@@ -1524,7 +1524,7 @@ int launch_down_t(const maya_moe_args& a, const DeviceState& st, hipStream_t s) 
 // tokens, 733 -> 143; IQ2_S gate/up with Q4_K down 4864 x 1280, eight tokens, 430 -> 89; Q8_0 2560 x 1280, six tokens, 148 -> 81.
 // The general kernels share a decode among an expert's tokens, these (but for Q8_0) decode for every entry, so the lead narrows with
 // the entries an expert, without turning over: 16 tokens on one expert of 2816 x 1280, Q4_K 158 -> 29, IQ2_S 111 -> 45; top-10 of 16
-// experts 498 -> 125 and 337 -> 172, IQ2_XXS gate/up with IQ2_S down 206 -> 94; all of 16 experts, IQ2_S 4096 x 2048, 451 -> 406.
+// experts 498 -> 125 and 337 -> 172, IQ2_XXS gate/up with IQ2_S down 276 -> 162; all of 16 experts, IQ2_S 4096 x 2048, 451 -> 406.
 static bool pos_row_ok(int n_embd) { return n_embd % 256 == 0 && n_embd >= 256 && n_embd <= 8192; }
 // A blob's matrices may lie in any order, but the position-mapped gate/up kernels hold the way from the gate rows to the up rows in 32
 // bits, and those of the stream packing read both inside down_off - gate_off bytes from the gate rows on (32 bits too, so down rows in
@@ -1777,21 +1777,15 @@ bool gate_up_iq2xxs_pos_ok(const maya_moe_args& a) {
     return l.gate_type == kIQ2_XXS && l.up_type == kIQ2_XXS && pos_row_ok(l.n_embd) && l.n_ff % 16 == 0 && gate_up_rows_ok(l);
 }
 int launch_gate_up_iq2xxs_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s) {
-    const dim3 grid((unsigned) (a.layout.n_ff / 16), (unsigned) (a.n_tokens * a.k));
-    // (compiled for 7 waves a SIMD: at 8 four registers are spilled, 51.9 -> 56.0 us for four tokens of 4096 x 2048, 275 -> 285 for 16 of 6144 x 2048)
-#define MAYA_XXS(NWV)                                                                                                                            \
-    if (a.layout.n_embd == 1024 * NWV) hipLaunchKernelGGL((gate_up_iq2xxs_pos_kernel<NWV, 16, 7, true>), grid, dim3(64 * NWV), 0, s, a, st.cb);   \
-    else hipLaunchKernelGGL((gate_up_iq2xxs_pos_kernel<NWV, 16, 7, false>), grid, dim3(64 * NWV), 0, s, a, st.cb);
-    switch (pos_waves(a.layout.n_embd)) {
-        case 2: MAYA_XXS(2) break;
-        case 3: MAYA_XXS(3) break;
-        case 4: MAYA_XXS(4) break;
-        case 5: MAYA_XXS(5) break;
-        case 6: MAYA_XXS(6) break;
-        case 7: MAYA_XXS(7) break;
-        default: MAYA_XXS(8) break;
-    }
-#undef MAYA_XXS
+    // Eight row pairs a wave where that leaves every SIMD three waves, else four (layers with IQ2_S down, four / eight: 6144 x 2048
+    // top-8, four tokens 84.8 / 79.5 us, 16 tokens 295 / 281; 4096 x 1536 top-8, two tokens, 3072 waves of eight, 30.5 / 29.6;
+    // 7168 x 2048 one token top-10, 2560 waves, 39.6 / 41.2, top-2 20.4 / 23.2).
+    // (compiled for 5 waves a SIMD: for 7 the form of four has 72 registers of the 76 it takes, and the layers above 5 to 10 % longer)
+    const int entries = a.n_tokens * a.k, n_ff = a.layout.n_ff;
+    if (n_ff % 32 == 0 && (long long) (n_ff / 8) * entries >= 3072)
+        hipLaunchKernelGGL((gate_up_iq2xxs_pos_kernel<8, 5>), dim3((unsigned) (n_ff / 32), (unsigned) entries), dim3(256), 0, s, a, st.cb);
+    else
+        hipLaunchKernelGGL((gate_up_iq2xxs_pos_kernel<4, 5>), dim3((unsigned) (n_ff / 16), (unsigned) entries), dim3(256), 0, s, a, st.cb);
     MAYA_LAUNCHED("gate_up_iq2xxs_pos_kernel");
     return MAYA_OK;
 }

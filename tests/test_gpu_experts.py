@@ -179,6 +179,49 @@ def test_iq2_xxs_gate_rows_at_any_two_byte_address(lib, oracle, n_embd, n_ff, ne
     assert np.array_equal(alone[0].view(np.int32), packed[nt - 1].view(np.int32))
 
 
+@pytest.mark.parametrize("n_embd,n_ff,ne,k,nt", (
+    (256, 256, 4, 2, 1),          # one block a row: a step of 8 lanes of 32
+    (1024, 512, 6, 4, 3),         # one whole step
+    (1280, 256, 5, 3, 16),        # a step and a part of one
+    (6144, 2048, 10, 8, 1),       # four row pairs a wave, one token
+    (6144, 2048, 10, 8, 2),       # eight
+    (2816, 1792, 12, 2, 7),       # next to the line between the two: 3136 waves of eight
+    (8192, 768, 12, 9, 3),        # the widest
+))
+def test_iq2_xxs_gate_rows_sum_as_the_general_kernel(lib, n_embd, n_ff, ne, k, nt):
+    """h of gate_up_iq2xxs_pos_kernel bit for bit gate_up_kernel's, which takes the same experts where their up rows lie in front of the
+    gate rows: the output of a layer hangs on h through int8 codes, so another order of the sums is another output."""
+    import ctypes as C
+    blobs = make_experts(16, 22, n_embd, n_ff, ne, 1650 + nt)
+    plain, _ = lib.layout(16, 22, n_embd, n_ff)
+    moved, _ = lib.layout(16, 22, n_embd, n_ff)
+    up = plain.down_off - plain.up_off
+    moved.up_off, moved.gate_off = 0, up
+    rng = np.random.default_rng(1651 + nt)
+    logits = rng.standard_normal((nt, ne)).astype(np.float32)
+    x = rng.standard_normal((nt, n_embd)).astype(np.float32)
+    x[0, :32] = -0.0
+    print("case", n_embd, n_ff, ne, k, nt, flush=True)
+    got = {}
+    for name, l, bs in (("pos", plain, blobs), ("general", moved, [np.concatenate([b[up:2 * up], b[:up], b[2 * up:]]) for b in blobs])):
+        store = lib.ExpertStore(bs, pack_layout=l)
+        ptr = lib.route_plan(dev(logits), k, store.table)[2]
+        xq, h = lib.quant_act(16, dev(x)), torch.full((nt * k, n_ff), float("nan"), device="cuda")
+        a = lib.Args()
+        a.layout, a.n_tokens, a.k = lib.copy_layout(l, lib.PACK_STREAM), nt, k
+        a.plan_ptr, a.x, a.h, a.limit = ptr.data_ptr(), xq.c(), h.data_ptr(), float("inf")
+        wts = torch.ones(nt * k, device="cuda")
+        a.plan_w = wts.data_ptr()
+        lib.check(lib.load().maya_moe_gate_up(C.byref(a), lib._stream(None)))
+        layer = lib.MoeLayer(16, 22, n_embd, n_ff, ne, k, max_tokens=nt, packing=lib.PACK_STREAM)
+        layer.layout = lib.copy_layout(l, lib.PACK_STREAM)
+        out = layer.forward(store.table, dev(logits), dev(x)).clone()
+        torch.cuda.synchronize()
+        got[name] = h, out
+    for p, g in zip(got["pos"], got["general"]):
+        assert not torch.isnan(g).any() and torch.equal(p.view(torch.int32), g.view(torch.int32))
+
+
 @pytest.mark.parametrize("gt,dt,n_embd,n_ff,ne,k,nt", (
     (22, 22, 2048, 256, 6, 1, 5),      # 8 positions a half wave, one slot; a grid of 16 rows a workgroup either way
     (19, 19, 4096, 1024, 12, 9, 2),    # full halves, more than 8 slots; 32 rows a workgroup for two tokens, 16 for one
@@ -329,7 +372,7 @@ def one_sign_rows(t, n_rows, k, rng, d=None):
 
 @pytest.mark.parametrize("where", ("up", "down"))
 @pytest.mark.parametrize("nt", (1, 3))
-@pytest.mark.parametrize("t", (8, 12, 22, 19, 29))
+@pytest.mark.parametrize("t", (8, 12, 16, 22, 19, 29))
 def test_an_infinite_scale_in_a_rows_last_block(lib, oracle, t, nt, where):
     """Rows that end inside a wave, every third with an infinite scale in its last block, all products positive: an up row gives
     +limit, a down row +Inf, in either packing - no lane past the row's end may make a NaN of it (which clamps to -limit)."""
