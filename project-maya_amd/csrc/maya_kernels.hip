@@ -2669,6 +2669,11 @@ static int layer_setup(const maya_moe_layout* l, const uint64_t* expert_table, i
 }
 
 enum { kLayerWhole = 0, kLayerBegin = 1, kLayerEnd = 2 };
+// Beside a shared expert on the second stream the head of several tokens is one launch for up to so many.  Its launches run in the head's
+// time, and what is left of them when the routed gate/up starts costs the more the more tokens there are.  One launch / two: Q4_K
+// 2048 x 768 top-8 with a Q4_K shared expert, 2 tokens 47.1 / 49.9 us, 3 48.7 / 49.5, 4 49.3 / 50.9, 8 74.2 / 72.1; IQ2_S 7168 x 2048
+// with Q4_K down, 2 tokens 92.1 / 92.8, 4 134.9 / 137.9, 8 224 / 227; IQ1_S 4096 x 1536 with an IQ2_S one, 4 tokens 69.2 / 71.2, 8 97.6 / 94.0.
+constexpr int kHeadBesideTokens = 4;
 static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, int k, const maya_router* router,
                              const float* logits, const void* x, int x_dtype, int n_tokens, float limit, const float* add,
                              int32_t* ids, float* weights, float* out, void* workspace, size_t workspace_bytes, void* stream,
@@ -2704,11 +2709,9 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
                                            : launch_gate_up_iq1s_pos(a, *st, s, &hd)))
             return rc;
         gate_up_done = true;
-    } else if (logits && n_tokens > 1 && !join && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 && x_dtype <= 2) {
-        // several tokens, one launch: route, plan, group and round x, for the routed experts' rows and a shared Q8_0 expert's.  (Not
-        // beside a shared expert on the second stream: its launches run in the head's time, and what is left of them when the
-        // routed gate/up starts costs more than the head gains: 8 tokens 235 us with two launches and 237 with one, 16 tokens
-        // 424 and 433.)
+    } else if (logits && n_tokens > 1 && n_tokens <= (join ? kHeadBesideTokens : MAYA_MAX_TOKENS) && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 &&
+               x_dtype <= 2) {
+        // several tokens, one launch: route, plan, group and round x, for the routed experts' rows and a shared Q8_0 expert's
         const bool q8k = q8k_act(l->gate_type);
         if (q80 && !q8k) sh.x = w.x;
         if ((rc = launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups,

@@ -253,3 +253,35 @@ def test_down_of_one_slot_combines_as_of_two(lib):
         (one, p1), (two, p2) = down(1, ptr1, wts, h), down(2, ptr2, w2, h2)
         assert torch.equal(one, two), (f, s)
         assert s or torch.equal(p1[::2], p2.view(T, 2, E)[::2, 0])
+
+
+@pytest.mark.parametrize("sigmoid", (False, True))
+def test_short_windows_beside_the_second_stream_take_the_one_launch_head(lib, sigmoid):
+    """Two to four tokens beside a shared expert of a type that has launches of its own: one launch less than more tokens have
+    (the head groups its plan itself), counted in captured graphs; the bits of the two calls either way."""
+    import ctypes as C
+    gt, st, E, FF, NE, TK = Q4_K, Q4_K, 2048, 768, 24, 8
+    w = build(lib, gt, gt, st, E, FF, NE, TK, 8, 620)
+    bias = torch.zeros(NE, device="cuda")
+    router = lib.Router(lib.ROUTER_SIGMOID, 1, bias.data_ptr(), 2.5) if sigmoid else None
+    dense = {T: lib.DenseExpert(st, st, E, FF, T, w["sh_packed"].data_ptr(), packing=lib.PACK_STREAM) for T in (2, 4, 5)}
+    hip, s, kernels = C.CDLL("libamdhip64.so"), torch.cuda.Stream(), {}
+    for T in dense:
+        logits, x, _ = inputs(E, NE, T, 621 + T)
+        sh = dense[T].forward(x)
+        want = w["layer"].forward(w["table"], logits, x, add=sh, router=router).clone()
+        got = w["layer"].forward(w["table"], logits, x, shared=dense[T], router=router).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), T
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g, stream=s):
+            w["layer"].forward(w["table"], logits, x, shared=dense[T], router=router, stream=torch.cuda.current_stream())
+        graph, n = C.c_void_p(g.raw_cuda_graph()), C.c_size_t(0)
+        assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+        nodes, kind = (C.c_void_p * n.value)(), C.c_int(0)
+        assert hip.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+        kernels[T] = 0
+        for node in nodes:
+            assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+            kernels[T] += kind.value == 0   # hipGraphNodeTypeKernel
+    assert kernels[2] == kernels[4] == kernels[5] - 1, kernels
