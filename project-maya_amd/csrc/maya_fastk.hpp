@@ -170,7 +170,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(MAYA_HEA
 // The leading arguments repeat fields of `a`: they arrive in scalar registers with the dispatch (down_iq2s_pos_kernel).  What
 // the kernel asks of memory first - the plan, the combine's weights, h - goes out side by side; it used to wait for the plan
 // before h, and the combine read plan and weights slot by slot at the end.
-// Measured: 2048 x 768 top-8, one token, 8.1 -> 4.6 us a launch (sixteen layers in a graph 249 -> 196 us); 7168 x 2048 top-1 5.5 -> 5.0.
+// Measured: 2048 x 768 top-8, one token, 8.1 -> 5.2 us a launch (sixteen layers in a graph 249 -> 196 us); 7168 x 2048 top-1 5.5 -> 5.0.
 template <int ROWS, int MINW, int SLOTS, int NU, bool AHEAD = false, bool PAIR = false>
 __global__ __launch_bounds__(64 * SLOTS, MINW) void down_q4k_pos_kernel(const uint64_t* __restrict__ plan_ptr, const float* __restrict__ plan_w,
                                                                   const float* __restrict__ h, const int32_t* __restrict__ skip,

@@ -1885,12 +1885,14 @@ int launch_down_q4k_pos(const maya_moe_args& a, hipStream_t s) {
                      : (long long) (n_embd / 16) * a.n_tokens < (a.k <= 2 ? 1024 : 256) && n_embd % 8 == 0 ? 8 : 16;
     const dim3 grid((unsigned) (n_embd / rows), (unsigned) a.n_tokens), block(64u * (unsigned) a.k);
     const bool full = a.layout.n_ff == 2048;
+    // (two rows a wave: compiled for 7 waves a SIMD, as at 8 two registers are spilled; layers of 8 / 7: 4096 x 1024 top-8, two tokens 27.7 / 26.9 us,
+    // eight 65.3 / 64.2, 6144 x 1024 eight 94.5 / 91.5, 2048 x 768 four 24.9 / 24.4, 7168 x 512 sixteen 124 / 126)
     const bool pair = a.layout.n_ff <= 1024;
 #define MAYA_DOWN(R, MINW, SLOTS, NU, AHEAD, PAIR) \
     hipLaunchKernelGGL((down_q4k_pos_kernel<R, MINW, SLOTS, NU, AHEAD, PAIR>), grid, block, 0, s, a.plan_ptr, a.plan_w, a.h, a.skip, a.hq.q, a.k, n_embd, a.layout.n_ff >> 5, a);
 #define MAYA_ROWS(R, MINW, AHEAD)                                    \
     if (a.k <= 8 && full) { MAYA_DOWN(R, MINW, 8, 64, AHEAD, false) } \
-    else if (a.k <= 8 && pair) { MAYA_DOWN(R, MINW, 8, 0, AHEAD, true) } \
+    else if (a.k <= 8 && pair) { MAYA_DOWN(R, (AHEAD ? MINW : 7), 8, 0, AHEAD, true) } \
     else if (a.k <= 8) { MAYA_DOWN(R, MINW, 8, 0, AHEAD, false) }     \
     else if (pair) { MAYA_DOWN(R, MINW, 16, 0, AHEAD, true) }         \
     else { MAYA_DOWN(R, MINW, 16, 0, AHEAD, false) }

@@ -43,17 +43,29 @@ def constant(text, name, known):
     return int(eval(re.search(r"\b%s = ([^,;]+)[,;]" % name, text).group(1), {}, known))
 
 
-def test_the_iq2s_prompt_kernels_have_no_lds_but_their_array():
-    """Their tables' look-ups count LDS addresses from 0: a second object there is refused at the first call, and seen here first."""
+def built():
     lib = os.path.join(ROOT, "project-maya_amd", "libmaya_moe.so")
     if not os.path.exists(lib):
         from maya_amd import build
         build.build()
+    return lib
+
+
+def test_kernels_of_rows_a_wave_spill_nothing():
+    """Register limits are chosen so that the loops over weight rows keep everything in registers."""
+    got = {n: k for n, k in kernels(built()).items() if "down_q4k_pos_kernel" in n or "gate_up_iq2xxs_pos_kernel" in n}
+    assert len(got) >= 10
+    for n, k in got.items():
+        assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, n
+
+
+def test_the_iq2s_prompt_kernels_have_no_lds_but_their_array():
+    """Their tables' look-ups count LDS addresses from 0: a second object there is refused at the first call, and seen here first."""
     text = open(os.path.join(CSRC, "maya_prefill.hip")).read() + open(os.path.join(CSRC, "maya_prefill_iq2s.hpp")).read()
     known = {}
     for name in ("kPfRows", "kPfPlane", "kPfDOffNoS", "kPfBufBytesNoS", "kIqSigns", "kIqScales", "kIqTables", "kIqLdsBytes"):
         known[name] = constant(text, name, known)
-    got = {n: k for n, k in kernels(lib).items() if "prefill_iq2s_kernel" in n}
+    got = {n: k for n, k in kernels(built()).items() if "prefill_iq2s_kernel" in n}
     assert len(got) == 2
     for n, k in got.items():
         assert k[".group_segment_fixed_size"] == known["kIqLdsBytes"], n
