@@ -384,8 +384,9 @@ int maya_moe_layer_decode_static(const maya_moe_layout* l, const uint64_t* exper
  * format of src/prefill/moe_fused_rdna4.cu:87-109 and its requantized H, :620-660).
  * Entry e = t * k + j is token t's j-th expert.  The plan sorts the entries by expert, stably: expert x's rows are
  * bounds[x] .. bounds[x + 1], row r serves entry row_entry[r], entry e sits at row entry_row[e] (-1: its expert is not
- * resident or its id is out of range).  Tiles of at most maya_moe_prefill_tile_rows() rows of one expert are what a
- * workgroup of the GEMM kernels takes; all counts stay on the device, so nothing here synchronises. */
+ * resident or its id is out of range).  The tiles are of at most maya_moe_prefill_tile_rows() rows of one expert; a workgroup
+ * of the GEMM kernels takes a listed tile, or two that follow each other in an expert's rows and on the list.  The rows of the listed
+ * tiles, and no others, are computed.  All counts stay on the device, so nothing here synchronises. */
 typedef struct maya_prefill_plan {
     int32_t* bounds;      /* [n_expert + 1] */
     int32_t* row_entry;   /* [n_entries] */

@@ -339,7 +339,6 @@ typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 // top-8 of 256 experts of 7168 x 2048 under a skewed routing (70 of its 93 experts with 24 rows or fewer), 627 -> 520 and 336 ->
 // 291.  What bounds it: on full tiles vector issue (59 % of the cycles) and matrix time (50 %), at the 1.75 GHz that this
 // load leaves of 2.4; few rows an expert stream their weights at 3.2 TB/s, of 5.2 without arithmetic.
-constexpr int kPfGroups = 4;                         // row groups of a workgroup at most: two of the plan's tiles
 constexpr int kPfRing = 4;                           // activations of a pass in LDS, three passes ahead
 constexpr int kPfPlane = 32 * 256;                   // codes of a pass
 constexpr int kPfSlotS = kPfPlane, kPfSlotD = kPfSlotS + 1024, kPfSlot = kPfSlotD + 256;   // codes [32][256], sums [32][16], scales [32]
@@ -676,15 +675,21 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
     });
 }
 
-// The workgroup's rows: the tile and, of the same expert, the next one.  False where there are none: past the last tile, or the
-// workgroup of the tile before takes them.
+// The workgroup's rows: a listed tile, and with it the next one on the list where that goes on with the expert's rows and starts in
+// the middle of 128 of them.  False where there are none: past the last tile, or the workgroup of the tile before takes them.
+// (Both sides read the list itself, so a caller's part of it is what is computed.)
+static_assert(2 * kPfRows == 4 * 32, "four row groups of a workgroup at most");
 struct PfTile { int ex, row0, nrows; };
 __device__ __forceinline__ bool pf_my_tile(const PfGemm& a, PfTile& t) {
-    const int tile = blockIdx.y;
-    if (tile >= *a.plan.n_tiles) return false;
+    const int tile = blockIdx.y, n = *a.plan.n_tiles;
+    if (tile >= n) return false;
     t.ex = a.plan.tile_expert[tile], t.row0 = a.plan.tile_row0[tile];
-    if ((t.row0 - a.plan.bounds[t.ex]) % (32 * kPfGroups) != 0) return false;
-    t.nrows = min(32 * kPfGroups, a.plan.bounds[t.ex + 1] - t.row0);
+    const int before = max(tile - 1, 0), behind = min(tile + 1, n - 1);
+    const int bx = a.plan.tile_expert[before], b0 = a.plan.tile_row0[before], nx = a.plan.tile_expert[behind], n0 = a.plan.tile_row0[behind];
+    const int first = a.plan.bounds[t.ex], at = (t.row0 - first) % (2 * kPfRows);
+    if (at == kPfRows && bx == t.ex && b0 == t.row0 - kPfRows) return false;
+    const bool two = at == 0 && nx == t.ex && n0 == t.row0 + kPfRows;
+    t.nrows = min(two ? 2 * kPfRows : kPfRows, a.plan.bounds[t.ex + 1] - t.row0);
     return true;
 }
 

@@ -234,6 +234,46 @@ def test_experts_of_every_number_of_row_groups(pf, oracle, t, n_embd, n_ff):
             assert rel_l2(part[row], want) <= 1e-5, (EDGE_ROWS[e], r)
 
 
+@pytest.mark.parametrize("t, n_embd, n_ff", [(Q4_K, 512, 256), (22, 512, 512)], ids=str)
+def test_a_part_of_the_tile_list(pf, oracle, t, n_embd, n_ff):
+    """A caller may hand on some of a plan's tiles - a chunk in two halves, every second tile, one tile, any order: their rows are the
+    whole list's bit for bit, and no other row is written."""
+    from maya_amd import lib
+    import synth
+    rows = [300, 64, 10, 129, 65]
+    ne = len(rows)
+    gen = np.random.default_rng(17)
+    blobs = make_blobs(oracle, ne, n_embd, n_ff, 17) if t == Q4_K else [synth.expert_blob(t, t, n_embd, n_ff, gen) for _ in range(ne)]
+    layout, _ = lib.layout(t, t, n_embd, n_ff)
+    table = lib.ExpertStore(blobs, pack_layout=layout)
+    layout = lib.copy_layout(layout, lib.PACK_STREAM)
+    ids = np.repeat(np.arange(ne, dtype=np.int32), rows)
+    gen.shuffle(ids)
+    x = dev(gen.standard_normal((ids.size, n_embd)).astype(np.float32))
+    p = pf.plan(dev(ids), table.table)
+    xq = pf.quant(x, p, 1)
+    hq = pf.gate_up(layout, table.table, p, xq)
+    part = pf.down(layout, table.table, p, hq)
+    n = int(p.n_tiles.item())
+    tile_ex, tile_row0, bounds = (v.cpu().numpy() for v in (p.tile_expert[:n], p.tile_row0[:n], p.bounds))
+    assert n == sum(-(-r // 64) for r in rows)
+    assert bool((hq.f32 != 0).any(1).all()) and bool((part != 0).any(1).all())
+    lists = [range(n // 2), range(n // 2, n), range(0, n, 2), range(1, n, 2), [3], [1, 2], [0, 2, 3], range(n - 1, -1, -1), []]
+    for which in lists:
+        which = list(which)
+        q = pf.plan(dev(ids), table.table)
+        want = np.zeros(ids.size, dtype=bool)
+        for i, j in enumerate(which):
+            q.tile_expert[i], q.tile_row0[i] = int(tile_ex[j]), int(tile_row0[j])
+            want[tile_row0[j]:min(tile_row0[j] + 64, bounds[tile_ex[j] + 1])] = True
+        q.n_tiles.fill_(len(which))
+        print("tiles", which, flush=True)
+        for whole, some in ((hq.f32, pf.gate_up(layout, table.table, q, xq).f32), (part, pf.down(layout, table.table, q, hq))):
+            on = torch.from_numpy(want).cuda()
+            assert torch.equal(some[on].view(torch.int32), whole[on].view(torch.int32)), which
+            assert not bool(some[~on].any()), which
+
+
 IQ_CASES = [
     # gate/up type, down type, n_embd, n_ff, n_expert, k, n_tokens, limit, experts that are not resident
     (22, 22, 512, 512, 6, 2, 41, 0.0, ()),
