@@ -352,6 +352,8 @@ int maya_moe_layer_decode_end(const maya_moe_layout* l, const uint64_t* expert_t
  *   entries, plan_ptr all its blob, plan_w all 1, its groups (one group of n_tokens entries), its own x / h / hq (NULL
  *   where the down kernel rounds h itself) / part buffers, `add` the layer's residual or NULL, `out` its own
  *   [n_tokens][n_embd] buffer (not the layer's out).
+ *   Its h and out are filled; x, hq and part are scratch, which a call fills where its launches use them (two launches on
+ *   `stream`: no hq, no part, and x only of several tokens beside routed rows that are not Q8_0).
  * The fork and the join are event records and waits, so the call may be captured in a HIP graph (maya_init() first).
  * Every refusal of the stages (status > 0) is found before the fork: such a call has launched nothing on either stream.
  * Calls on one device are serialised on the host by a lock.  The device has ONE such second stream: while `stream` is being

@@ -2626,8 +2626,6 @@ int maya_moe_layer_decode(const maya_moe_layout* l, const uint64_t* expert_table
 }
 }  // extern "C"
 
-// The layer's launches.  `q80`: a shared expert of Q8_0 rows, run between the layer's own launches on the same stream.  `join`: an event the down launch waits for (the shared expert's output, which `add` then points
-// at), *joined set once the stream waits for it.
 // The routed layer's refusals (status > 0) and its stage arguments over the carved workspace, without launching anything.
 static int layer_setup(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, int k, const maya_router* router,
                        const float* logits, const void* x, int x_dtype, int n_tokens, float limit, const float* add, int32_t* ids,
@@ -2676,6 +2674,8 @@ enum { kLayerWhole = 0, kLayerBegin = 1, kLayerEnd = 2 };
 // 2048 x 768 top-8 with a Q4_K shared expert, 2 tokens 47.1 / 49.9 us, 3 48.7 / 49.5, 4 49.3 / 50.9, 8 74.2 / 72.1; IQ2_S 7168 x 2048
 // with Q4_K down, 2 tokens 92.1 / 92.8, 4 134.9 / 137.9, 8 224 / 227; IQ1_S 4096 x 1536 with an IQ2_S one, 4 tokens 69.2 / 71.2, 8 97.6 / 94.0.
 constexpr int kHeadBesideTokens = 4;
+// The layer's launches.  `q80`: a shared expert of Q8_0 rows, run between the layer's own launches on the same stream.  `join`: an event
+// the down launch waits for (the shared expert's output, which `add` then points at), *joined set once the stream waits for it.
 static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, int k, const maya_router* router,
                              const float* logits, const void* x, int x_dtype, int n_tokens, float limit, const float* add,
                              int32_t* ids, float* weights, float* out, void* workspace, size_t workspace_bytes, void* stream,
@@ -2694,6 +2694,7 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
     const maya_act none{nullptr, nullptr, nullptr};
     const bool q80_down = down_q80_pos_ok(a);   // (that launch rounds h itself)
     maya_moe_args sh;
+    bool sh_rounded = false;
     if (q80) {
         sh = *q80;
         sh.hq = none, sh.part = nullptr;
@@ -2716,8 +2717,10 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
         // several tokens, one launch: route, plan, group and round x, for the routed experts' rows and a shared Q8_0 expert's
         const bool q8k = q8k_act(l->gate_type);
         if (q80 && !q8k) sh.x = w.x;
+        // (the head stores 16 codes and two sums at a time, maya_quant_act one: a caller's buffer that is not aligned for that is its)
+        sh_rounded = q80 && (((uintptr_t) sh.x.q & 15) | ((uintptr_t) sh.x.bsums & 3)) == 0;
         if ((rc = launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups,
-                                     x, x_dtype, l->n_embd, q8k ? w.x : none, !q8k ? w.x : q80 ? sh.x : none, as_stream(stream))))
+                                     x, x_dtype, l->n_embd, q8k ? w.x : none, !q8k ? w.x : sh_rounded ? sh.x : none, as_stream(stream))))
             return rc;
         grouped = true;
     } else if (logits && q8k_act(l->gate_type) && n_expert <= MAYA_MAX_EXPERTS && x_dtype >= 0 && x_dtype <= 2) {
@@ -2740,7 +2743,7 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
         if ((rc = maya_quant_act(l->gate_type, x, x_dtype, 0, n_tokens, l->n_embd, w.x, stream))) return rc;
     }
     if (q80 && n_tokens > 1) {
-        if (!grouped && (rc = maya_quant_act(kQ8_0, x, x_dtype, 0, n_tokens, l->n_embd, sh.x, stream))) return rc;
+        if (!sh_rounded && (rc = maya_quant_act(kQ8_0, x, x_dtype, 0, n_tokens, l->n_embd, sh.x, stream))) return rc;
         if ((rc = launch_gate_up_q80_pos(sh, as_stream(stream))) || (rc = launch_down_q80_pos(sh, as_stream(stream), true))) return rc;
     }
     if (n_tokens > 1) {

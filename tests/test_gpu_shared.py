@@ -255,17 +255,32 @@ def test_down_of_one_slot_combines_as_of_two(lib):
         assert s or torch.equal(p1[::2], p2.view(T, 2, E)[::2, 0])
 
 
+def kernels_of(call):
+    """The kernel launches of a call, counted in a captured graph."""
+    import ctypes as C
+    hip, g = C.CDLL("libamdhip64.so"), torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        call()
+    graph, n = C.c_void_p(g.raw_cuda_graph()), C.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+    nodes, kind, count = (C.c_void_p * n.value)(), C.c_int(0), 0
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+    for node in nodes:
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        count += kind.value == 0   # hipGraphNodeTypeKernel
+    return count
+
+
 @pytest.mark.parametrize("sigmoid", (False, True))
 def test_short_windows_beside_the_second_stream_take_the_one_launch_head(lib, sigmoid):
     """Two to four tokens beside a shared expert of a type that has launches of its own: one launch less than more tokens have
     (the head groups its plan itself), counted in captured graphs; the bits of the two calls either way."""
-    import ctypes as C
     gt, st, E, FF, NE, TK = Q4_K, Q4_K, 2048, 768, 24, 8
     w = build(lib, gt, gt, st, E, FF, NE, TK, 8, 620)
     bias = torch.zeros(NE, device="cuda")
     router = lib.Router(lib.ROUTER_SIGMOID, 1, bias.data_ptr(), 2.5) if sigmoid else None
     dense = {T: lib.DenseExpert(st, st, E, FF, T, w["sh_packed"].data_ptr(), packing=lib.PACK_STREAM) for T in (2, 4, 5)}
-    hip, s, kernels = C.CDLL("libamdhip64.so"), torch.cuda.Stream(), {}
+    kernels = {}
     for T in dense:
         logits, x, _ = inputs(E, NE, T, 621 + T)
         sh = dense[T].forward(x)
@@ -273,15 +288,24 @@ def test_short_windows_beside_the_second_stream_take_the_one_launch_head(lib, si
         got = w["layer"].forward(w["table"], logits, x, shared=dense[T], router=router).clone()
         torch.cuda.synchronize()
         assert torch.equal(got, want), T
-        g = torch.cuda.CUDAGraph(keep_graph=True)
-        with torch.cuda.graph(g, stream=s):
-            w["layer"].forward(w["table"], logits, x, shared=dense[T], router=router, stream=torch.cuda.current_stream())
-        graph, n = C.c_void_p(g.raw_cuda_graph()), C.c_size_t(0)
-        assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0
-        nodes, kind = (C.c_void_p * n.value)(), C.c_int(0)
-        assert hip.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
-        kernels[T] = 0
-        for node in nodes:
-            assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
-            kernels[T] += kind.value == 0   # hipGraphNodeTypeKernel
+        kernels[T] = kernels_of(lambda: w["layer"].forward(w["table"], logits, x, shared=dense[T], router=router, stream=torch.cuda.current_stream()))
     assert kernels[2] == kernels[4] == kernels[5] - 1, kernels
+
+
+def test_a_shared_q8_0_experts_sums_at_any_two_byte_address(lib):
+    """The head of several tokens stores two code sums at a time: where the caller's buffer is not aligned for that, x is rounded by a
+    launch of its own, as maya_quant_act takes any buffer - the same codes, sums and outputs."""
+    gt, E, FF, NE, TK, T = Q4_K, 2304, 768, 20, 4, 3
+    w = build(lib, gt, gt, Q8_0, E, FF, NE, TK, T, 640)
+    logits, x, _ = inputs(E, NE, T, 641)
+    call = lambda: w["layer"].forward(w["table"], logits, x, shared=w["dense"], stream=torch.cuda.current_stream())  # noqa: E731
+    want = call().clone()
+    torch.cuda.synchronize()
+    plain, sums = kernels_of(call), w["dense"].xq.bsums.clone()
+    off = torch.zeros(T * (E // 16) + 1, dtype=torch.int16, device="cuda")[1:]
+    assert off.data_ptr() % 4 == 2
+    w["dense"].args.x.bsums = off.data_ptr()
+    got = call().clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and torch.equal(off.view(T, -1), sums)
+    assert kernels_of(call) == plain + 1
