@@ -266,11 +266,6 @@ __device__ __forceinline__ float pf_swiglu(float g, float u, float limit) {
 }
 
 typedef unsigned short pf_u16x2 __attribute__((ext_vector_type(2)));
-// four 4-bit codes (one a byte) times a factor <= 7: no byte overflows, so one packed 16-bit multiply does it
-__device__ __forceinline__ uint32_t pf_scale_codes(uint32_t w, uint32_t f) {
-    const pf_u16x2 ff = {(unsigned short) f, (unsigned short) f};
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(pf_u16x2, w) * ff);
-}
 
 // LDS reads of the GEMM loop are written out by hand.  The compiler cannot tell which LDS buffer a direct-to-LDS copy
 // fills, so before any LDS read of its own it waits for every copy in flight - here that would be the copy of the
@@ -867,8 +862,7 @@ static int prefill_check(const char* what, const maya_moe_layout* l, const uint6
         return fail(MAYA_E_UNSUPPORTED, "%s: IQ2_S rows are taken in the stream packing (maya_moe_repack)", what);
     if (l->n_embd <= 0 || l->n_ff <= 0 || l->n_embd % 256 || l->n_ff % 256)
         return fail(MAYA_E_SHAPE, "%s: n_embd %d / n_ff %d: multiples of 256 wanted", what, l->n_embd, l->n_ff);
-    // (IQ2_S: refused since the kernel's first form, whose 16-byte copies wanted quads - 328 bytes a block - of a multiple of 16 bytes.
-    // The present one reads 8 bytes at a time; a last block of its own has not been tried on it.)
+    // (IQ2_S: the kernel's 16-byte copies into LDS want quads - 328 bytes a block - of a multiple of 16 bytes: an even number of blocks)
     if (type_a == kIQ2_S && k % 512) return fail(MAYA_E_SHAPE, "%s: IQ2_S rows of %lld values: a multiple of 512 wanted", what, (long long) k);
     if (type_a == kIQ2_S) {
         int rc = prefill_iq2s_lds_ok<true>(what);

@@ -130,14 +130,11 @@ template <bool GU> struct PfIq2s {
             wh[i] = (int) __builtin_amdgcn_perm((uint32_t) l.sc[3], (uint32_t) l.sc[2], q[i]);
         }
     }
-    __device__ __forceinline__ v4i codes(const Row&, int) const { return v4i{0, 0, 0, 0}; }   // (no tile of one plane)
 };
-// (a slot of the activations' ring; the sums' place in it stays empty, as the weights have no minimums)
-constexpr int kPfDOffNoS = kPfPlane + 1024, kPfBufBytesNoS = kPfDOffNoS + 256;
-static_assert(kPfDOffNoS == kPfSlotD && kPfBufBytesNoS == kPfSlot && kPfRing == 4 && PfIq2s<true>::kWave == 2816, "the sum below");
-constexpr int kIqLdsBytes = kIqTables + 4 * kPfBufBytesNoS + 2 * 4 * 2816;   // tables, ring, the weights [2][4 waves]
-static_assert(kIqLdsBytes == PfLds<PfIq2s<true>>::bytes);
-static_assert(kIqLdsBytes == PfLds<PfIq2s<false>>::bytes && kIqLdsBytes <= 80 * 1024, "two workgroups a compute unit");
+// tables, the activations' ring (the sums' place in a slot stays empty, as the weights have no minimums), the weights [2][4 waves]
+constexpr int kIqLdsBytes = 70912;
+static_assert(kIqLdsBytes == PfLds<PfIq2s<true>>::bytes && kIqLdsBytes == PfLds<PfIq2s<false>>::bytes);
+static_assert(kIqLdsBytes <= 80 * 1024, "two workgroups a compute unit");
 
 // grid (bands of weight rows, tiles at most)
 template <bool GU>

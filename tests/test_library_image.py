@@ -39,10 +39,6 @@ def code_object_kernels(e):
                 yield from ((k[".name"], k) for k in msgpack.unpackb(e[desc:desc + desc_size], strict_map_key=False)["amdhsa.kernels"])
 
 
-def constant(text, name, known):
-    return int(eval(re.search(r"\b%s = ([^,;]+)[,;]" % name, text).group(1), {}, known))
-
-
 def built():
     lib = os.path.join(ROOT, "project-maya_amd", "libmaya_moe.so")
     if not os.path.exists(lib):
@@ -61,11 +57,8 @@ def test_kernels_of_rows_a_wave_spill_nothing():
 
 def test_the_iq2s_prompt_kernels_have_no_lds_but_their_array():
     """Their tables' look-ups count LDS addresses from 0: a second object there is refused at the first call, and seen here first."""
-    text = open(os.path.join(CSRC, "maya_prefill.hip")).read() + open(os.path.join(CSRC, "maya_prefill_iq2s.hpp")).read()
-    known = {}
-    for name in ("kPfRows", "kPfPlane", "kPfDOffNoS", "kPfBufBytesNoS", "kIqSigns", "kIqScales", "kIqTables", "kIqLdsBytes"):
-        known[name] = constant(text, name, known)
+    lds = int(re.search(r"\bkIqLdsBytes = (\d+);", open(os.path.join(CSRC, "maya_prefill_iq2s.hpp")).read()).group(1))
     got = {n: k for n, k in kernels(built()).items() if "prefill_iq2s_kernel" in n}
     assert len(got) == 2
     for n, k in got.items():
-        assert k[".group_segment_fixed_size"] == known["kIqLdsBytes"], n
+        assert k[".group_segment_fixed_size"] == lds, n
