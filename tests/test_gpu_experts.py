@@ -129,9 +129,10 @@ def test_layer_matches_cpu_path(lib, oracle, gt, dt, n_embd, n_ff, ne, k, nt, pa
 @pytest.mark.parametrize("nt", (1, 3))
 @pytest.mark.parametrize("order", ("ugd", "gdu", "dgu"))
 @pytest.mark.parametrize("t,packing", ((16, 0), (22, 1), (12, 1), (8, 1), (19, 1), (29, 1)))
-def test_matrices_of_a_blob_in_any_order(lib, oracle, t, packing, order, nt):
+@pytest.mark.parametrize("n_embd,n_ff", ((1024, 512), (2816, 256)))
+def test_matrices_of_a_blob_in_any_order(lib, oracle, n_embd, n_ff, t, packing, order, nt):
     """The offsets of a layout say where a blob's matrices lie: up rows in front of the gate rows, down rows between or first."""
-    n_embd, n_ff, ne, k = 1024, 512, 5, 3
+    ne, k = 5, 3
     blobs = make_experts(t, t, n_embd, n_ff, ne, 900 + t)
     plain, nbytes = lib.layout(t, t, n_embd, n_ff)
     part = {"g": (0, plain.up_off), "u": (plain.up_off, plain.down_off), "d": (plain.down_off, nbytes)}
