@@ -122,8 +122,8 @@ def event_time(fn, reps, stream, rounds=ROUNDS):
 # HBM bytes a step (a launch of the named kernel for the prefill chunks) read from rocprofv3's FETCH_SIZE and WRITE_SIZE
 # counters, scaled by a plain copy of known size (profiles/other_configs_hbm_traffic_pmc.txt); they belong to the
 # synthetic inputs these workloads make (fixed seeds), so they are constants here
-TRAFFIC_BYTES = {"single_q4k": 25455616, "batch8_mixed": 1097086054, "exl3_verify": 339187098,
-                 "prefill_q4k": 2032205107, "prefill_iq2s": 1224389018, "prefill_mixed": 1224389018}
+TRAFFIC_BYTES = {"single_q4k": 25477477, "batch8_mixed": 1097310892, "exl3_verify": 339203348,
+                 "prefill_q4k": 2124163105, "prefill_iq2s": 1277753024, "prefill_mixed": 1278056808}
 
 
 def hbm_roofline(kernel, bytes_launch, seconds, traffic=None):

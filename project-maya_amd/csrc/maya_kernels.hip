@@ -987,7 +987,7 @@ __global__ __launch_bounds__(256) void group_kernel(const uint64_t* __restrict__
 // It takes 6.9 us for 4 tokens of 160 experts with the sigmoid router, where a routing launch and a grouping launch behind it took
 // 10.0; without x and with the softmax router 5.4, where exact routing in workgroup 0 with the grouping behind it took 10.4.  Layers:
 // IQ1_S 6144 x 2048, 2 tokens, 44.4 -> 41.7 us, 4 tokens 77.0 -> 75.4; IQ2_S 7168 x 2048 with Q4_K down, 8 tokens, 220 -> 214.5;
-// Q4_K 2048 x 768, 3 tokens, 30.1 -> 27.5; EXL3 6144 x 1536 at 3 bits, 4 tokens, 152.3 -> 148.6.
+// Q4_K 2048 x 768, 3 tokens, 30.1 -> 27.5; EXL3 6144 x 1536 at 3 bits, 4 tokens, 153.8 -> 150.7.
 constexpr int kHeadRoute = 4, kHeadRound = 32768;   // tokens of a routing workgroup, values of a rounding one
 template <int DT>
 __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restrict__ logits, const uint64_t* __restrict__ table,
