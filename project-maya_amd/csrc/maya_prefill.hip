@@ -6,7 +6,7 @@
 // takes 32 weight rows (gate/up: the gate rows of 16 features and their up rows, so the SwiGLU stays inside the wave).  A Q4_K
 // weight is two int8 planes (its code times the low and the high 3 bits of its sub-block's scale), and v_mfma_i32_32x32x32_i8 sums
 // a whole 256-value super-block of either exactly; the two F32 scales and the minimums' term are applied once an output a
-// super-block.  Weights and activations go from HBM to LDS without registers, two super-blocks and three row groups ahead.
+// super-block.  Weights and activations go from HBM to LDS without registers, about two super-blocks and two or three row groups ahead.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -322,9 +322,13 @@ typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 //
 // Weights and activations both go to LDS without registers, and a lane reads its pieces from there.  A lane that loads its
 // own weight row from memory makes each lane of the instruction a cache access of its own: 64 clocks a compute unit for
-// 1 KB out of L2, five such loads a wave a super-block, and the data path of the cache busy 85 % of the kernel.  A copy takes a
-// row's 144 bytes by nine lanes in a run (19 clocks).  A row in LDS is 36 banks on from the one before, so the 16-byte reads of
-// 16 rows meet every bank once.
+// 1 KB out of L2, five such loads a wave a super-block, and the data path of the cache busy 85 % of the kernel; a copy takes it by
+// eight lanes in a run (16 clocks).  Q4_K rows come in pieces of 128 bytes, not in blocks of 144: a block lies in two or three
+// cache lines, two of which its neighbours ask for again, and a compute unit has about 400 line requests in flight (32 copies of
+// 144-byte runs, 48 of 128-byte ones, before the next one waits).  The copies of a super-block wait 320 clocks to be issued
+// where they waited 1265, and chunks of few rows an expert take 6 to 10 % less: 64 tokens top-8 of 256 experts of 7168 x 2048 1047 ->
+// 945 us, 256 of 288 of 4096 x 2048 848 -> 765, 512 under a skewed routing 835 -> 814; where every expert fills its tiles
+// nothing changes (4096 tokens 2435).
 //
 // Tiles of up to 24 rows (NB blocks of 8) take the codes themselves to the matrix cores, one instruction a sub-block instead of
 // two planes': the sub-block sums of their few rows times the scales cost less on the vector ALU (4 multiply-adds a lane for 8
@@ -334,7 +338,6 @@ typedef _Float16 pf_v2h __attribute__((ext_vector_type(2)));
 // top-8 of 256 experts of 7168 x 2048 under a skewed routing (70 of its 93 experts with 24 rows or fewer), 627 -> 520 and 336 ->
 // 291.  What bounds it: on full tiles vector issue (59 % of the cycles) and matrix time (50 %), at the 1.75 GHz that this
 // load leaves of 2.4; few rows an expert stream their weights at 3.2 TB/s, of 5.2 without arithmetic.
-constexpr int kPfRing = 4;                           // activations of a pass in LDS, three passes ahead
 constexpr int kPfPlane = 32 * 256;                   // codes of a pass
 constexpr int kPfSlotS = kPfPlane, kPfSlotD = kPfSlotS + 1024, kPfSlot = kPfSlotD + 256;   // codes [32][256], sums [32][16], scales [32]
 
@@ -383,44 +386,52 @@ __device__ __forceinline__ pf_v2h pf_bytes_1024(uint32_t w, uint32_t sel) {
 // bytes), a lane's reads of its row's part of them, and the two planes of a sub-block out of the registers these filled.
 template <bool GU> struct PfQ4K {
     static constexpr bool kSums = true;
-    static constexpr int kLdsAt = 0, kWave = 32 * 144;
-    static constexpr int kMats = GU ? 2 : 1, kRows = 32 / kMats, kWhole = kRows * 9 / 64, kTail = kRows * 9 % 64;
-    static constexpr int kCopies = kMats * (kWhole + 1);
+    // A piece is 128 bytes of each of the 32 rows, 16-byte granule g of row r at g ^ (r / 2 & 7): the 16-byte reads of 16 rows meet
+    // every bank once.  A super-block's nine granules lie in two pieces, a ring of three holds the one behind them as well.  (A fourth,
+    // in the place of the activations' fourth slot or not, does not fit two workgroups' LDS; the fourth slot gave nothing.)
+    static constexpr int kPiece = 32 * 128, kLdsAt = 0, kWave = 3 * kPiece;
+    static constexpr int kCopies = 4, kRing = 3;   // (kRing: passes of activations in LDS, all but one of them ahead)
+    static constexpr int kOneGroupBut = kCopies;   // (the piece that every eighth super-block ends in was asked for one super-block ago)
     static constexpr int kHiFactor = 8, kLook = 0;   // (a sum is lo + 8 hi; LDS look-ups of a sub-block's planes)
-    __amdgpu_buffer_rsrc_t r[kMats];
-    uint32_t at[kWhole + 1], row_at, m_shift;
-    int lane;
+    __amdgpu_buffer_rsrc_t r[2];   // 16 rows each
+    uint32_t at[2], row_at, swizzle, m_shift;   // at: a lane's offsets in the piece to ask for next
+    int lane, left, cur;           // left: the pieces not asked for yet; cur: where the ring's first one sits
     pf_v2h m_mul, m_add;
     __device__ __forceinline__ void init(const PfGemm& a, const uint8_t* blob, int64_t n0, int lane_) {
-        lane = lane_;
+        const int row_bytes = (int) a.row_bytes;
+        lane = lane_, left = (row_bytes + 127) >> 7, cur = 0;
 #pragma unroll
-        for (int m = 0; m < kMats; ++m)
-            r[m] = __builtin_amdgcn_make_buffer_rsrc((void*) (blob + a.off[m] + (size_t) n0 * a.row_bytes), 0, (int) (kRows * a.row_bytes), 0x00020000);
-#pragma unroll
-        for (int i = 0; i <= kWhole; ++i) {   // 16 bytes a lane, the nine pieces of a row in a run
-            const int u = 64 * i + lane;
-            at[i] = (uint32_t) ((u / 9) * (int) a.row_bytes + (u % 9) * 16);
+        for (int i = 0; i < 2; ++i) {
+            r[i] = __builtin_amdgcn_make_buffer_rsrc((void*) (blob + a.off[GU ? i : 0] + (size_t) (n0 + (GU ? 0 : 16 * i)) * a.row_bytes), 0, 16 * row_bytes, 0x00020000);
+            at[i] = (uint32_t) ((8 * i + (lane >> 3)) * row_bytes + ((lane & 7) ^ (4 * i + (lane >> 4))) * 16);   // 8 rows a copy, 8 lanes a row
         }
         const int kh = lane >> 5;
-        row_at = (lane & 31) * 144 + 16 * kh;
+        row_at = (lane & 31) * 128;
+        swizzle = 16 * ((lane >> 1) & 7);
         m_shift = 2 * kh;
         m_mul = kh ? pf_v2h{(_Float16) 16.0f, (_Float16) 16.0f} : pf_v2h{(_Float16) 1.0f, (_Float16) 1.0f};
         m_add = kh ? pf_v2h{(_Float16) -16384.0f, (_Float16) -16384.0f} : pf_v2h{(_Float16) -1024.0f, (_Float16) -1024.0f};
     }
-    __device__ __forceinline__ void copy(uint8_t* to, int sb) const {
+    __device__ __forceinline__ int behind(int slot) const { return slot == 2 * kPiece ? 0 : slot + kPiece; }
+    // The next piece, to `to`.  (The piece is in the lanes' offsets, not in the scalar one, which need not take part in the buffer's range
+    // check: a row's last piece goes on into the row behind it, and behind the matrix there may be nothing.)
+    __device__ __forceinline__ void copy(uint8_t* to) {
+        if (left <= 0) return;
 #pragma unroll
-        for (int m = 0; m < kMats; ++m)
+        for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(r[i >> 1], (pf_lptr) (to + i * 1024), 16, at[i & 1], 0, 0, 0);
+        at[0] += 128, at[1] += 128, --left;
+    }
+    __device__ __forceinline__ void first(uint8_t* to) {
 #pragma unroll
-            for (int i = 0; i < kWhole; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + i * 1024), 16, at[i], sb * 144, 0, 0);
-        // (the lane number is hidden from the compiler: it would follow one `if` into the next, merge copies of different places and
-        // pick their LDS address by lane, which has to be the same for the wave)
-        int l = lane;
-        asm volatile("" : "+v"(l));
-        if (l < kTail) {
-#pragma unroll
-            for (int m = 0; m < kMats; ++m)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + m * kRows * 144 + kWhole * 1024), 16, at[kWhole], sb * 144, 0, 0);
+        for (int i = 0; i < 3; ++i) copy(to + i * kPiece);
+    }
+    // super-block sb is in registers: the one or two pieces that it was the last to want make room
+    __device__ __forceinline__ void next(uint8_t* to, int sb) {
+        copy(to + cur);
+        cur = behind(cur);
+        if ((sb & 7) == 7) {
+            copy(to + cur);
+            cur = behind(cur);
         }
     }
     struct Row {   // a lane's part of its row: the header, four 16-byte pieces of the codes (bytes 32 c + 16 kh of their 128: the low
@@ -431,13 +442,15 @@ template <bool GU> struct PfQ4K {
         pf_u16x2 flo[2][2], fhi[2][2];
         pf_v8h mb;
     };
-    __device__ __forceinline__ void read(Row& w, uint32_t base) const {
-        const uint32_t at = base + row_at;
-        w.hdr = pf_lds_i32x4<0>(base + (lane & 31) * 144);
-        w.q[0] = pf_lds_i32x4<16>(at);
-        w.q[1] = pf_lds_i32x4<48>(at);
-        w.q[2] = pf_lds_i32x4<80>(at);
-        w.q[3] = pf_lds_i32x4<112>(at);
+    __device__ __forceinline__ void read(Row& w, uint32_t base, int sb) const {
+        const uint32_t here = base + row_at + cur, behind_it = base + row_at + behind(cur);
+        const uint32_t g = 16 * (sb & 7);   // (granule 9 sb, in its piece)
+        w.hdr = pf_lds_i32x4<0>(here + (g ^ swizzle));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t at = (16 * (lane >> 5) + g + 16 + 32 * c) ^ swizzle;   // (bit 7: in the piece behind)
+            w.q[c] = pf_lds_i32x4<0>((at & 128 ? behind_it : here) + (at & 0x70));
+        }
     }
     template <int BUT> __device__ __forceinline__ void wait(Row& w) const {
         asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(w.hdr), "+v"(w.q[0]), "+v"(w.q[1]), "+v"(w.q[2]), "+v"(w.q[3]) : "n"(BUT));
@@ -485,8 +498,8 @@ template <bool GU> struct PfQ4K {
     }
 };
 
-template <typename W> struct PfLds {   // the weight type's tables, the activations' ring, the weights [2][4 waves]
-    static constexpr int ring = W::kLdsAt, w = ring + kPfRing * kPfSlot, w_step = 4 * W::kWave, bytes = w + 2 * w_step;
+template <typename W> struct PfLds {   // the weight type's tables, the activations' ring, the weights of the 4 waves
+    static constexpr int ring = W::kLdsAt, w = ring + W::kRing * kPfSlot, bytes = w + 4 * W::kWave;
 };
 
 // NB: 0, or the blocks of 8 rows of a tile that takes the codes themselves to the matrix cores
@@ -509,17 +522,17 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
     dma.init(a, row0, nrows, NM, wave, lane);
     W wts;
     uint8_t* const wlds = lds + S::w + wave * W::kWave;
-    // the copies of pass (sb, m) + 3 go into the slot of the pass before (sb, m); in the prologue, of passes 0..2
-    auto copy_pass = [&](auto mc, int sb, int slot) {   // (M in 0 .. NM + 2: pass M of super-block sb on)
+    // the copies of pass (sb, m) + kAhead go into the slot of the pass before (sb, m); in the prologue, of the first kAhead passes
+    constexpr int kAhead = W::kRing - 1;
+    auto copy_pass = [&](auto mc, int sb, int slot) {   // (M in 0 .. NM - 1 + kAhead: pass M of super-block sb on)
         constexpr int M = decltype(mc)::value, m = M % NM;
         const int b = sb + M / NM;
         if (b < nsb) dma.template copy<m == NM - 1>(lds + S::ring + slot * kPfSlot, b, m);
     };
-    pf_for_m<0, 3>([&](auto mc) { copy_pass(mc, 0, decltype(mc)::value); });
+    pf_for_m<0, kAhead>([&](auto mc) { copy_pass(mc, 0, decltype(mc)::value); });
     int slot = 0;
     wts.init(a, blob, n0, lane);
-    wts.copy(wlds, 0);
-    if (nsb > 1) wts.copy(wlds + S::w_step, 1);
+    wts.first(wlds);
     // a lane's 16 codes of sub-block j: the row's 16-byte chunk 2 j + kh, which sits at that index ^ (the row & 15)
     const uint32_t a_base = ln * 256 + (((ln & 15) ^ kh) << 4);
     const uint32_t lbase = pf_lds_addr(lds) + S::ring, wbase = pf_lds_addr(wlds);
@@ -529,17 +542,21 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
         typename W::Row w;
         pf_for_m<0, NM>([&](auto mc) {
             constexpr int m = decltype(mc)::value;
-            // What this pass reads has landed once only what was issued after it is in flight: the activations of the two passes
-            // behind it (at least two copies a wave each) and the weights issued in the three passes before this one; the weights
-            // of a tile of one group were issued two passes ago, behind the next pass's activations.
-            constexpr int kIssued = ((m + 4 * NM - 1) % NM == 0) + ((m + 4 * NM - 2) % NM == 0) + ((m + 4 * NM - 3) % NM == 0);
-            constexpr int kBut = NM == 1 ? 2 + W::kCopies : 4 + W::kCopies * kIssued;
+            // What this pass reads has landed once only what was issued after it is in flight: the activations of the passes behind it
+            // (at least two copies a wave each) and the weights issued in the passes since its own activations were; with one group a
+            // super-block its weights decide.
+            constexpr int kIssued = [] {
+                int n = 0;
+                for (int i = 1; i <= kAhead; ++i) n += (m + 4 * NM - i) % NM == 0;
+                return n;
+            }();
+            constexpr int kActs = 2 * (kAhead - 1) + W::kCopies * kIssued, kBut = NM == 1 && W::kOneGroupBut < kActs ? W::kOneGroupBut : kActs;
             if (!steady || (m == 0 && sb == 0)) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
             else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBut) : "memory");
             const uint32_t lbuf = lbase + slot * kPfSlot;
-            if constexpr (m == 0) wts.read(w, wbase + (sb & 1) * S::w_step);
-            copy_pass(std::integral_constant<int, m + 3>{}, sb, (slot + 3) & 3);
-            slot = (slot + 1) & 3;
+            if constexpr (m == 0) wts.read(w, wbase, sb);
+            copy_pass(std::integral_constant<int, m + kAhead>{}, sb, slot ? slot - 1 : kAhead);
+            slot = slot == kAhead ? 0 : slot + 1;
             // The two plane products of the block, int32, a matrix instruction a sub-block and plane, accumulated over the 8
             // sub-blocks.  The activation operand is requested from LDS two sub-blocks ahead.
             pf_v16i dot[2];
@@ -564,8 +581,7 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
             };
             if constexpr (m == 0) {
                 wts.template wait<2>(w);
-                // (the wave's weights are in registers: their LDS takes the super-block after the next one's)
-                if (steady) wts.copy(wlds + (sb & 1) * S::w_step, sb + 2);
+                wts.next(wlds, sb);
                 wts.open(w);
                 wts.template look<0>(w);
             }

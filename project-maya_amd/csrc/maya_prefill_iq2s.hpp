@@ -23,8 +23,8 @@ constexpr int kIqMags = 0, kIqSigns = 8192, kIqScales = kIqSigns + 2048, kIqTabl
 // pieces sit in LDS at their index ^ twice the quad, so that a sub-block's words of 32 rows meet every bank once.
 template <bool GU> struct PfIq2s {
     static constexpr bool kSums = false;
-    static constexpr int kLdsAt = kIqTables, kWave = 2048 + 512 + 64 + 192;   // (a multiple of 256: addresses below are xor-ed)
-    static constexpr int kMats = GU ? 2 : 1, kQuads = 8 / kMats, kCopies = GU ? 6 : 5;
+    static constexpr int kLdsAt = kIqTables, kStep = 2048 + 512 + 64 + 192, kWave = 2 * kStep;   // (multiples of 256: addresses below are xor-ed)
+    static constexpr int kMats = GU ? 2 : 1, kQuads = 8 / kMats, kCopies = GU ? 6 : 5, kOneGroupBut = 2 + kCopies, kRing = 4;
     static constexpr int kHiFactor = 256, kLook = 5;
     static constexpr float kOutFactor = 0.125f;
     __amdgpu_buffer_rsrc_t r[kMats];
@@ -56,13 +56,23 @@ template <bool GU> struct PfIq2s {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r[GU ? i : 0], (pf_lptr) (to + 2048 + i * 256), 4, pat[GU ? 0 : i], sb * 64, 0, 0);
-        int l = lane;   // (hidden from the compiler, as in PfQ4K's copies)
+        // (the lane number is hidden from the compiler: it would follow one `if` into the next, merge copies of different places and
+        // pick their LDS address by lane, which has to be the same for the wave)
+        int l = lane;
         asm volatile("" : "+v"(l));
         if (l < 2 * kQuads) {
 #pragma unroll
             for (int m = 0; m < kMats; ++m)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + 2560 + m * 32), 4, sat, sb * 8, 0, 0);
         }
+    }
+    __device__ __forceinline__ void first(uint8_t* to) const {
+        copy(to, 0);
+        if (nsb > 1) copy(to + kStep, 1);
+    }
+    // super-block sb is in registers: its LDS takes the super-block after the next one's
+    __device__ __forceinline__ void next(uint8_t* to, int sb) const {
+        if (sb + 2 < nsb) copy(to + (sb & 1) * kStep, sb + 2);
     }
     struct Look {   // the LDS look-ups of one sub-block: selectors and signs of the lane's two grid entries, its group's digits
         pf_i2 m0, m1, s0, s1;
@@ -77,7 +87,8 @@ template <bool GU> struct PfIq2s {
         uint32_t e0[2], e1[2], sc[2];   // a byte a sub-block: the two entries' high bits, 16 ls
         Look lk[2];
     };
-    __device__ __forceinline__ void read(Row& w, uint32_t base) const {
+    __device__ __forceinline__ void read(Row& w, uint32_t base, int sb) const {
+        base += (sb & 1) * kStep;
         const uint32_t at = base + ix_at;
 #pragma unroll
         for (int j = 0; j < 8; ++j) w.is[j] = pf_lds_b64<0>(at ^ (32 * j));
@@ -131,7 +142,7 @@ template <bool GU> struct PfIq2s {
         }
     }
 };
-// tables, the activations' ring (the sums' place in a slot stays empty, as the weights have no minimums), the weights [2][4 waves]
+// tables, the activations' ring (the sums' place in a slot stays empty, as the weights have no minimums), the weights [4 waves][2]
 constexpr int kIqLdsBytes = 70912;
 static_assert(kIqLdsBytes == PfLds<PfIq2s<true>>::bytes && kIqLdsBytes == PfLds<PfIq2s<false>>::bytes);
 static_assert(kIqLdsBytes <= 80 * 1024, "two workgroups a compute unit");

@@ -1,6 +1,8 @@
 """The prompt-chunk path on the GPU through the C ABI: plan (count / scan / stable scatter / tiles), Q8_K activation
 rows, the grouped int8-MFMA GEMMs over Q4_K experts and the combine, against the CPU checker's restatement of the
 reference's CPU expert path, stage by stage: every row of the chunk is that path's expert on the row's token."""
+import sys
+
 import numpy as np
 import pytest
 
@@ -272,6 +274,14 @@ def test_a_part_of_the_tile_list(pf, oracle, t, n_embd, n_ff):
             on = torch.from_numpy(want).cuda()
             assert torch.equal(some[on].view(torch.int32), whole[on].view(torch.int32)), which
             assert not bool(some[~on].any()), which
+
+
+@pytest.mark.parametrize("n_embd, n_ff", [(1792, 2048), (2304, 4096), (4352, 2560)], ids=str)
+def test_rows_of_more_blocks_than_a_round_of_pieces(pf, oracle, monkeypatch, n_embd, n_ff):
+    """Q4_K rows reach LDS in pieces of 128 bytes, nine of them eight super-blocks: rows that end before, at and behind such a round (7, 8,
+    9, 10, 16 and 17 super-blocks), in tiles of every form, to the bounds of the test above."""
+    monkeypatch.setattr(sys.modules[__name__], "EDGE_ROWS", [1, 9, 24, 25, 33, 65, 97, 128])
+    test_experts_of_every_number_of_row_groups(pf, oracle, Q4_K, n_embd, n_ff)
 
 
 IQ_CASES = [
