@@ -803,6 +803,32 @@ __global__ __launch_bounds__(256) void router_kernel(const float* __restrict__ l
     }
 }
 
+// The softmax router of many tokens, a wave each (up to 64 R experts): a workgroup a token, three of whose waves wait for one while it
+// adds and picks.  4096 tokens of 288 experts 40.3 -> 14.1 us, of 256 18.4 -> 11.6, 512 of 256 6.5 -> 5.7; one of 288 8.2 -> 6.2; up to
+// 256 tokens of up to 256 experts nothing in it (5.0 to 5.5 us, either way the shorter by 0.1), so these stay as they are.
+template <int R>
+__global__ __launch_bounds__(256) void router_waves_kernel(const float* __restrict__ logits, int n_tokens, int n_expert, int k,
+                                                           int32_t* __restrict__ ids, float* __restrict__ weights) {
+    const int t = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= n_tokens) return;
+    const float* l = logits + (size_t) t * n_expert;
+    float lv[R], mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < R; ++r) lv[r] = 64 * r + lane < n_expert ? l[64 * r + lane] : -INFINITY;
+#pragma unroll
+    for (int r = 0; r < R; ++r) mx = fmaxf(mx, lv[r]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    double ex[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) ex[r] = 64 * r + lane < n_expert ? exp((double) lv[r] - (double) mx) : 0.0;
+    int id;
+    float w;
+    uint64_t ptr;
+    route_narrow_regs(n_expert, k, ex, nullptr, id, w, ptr);
+    if (lane < k) ids[(size_t) t * k + lane] = id, weights[(size_t) t * k + lane] = w;
+}
+
 // The layer's head in one launch, grid (1 + n_embd / 256, n_tokens): workgroup 0 of a token routes it, writes its
 // plan slots (blob addresses from the residency table); the other workgroups round one 256-value block of the hidden
 // state each to Q8_K.
@@ -2259,6 +2285,13 @@ static int route_impl(const char* what, const float* logits, int n_tokens, int n
     if (n_tokens <= 0 || n_tokens > 65535 || n_expert <= 0 || n_expert > MAYA_MAX_EXPERTS || k <= 0 || k > MAYA_MAX_K || k > n_expert)
         return fail(MAYA_E_SHAPE, "%s: tokens %d experts %d k %d (limits %d experts, k %d)", what, n_tokens, n_expert, k,
                     MAYA_MAX_EXPERTS, MAYA_MAX_K);
+    if (r.kind == MAYA_ROUTER_SOFTMAX && n_expert <= 512 && (n_expert > 256 || n_tokens > 256)) {
+        const dim3 grid((unsigned) ((n_tokens + 3) / 4));
+        if (n_expert <= 256) hipLaunchKernelGGL(router_waves_kernel<4>, grid, dim3(256), 0, as_stream(stream), logits, n_tokens, n_expert, k, ids, weights);
+        else hipLaunchKernelGGL(router_waves_kernel<8>, grid, dim3(256), 0, as_stream(stream), logits, n_tokens, n_expert, k, ids, weights);
+        MAYA_LAUNCHED("router_waves_kernel");
+        return MAYA_OK;
+    }
     hipLaunchKernelGGL(router_kernel, dim3((unsigned) n_tokens), dim3(256), 0, as_stream(stream), logits, n_expert, k, r, ids, weights);
     MAYA_LAUNCHED("router_kernel");
     return MAYA_OK;

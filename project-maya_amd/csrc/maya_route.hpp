@@ -18,30 +18,31 @@ __device__ __forceinline__ int wave_max_i32(int v) {
     return __builtin_amdgcn_readlane(v, 63);
 }
 
-// Up to 256 experts, ONE wave, sm.ex filled: lane L keeps experts L, L + 64, L + 128, L + 192 in registers from the sum
+// Up to 64 R experts, ONE wave, sm.ex filled: lane L keeps experts L, L + 64, L + 128, ... in registers from the sum
 // to the weights, so nothing but the result touches LDS and no workgroup barrier sits on the path.
 //  * the sum: ascending, one add after the other (the reference's order).  The chain of dependent double adds is the
 //    critical path, so every add takes its operand from a lane by v_readlane, eight fetched ahead; all lanes carry the sum.
 //  * the k largest: k rounds of the reference's strict-> arg-max with the lower index on ties
 //    (src/kernels/cuda/router_top10.cu:140-176).  Probabilities are non-negative, so their bit patterns order like the
-//    values as signed integers and -1 marks "taken" or "no such expert"; a round is a 4-way maximum a lane, the wave
+//    values as signed integers and -1 marks "taken" or "no such expert"; a round is an R-way maximum a lane, the wave
 //    maximum, and the first lane (lowest expert: lower register first, then lower lane) that holds it.
 //  * renormalisation: the k weights summed in slot order in double, one division a lane.
-// (the token's exponentials already 4 a lane in ex; the wave's lane i < k returns slot i: its expert and weight.  `tab`:
-// the residency table's entries of the lane's four experts, NULL when no plan is wanted; the slot's blob address then
+// (the token's exponentials already R a lane in ex; the wave's lane i < k returns slot i: its expert and weight.  `tab`:
+// the residency table's entries of the lane's experts, NULL when no plan is wanted; the slot's blob address then
 // comes back in my_ptr - read from the chosen expert's lane, no second trip to memory.)
-__device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const double (&ex)[4], const uint64_t* tab, int& my_id,
+template <int R>
+__device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const double (&ex)[R], const uint64_t* tab, int& my_id,
                                                   float& my_weight, uint64_t& my_ptr) {
     const int lane = threadIdx.x & 63;
-    int lo[4], hi[4];
+    int lo[R], hi[R];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < R; ++r) {
         lo[r] = __double2loint(ex[r]);
         hi[r] = __double2hiint(ex[r]);
     }
     double sum = 0.0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < R; ++r) {
         if (64 * r < n_expert) {
 #pragma unroll
             for (int j0 = 0; j0 < 64; j0 += 8) {
@@ -57,24 +58,34 @@ __device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const dou
         }
     }
     const float inv = (float) (1.0 / sum);
-    int key[4];
+    int key[R];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) key[r] = 64 * r + lane < n_expert ? __float_as_int((float) (ex[r] * (double) inv)) : -1;
+    for (int r = 0; r < R; ++r) {
+        key[r] = 64 * r + lane < n_expert ? __float_as_int((float) (ex[r] * (double) inv)) : -1;
+        // (a row with an infinity or a NaN is all NaN, of the sign the division gave it; beyond 256 experts such rows come out with
+        // their lowest experts, as from route_token, whose keys are unsigned)
+        if (R > 4 && 64 * r + lane < n_expert && key[r] < 0) key[r] = 0x7fffffff;
+    }
     int id = 0, my_w = 0;
     uint64_t ptr = 0ull;
     for (int i = 0; i < k; ++i) {
-        const int top = wave_max_i32(max(max(key[0], key[1]), max(key[2], key[3])));
+        int best = max(key[0], key[1]);
+#pragma unroll
+        for (int q = 2; q < R; ++q) best = max(best, key[q]);
+        const int top = wave_max_i32(best);
         unsigned long long b = __ballot(key[0] == top);
         int r = 0;
-        if (b == 0ull) b = __ballot(key[1] == top), r = 1;
-        if (b == 0ull) b = __ballot(key[2] == top), r = 2;
-        if (b == 0ull) b = __ballot(key[3] == top), r = 3;
+#pragma unroll
+        for (int q = 1; q < R; ++q)
+            if (b == 0ull) b = __ballot(key[q] == top), r = q;
         const int at = __builtin_amdgcn_readfirstlane(__builtin_ctzll(b));
 #pragma unroll
-        for (int q = 0; q < 4; ++q) key[q] = (q == r && lane == at) ? -1 : key[q];
-        if (lane == i) id = 64 * r + at, my_w = top;
+        for (int q = 0; q < R; ++q) key[q] = (q == r && lane == at) ? -1 : key[q];
+        if (lane == i) id = 64 * r + at, my_w = R > 4 && top == 0x7fffffff ? (int) 0xffc00000 : top;
         if (tab) {
-            const uint64_t tq = r == 0 ? tab[0] : r == 1 ? tab[1] : r == 2 ? tab[2] : tab[3];
+            uint64_t tq = tab[0];
+#pragma unroll
+            for (int q = 1; q < R; ++q) tq = r == q ? tab[q] : tq;
             const uint32_t plo = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) tq, at);
             const uint32_t phi = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) (tq >> 32), at);
             if (lane == i) ptr = ((uint64_t) phi << 32) | plo;

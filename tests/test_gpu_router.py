@@ -167,6 +167,31 @@ def test_sigmoid_router_ties_bias_and_tiny_sums(lib, oracle):
     assert L.maya_moe_route_sigmoid(x.data_ptr(), 0, 1, 8, 9, 1.0, 1, o.data_ptr(), o.data_ptr(), 0) == 2   # k > experts
 
 
+@pytest.mark.parametrize("ne,k,nt", ((64, 6, 257), (256, 8, 515), (200, 1, 300), (257, 8, 1), (288, 8, 6), (320, 16, 259), (512, 10, 33)))
+def test_softmax_router_a_wave_a_token(lib, oracle, ne, k, nt):
+    """Many tokens, and more than 256 experts up to 512: the same bits as the routing launch with the plan, which gives a token a workgroup,
+    on ties, underflow and rows of infinities and NaN; ids of finite rows also against the CPU checker."""
+    rng = np.random.default_rng(ne + k + nt)
+    logits = rng.standard_normal((nt, ne)).astype(np.float32)
+    logits[nt // 2:] = np.round(logits[nt // 2:] * 4) / 4
+    odd = {}
+    if nt > 5:
+        logits[0] = 0.25
+        logits[1] = -200 * rng.random(ne)
+        logits[2, ne // 3] = np.inf
+        logits[3, ne - 1] = np.nan
+        logits[4] = -np.inf
+        odd = {2, 3, 4}
+    ld = torch.from_numpy(logits).cuda()
+    ids, w = lib.route_topk(ld, k)
+    ids2, w2, _ = lib.route_plan(ld, k, torch.arange(1, ne + 1, dtype=torch.int64, device="cuda") * 4096)
+    torch.cuda.synchronize()
+    assert torch.equal(ids, ids2) and torch.equal(w.view(torch.int32), w2.view(torch.int32))
+    rows = [t for t in range(nt) if t not in odd]
+    wi, _ = oracle.router_topk(logits[rows], k)
+    assert np.array_equal(ids.cpu().numpy()[rows], wi)
+
+
 def test_route_plan_in_one_launch(lib):
     rng = np.random.default_rng(31)
     for ne, k, nt in ((256, 8, 5), (300, 6, 3), (8, 2, 1)):
