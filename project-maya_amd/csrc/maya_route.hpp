@@ -28,7 +28,7 @@ __device__ __forceinline__ int wave_max_i32(int v) {
 //    maximum, and the first lane (lowest expert: lower register first, then lower lane) that holds it.
 //  * renormalisation: the k weights summed in slot order in double, one division a lane.
 // (the token's exponentials already R a lane in ex; the wave's lane i < k returns slot i: its expert and weight.  `tab`:
-// the residency table's entries of the lane's experts, NULL when no plan is wanted; the slot's blob address then
+// the residency table's entries of the lane's experts (R = 4), NULL when no plan is wanted; the slot's blob address then
 // comes back in my_ptr - read from the chosen expert's lane, no second trip to memory.)
 template <int R>
 __device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const double (&ex)[R], const uint64_t* tab, int& my_id,
@@ -82,10 +82,10 @@ __device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const dou
 #pragma unroll
         for (int q = 0; q < R; ++q) key[q] = (q == r && lane == at) ? -1 : key[q];
         if (lane == i) id = 64 * r + at, my_w = R > 4 && top == 0x7fffffff ? (int) 0xffc00000 : top;
-        if (tab) {
-            uint64_t tq = tab[0];
-#pragma unroll
-            for (int q = 1; q < R; ++q) tq = r == q ? tab[q] : tq;
+        if (R == 4 && tab) {
+            // (written out: as a loop over tab the select becomes an index, the table memory, and a kernel with scratch memory starts
+            // 10 us later)
+            const uint64_t tq = r == 0 ? tab[0] : r == 1 ? tab[1] : r == 2 ? tab[2] : tab[3];
             const uint32_t plo = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) tq, at);
             const uint32_t phi = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) (tq >> 32), at);
             if (lane == i) ptr = ((uint64_t) phi << 32) | plo;
