@@ -519,25 +519,33 @@ struct LayerHeadIn {
 // scale to the up lanes through LDS.  y: the position's 32 codes in that order, d: its block's scale, blob: the expert of
 // slot blockIdx.y.  A lane past the row's last position (`on` false; u is then its own index, o0 and o1 the last
 // position's) gets zero codes and a zero scale.  False: the thread has nothing more to do in this launch.
-template <int NW>
+// R: the experts a lane of the picking wave holds: 4 (up to 256), 8 (up to 512: a chosen expert's blob address is then read from the
+// table's copy in LDS wherever the router needs it).
+template <int NW, int R>
 __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent, const int32_t* skip, bool is_up, bool on, int u, int o0,
                                                 int o1, int (&y)[8], float& d, uint64_t& blob) {
     constexpr int NU = 32 * NW;
     __shared__ uint64_t s_blob[MAYA_MAX_K];
-    __shared__ float s_lv[256];
-    __shared__ uint64_t s_tab[256];
+    __shared__ float s_lv[64 * R];
+    __shared__ uint64_t s_tab[64 * R];
     __shared__ int s_y[9][NU];
     const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert;
     const bool picker = t >= 64 * (NW - 1), sigm = hd.sigmoid != 0;
-    float lv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    uint64_t tab[4] = {0ull, 0ull, 0ull, 0ull};
+    float lv[R], bv[R];
+    uint64_t tab[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) lv[r] = bv[r] = 0.0f, tab[r] = 0ull;
     if (picker) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < R; ++r) {
             const int x = 64 * r + lane;
             lv[r] = x < ne ? hd.logits[x] : -INFINITY;
             tab[r] = x < ne ? hd.table[x] : 0ull;
             if (hd.bias) bv[r] = x < ne ? hd.bias[x] : 0.0f;
+        }
+        if constexpr (R > 4) {   // (16 registers less than the kernel would need behind this)
+#pragma unroll
+            for (int r = 0; r < R; ++r) s_tab[64 * r + lane] = tab[r];
         }
     }
     if (blockIdx.x == gridDim.x - 1) {   // the router (it looks at no skip flag, like the head kernel)
@@ -546,12 +554,13 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
         float w;
         uint64_t ptr;
         if (sigm) {
-            float pr[4], sc[4];
+            float pr[R], sc[R];
             const bool fin = sigmoid_scores(lv, bv, hd.bias != nullptr, ne, pr, sc);
             route_wave_sigmoid(pr, sc, fin, tab, ne, n_ent, hd.out.norm, hd.out.w_scale, id, w, ptr);
         } else {
             route_wave_softmax(lv, tab, ne, n_ent, id, w, ptr);
         }
+        if constexpr (R > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
         if (lane < n_ent) {
             hd.out.ids[lane] = id;
             hd.out.weights[lane] = w;
@@ -562,25 +571,29 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
     if (skip && *skip) return false;
     if (picker) {
         __builtin_amdgcn_s_setprio(3);   // the workgroup waits for this wave: it goes first on its SIMD
+        if constexpr (R <= 4) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s_tab[64 * r + lane] = tab[r];
+            for (int r = 0; r < R; ++r) s_tab[64 * r + lane] = tab[r];
+        }
         int id;
         uint64_t ptr;
         if (sigm) {
             // the scores are the exact router's own keys: any strictly descending order of the picks is its order
-            float pr[4], sc[4];
+            float pr[R], sc[R];
             const bool fin = sigmoid_scores(lv, bv, hd.bias != nullptr, ne, pr, sc);
             if (route_wave_order_only(sc, fin, ne, n_ent, s_lv, 0.0f, INFINITY, id)) {
                 ptr = s_tab[lane < n_ent ? id : 0];
             } else {
                 float w;
                 route_wave_sigmoid(pr, sc, fin, tab, ne, n_ent, hd.out.norm, hd.out.w_scale, id, w, ptr);
+                if constexpr (R > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
             }
         } else if (route_wave_order_only(lv, true, ne, n_ent, s_lv, 1e-6f, 60.0f, id)) {
             ptr = s_tab[lane < n_ent ? id : 0];
         } else {
             float w;
             route_wave_softmax(lv, tab, ne, n_ent, id, w, ptr);
+            if constexpr (R > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
         }
         if (lane < n_ent) s_blob[lane] = ptr;
         __builtin_amdgcn_s_setprio(0);
@@ -645,11 +658,11 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
 
 // The leading arguments are what the kernel asks of memory first; as plain pointers and integers at the head of the
 // argument list they arrive in scalar registers with the dispatch (a structure passed by value is read from memory
-// first).  HEAD: p0 = the logits [n_expert], p1 = the table [n_expert] of blob addresses (0 = absent), p2 = x [n_embd] of
+// first).  HEAD (4 or 8: the experts a lane of the picking wave holds, up to 256 or 512 in all; 0: no head): p0 = the logits [n_expert], p1 = the table [n_expert] of blob addresses (0 = absent), p2 = x [n_embd] of
 // dtype `mode & 255`, bias = the sigmoid router's (bit 8 of mode: the sigmoid router) or NULL; else p0 = the plan's blob
 // addresses (a.plan_ptr), p1 = the codes of x (a.x.q), p2 = their scales (a.x.d).  mode >> 16 = n_embd / 32, the
 // sub-blocks a row.
-template <int NW, int MINW, bool HEAD>
+template <int NW, int MINW, int HEAD>
 __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_kernel(const void* __restrict__ p0, const void* __restrict__ p1,
                                                                                       const void* __restrict__ p2,
                                                                                       const uint64_t* __restrict__ iq2s_grid,
@@ -661,8 +674,8 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
     __shared__ __align__(16) int lds[kFastLdsWords];
     __shared__ float part[2][2 * NW][8];
     __shared__ uint64_t s_blob[HEAD ? MAYA_MAX_K : 1];
-    __shared__ float s_lv[HEAD ? 256 : 1];              // the picker's scratch: the logits, the table
-    __shared__ uint64_t s_tab[HEAD ? 256 : 1];
+    __shared__ float s_lv[HEAD ? 64 * HEAD : 1];              // the picker's scratch: the logits, the table
+    __shared__ uint64_t s_tab[HEAD ? 64 * HEAD : 1];
     __shared__ int s_y[HEAD ? 9 : 1][HEAD ? NU : 1];   // a position's codes and scale, from its gate lane to its up lane
     const uint2* grid = (const uint2*) lds;
     const uint2* stab = (const uint2*) (lds + 2048);
@@ -686,15 +699,21 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
         const bool picker = t >= 64 * (NW - 1);
         const int x_dtype = mode & 255;
         const bool sigm = (mode & 256) != 0;
-        float lv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        uint64_t tab[4] = {0ull, 0ull, 0ull, 0ull};
+        float lv[HEAD], bv[HEAD];
+        uint64_t tab[HEAD];
+#pragma unroll
+        for (int r = 0; r < HEAD; ++r) lv[r] = bv[r] = 0.0f, tab[r] = 0ull;
         if (picker) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < HEAD; ++r) {
                 const int e = 64 * r + lane;
                 lv[r] = e < ne ? logits[e] : -INFINITY;
                 tab[r] = e < ne ? table[e] : 0ull;
                 if (bias) bv[r] = e < ne ? bias[e] : 0.0f;
+            }
+            if constexpr (HEAD > 4) {   // (16 registers less than the kernel would need behind this)
+#pragma unroll
+                for (int r = 0; r < HEAD; ++r) s_tab[64 * r + lane] = tab[r];
             }
         }
         table_request(iq2s_grid, tp);   // (behind the picker's loads: loads come back in the order they were asked for)
@@ -704,12 +723,13 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
             float w;
             uint64_t ptr;
             if (sigm) {
-                float p[4], sc[4];
+                float p[HEAD], sc[HEAD];
                 const bool fin = sigmoid_scores(lv, bv, bias != nullptr, ne, p, sc);
                 route_wave_sigmoid(p, sc, fin, tab, ne, n_ent, hd.norm, hd.w_scale, id, w, ptr);
             } else {
                 route_wave_softmax(lv, tab, ne, n_ent, id, w, ptr);
             }
+            if constexpr (HEAD > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
             if (lane < n_ent) {
                 hd.ids[lane] = id;
                 hd.weights[lane] = w;
@@ -722,25 +742,29 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
         if (skipv) return;
         if (picker) {   // (before x is loaded: the values of x then take no registers here)
             __builtin_amdgcn_s_setprio(3);   // the workgroup waits for this wave: it goes first on its SIMD
+            if constexpr (HEAD <= 4) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s_tab[64 * r + lane] = tab[r];
+                for (int r = 0; r < HEAD; ++r) s_tab[64 * r + lane] = tab[r];
+            }
             int id;
             uint64_t ptr;
             if (sigm) {
                 // the scores are the exact router's own keys: any strictly descending order of the picks is its order
-                float p[4], sc[4];
+                float p[HEAD], sc[HEAD];
                 const bool fin = sigmoid_scores(lv, bv, bias != nullptr, ne, p, sc);
                 if (route_wave_order_only(sc, fin, ne, n_ent, s_lv, 0.0f, INFINITY, id)) {
                     ptr = s_tab[lane < n_ent ? id : 0];
                 } else {
                     float w;
                     route_wave_sigmoid(p, sc, fin, tab, ne, n_ent, hd.norm, hd.w_scale, id, w, ptr);
+                    if constexpr (HEAD > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
                 }
             } else if (route_wave_order_only(lv, true, ne, n_ent, s_lv, 1e-6f, 60.0f, id)) {
                 ptr = s_tab[lane < n_ent ? id : 0];
             } else {
                 float w;
                 route_wave_softmax(lv, tab, ne, n_ent, id, w, ptr);
+                if constexpr (HEAD > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
             }
             if (lane < n_ent) s_blob[lane] = ptr;
             __builtin_amdgcn_s_setprio(0);

@@ -737,12 +737,13 @@ __device__ __forceinline__ void route_any(const float* __restrict__ l, int n_exp
 // lv / bv / tab of experts L, L + 64, ...; bv all zero without a bias).  sc: the lane's four scores p + bias as the
 // caller already made them with sigmoid_scores (the same instructions, so the same bits).  Lane i < k returns slot i; a
 // row with a non-finite logit or score returns id -1, weight 0, no blob.
-__device__ __forceinline__ bool sigmoid_scores(const float (&lv)[4], const float (&bv)[4], bool has_bias, int n_expert, float (&p)[4],
-                                               float (&sc)[4]) {
+template <int R>
+__device__ __forceinline__ bool sigmoid_scores(const float (&lv)[R], const float (&bv)[R], bool has_bias, int n_expert, float (&p)[R],
+                                               float (&sc)[R]) {
     const int lane = threadIdx.x & 63;
     bool fin = true;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int r = 0; r < R; ++r) {
         const bool have = 64 * r + lane < n_expert;
         const float le = have ? lv[r] : 0.0f;
         p[r] = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf(-le)));
@@ -801,6 +802,46 @@ __global__ __launch_bounds__(256) void router_kernel(const float* __restrict__ l
         ids[(size_t) t * k + threadIdx.x] = sm.id[threadIdx.x];
         weights[(size_t) t * k + threadIdx.x] = sm.w[threadIdx.x];
     }
+}
+
+// The same for up to 512 experts, 8 a lane, without the blobs' addresses (what is read of a chosen expert is read lane by register and
+// then selected: as an indexed register array it would be memory).
+__device__ __forceinline__ void route_wave_sigmoid(const float (&p)[8], const float (&sc)[8], bool fin, const uint64_t (&)[8], int n_expert,
+                                                   int k, int norm, float w_scale, int& my_id, float& my_w, uint64_t& my_ptr) {
+    const int lane = threadIdx.x & 63;
+    constexpr int kNone = (int) 0x80000000;
+    const bool bad = __any(!fin) != 0;
+    int key[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) key[r] = 64 * r + lane < n_expert ? float_order_key(sc[r]) : kNone;
+    int id = 0;
+    float pw = 0.0f;
+    for (int i = 0; i < k; ++i) {
+        int best = key[0];
+#pragma unroll
+        for (int r = 1; r < 8; ++r) best = max(best, key[r]);
+        const int top = wave_max_i32(best);
+        unsigned long long b = __ballot(key[0] == top);
+        int q = 0;
+#pragma unroll
+        for (int r = 1; r < 8; ++r)
+            if (b == 0ull) b = __ballot(key[r] == top), q = r;
+        const int at = __builtin_amdgcn_readfirstlane(__builtin_ctzll(b));
+        int pv = 0;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            key[r] = r == q && lane == at ? kNone : key[r];
+            const int v = __builtin_amdgcn_readlane(__float_as_int(p[r]), at);
+            pv = r == q ? v : pv;
+        }
+        if (lane == i) id = 64 * q + at, pw = __int_as_float(pv);
+    }
+    double s = 0.0;
+    for (int i = 0; i < k; ++i) s += (double) __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pw), i));
+    const float inv = (float) (norm == 0 ? 1.0 : norm == 2 ? 1.0 / (s + 1e-20) : 1.0 / fmax(s, 6.103515625e-05));
+    my_id = bad ? -1 : id;
+    my_w = bad ? 0.0f : (float) ((double) pw * (double) inv * (double) w_scale);
+    my_ptr = 0ull;
 }
 
 // The softmax router of many tokens, a wave each (up to 64 R experts): a workgroup a token, three of whose waves wait for one while it
@@ -1004,7 +1045,7 @@ __global__ __launch_bounds__(256) void group_kernel(const uint64_t* __restrict__
     group_entries(g, n, grp_ptr, grp_start, grp_ent, n_groups);
 }
 
-// The head of several tokens in ONE launch (up to 16, either router, up to 256 experts, 256 entries): route, plan, group, Q8_K of x.
+// The head of several tokens in ONE launch (up to 16, either router, up to 64 R experts, 256 entries): route, plan, group, Q8_K of x.
 // Workgroup 0 has a wave a token: it picks the token's experts from the ORDER of the logits (route_wave_order_only; the exact
 // router on the same wave where that does not settle it), writes the plan and groups it itself (group_kernel's arithmetic).  The
 // workgroups 1 ... ceil(tokens / 4) route four tokens each exactly, a wave each, for ids and weights, which nothing in the launch
@@ -1014,16 +1055,21 @@ __global__ __launch_bounds__(256) void group_kernel(const uint64_t* __restrict__
 // 10.0; without x and with the softmax router 5.4, where exact routing in workgroup 0 with the grouping behind it took 10.4.  Layers:
 // IQ1_S 6144 x 2048, 2 tokens, 44.4 -> 41.7 us, 4 tokens 77.0 -> 75.4; IQ2_S 7168 x 2048 with Q4_K down, 8 tokens, 220 -> 214.5;
 // Q4_K 2048 x 768, 3 tokens, 30.1 -> 27.5; EXL3 6144 x 1536 at 3 bits, 4 tokens, 153.8 -> 150.7.
+// R = 8 takes 257 to 512 experts (and one token of them, where no gate/up launch carries the head), whose routing was a workgroup a
+// token with a 64-bit key an expert: Q8_0 2048 x 512 top-8 of 300, 1 token, 21.7 -> 16.9 us; Q4_K 2048 x 768 of 384, 2 tokens, 25.5 ->
+// 21.4; of 512, 4 tokens, 36.5 -> 32.8; IQ1_M 6144 x 1536 of 270, 9 tokens, 48.8 -> 43.6.  Up to 256 the form of 4 a lane is the
+// shorter: Q4_K 2048 x 768 of 256, 3 tokens, sigmoid, 22.2 us with R = 4, 23.9 with 8; of 128, 4 tokens, 24.2 / 24.9 (one token, its head in
+// the gate/up launch: IQ1_S 5120 x 1536 of 160 20.5 / 21.1, IQ2_S 7168 x 2048 of 256 29.1 / 29.3).
 constexpr int kHeadRoute = 4, kHeadRound = 32768;   // tokens of a routing workgroup, values of a rounding one
-template <int DT>
+template <int DT, int R>
 __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restrict__ logits, const uint64_t* __restrict__ table,
                                                            const void* __restrict__ x, int n_expert, int k, int n_tokens, int n_embd, RouterSpec rs,
                                                            int32_t* __restrict__ ids, float* __restrict__ weights, uint64_t* __restrict__ plan,
                                                            uint64_t* __restrict__ grp_ptr, int32_t* __restrict__ grp_start,
                                                            int32_t* __restrict__ grp_ent, int32_t* __restrict__ n_groups, maya_act xq, maya_act xs) {
     __shared__ GroupLds g;
-    __shared__ float s_lv[MAYA_MAX_TOKENS][256];
-    __shared__ uint64_t s_tab[256];
+    __shared__ float s_lv[MAYA_MAX_TOKENS][64 * R];
+    __shared__ uint64_t s_tab[64 * R];
     const int tid = threadIdx.x, lane = tid & 63, n_route = (n_tokens + kHeadRoute - 1) / kHeadRoute;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if ((int) blockIdx.x > n_route) {
@@ -1056,10 +1102,10 @@ __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restri
     const int t = pick ? wave : wave < kHeadRoute ? ((int) blockIdx.x - 1) * kHeadRoute + wave : n_tokens;
     if (t < n_tokens) {
         const float* l = logits + (size_t) t * n_expert;
-        float lv[4], bv[4], pr[4], sc[4];
-        uint64_t tab[4];
+        float lv[R], bv[R], pr[R], sc[R];
+        uint64_t tab[R];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < R; ++r) {
             const int e = 64 * r + lane;
             lv[r] = e < n_expert ? l[e] : -INFINITY;
             tab[r] = e < n_expert ? table[e] : 0ull;
@@ -1073,7 +1119,7 @@ __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restri
         bool exact = !pick || k >= n_expert;
         if (pick) {   // (every wave writes the whole table and reads it behind its own writes)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s_tab[64 * r + lane] = tab[r];
+            for (int r = 0; r < R; ++r) s_tab[64 * r + lane] = tab[r];
         }
         if (!exact) {
             exact = !(sigm ? route_wave_order_only(sc, fin, n_expert, k, s_lv[t], 0.0f, INFINITY, id)
@@ -1083,6 +1129,7 @@ __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restri
         if (exact) {
             if (sigm) route_wave_sigmoid(pr, sc, fin, tab, n_expert, k, rs.norm, rs.w_scale, id, w, ptr);
             else route_wave_softmax(lv, tab, n_expert, k, id, w, ptr);
+            if (R > 4 && pick) ptr = lane < k && id >= 0 ? s_tab[id] : 0ull;
         }
         if (lane < k) {
             if (pick) {
@@ -1103,14 +1150,18 @@ __global__ __launch_bounds__(1024) void window_head_kernel(const float* __restri
 }
 // what it covers
 inline bool window_head_ok(int n_tokens, int n_expert, int k) {
-    return n_tokens >= 1 && n_tokens <= MAYA_MAX_TOKENS && n_expert >= 1 && n_expert <= 256 && k >= 1 && k <= MAYA_MAX_K && k <= n_expert && n_tokens * k <= 256;
+    return n_tokens >= 1 && n_tokens <= MAYA_MAX_TOKENS && n_expert >= 1 && n_expert <= 512 && k >= 1 && k <= MAYA_MAX_K && k <= n_expert && n_tokens * k <= 256;
 }
 static int launch_window_head(const RouterSpec& rs, const float* logits, int n_tokens, int n_expert, int k, const uint64_t* table, int32_t* ids,
                               float* weights, uint64_t* plan, uint64_t* grp_ptr, int32_t* grp_start, int32_t* grp_ent, int32_t* n_groups,
                               const void* x, int x_dtype, int n_embd, maya_act xq, maya_act xs, hipStream_t s) {
     const int64_t rounding = ((int64_t) n_tokens * n_embd + kHeadRound - 1) / kHeadRound * ((xq.q != nullptr) + (xs.q != nullptr));
     const dim3 grid((unsigned) (1 + (n_tokens + kHeadRoute - 1) / kHeadRoute + rounding)), block(1024);
-#define MAYA_WH(DT) hipLaunchKernelGGL(window_head_kernel<DT>, grid, block, 0, s, logits, table, x, n_expert, k, n_tokens, n_embd, rs, ids, weights, plan, grp_ptr, grp_start, grp_ent, n_groups, xq, xs)
+#define MAYA_WH(DT)                                                                                                                              \
+    if (n_expert <= 256) hipLaunchKernelGGL((window_head_kernel<DT, 4>), grid, block, 0, s, logits, table, x, n_expert, k, n_tokens, n_embd, rs, ids,  \
+                                            weights, plan, grp_ptr, grp_start, grp_ent, n_groups, xq, xs);                                       \
+    else hipLaunchKernelGGL((window_head_kernel<DT, 8>), grid, block, 0, s, logits, table, x, n_expert, k, n_tokens, n_embd, rs, ids, weights, plan, \
+                            grp_ptr, grp_start, grp_ent, n_groups, xq, xs)
     switch (rounding ? x_dtype : MAYA_DT_F32) {
         case MAYA_DT_BF16: MAYA_WH(MAYA_DT_BF16); break;
         case MAYA_DT_F16: MAYA_WH(MAYA_DT_F16); break;
@@ -1607,8 +1658,10 @@ int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hip
     static int per_cu = 0;
     if (per_cu == 0) {
         int n = 0, m = 0;
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gate_up_iq2s_tiles_kernel<NW, kMinW, false>, 64 * NW, 0));
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, kMinW, true>, 64 * NW, 0));
+        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gate_up_iq2s_tiles_kernel<NW, kMinW, 0>, 64 * NW, 0));
+        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, kMinW, 4>, 64 * NW, 0));
+        n = m < n ? m : n;
+        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, kMinW, 8>, 64 * NW, 0));
         n = m < n ? m : n;
         per_cu = n > kMostPerCu ? kMostPerCu : n > 0 ? n : 1;
     }
@@ -1617,27 +1670,29 @@ int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hip
     const unsigned walkers = (unsigned) (wgs < n_tiles ? wgs : n_tiles);
     const int nu = a.layout.n_embd >> 5;   // sub-blocks a row, in the upper half of `mode`
     if (hd) {   // workgroup 0 routes, the others walk the tiles
-        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, true>), dim3(walkers + 1), dim3(64 * NW), 0, s, (const void*) hd->logits,
-                           (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias, a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a,
-                           hd->out);
+        auto kern = hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8>;
+        hipLaunchKernelGGL(kern, dim3(walkers + 1), dim3(64 * NW), 0, s, (const void*) hd->logits, (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias,
+                           a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a, hd->out);
     } else {
-        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, false>), dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
+        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, 0>), dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
                            (const void*) a.x.q, (const void*) a.x.d, st.cb.iq2s, (const float*) nullptr, a.skip, 0, nu << 16, a.k, a, LayerHead{});
     }
     MAYA_LAUNCHED("gate_up_iq2s_tiles_kernel");
     return MAYA_OK;
 }
-// The single-token layer whose head rides in the gate/up launch (gate_up_iq2s_tiles_kernel<.., true>,
-// gate_up_q4k_pos_kernel<.., true>): either router over up to 256 experts with more experts than slots, x aligned for
+// The single-token layer whose head rides in the gate/up launch (gate_up_iq2s_tiles_kernel<.., 4 or 8>,
+// gate_up_q4k_pos_kernel<.., 4 or 8>): either router over up to 512 experts with more experts than slots, x aligned for
 // 16-byte loads, IQ2_S, Q4_K or IQ1_S gate/up rows in the stream packing's shapes.  (IQ1_M keeps its head launch: its
 // gate/up kernel with the head in it was 6.3 us slower a launch than without, more than the 4.8 us head launch it replaces;
 // IQ1_S gains 1.4 us a layer, Q4_K 0.6, and the one-expert Q4_K layer of few workgroups 2.7 of 16.)
+// 257 to 512 experts (8 a lane) gain more, as their routing launch is longer: Q4_K 2048 x 768 top-8 of 288 18.5 -> 12.3 us, 7168 x 2048
+// of 288 43.0 -> 39.2, IQ2_S 7168 x 1024 of 384 28.7 -> 22.6, IQ1_S 5120 x 1536 of 384 27.3 -> 20.4.
 bool gate_up_q4k_pos_ok(const maya_moe_args& a);
 bool gate_up_iq1s_pos_ok(const maya_moe_args& a);
 static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& rs, const float* logits, int n_expert, const void* x,
                                      int x_dtype) {
     const maya_moe_layout& l = a.layout;
-    if (!(logits && a.n_tokens == 1 && n_expert <= 256 && a.k < n_expert && x_dtype >= 0 && x_dtype <= 2 && ((uintptr_t) x & 15) == 0))
+    if (!(logits && a.n_tokens == 1 && n_expert <= 512 && a.k < n_expert && x_dtype >= 0 && x_dtype <= 2 && ((uintptr_t) x & 15) == 0))
         return false;
     if (l.gate_type == kQ4_K) return gate_up_q4k_pos_ok(a);
     if (l.gate_type == kIQ1_S) return gate_up_iq1s_pos_ok(a);
@@ -1780,8 +1835,9 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_IQ1(NWV)                                                                                                          \
-    if (hd && fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
-    else if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);   \
+    if (hd && hd->n_expert > 256) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, 8>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
+    else if (hd && fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
+    else if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);   \
     else if (fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);         \
     else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, false>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);
     switch (pos_waves(a.layout.n_embd)) {
@@ -1880,13 +1936,18 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd ? 1u : 0u), (unsigned) (a.n_tokens * a.k));
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
+    const bool wide = hd && hd->n_expert > 256;   // (their rows take the form that any length has)
 #define MAYA_Q4F(NWV, F)                                                                                                    \
-    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);   \
-    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);     \
+    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);      \
+    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);        \
     else if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);          \
     else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8, F>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
+#define MAYA_Q4W(NWV)                                                                                                       \
+    if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, false, true, 8>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);        \
+    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, false, false, 8>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
 #define MAYA_Q4(NWV)                         \
-    if (fit) { MAYA_Q4F(NWV, true) }        \
+    if (wide) { MAYA_Q4W(NWV) }             \
+    else if (fit) { MAYA_Q4F(NWV, true) }   \
     else { MAYA_Q4F(NWV, false) }
     switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_Q4(2) break;
@@ -1899,6 +1960,7 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     }
 #undef MAYA_Q4
 #undef MAYA_Q4F
+#undef MAYA_Q4W
     MAYA_LAUNCHED("gate_up_q4k_pos_kernel");
     return MAYA_OK;
 }
@@ -2745,13 +2807,13 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
                                            : launch_gate_up_iq1s_pos(a, *st, s, &hd)))
             return rc;
         gate_up_done = true;
-    } else if (logits && n_tokens > 1 && n_tokens <= (join ? kHeadBesideTokens : MAYA_MAX_TOKENS) && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 &&
+    } else if (logits && (n_tokens > 1 || n_expert > 256) && n_tokens <= (join ? kHeadBesideTokens : MAYA_MAX_TOKENS) && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 &&
                x_dtype <= 2) {
         // several tokens, one launch: route, plan, group and round x, for the routed experts' rows and a shared Q8_0 expert's
         const bool q8k = q8k_act(l->gate_type);
         if (q80 && !q8k) sh.x = w.x;
         // (the head stores 16 codes and two sums at a time, maya_quant_act one: a caller's buffer that is not aligned for that is its)
-        sh_rounded = q80 && (((uintptr_t) sh.x.q & 15) | ((uintptr_t) sh.x.bsums & 3)) == 0;
+        sh_rounded = q80 && n_tokens > 1 && (((uintptr_t) sh.x.q & 15) | ((uintptr_t) sh.x.bsums & 3)) == 0;
         if ((rc = launch_window_head(rs, logits, n_tokens, n_expert, k, expert_table, ids, weights, w.plan_ptr, w.grp_ptr, w.grp_start, w.grp_ent, w.n_groups,
                                      x, x_dtype, l->n_embd, q8k ? w.x : none, !q8k ? w.x : sh_rounded ? sh.x : none, as_stream(stream))))
             return rc;

@@ -1,4 +1,4 @@
-// maya_route.hpp - the softmax router on one wave (up to 256 experts), exactly and by the order of the logits alone: what the kernels
+// maya_route.hpp - the softmax router on one wave (up to 512 experts), exactly and by the order of the logits alone: what the kernels
 // that route for themselves share (the routing kernels, the decode layers whose head rides in their gate/up launch).
 #pragma once
 
@@ -83,8 +83,8 @@ __device__ __forceinline__ void route_narrow_regs(int n_expert, int k, const dou
         for (int q = 0; q < R; ++q) key[q] = (q == r && lane == at) ? -1 : key[q];
         if (lane == i) id = 64 * r + at, my_w = R > 4 && top == 0x7fffffff ? (int) 0xffc00000 : top;
         if (R == 4 && tab) {
-            // (written out: as a loop over tab the select becomes an index, the table memory, and a kernel with scratch memory starts
-            // 10 us later)
+            // (written out: as a loop over tab the select becomes an index, the table goes to memory, and the kernels whose launch holds
+            // this router take 11 us longer)
             const uint64_t tq = r == 0 ? tab[0] : r == 1 ? tab[1] : r == 2 ? tab[2] : tab[3];
             const uint32_t plo = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) tq, at);
             const uint32_t phi = (uint32_t) __builtin_amdgcn_readlane((int) (uint32_t) (tq >> 32), at);
@@ -103,17 +103,21 @@ __device__ __forceinline__ int float_order_key(float v) {
     const int b = __float_as_int(v);
     return b >= 0 ? b : b ^ 0x7fffffff;
 }
-// The softmax router on ONE wave, nothing but registers (up to 256 experts, 4 a lane: lane L holds experts L, L + 64, ...;
-// lv = -inf and tab = 0 past the end): the maximum, the exponentials, then route_narrow_regs.  Lane i < k returns slot i.
-__device__ __forceinline__ void route_wave_softmax(const float (&lv)[4], const uint64_t (&tab)[4], int n_expert, int k, int& id,
+// The softmax router on ONE wave, nothing but registers (up to 64 R experts, R a lane: lane L holds experts L, L + 64, ...;
+// lv = -inf and tab = 0 past the end): the maximum, the exponentials, then route_narrow_regs.  Lane i < k returns slot i (its blob's
+// address for R = 4 only).
+template <int R>
+__device__ __forceinline__ void route_wave_softmax(const float (&lv)[R], const uint64_t (&tab)[R], int n_expert, int k, int& id,
                                                    float& w, uint64_t& ptr) {
     const int lane = threadIdx.x & 63;
-    float mx = fmaxf(fmaxf(lv[0], lv[1]), fmaxf(lv[2], lv[3]));
+    float mx = fmaxf(lv[0], lv[1]);
+#pragma unroll
+    for (int r = 2; r < R; ++r) mx = fmaxf(mx, lv[r]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
-    double ex[4];
+    double ex[R];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ex[r] = 64 * r + lane < n_expert ? exp((double) lv[r] - (double) mx) : 0.0;
+    for (int r = 0; r < R; ++r) ex[r] = 64 * r + lane < n_expert ? exp((double) lv[r] - (double) mx) : 0.0;
     route_narrow_regs(n_expert, k, ex, tab, id, w, ptr);
 }
 
@@ -126,43 +130,41 @@ __device__ __forceinline__ void route_wave_softmax(const float (&lv)[4], const u
 // Anything else (ties, near ties, the sub-normal range, NaN / Inf) returns false and the caller runs the exact router.
 //
 // A round must be short (k + 1 of them run one after the other on one wave while its workgroup waits), so a key is one
-// word that names its expert: the logit's ordered bits with the low byte replaced by 255 - index.  The largest key of
-// the wave IS the pick, with no search for the lane that holds it.  The 8 bits given up make picks inside one
+// word that names its expert: the logit's ordered bits with the low byte (R = 8: nine bits) replaced by 255 - index.  The largest key
+// of the wave IS the pick, with no search for the lane that holds it.  The bits given up make picks inside one
 // 256-ulp bucket come out in index order: the check below therefore compares the picks' TRUE logits (a wrong order
 // shows as a negative gap), and holds the k-th pick against the upper end of the (k + 1)-th pick's bucket, above which
-// nothing unpicked can lie.  One wave, k < n_expert <= 256, k + 1 <= 64; s_lv [256] floats of LDS scratch; lane i < k
+// nothing unpicked can lie.  One wave, k < n_expert <= 64 R, k + 1 <= 64; s_lv [64 R] floats of LDS scratch; lane i < k
 // gets slot i's expert.
 // (The sigmoid router picks by the score p + bias itself, so its keys ARE the exact router's: margin 0 - any strictly
 // descending order is the router's - and no range to keep; `fin` then says that no logit and no score is non-finite.)
-__device__ __forceinline__ bool route_wave_order_only(const float (&lv)[4], bool fin, int n_expert, int k, float* s_lv, float margin,
+template <int R>
+__device__ __forceinline__ bool route_wave_order_only(const float (&lv)[R], bool fin, int n_expert, int k, float* s_lv, float margin,
                                                       float range, int& my_id) {
     const int lane = threadIdx.x & 63;
-    constexpr int kNone = (int) 0x80000000;
-    int k0, k1, k2, k3;
-    {
-        int key[4];
+    constexpr int kNone = (int) 0x80000000, kIndex = 64 * R - 1;
+    int key[R];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = 64 * r + lane;
-            const bool have = e < n_expert;
-            key[r] = have ? (int) (((uint32_t) float_order_key(lv[r]) & 0xffffff00u) | (uint32_t) (255 - e)) : kNone;
-            fin = fin && (!have || isfinite(lv[r]));
-            s_lv[e] = lv[r];
-        }
-        k0 = key[0], k1 = key[1], k2 = key[2], k3 = key[3];
+    for (int r = 0; r < R; ++r) {
+        const int e = 64 * r + lane;
+        const bool have = e < n_expert;
+        key[r] = have ? (int) (((uint32_t) float_order_key(lv[r]) & ~(uint32_t) kIndex) | (uint32_t) (kIndex - e)) : kNone;
+        fin = fin && (!have || isfinite(lv[r]));
+        s_lv[e] = lv[r];
     }
     int my_key = kNone;
     for (int i = 0; i <= k; ++i) {
-        const int top = wave_max_i32(max(max(k0, k1), max(k2, k3)));
-        k0 = k0 == top ? kNone : k0;
-        k1 = k1 == top ? kNone : k1;
-        k2 = k2 == top ? kNone : k2;
-        k3 = k3 == top ? kNone : k3;
+        int best = max(max(key[0], key[1]), max(key[2], key[3]));
+#pragma unroll
+        for (int r = 4; r < R; ++r) best = max(best, key[r]);
+        const int top = wave_max_i32(best);
+#pragma unroll
+        for (int r = 0; r < R; ++r) key[r] = key[r] == top ? kNone : key[r];
         my_key = lane == i ? top : my_key;
     }
-    const int id = 255 - (my_key & 255);
+    const int id = kIndex - (my_key & kIndex);
     const float val = lane <= k ? s_lv[id] : 0.0f;
-    const int ub_key = my_key | 255;
+    const int ub_key = my_key | kIndex;
     const float ub = __int_as_float(ub_key >= 0 ? ub_key : ub_key ^ 0x7fffffff);   // the bucket's upper end
     const float nxt = __shfl_down(lane == k ? ub : val, 1, kWave);
     const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), 0));

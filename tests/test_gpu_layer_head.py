@@ -354,3 +354,55 @@ def test_other_types_head_in_the_gate_up_launch(lib, oracle, ty, n_embd, n_ff, n
     out = fused.forward(store.table, dev(lg), xin.cuda().view(1, -1)).cpu().numpy()
     wi, ww, wout = oracle_layer(oracle, ty, ty, blobs, k, n_embd, n_ff, lg, x32.reshape(1, -1))
     assert np.array_equal(fused.ids.cpu().numpy(), wi) and rel_l2(out[0], wout[0]) <= 1e-3
+
+
+def wide_logits(ne, seed):
+    """Rows of `ne` logits: the edge cases of logit_cases, spread so that what decides sits on either side of 256."""
+    rng = np.random.default_rng(seed)
+    base = rng.standard_normal(ne).astype(np.float32)
+    rows = [base.copy() for _ in range(10)]
+    rows[1][[ne - 1, 3, 256]] = np.float32(4.5)
+    order = np.argsort(-base)
+    rows[2][order[8]] = rows[2][order[7]]
+    rows[3][order[3]] = np.nextafter(rows[3][order[2]], np.float32(-10))
+    rows[3][order[8]] = np.nextafter(rows[3][order[7]], np.float32(-10))
+    rows[4][:] = 0.0
+    rows[5][ne - 1] = np.float32(300.0)
+    rows[6] = (base * np.float32(40.0)).astype(np.float32)
+    rows[7][256] = np.float32(np.inf)
+    rows[8][ne - 1] = np.float32(np.nan)
+    rows[9] = np.arange(ne, dtype=np.float32) * np.float32(5e-7)
+    return rows
+
+
+@pytest.mark.parametrize("sigmoid", (False, True))
+@pytest.mark.parametrize("ty,n_embd,n_ff,ne,nt", ((12, 2048, 256, 257, 1), (12, 3072, 2048, 512, 1), (22, 4352, 256, 300, 1), (19, 2304, 256, 512, 1),
+                                                  (8, 2048, 256, 288, 1), (12, 2048, 256, 512, 3), (8, 2048, 256, 257, 10), (22, 2048, 256, 300, 16)))
+def test_heads_of_more_than_256_experts(lib, ty, n_embd, n_ff, ne, nt, sigmoid):
+    """257 to 512 experts, the head in the gate/up launch or in one of its own: ids and weights bit for bit the routing launch's, the
+    output that of the layer given these ids and weights; x also from an address that is not 16-byte aligned."""
+    k, kinds = 8, 9
+    blobs = make_experts(ty, ty, n_embd, n_ff, kinds, 5 * ne + ty)
+    store = lib.ExpertStore(blobs, pack_layout=lib.layout(ty, ty, n_embd, n_ff)[0])
+    table = store.table[torch.arange(ne, device="cuda") % kinds].contiguous()
+    table[5::11] = 0                                            # not resident
+    rng = np.random.default_rng(ne + nt)
+    bias = dev((rng.standard_normal(ne) * 0.1).astype(np.float32))
+    router = lib.Router(lib.ROUTER_SIGMOID, 1, bias.data_ptr(), 2.5) if sigmoid else None
+    layer, given = (lib.MoeLayer(ty, ty, n_embd, n_ff, ne, k, max_tokens=nt, packing=1) for _ in range(2))
+    x = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda()
+    rows = wide_logits(ne, ne)
+    for first in range(0, len(rows), nt):
+        print("rows from", first, flush=True)
+        lg = dev(np.stack([rows[(first + i) % len(rows)] for i in range(nt)]))
+        out = layer.forward(table, lg, x, router=router).clone()
+        ids, w, _ = lib.route_plan(lg, k, table, router)
+        want = given.forward(table, None, x, routed=(ids, w)).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(layer.ids, ids) and torch.equal(layer.weights.view(torch.int32), w.view(torch.int32)), first
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32)), first
+        buf = torch.empty(x.numel() + 1, device="cuda")
+        buf[1:] = x.reshape(-1)
+        out = layer.forward(table, lg, buf[1:].reshape(nt, n_embd), router=router)
+        torch.cuda.synchronize()
+        assert torch.equal(layer.ids, ids) and torch.equal(out.view(torch.int32), want.view(torch.int32)), first
