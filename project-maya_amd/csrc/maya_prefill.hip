@@ -9,6 +9,7 @@
 // super-block.  Weights and activations go from HBM to LDS without registers, about two super-blocks and two or three row groups ahead.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <math.h>
 #include <stdint.h>
@@ -33,10 +34,28 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // one workgroup scattering all 32 chunks a wave, 11.9 us like this; 4096 entries over 256: 12 us, 7.5 us.
 // dynamic LDS: [kPlanWaves][n_expert] 64-bit lane masks (with_masks), seg[kPlanWaves][n_expert] counts -> bases,
 // before[n_expert], total[n_expert], base[n_expert + 1], tbase[n_expert + 1]
+// What a layer call's GEMMs are to do, a row of their grids an item (a stage call has the plan's tiles only).  Every row of the grid
+// but the last ones has work.  With a workgroup for each tile of 64 rows, the second tile of every pair was a workgroup that
+// returned at once; workgroups go to an XCD's shader engines in turn whatever they do and in order, so with few bands of weight rows an
+// XCD some engines got the work and the others the returns.  Microseconds a layer call, tiles and items: 128 experts
+// of 4096 x 512 (8 bands), 94 rows each, Q4_K 393 -> 327, IQ2_S 379 -> 305; 288 of 3072 x 1536 (24 bands) 1445 -> 1314; 512 tokens,
+// skewed, of 256 experts of 7168 x 2048 (32 and 56) 836 -> 808; 4096 tokens of 288 of 4096 x 2048 (32) 2490 -> 2462.
+// Workgroups that stay and take item after item from a counter were slower than one an item: 4096 tokens 2470, the skewed 512
+// 832 (an item's stores have to land before the next one's copies can be told apart from them; a new workgroup does not wait).
+// So was finding the leading tiles in the GEMM from the plan's list: 2595.
+struct PfItem {
+    uint64_t blob;   // an expert's bytes
+    int32_t row0, nrows;   // of its rows
+};
+struct PfWork {
+    PfItem* list;
+    int32_t* n;      // [1] items
+    int rows;
+};
 constexpr int kPlanMaxGroups = 64;   // (at 1 << 20 entries the counting would outweigh the scatter)
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_t* __restrict__ ids, int n_entries,
                                                                     const uint64_t* __restrict__ table, int n_expert,
-                                                                    maya_prefill_plan p, int max_tiles, int with_masks) {
+                                                                    maya_prefill_plan p, int max_tiles, int with_masks, PfWork work) {
     extern __shared__ __attribute__((aligned(16))) int32_t sm[];
     unsigned long long* mask = with_masks ? (unsigned long long*) sm : nullptr;
     int32_t* seg = sm + (with_masks ? 2 * kPlanWaves * n_expert : 0);
@@ -87,10 +106,8 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
     }
     __syncthreads();
     // the experts' first rows (wave 0) and first tiles (wave 1): a lane a run of experts, a scan over the lanes between two passes
-    if (wave < 2) {
+    auto first_of = [&](auto size, int32_t* o) {
         const int per_lane = (n_expert + 63) >> 6, x0 = lane * per_lane;
-        int32_t* o = wave ? tbase : base;
-        auto size = [&](int x) { return wave ? (total[x] + kPfRows - 1) / kPfRows : total[x]; };
         int local = 0;
         for (int i = 0; i < per_lane; ++i)
             if (x0 + i < n_expert) local += size(x0 + i);
@@ -107,7 +124,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
                 run += size(x0 + i);
                 if (x0 + i == n_expert - 1) o[n_expert] = run;
             }
-    }
+    };
+    if (wave == 0) first_of([&](int x) { return total[x]; }, base);
+    if (wave == 1) first_of([&](int x) { return (total[x] + kPfRows - 1) / kPfRows; }, tbase);
     __syncthreads();
     if (blockIdx.x == 0) {
         for (int x = tid; x <= n_expert; x += kPlanThreads) p.bounds[x] = base[x];
@@ -118,6 +137,16 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
                 p.tile_row0[t] = base[x] + (t - tbase[x]) * kPfRows;
             }
         if (tid == 0) *p.n_tiles = min(tbase[n_expert], max_tiles);
+    }
+    if (work.list != nullptr && blockIdx.x == min(1u, gridDim.x - 1)) {   // the GEMMs' work list: every expert's rows in runs of work.rows
+        __syncthreads();   // (tbase's readers above)
+        if (wave == 0) {
+            first_of([&](int x) { return (total[x] + work.rows - 1) / work.rows; }, tbase);
+            if (lane == 0) *work.n = tbase[n_expert];
+        }
+        __syncthreads();
+        for (int x = tid; x < n_expert; x += kPlanThreads)
+            for (int r = 0, t = tbase[x]; r < total[x]; r += work.rows, ++t) work.list[t] = {table[x], base[x] + r, min(work.rows, total[x] - r)};
     }
     // the stable scatter: 64 entries a step, a lane's rank = the earlier lanes of the step with its expert
     for (int c0 = lo; c0 < hi; c0 += 64) {
@@ -243,11 +272,13 @@ struct PfGemm {
     maya_prefill_act x;    // the tile rows' activations [rows][k]
     float* out;            // gate/up: the SwiGLU outputs [rows][n] F32; down: part [rows][n]
     float limit;
+    PfWork work;           // (list null: the plan's tiles, a workgroup each)
 };
 
 // The codes of a group of rows in LDS: 256 bytes a row, 16-byte chunk c of row r at position c ^ (r & 15): the 16 rows x 4
 // k-groups of a matrix-core operand read then hit distinct banks.
 typedef __attribute__((address_space(3))) void* pf_lptr;
+typedef __attribute__((address_space(3))) uint8_t* pf_lds8;
 // the 8 six-bit scales and 8 six-bit minimums of a Q4_K block's 12 bytes, as bytes of two words each
 // (get_scale_min_k4, include/strata/artifact/dequant.hpp:162-172)
 __device__ __forceinline__ void q4k_unpack_scales(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t (&sc)[2], uint32_t (&mn)[2]) {
@@ -271,9 +302,7 @@ typedef unsigned short pf_u16x2 __attribute__((ext_vector_type(2)));
 // fills, so before any LDS read of its own it waits for every copy in flight - here that would be the copy of the
 // super-block two ahead, issued moments earlier.  These reads it does not see; each group is followed by a wait
 // on the registers it filled (the values pass through the wait, so nothing that uses them can move above it).
-__device__ __forceinline__ uint32_t pf_lds_addr(const void* p) {
-    return (uint32_t) (uintptr_t) (const __attribute__((address_space(3))) void*) p;
-}
+__device__ __forceinline__ uint32_t pf_lds_addr(pf_lds8 p) { return (uint32_t) (uintptr_t) p; }
 typedef int pf_i2 __attribute__((ext_vector_type(2)));
 template <int OFF> __device__ __forceinline__ pf_i2 pf_lds_b64(uint32_t addr) {
     pf_i2 v;
@@ -366,7 +395,7 @@ template <bool SUMS> struct PfRowsDma {   // SUMS: with the code sums that a typ
         od = (uint32_t) ((lane & 31) * (k >> 8) * 4);
         ld = (uint32_t) (min(l0 + (lane & 31), last) * (k >> 8) * 4);
     }
-    template <bool LAST> __device__ __forceinline__ void copy(uint8_t* buf, int sb, int m) const {
+    template <bool LAST> __device__ __forceinline__ void copy(pf_lds8 buf, int sb, int m) const {
         const int at = LAST ? 0 : 32 * m;
 #pragma unroll
         for (int n = 0; n < 2; ++n)
@@ -415,18 +444,18 @@ template <bool GU> struct PfQ4K {
     __device__ __forceinline__ int behind(int slot) const { return slot == 2 * kPiece ? 0 : slot + kPiece; }
     // The next piece, to `to`.  (The piece is in the lanes' offsets, not in the scalar one, which need not take part in the buffer's range
     // check: a row's last piece goes on into the row behind it, and behind the matrix there may be nothing.)
-    __device__ __forceinline__ void copy(uint8_t* to) {
+    __device__ __forceinline__ void copy(pf_lds8 to) {
         if (left <= 0) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(r[i >> 1], (pf_lptr) (to + i * 1024), 16, at[i & 1], 0, 0, 0);
         at[0] += 128, at[1] += 128, --left;
     }
-    __device__ __forceinline__ void first(uint8_t* to) {
+    __device__ __forceinline__ void first(pf_lds8 to) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) copy(to + i * kPiece);
     }
     // super-block sb is in registers: the one or two pieces that it was the last to want make room
-    __device__ __forceinline__ void next(uint8_t* to, int sb) {
+    __device__ __forceinline__ void next(pf_lds8 to, int sb) {
         copy(to + cur);
         cur = behind(cur);
         if ((sb & 7) == 7) {
@@ -502,11 +531,17 @@ template <typename W> struct PfLds {   // the weight type's tables, the activati
     static constexpr int ring = W::kLdsAt, w = ring + W::kRing * kPfSlot, bytes = w + 4 * W::kWave;
 };
 
+// the rows that a workgroup computes, of the expert whose bytes are at blob
+struct PfTile {
+    const uint8_t* blob;
+    int row0, nrows;
+};
+
 // NB: 0, or the blocks of 8 rows of a tile that takes the codes themselves to the matrix cores
 template <typename W, bool GU, int NM, int NB = 0>
-__device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, int row0, int nrows) {
+__device__ __forceinline__ void pf_tile(const PfGemm& a, pf_lds8 lds, const PfTile& t) {
+    const int row0 = t.row0, nrows = t.nrows;
     typedef PfLds<W> S;
-    const uint8_t* blob = (const uint8_t*) a.table[ex];
     const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the wave's first feature (gate/up) or output row (down): n is a multiple of 256, every workgroup has all its rows
@@ -521,7 +556,7 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
     PfRowsDma<W::kSums> dma;
     dma.init(a, row0, nrows, NM, wave, lane);
     W wts;
-    uint8_t* const wlds = lds + S::w + wave * W::kWave;
+    const pf_lds8 wlds = lds + S::w + wave * W::kWave;
     // the copies of pass (sb, m) + kAhead go into the slot of the pass before (sb, m); in the prologue, of the first kAhead passes
     constexpr int kAhead = W::kRing - 1;
     auto copy_pass = [&](auto mc, int sb, int slot) {   // (M in 0 .. NM - 1 + kAhead: pass M of super-block sb on)
@@ -531,7 +566,7 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
     };
     pf_for_m<0, kAhead>([&](auto mc) { copy_pass(mc, 0, decltype(mc)::value); });
     int slot = 0;
-    wts.init(a, blob, n0, lane);
+    wts.init(a, t.blob, n0, lane);
     wts.first(wlds);
     // a lane's 16 codes of sub-block j: the row's 16-byte chunk 2 j + kh, which sits at that index ^ (the row & 15)
     const uint32_t a_base = ln * 256 + (((ln & 15) ^ kh) << 4);
@@ -690,36 +725,46 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, uint8_t* lds, int ex, i
 // the middle of 128 of them.  False where there are none: past the last tile, or the workgroup of the tile before takes them.
 // (Both sides read the list itself, so a caller's part of it is what is computed.)
 static_assert(2 * kPfRows == 4 * 32, "four row groups of a workgroup at most");
-struct PfTile { int ex, row0, nrows; };
 __device__ __forceinline__ bool pf_my_tile(const PfGemm& a, PfTile& t) {
     const int tile = blockIdx.y, n = *a.plan.n_tiles;
     if (tile >= n) return false;
-    t.ex = a.plan.tile_expert[tile], t.row0 = a.plan.tile_row0[tile];
+    const int ex = a.plan.tile_expert[tile];
+    t.row0 = a.plan.tile_row0[tile];
     const int before = max(tile - 1, 0), behind = min(tile + 1, n - 1);
     const int bx = a.plan.tile_expert[before], b0 = a.plan.tile_row0[before], nx = a.plan.tile_expert[behind], n0 = a.plan.tile_row0[behind];
-    const int first = a.plan.bounds[t.ex], at = (t.row0 - first) % (2 * kPfRows);
-    if (at == kPfRows && bx == t.ex && b0 == t.row0 - kPfRows) return false;
-    const bool two = at == 0 && nx == t.ex && n0 == t.row0 + kPfRows;
-    t.nrows = min(two ? 2 * kPfRows : kPfRows, a.plan.bounds[t.ex + 1] - t.row0);
+    const int first = a.plan.bounds[ex], at = (t.row0 - first) % (2 * kPfRows);
+    if (at == kPfRows && bx == ex && b0 == t.row0 - kPfRows) return false;
+    const bool two = at == 0 && nx == ex && n0 == t.row0 + kPfRows;
+    t.nrows = min(two ? 2 * kPfRows : kPfRows, a.plan.bounds[ex + 1] - t.row0);
+    t.blob = (const uint8_t*) a.table[ex];
+    return true;
+}
+
+// the same from the work list where there is one
+__device__ __forceinline__ bool pf_my_rows(const PfGemm& a, PfTile& t) {
+    if (a.work.list == nullptr) return pf_my_tile(a, t);
+    if ((int) blockIdx.y >= *a.work.n) return false;
+    const PfItem i = a.work.list[blockIdx.y];
+    t.blob = (const uint8_t*) i.blob, t.row0 = i.row0, t.nrows = i.nrows;
     return true;
 }
 
 #include "maya_prefill_iq2s.hpp"
 
-// grid (bands of weight rows, tiles at most)
+// grid (bands of weight rows, items or tiles at most)
 template <bool GU>
 __global__ __launch_bounds__(256, 2) void prefill_q4k_kernel(PfGemm a) {
     typedef PfQ4K<GU> W;
     __shared__ __attribute__((aligned(256))) uint8_t lds[PfLds<W>::bytes];
     PfTile t;
-    if (!pf_my_tile(a, t)) return;
-    if (t.nrows <= 8) pf_tile<W, GU, 1, 1>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 16) pf_tile<W, GU, 1, 2>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 24) pf_tile<W, GU, 1, 3>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 32) pf_tile<W, GU, 1>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 64) pf_tile<W, GU, 2>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 96) pf_tile<W, GU, 3>(a, lds, t.ex, t.row0, t.nrows);
-    else pf_tile<W, GU, 4>(a, lds, t.ex, t.row0, t.nrows);
+    if (!pf_my_rows(a, t)) return;
+    if (t.nrows <= 8) pf_tile<W, GU, 1, 1>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 16) pf_tile<W, GU, 1, 2>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 24) pf_tile<W, GU, 1, 3>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 32) pf_tile<W, GU, 1>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 64) pf_tile<W, GU, 2>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 96) pf_tile<W, GU, 3>(a, (pf_lds8) lds, t);
+    else pf_tile<W, GU, 4>(a, (pf_lds8) lds, t);
 }
 
 template <int ODT>
@@ -808,27 +853,21 @@ static bool plan_ok(const maya_prefill_plan* p) {
 static bool act_ok(const maya_prefill_act& a) {
     return a.q && a.d && a.s && (((uintptr_t) a.q | (uintptr_t) a.s) & 15) == 0 && ((uintptr_t) a.d & 3) == 0;
 }
+// The rows of a GEMM's grid: every tile of a plan, or the items that a list can hold.
+static unsigned pf_grid_rows(const PfWork& work, int n_entries, int n_expert) {
+    return work.list ? (unsigned) (n_entries / work.rows + std::min(n_entries, n_expert)) : (unsigned) maya_moe_prefill_max_tiles(n_entries, n_expert);
+}
 template <bool GU>
-static int pf_launch(const PfGemm& a, dim3 grid, hipStream_t s) {
+static void pf_launch(const PfGemm& a, dim3 grid, hipStream_t s) {
     hipLaunchKernelGGL(prefill_q4k_kernel<GU>, grid, dim3(256), 0, s, a);
-    return MAYA_OK;
 }
 
 }  // namespace maya
 
 using namespace maya;
 
-extern "C" {
-
-int maya_moe_prefill_tile_rows(void) { return kPfRows; }
-int maya_moe_prefill_max_tiles(int n_entries, int n_expert) {
-    if (n_entries <= 0 || n_expert <= 0) return 0;
-    return (n_entries + kPfRows - 1) / kPfRows + n_expert;
-}
-int maya_moe_prefill_supported(int type) { return type == kQ4_K || type == kIQ2_S ? 1 : 0; }
-
-int maya_moe_prefill_plan(const int32_t* ids, int n_entries, const uint64_t* expert_table, int n_expert,
-                          const maya_prefill_plan* plan, void* stream) {
+static int pf_plan(const int32_t* ids, int n_entries, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan,
+                   const PfWork& work, void* stream) {
     DeviceState* st;
     if (const int rc = current_state(&st)) return rc;
     if (!ids || !expert_table || !plan_ok(plan)) return fail(MAYA_E_ARG, "prefill_plan: null pointer");
@@ -842,9 +881,103 @@ int maya_moe_prefill_plan(const int32_t* ids, int n_entries, const uint64_t* exp
     if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) prefill_plan_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
     const int groups = (n_entries + kPlanThreads - 1) / kPlanThreads;
     hipLaunchKernelGGL(prefill_plan_kernel, dim3(groups < kPlanMaxGroups ? groups : kPlanMaxGroups), dim3(kPlanThreads), lds, as_stream(stream),
-                       ids, n_entries, expert_table, n_expert, *plan, maya_moe_prefill_max_tiles(n_entries, n_expert), with_masks);
+                       ids, n_entries, expert_table, n_expert, *plan, maya_moe_prefill_max_tiles(n_entries, n_expert), with_masks, work);
     MAYA_LAUNCHED("prefill_plan_kernel");
     return MAYA_OK;
+}
+
+static int prefill_check(const char* what, const maya_moe_layout* l, const uint64_t* table, int n_expert, const maya_prefill_plan* plan,
+                         int n_entries, int type_a, int type_b, int64_t k) {
+    if (!l || !table || !plan_ok(plan)) return fail(MAYA_E_ARG, "%s: null pointer", what);
+    if (type_a != type_b || (type_a != kQ4_K && type_a != kIQ2_S))
+        return fail(MAYA_E_UNSUPPORTED, "%s: weight types %d / %d (Q4_K or IQ2_S, gate and up alike)", what, type_a, type_b);
+    if (l->packing != MAYA_PACK_GGUF && l->packing != MAYA_PACK_STREAM) return fail(MAYA_E_UNSUPPORTED, "%s: packing %d", what, l->packing);
+    if (type_a == kIQ2_S && l->packing != MAYA_PACK_STREAM)
+        return fail(MAYA_E_UNSUPPORTED, "%s: IQ2_S rows are taken in the stream packing (maya_moe_repack)", what);
+    if (l->n_embd <= 0 || l->n_ff <= 0 || l->n_embd % 256 || l->n_ff % 256)
+        return fail(MAYA_E_SHAPE, "%s: n_embd %d / n_ff %d: multiples of 256 wanted", what, l->n_embd, l->n_ff);
+    // (IQ2_S: the kernel's 16-byte copies into LDS want quads - 328 bytes a block - of a multiple of 16 bytes: an even number of blocks)
+    if (type_a == kIQ2_S && k % 512) return fail(MAYA_E_SHAPE, "%s: IQ2_S rows of %lld values: a multiple of 512 wanted", what, (long long) k);
+    if (type_a == kIQ2_S)
+        if (const int rc = prefill_iq2s_lds_ok(what)) return rc;
+    if ((l->gate_off | l->up_off | l->down_off) & 15) return fail(MAYA_E_ARG, "%s: matrix offsets not 16-byte aligned", what);
+    // (an entry is a row of the second grid dimension in the quantizers' launches)
+    if (n_entries <= 0 || n_entries > 65535 || n_expert <= 0) return fail(MAYA_E_SHAPE, "%s: entries %d (1..65535) experts %d", what, n_entries, n_expert);
+    return MAYA_OK;
+}
+
+static int pf_gate_up(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan, int n_entries,
+                      maya_prefill_act xq, float limit, float* h, maya_prefill_act hq, const PfWork& work, void* stream) {
+    DeviceState* st;
+    if (const int rc = current_state(&st)) return rc;
+    if (const int rc = prefill_check("prefill_gate_up", l, expert_table, n_expert, plan, n_entries, l ? l->gate_type : 0, l ? l->up_type : 0, l ? l->n_embd : 0)) return rc;
+    if (!act_ok(xq) || !act_ok(hq) || !h) return fail(MAYA_E_ARG, "prefill_gate_up: null or misaligned activations");
+    PfGemm a{};
+    a.table = expert_table;
+    a.plan = *plan;
+    a.off[0] = l->gate_off;
+    a.off[1] = l->up_off;
+    a.k = l->n_embd;
+    a.n = l->n_ff;
+    a.row_bytes = (int64_t) (l->n_embd / 256) * 144;
+    a.x = xq;
+    a.out = h;
+    a.limit = limit;
+    a.work = work;
+    const dim3 grid((unsigned) (l->n_ff / 64), pf_grid_rows(work, n_entries, n_expert));
+    if (l->gate_type == kIQ2_S) {
+        hipLaunchKernelGGL(prefill_iq2s_kernel<true>, grid, dim3(256), 0, as_stream(stream), a, st->cb);
+        MAYA_LAUNCHED("prefill_iq2s_kernel<gate_up>");
+    } else {
+        pf_launch<true>(a, grid, as_stream(stream));
+        MAYA_LAUNCHED("prefill_q4k_kernel<gate_up>");
+    }
+    const dim3 qgrid((unsigned) ((l->n_ff + 8191) / 8192), (unsigned) n_entries);
+    hipLaunchKernelGGL(prefill_quant_rows_kernel, qgrid, dim3(256), 0, as_stream(stream), (const float*) h, *plan, n_expert, (int64_t) l->n_ff, hq);
+    MAYA_LAUNCHED("prefill_quant_rows_kernel");
+    return MAYA_OK;
+}
+
+static int pf_down(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan, int n_entries,
+                   maya_prefill_act hq, float* part, const PfWork& work, void* stream) {
+    DeviceState* st;
+    if (const int rc = current_state(&st)) return rc;
+    if (const int rc = prefill_check("prefill_down", l, expert_table, n_expert, plan, n_entries, l ? l->down_type : 0, l ? l->down_type : 0, l ? l->n_ff : 0)) return rc;
+    if (!act_ok(hq) || !part) return fail(MAYA_E_ARG, "prefill_down: null or misaligned pointer");
+    if (l->n_embd % 32) return fail(MAYA_E_SHAPE, "prefill_down: n_embd %d", l->n_embd);
+    PfGemm a{};
+    a.table = expert_table;
+    a.plan = *plan;
+    a.off[0] = l->down_off;
+    a.k = l->n_ff;
+    a.n = l->n_embd;
+    a.row_bytes = (int64_t) (l->n_ff / 256) * 144;
+    a.x = hq;
+    a.out = part;
+    a.work = work;
+    const dim3 grid((unsigned) ((l->n_embd + 127) / 128), pf_grid_rows(work, n_entries, n_expert));
+    if (l->down_type == kIQ2_S) {
+        hipLaunchKernelGGL(prefill_iq2s_kernel<false>, grid, dim3(256), 0, as_stream(stream), a, st->cb);
+        MAYA_LAUNCHED("prefill_iq2s_kernel<down>");
+    } else {
+        pf_launch<false>(a, grid, as_stream(stream));
+        MAYA_LAUNCHED("prefill_q4k_kernel<down>");
+    }
+    return MAYA_OK;
+}
+
+extern "C" {
+
+int maya_moe_prefill_tile_rows(void) { return kPfRows; }
+int maya_moe_prefill_max_tiles(int n_entries, int n_expert) {
+    if (n_entries <= 0 || n_expert <= 0) return 0;
+    return (n_entries + kPfRows - 1) / kPfRows + n_expert;
+}
+int maya_moe_prefill_supported(int type) { return type == kQ4_K || type == kIQ2_S ? 1 : 0; }
+
+int maya_moe_prefill_plan(const int32_t* ids, int n_entries, const uint64_t* expert_table, int n_expert,
+                          const maya_prefill_plan* plan, void* stream) {
+    return pf_plan(ids, n_entries, expert_table, n_expert, plan, PfWork{}, stream);
 }
 
 int maya_moe_prefill_quant(const void* x, int x_dtype, int64_t x_stride, const maya_prefill_plan* plan, int n_entries,
@@ -868,85 +1001,14 @@ int maya_moe_prefill_quant(const void* x, int x_dtype, int64_t x_stride, const m
     return MAYA_OK;
 }
 
-static int prefill_check(const char* what, const maya_moe_layout* l, const uint64_t* table, int n_expert, const maya_prefill_plan* plan,
-                         int n_entries, int type_a, int type_b, int64_t k) {
-    if (!l || !table || !plan_ok(plan)) return fail(MAYA_E_ARG, "%s: null pointer", what);
-    if (type_a != type_b || (type_a != kQ4_K && type_a != kIQ2_S))
-        return fail(MAYA_E_UNSUPPORTED, "%s: weight types %d / %d (Q4_K or IQ2_S, gate and up alike)", what, type_a, type_b);
-    if (l->packing != MAYA_PACK_GGUF && l->packing != MAYA_PACK_STREAM) return fail(MAYA_E_UNSUPPORTED, "%s: packing %d", what, l->packing);
-    if (type_a == kIQ2_S && l->packing != MAYA_PACK_STREAM)
-        return fail(MAYA_E_UNSUPPORTED, "%s: IQ2_S rows are taken in the stream packing (maya_moe_repack)", what);
-    if (l->n_embd <= 0 || l->n_ff <= 0 || l->n_embd % 256 || l->n_ff % 256)
-        return fail(MAYA_E_SHAPE, "%s: n_embd %d / n_ff %d: multiples of 256 wanted", what, l->n_embd, l->n_ff);
-    // (IQ2_S: the kernel's 16-byte copies into LDS want quads - 328 bytes a block - of a multiple of 16 bytes: an even number of blocks)
-    if (type_a == kIQ2_S && k % 512) return fail(MAYA_E_SHAPE, "%s: IQ2_S rows of %lld values: a multiple of 512 wanted", what, (long long) k);
-    if (type_a == kIQ2_S) {
-        int rc = prefill_iq2s_lds_ok<true>(what);
-        if (!rc) rc = prefill_iq2s_lds_ok<false>(what);
-        if (rc) return rc;
-    }
-    if ((l->gate_off | l->up_off | l->down_off) & 15) return fail(MAYA_E_ARG, "%s: matrix offsets not 16-byte aligned", what);
-    // (an entry is a row of the second grid dimension in the quantizers' launches)
-    if (n_entries <= 0 || n_entries > 65535 || n_expert <= 0) return fail(MAYA_E_SHAPE, "%s: entries %d (1..65535) experts %d", what, n_entries, n_expert);
-    return MAYA_OK;
-}
-
 int maya_moe_prefill_gate_up(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan,
                              int n_entries, maya_prefill_act xq, float limit, float* h, maya_prefill_act hq, void* stream) {
-    DeviceState* st;
-    if (const int rc = current_state(&st)) return rc;
-    if (const int rc = prefill_check("prefill_gate_up", l, expert_table, n_expert, plan, n_entries, l ? l->gate_type : 0, l ? l->up_type : 0, l ? l->n_embd : 0)) return rc;
-    if (!act_ok(xq) || !act_ok(hq) || !h) return fail(MAYA_E_ARG, "prefill_gate_up: null or misaligned activations");
-    PfGemm a{};
-    a.table = expert_table;
-    a.plan = *plan;
-    a.off[0] = l->gate_off;
-    a.off[1] = l->up_off;
-    a.k = l->n_embd;
-    a.n = l->n_ff;
-    a.row_bytes = (int64_t) (l->n_embd / 256) * 144;
-    a.x = xq;
-    a.out = h;
-    a.limit = limit;
-    const dim3 grid((unsigned) (l->n_ff / 64), (unsigned) maya_moe_prefill_max_tiles(n_entries, n_expert));
-    if (l->gate_type == kIQ2_S) {
-        hipLaunchKernelGGL(prefill_iq2s_kernel<true>, grid, dim3(256), 0, as_stream(stream), a, st->cb);
-        MAYA_LAUNCHED("prefill_iq2s_kernel<gate_up>");
-    } else {
-        if (const int rc = pf_launch<true>(a, grid, as_stream(stream))) return rc;
-        MAYA_LAUNCHED("prefill_q4k_kernel<gate_up>");
-    }
-    const dim3 qgrid((unsigned) ((l->n_ff + 8191) / 8192), (unsigned) n_entries);
-    hipLaunchKernelGGL(prefill_quant_rows_kernel, qgrid, dim3(256), 0, as_stream(stream), (const float*) h, *plan, n_expert, (int64_t) l->n_ff, hq);
-    MAYA_LAUNCHED("prefill_quant_rows_kernel");
-    return MAYA_OK;
+    return pf_gate_up(l, expert_table, n_expert, plan, n_entries, xq, limit, h, hq, PfWork{}, stream);
 }
 
 int maya_moe_prefill_down(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan,
                           int n_entries, maya_prefill_act hq, float* part, void* stream) {
-    DeviceState* st;
-    if (const int rc = current_state(&st)) return rc;
-    if (const int rc = prefill_check("prefill_down", l, expert_table, n_expert, plan, n_entries, l ? l->down_type : 0, l ? l->down_type : 0, l ? l->n_ff : 0)) return rc;
-    if (!act_ok(hq) || !part) return fail(MAYA_E_ARG, "prefill_down: null or misaligned pointer");
-    if (l->n_embd % 32) return fail(MAYA_E_SHAPE, "prefill_down: n_embd %d", l->n_embd);
-    PfGemm a{};
-    a.table = expert_table;
-    a.plan = *plan;
-    a.off[0] = l->down_off;
-    a.k = l->n_ff;
-    a.n = l->n_embd;
-    a.row_bytes = (int64_t) (l->n_ff / 256) * 144;
-    a.x = hq;
-    a.out = part;
-    const dim3 grid((unsigned) ((l->n_embd + 127) / 128), (unsigned) maya_moe_prefill_max_tiles(n_entries, n_expert));
-    if (l->down_type == kIQ2_S) {
-        hipLaunchKernelGGL(prefill_iq2s_kernel<false>, grid, dim3(256), 0, as_stream(stream), a, st->cb);
-        MAYA_LAUNCHED("prefill_iq2s_kernel<down>");
-    } else {
-        if (const int rc = pf_launch<false>(a, grid, as_stream(stream))) return rc;
-        MAYA_LAUNCHED("prefill_q4k_kernel<down>");
-    }
-    return MAYA_OK;
+    return pf_down(l, expert_table, n_expert, plan, n_entries, hq, part, PfWork{}, stream);
 }
 
 int maya_moe_prefill_combine(const maya_prefill_plan* plan, const float* weights, const float* part, int n_tokens, int k,
@@ -979,6 +1041,7 @@ int maya_moe_prefill_combine(const maya_prefill_plan* plan, const float* weights
 
 struct PrefillWs {
     maya_prefill_plan plan;
+    PfWork work;
     maya_prefill_act x, h;
     float *hf, *part;
     size_t bytes;
@@ -999,6 +1062,9 @@ static PrefillWs prefill_carve(const maya_moe_layout& l, int n_tokens, int k, in
     w.plan.tile_expert = (int32_t*) take(4 * mt);
     w.plan.tile_row0 = (int32_t*) take(4 * mt);
     w.plan.n_tiles = (int32_t*) take(4);
+    w.work.rows = 2 * kPfRows;
+    w.work.list = (PfItem*) take(sizeof(PfItem) * mt);   // (fewer than the tiles)
+    w.work.n = (int32_t*) take(4);
     auto take_act = [&](maya_prefill_act& a, size_t k) {
         a.q = (int8_t*) take(ne * k);
         a.d = (float*) take(ne * (k / 256) * 4);
@@ -1042,10 +1108,10 @@ int maya_moe_prefill_layer(const maya_moe_layout* l, const uint64_t* expert_tabl
     const int ne = n_tokens * k;
     int rc;
     if (logits && (rc = maya_moe_route_topk(logits, n_tokens, n_expert, k, ids, weights, stream))) return rc;   // (null: ids / weights are given)
-    if ((rc = maya_moe_prefill_plan(ids, ne, expert_table, n_expert, &w.plan, stream))) return rc;
+    if ((rc = pf_plan(ids, ne, expert_table, n_expert, &w.plan, w.work, stream))) return rc;
     if ((rc = maya_moe_prefill_quant(x, x_dtype, 0, &w.plan, ne, n_expert, k, l->n_embd, w.x, stream))) return rc;
-    if ((rc = maya_moe_prefill_gate_up(l, expert_table, n_expert, &w.plan, ne, w.x, limit, w.hf, w.h, stream))) return rc;
-    if ((rc = maya_moe_prefill_down(l, expert_table, n_expert, &w.plan, ne, w.h, w.part, stream))) return rc;
+    if ((rc = pf_gate_up(l, expert_table, n_expert, &w.plan, ne, w.x, limit, w.hf, w.h, w.work, stream))) return rc;
+    if ((rc = pf_down(l, expert_table, n_expert, &w.plan, ne, w.h, w.part, w.work, stream))) return rc;
     return maya_moe_prefill_combine(&w.plan, weights, w.part, n_tokens, k, l->n_embd, add, out, out_dtype, stream);
 }
 

@@ -49,7 +49,7 @@ template <bool GU> struct PfIq2s {
         pair_sel = row & 1 ? 0x07030602u : 0x05010400u;   // of two sub-blocks' words: the row's high bits, its scales
         word_sel = kh ? 0x07060302u : 0x05040100u;     // the half of the index word, the half of the sign word
     }
-    __device__ __forceinline__ void copy(uint8_t* to, int sb) const {
+    __device__ __forceinline__ void copy(pf_lds8 to, int sb) const {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r[GU ? i : 0], (pf_lptr) (to + i * 1024), 16, wat[i], sb * 256, 0, 0);
@@ -66,12 +66,12 @@ template <bool GU> struct PfIq2s {
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(r[m], (pf_lptr) (to + 2560 + m * 32), 4, sat, sb * 8, 0, 0);
         }
     }
-    __device__ __forceinline__ void first(uint8_t* to) const {
+    __device__ __forceinline__ void first(pf_lds8 to) const {
         copy(to, 0);
         if (nsb > 1) copy(to + kStep, 1);
     }
     // super-block sb is in registers: its LDS takes the super-block after the next one's
-    __device__ __forceinline__ void next(uint8_t* to, int sb) const {
+    __device__ __forceinline__ void next(pf_lds8 to, int sb) const {
         if (sb + 2 < nsb) copy(to + (sb & 1) * kStep, sb + 2);
     }
     struct Look {   // the LDS look-ups of one sub-block: selectors and signs of the lane's two grid entries, its group's digits
@@ -147,16 +147,7 @@ constexpr int kIqLdsBytes = 70912;
 static_assert(kIqLdsBytes == PfLds<PfIq2s<true>>::bytes && kIqLdsBytes == PfLds<PfIq2s<false>>::bytes);
 static_assert(kIqLdsBytes <= 80 * 1024, "two workgroups a compute unit");
 
-// grid (bands of weight rows, tiles at most)
-template <bool GU>
-__global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebooks cb) {
-    // ONE array, so that it starts at LDS address 0 and the tables' addresses need no base added (five additions a sub-block):
-    // prefill_iq2s_lds_ok holds the built kernel against that before a launch
-    __shared__ __attribute__((aligned(256))) uint8_t lds[kIqLdsBytes];
-    uint8_t* tables = lds;
-    PfTile t;
-    if (!pf_my_tile(a, t)) return;
-    const int tid = threadIdx.x;
+__device__ __forceinline__ void pf_iq2s_tables(uint8_t* tables, const Codebooks& cb, int tid) {
     // the magnitudes 8, 25, 43 as 0, 1, 2 (their bits 4 and 5)
 #pragma unroll
     for (int i = 0; i < 4; ++i) ((uint64_t*) (tables + kIqMags))[tid + 256 * i] = (cb.iq2s[tid + 256 * i] >> 4) & 0x0303030303030303ull;
@@ -179,24 +170,41 @@ __global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebook
         }
         ((v4i*) (tables + kIqScales))[tid] = e;
     }
-    // (the tile's first barrier is in front of the first look-up)
+}
+
+// The kernels' LDS is ONE array, so that it starts at LDS address 0 and the tables' addresses need no base added (five additions a
+// sub-block): prefill_iq2s_lds_ok holds the built kernels against that before a launch.
+// grid (bands of weight rows, items or tiles at most)
+template <bool GU>
+__global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebooks cb) {
+    __shared__ __attribute__((aligned(256))) uint8_t lds[kIqLdsBytes];
+    PfTile t;
+    if (!pf_my_rows(a, t)) return;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // (nothing made of it for the tables stays in a register)
+    pf_iq2s_tables(lds, cb, tid);   // (the tile's first barrier is in front of the first look-up)
     typedef PfIq2s<GU> W;
-    if (t.nrows <= 32) pf_tile<W, GU, 1>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 64) pf_tile<W, GU, 2>(a, lds, t.ex, t.row0, t.nrows);
-    else if (t.nrows <= 96) pf_tile<W, GU, 3>(a, lds, t.ex, t.row0, t.nrows);
-    else pf_tile<W, GU, 4>(a, lds, t.ex, t.row0, t.nrows);
+    if (t.nrows <= 32) pf_tile<W, GU, 1>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 64) pf_tile<W, GU, 2>(a, (pf_lds8) lds, t);
+    else if (t.nrows <= 96) pf_tile<W, GU, 3>(a, (pf_lds8) lds, t);
+    else pf_tile<W, GU, 4>(a, (pf_lds8) lds, t);
 }
 // Refuses a built kernel that has other LDS than its array (a second __shared__ object may be placed in front of it, and the
 // tables would be read from the wrong addresses).  Asked of the runtime once a kernel.
-template <bool GU>
-static int prefill_iq2s_lds_ok(const char* what) {
+template <void (*KERNEL)(PfGemm, Codebooks), int BYTES>
+static int prefill_iq2s_kernel_lds_ok(const char* what) {
     static std::atomic<size_t> bytes{0};
     if (bytes.load(std::memory_order_relaxed) == 0) {
         hipFuncAttributes at{};
-        MAYA_HIP(hipFuncGetAttributes(&at, (const void*) prefill_iq2s_kernel<GU>));
+        MAYA_HIP(hipFuncGetAttributes(&at, (const void*) KERNEL));
         bytes.store(at.sharedSizeBytes, std::memory_order_relaxed);
     }
     const size_t got = bytes.load(std::memory_order_relaxed);
-    if (got != (size_t) kIqLdsBytes) return fail(MAYA_E_UNSUPPORTED, "%s: the IQ2_S kernel was built with %zu bytes of LDS, its array has %d", what, got, kIqLdsBytes);
+    if (got != (size_t) BYTES) return fail(MAYA_E_UNSUPPORTED, "%s: an IQ2_S kernel was built with %zu bytes of LDS, its array has %d", what, got, BYTES);
     return MAYA_OK;
+}
+static int prefill_iq2s_lds_ok(const char* what) {
+    int rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_kernel<true>, kIqLdsBytes>(what);
+    if (!rc) rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_kernel<false>, kIqLdsBytes>(what);
+    return rc;
 }

@@ -236,6 +236,40 @@ def test_experts_of_every_number_of_row_groups(pf, oracle, t, n_embd, n_ff):
             assert rel_l2(part[row], want) <= 1e-5, (EDGE_ROWS[e], r)
 
 
+@pytest.mark.parametrize("t, n_embd, n_ff", [(Q4_K, 512, 512), (Q4_K, 1280, 256), (22, 512, 512), (22, 1536, 1024)], ids=str)
+def test_layer_calls_equal_the_stages(pf, t, n_embd, n_ff):
+    """A layer call's products take a list of their own, a stage call's the plan's tiles: the same bits, for experts of EDGE_ROWS rows
+    each among experts that are not resident or have no rows."""
+    from maya_amd import lib
+    import synth
+    gen = np.random.default_rng(n_embd + t)
+    ne, k = len(EDGE_ROWS), 1
+    blobs = [synth.expert_blob(t, t, n_embd, n_ff, gen) for _ in range(ne)]
+    layout, _ = lib.layout(t, t, n_embd, n_ff)
+    store = lib.ExpertStore(blobs, pack_layout=layout)
+    layout = lib.copy_layout(layout, lib.PACK_STREAM)
+    ids = np.repeat(np.arange(ne, dtype=np.int32), EDGE_ROWS)
+    gen.shuffle(ids)
+    x = dev(gen.standard_normal((ids.size, n_embd)).astype(np.float32))
+    weights = dev(gen.random((ids.size, k)).astype(np.float32) + 0.5)
+    outs = []
+    for idle in (0, 7, 300):   # (300: fewer than 8 rows an expert on average)
+        table = torch.cat([store.table, store.table[:1].expand(idle)]).contiguous()
+        table[3] = 0
+        n_expert = ne + idle
+        p = pf.plan(dev(ids), table)
+        part = pf.down(layout, table, p, pf.gate_up(layout, table, p, pf.quant(x, p, k)))
+        want = pf.combine(p, weights, part, ids.size, k)
+        layer = pf.PrefillLayer(layout, n_expert, k, ids.size, out_dtype=torch.float32)
+        for _ in range(2):
+            got = layer.forward(table, None, x, routed=(dev(ids)[:, None], weights)).clone()
+            assert torch.equal(got.view(torch.int32), want.view(torch.int32)), idle
+        on = dev(ids) != 3
+        assert bool((got[on] != 0).any(1).all()) and not bool(got[~on].any())
+        outs.append(got)
+    assert all(torch.equal(o.view(torch.int32), outs[0].view(torch.int32)) for o in outs)
+
+
 @pytest.mark.parametrize("t, n_embd, n_ff", [(Q4_K, 512, 256), (22, 512, 512)], ids=str)
 def test_a_part_of_the_tile_list(pf, oracle, t, n_embd, n_ff):
     """A caller may hand on some of a plan's tiles - a chunk in two halves, every second tile, one tile, any order: their rows are the
