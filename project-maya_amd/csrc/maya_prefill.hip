@@ -926,7 +926,7 @@ static int pf_gate_up(const maya_moe_layout* l, const uint64_t* expert_table, in
     a.work = work;
     const dim3 grid((unsigned) (l->n_ff / 64), pf_grid_rows(work, n_entries, n_expert));
     if (l->gate_type == kIQ2_S) {
-        hipLaunchKernelGGL(prefill_iq2s_kernel<true>, grid, dim3(256), 0, as_stream(stream), a, st->cb);
+        prefill_iq2s_launch<true>(a, st->cb, grid, n_entries, n_expert, as_stream(stream));
         MAYA_LAUNCHED("prefill_iq2s_kernel<gate_up>");
     } else {
         pf_launch<true>(a, grid, as_stream(stream));
@@ -957,7 +957,7 @@ static int pf_down(const maya_moe_layout* l, const uint64_t* expert_table, int n
     a.work = work;
     const dim3 grid((unsigned) ((l->n_embd + 127) / 128), pf_grid_rows(work, n_entries, n_expert));
     if (l->down_type == kIQ2_S) {
-        hipLaunchKernelGGL(prefill_iq2s_kernel<false>, grid, dim3(256), 0, as_stream(stream), a, st->cb);
+        prefill_iq2s_launch<false>(a, st->cb, grid, n_entries, n_expert, as_stream(stream));
         MAYA_LAUNCHED("prefill_iq2s_kernel<down>");
     } else {
         pf_launch<false>(a, grid, as_stream(stream));
@@ -1062,7 +1062,8 @@ static PrefillWs prefill_carve(const maya_moe_layout& l, int n_tokens, int k, in
     w.plan.tile_expert = (int32_t*) take(4 * mt);
     w.plan.tile_row0 = (int32_t*) take(4 * mt);
     w.plan.n_tiles = (int32_t*) take(4);
-    w.work.rows = 2 * kPfRows;
+    // Items of 128 rows, a workgroup's most; of 64 where the IQ2_S kernel of few rows takes them.
+    w.work.rows = l.gate_type == kIQ2_S && prefill_iq2s_few((int) ne, n_expert) ? kPfRows : 2 * kPfRows;
     w.work.list = (PfItem*) take(sizeof(PfItem) * mt);   // (fewer than the tiles)
     w.work.n = (int32_t*) take(4);
     auto take_act = [&](maya_prefill_act& a, size_t k) {

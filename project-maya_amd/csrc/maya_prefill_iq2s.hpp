@@ -21,10 +21,10 @@ constexpr int kIqMags = 0, kIqSigns = 8192, kIqScales = kIqSigns + 2048, kIqTabl
 // A quad of rows (the stream packing's unit) holds, a super-block, 256 bytes of (index, sign) words [sub-block][row], 64 of (high
 // bits, scales) pairs [sub-block][row] and 8 of block scales [row]: three copies of a wave's eight quads.  The words' 16-byte
 // pieces sit in LDS at their index ^ twice the quad, so that a sub-block's words of 32 rows meet every bank once.
-template <bool GU> struct PfIq2s {
+template <bool GU, int RING = 4> struct PfIq2s {
     static constexpr bool kSums = false;
     static constexpr int kLdsAt = kIqTables, kStep = 2048 + 512 + 64 + 192, kWave = 2 * kStep;   // (multiples of 256: addresses below are xor-ed)
-    static constexpr int kMats = GU ? 2 : 1, kQuads = 8 / kMats, kCopies = GU ? 6 : 5, kOneGroupBut = 2 + kCopies, kRing = 4;
+    static constexpr int kMats = GU ? 2 : 1, kQuads = 8 / kMats, kCopies = GU ? 6 : 5, kOneGroupBut = 2 + kCopies, kRing = RING;
     static constexpr int kHiFactor = 256, kLook = 5;
     static constexpr float kOutFactor = 0.125f;
     __amdgpu_buffer_rsrc_t r[kMats];
@@ -189,6 +189,24 @@ __global__ __launch_bounds__(256, 2) void prefill_iq2s_kernel(PfGemm a, Codebook
     else if (t.nrows <= 96) pf_tile<W, GU, 3>(a, (pf_lds8) lds, t);
     else pf_tile<W, GU, 4>(a, (pf_lds8) lds, t);
 }
+// Chunks of few rows an expert: one group of 32 rows at a time, in registers and LDS that leave room for three workgroups a
+// compute unit, as the look-ups, the vector instructions and the matrix instructions take turns with two (LDS busy 57 % of the cycles, vector issue
+// 44 %, matrix cores 23 %).  75 tokens of 160 experts of 6144 x 1536 530 -> 483 us, 17 tokens 321 -> 293, with 10.3 waves a compute unit
+// where there were 7.1.  An item of more than 32 rows decodes its weights once a group.
+constexpr int kIqFewRing = 2, kIqFewLdsBytes = PfLds<PfIq2s<true, kIqFewRing>>::bytes;
+static_assert(kIqFewLdsBytes == PfLds<PfIq2s<false, kIqFewRing>>::bytes && kIqFewLdsBytes <= 160 * 1024 / 3, "three workgroups a compute unit");
+template <bool GU>
+__global__ __launch_bounds__(256, 3) void prefill_iq2s_few_kernel(PfGemm a, Codebooks cb) {
+    __shared__ __attribute__((aligned(256))) uint8_t lds[kIqFewLdsBytes];
+    PfTile t;
+    if (!pf_my_rows(a, t)) return;
+    pf_iq2s_tables(lds, cb, threadIdx.x);
+    typedef PfIq2s<GU, kIqFewRing> W;
+    for (int r = 0; r < t.nrows; r += 32) {
+        if (r) __syncthreads();   // (the copies of these rows go where the others may still be read)
+        pf_tile<W, GU, 1>(a, (pf_lds8) lds, {t.blob, t.row0 + r, min(32, t.nrows - r)});
+    }
+}
 // Refuses a built kernel that has other LDS than its array (a second __shared__ object may be placed in front of it, and the
 // tables would be read from the wrong addresses).  Asked of the runtime once a kernel.
 template <void (*KERNEL)(PfGemm, Codebooks), int BYTES>
@@ -206,5 +224,17 @@ static int prefill_iq2s_kernel_lds_ok(const char* what) {
 static int prefill_iq2s_lds_ok(const char* what) {
     int rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_kernel<true>, kIqLdsBytes>(what);
     if (!rc) rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_kernel<false>, kIqLdsBytes>(what);
+    if (!rc) rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_few_kernel<true>, kIqFewLdsBytes>(what);
+    if (!rc) rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_few_kernel<false>, kIqFewLdsBytes>(what);
     return rc;
+}
+// Whether a chunk's IQ2_S products run on the kernel for few rows an expert: on the average of them, as the host does not know the
+// routing.  Microseconds a layer call, 160 experts of 6144 x 1536, kernel of 128 rows and this one: 8 rows an expert on average 564 and 520
+// (routing skewed by 0.6 518 and 503, by 1.1 338 and 345), 12 rows 585 and 531 (590 and 578, 377 and 404), 24 rows 640 and 619 (714 and 760, 549 and
+// 618); of 3072 x 1536, 8 rows 301 and 278 (283 and 269, 188 and 185).
+static bool prefill_iq2s_few(int n_entries, int n_expert) { return n_entries <= 8 * n_expert; }
+template <bool GU>
+static void prefill_iq2s_launch(const PfGemm& a, const Codebooks& cb, dim3 grid, int n_entries, int n_expert, hipStream_t s) {
+    if (prefill_iq2s_few(n_entries, n_expert)) hipLaunchKernelGGL(prefill_iq2s_few_kernel<GU>, grid, dim3(256), 0, s, a, cb);
+    else hipLaunchKernelGGL(prefill_iq2s_kernel<GU>, grid, dim3(256), 0, s, a, cb);
 }
