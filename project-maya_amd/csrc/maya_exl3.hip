@@ -800,9 +800,15 @@ int launch_exl3_gate_up(const maya_exl3_args& a, const DeviceState& st, hipStrea
 // Slices a workgroup walks: as many as leave the call three workgroups a compute unit, at least one.  Three is what the registers of
 // the two-token kernels (70) let a compute unit hold at once; one token's hold four (58) or three (70, the down launch that makes h),
 // the four-token ones two (96 to 100): a call of theirs that is cut for three runs its last third as a second round.
-static int slices_per_wg(long long wgs, int S, const DeviceState& st) {
+// And half as many slices where the call then still has less than twice that and a workgroup 16 blocks of rows: a compute unit's three
+// end one after the other (the wave that came first issues first), with nothing to take their place, or a second round of workgroups is a part
+// of one.  Six a compute unit, three before: 4 tokens top-8 of 6144 x 1536 at 3 bits 145.5 -> 142.2 us, 5 tokens 204 -> 188, 8 tokens
+// top-6 of 4096 x 1536 148.5 -> 141.5, 4 tokens top-8 of 7168 x 2048 at 5 bits 235 -> 229.  Shorter workgroups do not pay: 2 tokens of 6144 x 1536
+// (12 blocks) 78.3 -> 79.2, 3 of 4096 x 1024 (8 blocks) 61.7 -> 64.2.
+static int slices_per_wg(long long wgs, int S, int blocks, const DeviceState& st) {
     int sp = S;
     while (sp > 1 && (S % sp != 0 || wgs * (S / sp) < 3ll * st.n_cu)) --sp;
+    if (sp % 2 == 0 && wgs * (S / sp) < 6ll * st.n_cu && blocks / S * (sp / 2) >= 16) sp /= 2;
     return sp;
 }
 template <int NT, bool DOWN, bool COMB, bool HEAD = false>
@@ -810,7 +816,7 @@ int launch_exl3_slices(const maya_exl3_args& a, int S, const __half* hr, const f
                        const DeviceState& st, hipStream_t s, const Exl3Head& hd = Exl3Head{}) {
     const maya_exl3_layout& l = a.layout;
     const int k = DOWN ? l.n_ff : l.n_embd, n = DOWN ? l.n_embd : l.n_ff, mats = DOWN ? 1 : 2;
-    int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, st);
+    int SP = slices_per_wg((long long) (n / 128) * a.n_tokens * a.k * mats, S, k / 128, st);
     while (SP * NT > 8) SP >>= 1;   // (the closing rotation takes a block of 128 sums a wave)
     const int rows = ((k / 128 + S - 1) / S) * SP * 128;   // the longest workgroup's
     size_t lds = (size_t) NT * rows * 2 + (size_t) SP * NT * 128 * 4;

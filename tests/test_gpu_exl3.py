@@ -175,7 +175,8 @@ def test_stage_calls_take_group_arrays_that_end_with_the_groups(ex, k2):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and float(got[0][1].abs().max()) > 0
 
 
-@pytest.mark.parametrize("n_embd,n_ff,k2,cb,nt", [(640, 384, 6, 2, 4), (2048, 1536, 8, 2, 16), (6144, 1536, 6, 2, 4), (1024, 512, 4, 1, 13)])
+@pytest.mark.parametrize("n_embd,n_ff,k2,cb,nt", [(640, 384, 6, 2, 4), (2048, 1536, 8, 2, 16), (6144, 1536, 6, 2, 4), (1024, 512, 4, 1, 13),
+                                                    (4224, 1536, 6, 2, 6)])   # (its gate/up workgroups: two slices of 8 or 9 blocks)
 def test_a_layers_window_is_its_tokens(ex, n_embd, n_ff, k2, cb, nt):
     """The layer on a window (several slices a workgroup, two tokens a walk) gives the bits of its tokens one at a time."""
     from maya_amd import lib
