@@ -501,6 +501,7 @@ struct LayerHeadIn {
     const float* bias;   // the sigmoid router's, or NULL
     int n_expert, x_dtype, sigmoid;
     LayerHead out;
+    int n_embd;
 };
 // What such a launch asks of memory first, as plain pointers and integers at the head of its arguments (they arrive in scalar
 // registers with the dispatch; a structure passed by value is read from memory first): the fields of LayerHeadIn, a.skip, a.k
@@ -510,8 +511,8 @@ struct LayerHeadIn {
         const int32_t *__restrict__ skip, int n_expert, int mode, int n_ent
 #define MAYA_HEAD_ARGS(hd, a)                                                                                   \
     hd.logits, hd.table, hd.x, hd.bias, a.skip, hd.n_expert, hd.x_dtype | (hd.sigmoid ? 256 : 0) | (a.layout.n_embd >> 5) << 16, a.k
-// The head of a one-token layer inside a gate/up launch whose workgroups are a (gate row, up row) pair's 2 * 32 NW
-// positions, grid (row blocks + 1, k): called by every thread once.  The workgroup (last column, 0) is the exact router
+// The head of a layer inside a gate/up launch whose workgroups are a (gate row, up row) pair's 2 * 32 NW
+// positions, grid (row blocks + 1, k, tokens): called by every thread once.  A token's workgroup (last column, 0) is its exact router
 // (ids, weights, plan: hd.out); the rest of that column leaves.  Every other workgroup picks the experts on its last
 // wave (up lanes only) from the ORDER of the logits - the exact router on the same wave when two of them are too close to
 // call - while the waves with gate lanes round their positions' x to Q8_K in registers (a 256-value block is 8 lanes: the
@@ -529,7 +530,7 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
     __shared__ float s_lv[64 * R];
     __shared__ uint64_t s_tab[64 * R];
     __shared__ int s_y[9][NU];
-    const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert;
+    const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert, tok = (int) blockIdx.z;
     const bool picker = t >= 64 * (NW - 1), sigm = hd.sigmoid != 0;
     float lv[R], bv[R];
     uint64_t tab[R];
@@ -539,7 +540,7 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int x = 64 * r + lane;
-            lv[r] = x < ne ? hd.logits[x] : -INFINITY;
+            lv[r] = x < ne ? hd.logits[tok * ne + x] : -INFINITY;
             tab[r] = x < ne ? hd.table[x] : 0ull;
             if (hd.bias) bv[r] = x < ne ? hd.bias[x] : 0.0f;
         }
@@ -562,9 +563,9 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
         }
         if constexpr (R > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
         if (lane < n_ent) {
-            hd.out.ids[lane] = id;
-            hd.out.weights[lane] = w;
-            hd.out.plan[lane] = ptr;
+            hd.out.ids[tok * n_ent + lane] = id;
+            hd.out.weights[tok * n_ent + lane] = w;
+            hd.out.plan[tok * n_ent + lane] = ptr;
         }
         return false;
     }
@@ -600,6 +601,7 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
     }
     float v[32];
     if (!is_up) {
+        o0 += tok * hd.n_embd, o1 += tok * hd.n_embd;   // (whole blocks: the low eight bits stay)
         if (hd.x_dtype == MAYA_DT_F32) {
             const float4 *xa = (const float4*) ((const float*) hd.x + o0), *xb = (const float4*) ((const float*) hd.x + o1);
 #pragma unroll

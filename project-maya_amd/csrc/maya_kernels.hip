@@ -1680,7 +1680,7 @@ int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hip
     MAYA_LAUNCHED("gate_up_iq2s_tiles_kernel");
     return MAYA_OK;
 }
-// The single-token layer whose head rides in the gate/up launch (gate_up_iq2s_tiles_kernel<.., 4 or 8>,
+// The layer whose head rides in the gate/up launch, one token's always, several tokens' where that pays (gate_up_iq2s_tiles_kernel<.., 4 or 8>,
 // gate_up_q4k_pos_kernel<.., 4 or 8>): either router over up to 512 experts with more experts than slots, x aligned for
 // 16-byte loads, IQ2_S, Q4_K or IQ1_S gate/up rows in the stream packing's shapes.  (IQ1_M keeps its head launch: its
 // gate/up kernel with the head in it was 6.3 us slower a launch than without, more than the 4.8 us head launch it replaces;
@@ -1689,10 +1689,30 @@ int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hip
 // of 288 43.0 -> 39.2, IQ2_S 7168 x 1024 of 384 28.7 -> 22.6, IQ1_S 5120 x 1536 of 384 27.3 -> 20.4.
 bool gate_up_q4k_pos_ok(const maya_moe_args& a);
 bool gate_up_iq1s_pos_ok(const maya_moe_args& a);
+bool gate_up_by_entries(const maya_moe_args& a);
+bool down_by_entries(const maya_moe_args& a);
+// The head of several tokens in the gate/up launch: a launch and its gap less (4 to 5 us), against a picking wave and the rounding
+// of x in every workgroup, fewer waves a compute unit (the registers of the head) and entries of one expert that no longer run side by side.
+// So: few weights to go through; IQ1_S up to 2^27 (its kernel is bound by vector instructions, which the head adds to); Q4_K up to 2^26, and up to
+// 2^28 where few of the tokens share experts and rows are of at most 4096 values (workgroups of up to four waves: those of five
+// or six lose a third of a compute unit's waves).  Microseconds a layer, head in a launch of its own / in this one:
+//   Q4_K 2048 x 768 top-8 of 128, 2 tokens 19.0 / 15.1, 4 24.1 / 20.3, 6 30.5 / 27.1, 16 (201 M) 51.8 / 54.9;  4096 x 512 of 200, 3 27.5 / 22.5;
+//   4096 x 1536 of 128, 2 36.7 / 32.2, 5 (252 M) 85.7 / 82.3;  4096 x 1024 top-4 of 64, 8 (experts shared) 36.9 / 37.4, 4096 x 512 top-6 of 96, 8 34.6 / 36.5;
+//   5120 x 1536 top-10 of 160, 2 54.3 / 55.2;  6144 x 1536 top-10 of 100, 3 96.2 / 99.6;  7168 x 2048 top-1 of 16, 4 (59 M) 27.3 / 25.1
+//   IQ1_S 2048 x 768, 2 18.8 / 14.6, 10 (126 M) 35.9 / 33.5;  4096 x 512, 4 25.6 / 21.8;  5120 x 1024 top-4 of 32, 4 (84 M) 23.9 / 24.1;
+//   6144 x 1536 top-10, 2 (189 M) 43.4 / 45.7;  7168 x 2048 top-8, 2 (235 M) 43.7 / 45.3, 4 75.5 / 82.5
+static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert) {
+    const maya_moe_layout& l = a.layout;
+    const int entries = a.n_tokens * a.k;
+    const long long weights = (long long) entries * l.n_ff * l.n_embd;   // (of one matrix)
+    if (!(gate_up_by_entries(a) && down_by_entries(a))) return false;   // (the others want the entries grouped)
+    if (l.gate_type == kIQ1_S) return weights <= 1ll << 27;
+    return l.gate_type == kQ4_K && (weights <= 1ll << 26 || (weights <= 1ll << 28 && 5 * entries <= 2 * n_expert && l.n_embd <= 4096));
+}
 static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& rs, const float* logits, int n_expert, const void* x,
                                      int x_dtype) {
     const maya_moe_layout& l = a.layout;
-    if (!(logits && a.n_tokens == 1 && n_expert <= 512 && a.k < n_expert && x_dtype >= 0 && x_dtype <= 2 && ((uintptr_t) x & 15) == 0))
+    if (!(logits && (a.n_tokens == 1 || window_head_in_gate_up_pays(a, n_expert)) && n_expert <= 512 && a.k < n_expert && x_dtype >= 0 && x_dtype <= 2 && ((uintptr_t) x & 15) == 0))
         return false;
     if (l.gate_type == kQ4_K) return gate_up_q4k_pos_ok(a);
     if (l.gate_type == kIQ1_S) return gate_up_iq1s_pos_ok(a);
@@ -1809,8 +1829,8 @@ bool down_iq1s_pos_ok(const maya_moe_args& a) {
            l.n_embd % 16 == 0 && (l.down_off & 15) == 0;
 }
 int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd = nullptr) {
-    // (IQ1_S with the head in the launch: one more column, whose first workgroup is the router)
-    const dim3 grid((unsigned) (a.layout.n_ff / 16) + (hd ? 1u : 0u), (unsigned) (a.n_tokens * a.k));
+    // (IQ1_S with the head in the launch: one more column, whose first workgroup is the token's router)
+    const dim3 grid((unsigned) (a.layout.n_ff / 16) + (hd ? 1u : 0u), (unsigned) (hd ? a.k : a.n_tokens * a.k), (unsigned) (hd ? a.n_tokens : 1));
     if (a.layout.gate_type == kIQ1_M) {
         // Compiled for 8 waves a SIMD where rows fill their lanes, 7 where they do not.  At 8 some of either spill two registers; at
         // 64 experts top-8 the former lose nothing by it (7168 x 2048, 16 tokens, 315 us against 320 at 7; 4096 x 2048, four tokens,
@@ -1932,8 +1952,8 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     // 16 rows a workgroup, 8 - all requested up front - when the call has so few entries that 16 would leave compute units idle
     const bool small = (long long) (a.layout.n_ff / 16) * a.n_tokens * a.k < 512;
     const int rows = small ? 8 : 16;
-    // (with the head in the launch: one more column, whose first workgroup is the router)
-    const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd ? 1u : 0u), (unsigned) (a.n_tokens * a.k));
+    // (with the head in the launch: one more column, whose first workgroup is the token's router)
+    const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd ? 1u : 0u), (unsigned) (hd ? a.k : a.n_tokens * a.k), (unsigned) (hd ? a.n_tokens : 1));
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
     const bool wide = hd && hd->n_expert > 256;   // (their rows take the form that any length has)
@@ -2797,8 +2817,9 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
     }
     if (!head) {
         // (the second half of a call made in two: the plan, the groups and h are in the workspace)
-    } else if (layer_head_in_gate_up_ok(a, rs, logits, n_expert, x, x_dtype)) {
-        // one token of IQ2_S, Q4_K or IQ1_S experts: route, plan, Q8_K of x and gate/up in one launch
+    } else if ((n_tokens == 1 || (!q80 && !join)) && layer_head_in_gate_up_ok(a, rs, logits, n_expert, x, x_dtype)) {
+        // IQ2_S, Q4_K or IQ1_S experts: route, plan, Q8_K of x and gate/up in one launch (a window beside a shared expert keeps the head
+        // of its own: it rounds x for a Q8_0 one too, and runs in the time of one on the second stream; where this runs, the down launch takes the entries one by one, ungrouped)
         const LayerHeadIn hd{logits, expert_table, x, rs.bias, n_expert, x_dtype, rs.kind == MAYA_ROUTER_SIGMOID ? 1 : 0,
                              LayerHead{ids, weights, w.plan_ptr, rs.w_scale, rs.norm}};
         hipStream_t s = as_stream(stream);
@@ -2806,7 +2827,7 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
                   : l->gate_type == kIQ2_S ? launch_layer_gate_up_iq2s(a, hd, *st, s)
                                            : launch_gate_up_iq1s_pos(a, *st, s, &hd)))
             return rc;
-        gate_up_done = true;
+        gate_up_done = grouped = true;
     } else if (logits && (n_tokens > 1 || n_expert > 256) && n_tokens <= (join ? kHeadBesideTokens : MAYA_MAX_TOKENS) && window_head_ok(n_tokens, n_expert, k) && x_dtype >= 0 &&
                x_dtype <= 2) {
         // several tokens, one launch: route, plan, group and round x, for the routed experts' rows and a shared Q8_0 expert's

@@ -360,8 +360,8 @@ def wide_logits(ne, seed):
     """Rows of `ne` logits: the edge cases of logit_cases, spread so that what decides sits on either side of 256."""
     rng = np.random.default_rng(seed)
     base = rng.standard_normal(ne).astype(np.float32)
-    rows = [base.copy() for _ in range(10)]
-    rows[1][[ne - 1, 3, 256]] = np.float32(4.5)
+    rows, mid = [base.copy() for _ in range(10)], 256 if ne > 256 else ne // 2
+    rows[1][[ne - 1, 3, mid]] = np.float32(4.5)
     order = np.argsort(-base)
     rows[2][order[8]] = rows[2][order[7]]
     rows[3][order[3]] = np.nextafter(rows[3][order[2]], np.float32(-10))
@@ -369,7 +369,7 @@ def wide_logits(ne, seed):
     rows[4][:] = 0.0
     rows[5][ne - 1] = np.float32(300.0)
     rows[6] = (base * np.float32(40.0)).astype(np.float32)
-    rows[7][256] = np.float32(np.inf)
+    rows[7][mid] = np.float32(np.inf)
     rows[8][ne - 1] = np.float32(np.nan)
     rows[9] = np.arange(ne, dtype=np.float32) * np.float32(5e-7)
     return rows
@@ -406,3 +406,46 @@ def test_heads_of_more_than_256_experts(lib, ty, n_embd, n_ff, ne, nt, sigmoid):
         out = layer.forward(table, lg, buf[1:].reshape(nt, n_embd), router=router)
         torch.cuda.synchronize()
         assert torch.equal(layer.ids, ids) and torch.equal(out.view(torch.int32), want.view(torch.int32)), first
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
+@pytest.mark.parametrize("sigmoid", (False, True))
+@pytest.mark.parametrize("ty,n_embd,n_ff,ne,k,nt", ((12, 2048, 256, 40, 8, 2), (12, 2304, 512, 40, 8, 7), (12, 4096, 512, 200, 8, 8), (12, 7168, 256, 9, 1, 16),
+                                                    (12, 2048, 256, 400, 8, 3), (19, 2048, 256, 40, 8, 2), (19, 5376, 512, 40, 8, 5), (19, 2048, 512, 512, 8, 16),
+                                                    (19, 2816, 256, 17, 16, 4)))
+def test_several_tokens_head_in_the_gate_up_launch(lib, ty, n_embd, n_ff, ne, k, nt, sigmoid, dtype):
+    """Windows whose head rides in the gate/up launch (Q4_K, IQ1_S): ids and weights bit for bit the routing launch's, the output that
+    of the layer given these ids and weights, which orders and rounds in launches of its own; the same in two calls and replayed
+    from a graph, with experts that are not resident."""
+    blobs = make_experts(ty, ty, n_embd, n_ff, 9, 3 * ne + ty)
+    store = lib.ExpertStore(blobs, pack_layout=lib.layout(ty, ty, n_embd, n_ff)[0])
+    table = store.table[torch.arange(ne, device="cuda") % 9].contiguous()
+    table[5::11] = 0
+    rng = np.random.default_rng(ne + nt)
+    bias = dev((rng.standard_normal(ne) * 0.1).astype(np.float32))
+    more = {"router": lib.Router(lib.ROUTER_SIGMOID, 1, bias.data_ptr(), 2.5)} if sigmoid else {}
+    layer, given, halves = (lib.MoeLayer(ty, ty, n_embd, n_ff, ne, k, max_tokens=nt, packing=1) for _ in range(3))
+    halves.ws.fill_(0x5a)                                       # (nothing is expected of the workspace)
+    x = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda().to(dtype)
+    rows = wide_logits(ne, ne)
+    lg = torch.empty((nt, ne), device="cuda")
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    replayed = lib.MoeLayer(ty, ty, n_embd, n_ff, ne, k, max_tokens=nt, packing=1)
+    lg.copy_(dev(np.stack([rows[i % len(rows)] for i in range(nt)])))
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        replayed.forward(table, lg, x, **more)
+    for first in range(0, len(rows), nt):
+        print("rows from", first, flush=True)
+        lg.copy_(dev(np.stack([rows[(first + i) % len(rows)] for i in range(nt)])))
+        out = layer.forward(table, lg, x, **more).clone()
+        ids, w, _ = lib.route_plan(lg, k, table, more.get("router"))
+        want = given.forward(table, None, x, routed=(ids, w)).clone()
+        halves.forward(table, lg, x, half="begin", **more)
+        halves.forward(table, lg, x, half="end", **more)
+        graph.replay()
+        torch.cuda.synchronize()
+        for got in (layer, halves, replayed):
+            assert torch.equal(got.ids, ids) and torch.equal(got.weights.view(torch.int32), w.view(torch.int32)), first
+            assert torch.equal(got.out[:nt].view(torch.int32), want.view(torch.int32)), first
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32)), first
