@@ -479,7 +479,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq2s_pos_kernel(maya_mo
 // workgroup pays the cold start (arguments, plan, tables, first weights: three memory round trips one after the other)
 // once instead of once per 16 rows, and no second round of workgroups starts behind the first.
 //
-// HEAD: the layer's head rides in the same launch, and no workgroup waits for another.  Workgroup 0 is the router: one
+// HEAD: the layer's head rides in the same launch, and no workgroup waits for another (of several tokens: a row of the grid each).  Workgroup 0 is the router: one
 // wave routes the token exactly (route_wave_softmax) and writes ids, weights and the plan for the down launch and the
 // caller.  Every other workgroup finds out for itself which experts were picked - the order of the k + 1 largest logits
 // (route_wave_order_only; the exact router on its first wave in the rare case that this does not settle it) - and rounds
@@ -686,7 +686,8 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
     const int nu = mode >> 16, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
     const bool on = lu < nu;
     const int u = on ? lu : nu - 1;
-    // (n_ent = a.k: one token, entry = plan slot)
+    // (n_ent = a.k: one token a row of the grid, entry = its plan slot)
+    const int tok = HEAD ? (int) blockIdx.y : 0;
     int y[8];
     float dy8;
     int first_tile = blockIdx.x, tile_step = gridDim.x;
@@ -696,7 +697,7 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
         // The workgroup's last wave holds up rows only; it picks the experts while the gate lanes round x (a gate lane and
         // the up lane of the same position need the same codes: the gate lane rounds, the up lane takes them from LDS).
         const int ne = n_expert;
-        const float* logits = (const float*) p0;
+        const float* logits = (const float*) p0 + tok * ne;
         const uint64_t* table = (const uint64_t*) p1;
         const bool picker = t >= 64 * (NW - 1);
         const int x_dtype = mode & 255;
@@ -733,9 +734,9 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
             }
             if constexpr (HEAD > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
             if (lane < n_ent) {
-                hd.ids[lane] = id;
-                hd.weights[lane] = w;
-                hd.plan[lane] = ptr;
+                hd.ids[tok * n_ent + lane] = id;
+                hd.weights[tok * n_ent + lane] = w;
+                hd.plan[tok * n_ent + lane] = ptr;
             }
             return;
         }
@@ -774,14 +775,14 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
         float v[32];
         if (!is_up) {
             if (x_dtype == MAYA_DT_F32) {
-                const float4* xv = (const float4*) p2 + 8 * u;
+                const float4* xv = (const float4*) p2 + 8 * (tok * nu + u);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float4 q = xv[i];
                     v[4 * i] = q.x, v[4 * i + 1] = q.y, v[4 * i + 2] = q.z, v[4 * i + 3] = q.w;
                 }
             } else {
-                const uint4* xv = (const uint4*) p2 + 4 * u;
+                const uint4* xv = (const uint4*) p2 + 4 * (tok * nu + u);
                 uint32_t w4[16];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -909,7 +910,7 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
                 g += part[buf][w][t];
                 up += part[buf][NW + w][t];
             }
-            if (present) a.h[(size_t) e * n_ff + 8 * rb + t] = swiglu(g, up, a.limit);
+            if (present) a.h[(size_t) (tok * n_ent + e) * n_ff + 8 * rb + t] = swiglu(g, up, a.limit);
         }
         if (!more) break;
         tile = nt, e = ne, rb = nrb, rs = nrs, blob = nblob, buf ^= 1;

@@ -1651,7 +1651,7 @@ int launch_gate_up_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
 // with the head's prologue in it the kernel needs 73-77 registers, and at 64 it spilled 36 bytes a lane to scratch
 // memory: 6.8 MB written and read back a launch, 2.1 us of the layer.  Windows keep gate_up_iq2s_pos_kernel: the tile
 // stream with the resident workgroups shared out among the tokens (a token's codes in a workgroup's registers) was built
-// and is slower there (configs[2]: 260 us against 234).
+// and is slower on long ones (eight tokens of 7168 x 2048 260 us against 234); window_head_in_gate_up_pays says where it is not.
 template <int NW>
 int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd = nullptr) {
     constexpr int kMinW = NW <= 3 ? 5 : 6, kMostPerCu = NW == 2 ? 12 : 3;
@@ -1666,12 +1666,12 @@ int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hip
         per_cu = n > kMostPerCu ? kMostPerCu : n > 0 ? n : 1;
     }
     const int n_tiles = a.k * (a.layout.n_ff / 8);
-    const int wgs = per_cu * st.n_cu;
+    const int wgs = per_cu * st.n_cu / (hd ? a.n_tokens : 1);   // (the resident workgroups shared out among the tokens)
     const unsigned walkers = (unsigned) (wgs < n_tiles ? wgs : n_tiles);
     const int nu = a.layout.n_embd >> 5;   // sub-blocks a row, in the upper half of `mode`
     if (hd) {   // workgroup 0 routes, the others walk the tiles
         auto kern = hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8>;
-        hipLaunchKernelGGL(kern, dim3(walkers + 1), dim3(64 * NW), 0, s, (const void*) hd->logits, (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias,
+        hipLaunchKernelGGL(kern, dim3(walkers + 1, (unsigned) a.n_tokens), dim3(64 * NW), 0, s, (const void*) hd->logits, (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias,
                            a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a, hd->out);
     } else {
         hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, 0>), dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
@@ -1701,12 +1701,17 @@ bool down_by_entries(const maya_moe_args& a);
 //   5120 x 1536 top-10 of 160, 2 54.3 / 55.2;  6144 x 1536 top-10 of 100, 3 96.2 / 99.6;  7168 x 2048 top-1 of 16, 4 (59 M) 27.3 / 25.1
 //   IQ1_S 2048 x 768, 2 18.8 / 14.6, 10 (126 M) 35.9 / 33.5;  4096 x 512, 4 25.6 / 21.8;  5120 x 1024 top-4 of 32, 4 (84 M) 23.9 / 24.1;
 //   6144 x 1536 top-10, 2 (189 M) 43.4 / 45.7;  7168 x 2048 top-8, 2 (235 M) 43.7 / 45.3, 4 75.5 / 82.5
+// IQ2_S rows share the resident workgroups of the tile walk out among the tokens: up to 2^27, two and three tokens up to 2^28 (the
+// kernel of a launch behind a head of its own has more waves a compute unit, which tells on longer launches).
+//   IQ2_S 2048 x 768 top-8 of 128, 2 18.9 / 15.5, 10 (126 M) 40.5 / 33.8;  4096 x 1536, 2 31.5 / 29.8, 3 (151 M) 41.4 / 36.1, 5 (252 M) 58.4 / 61.6;
+//   7168 x 2048 of 100, 2 (235 M) 53.0 / 49.5;  with Q4_K down rows 3 (352 M) 92.5 / 93.6, 8 197 / 206;  3072 x 1024 top-6, 8 (151 M) 39.1 / 40.2
 static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert) {
     const maya_moe_layout& l = a.layout;
     const int entries = a.n_tokens * a.k;
     const long long weights = (long long) entries * l.n_ff * l.n_embd;   // (of one matrix)
     if (!(gate_up_by_entries(a) && down_by_entries(a))) return false;   // (the others want the entries grouped)
     if (l.gate_type == kIQ1_S) return weights <= 1ll << 27;
+    if (l.gate_type == kIQ2_S) return weights <= 1ll << 27 || (weights <= 1ll << 28 && a.n_tokens <= 3);
     return l.gate_type == kQ4_K && (weights <= 1ll << 26 || (weights <= 1ll << 28 && 5 * entries <= 2 * n_expert && l.n_embd <= 4096));
 }
 static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& rs, const float* logits, int n_expert, const void* x,

@@ -412,9 +412,10 @@ def test_heads_of_more_than_256_experts(lib, ty, n_embd, n_ff, ne, nt, sigmoid):
 @pytest.mark.parametrize("sigmoid", (False, True))
 @pytest.mark.parametrize("ty,n_embd,n_ff,ne,k,nt", ((12, 2048, 256, 40, 8, 2), (12, 2304, 512, 40, 8, 7), (12, 4096, 512, 200, 8, 8), (12, 7168, 256, 9, 1, 16),
                                                     (12, 2048, 256, 400, 8, 3), (19, 2048, 256, 40, 8, 2), (19, 5376, 512, 40, 8, 5), (19, 2048, 512, 512, 8, 16),
-                                                    (19, 2816, 256, 17, 16, 4)))
+                                                    (19, 2816, 256, 17, 16, 4), (22, 2048, 256, 40, 8, 2), (22, 5376, 512, 40, 8, 3), (22, 2304, 512, 300, 8, 11),
+                                                    (22, 7168, 256, 17, 16, 4), (22, 3072, 768, 9, 1, 16)))
 def test_several_tokens_head_in_the_gate_up_launch(lib, ty, n_embd, n_ff, ne, k, nt, sigmoid, dtype):
-    """Windows whose head rides in the gate/up launch (Q4_K, IQ1_S): ids and weights bit for bit the routing launch's, the output that
+    """Windows whose head rides in the gate/up launch (Q4_K, IQ1_S, IQ2_S): ids and weights bit for bit the routing launch's, the output that
     of the layer given these ids and weights, which orders and rounds in launches of its own; the same in two calls and replayed
     from a graph, with experts that are not resident."""
     blobs = make_experts(ty, ty, n_embd, n_ff, 9, 3 * ne + ty)
