@@ -377,9 +377,9 @@ def wide_logits(ne, seed):
 
 @pytest.mark.parametrize("sigmoid", (False, True))
 @pytest.mark.parametrize("ty,n_embd,n_ff,ne,nt", ((12, 2048, 256, 257, 1), (12, 3072, 2048, 512, 1), (22, 4352, 256, 300, 1), (19, 2304, 256, 512, 1),
-                                                  (8, 2048, 256, 288, 1), (12, 2048, 256, 512, 3), (8, 2048, 256, 257, 10), (22, 2048, 256, 300, 16)))
+                                                  (8, 2048, 256, 288, 1), (12, 2048, 256, 512, 3), (8, 2048, 256, 257, 10), (22, 2048, 256, 300, 16), (8, 2304, 256, 40, 1)))
 def test_heads_of_more_than_256_experts(lib, ty, n_embd, n_ff, ne, nt, sigmoid):
-    """257 to 512 experts, the head in the gate/up launch or in one of its own: ids and weights bit for bit the routing launch's, the
+    """257 to 512 experts, and Q8_0 rows of fewer, the head in the gate/up launch or in one of its own: ids and weights bit for bit the routing launch's, the
     output that of the layer given these ids and weights; x also from an address that is not 16-byte aligned."""
     k, kinds = 8, 9
     blobs = make_experts(ty, ty, n_embd, n_ff, kinds, 5 * ne + ty)
