@@ -1704,13 +1704,15 @@ bool down_by_entries(const maya_moe_args& a);
 // IQ2_S rows share the resident workgroups of the tile walk out among the tokens: up to 2^27, two and three tokens up to 2^28 (the
 // kernel of a launch behind a head of its own has more waves a compute unit, which tells on longer launches).
 //   IQ2_S 2048 x 768 top-8 of 128, 2 18.9 / 15.5, 10 (126 M) 40.5 / 33.8;  4096 x 1536, 2 31.5 / 29.8, 3 (151 M) 41.4 / 36.1, 5 (252 M) 58.4 / 61.6;
-//   7168 x 2048 of 100, 2 (235 M) 53.0 / 49.5;  with Q4_K down rows 3 (352 M) 92.5 / 93.6, 8 197 / 206;  3072 x 1024 top-6, 8 (151 M) 39.1 / 40.2
+//   7168 x 2048 of 100, 2 (235 M) 53.0 / 49.5;  with Q4_K down rows 3 (352 M) 92.5 / 93.6, 8 197 / 206;  3072 x 1024 top-6, 8 (151 M) 39.1 / 40.2;
+//   more slots than eight and rows that leave lanes idle: top-10 2304 x 1792, 3 (124 M) 47.4 / 48.9, 4864 x 2048, 2 (199 M) 63.0 / 64.5
 static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert) {
     const maya_moe_layout& l = a.layout;
     const int entries = a.n_tokens * a.k;
     const long long weights = (long long) entries * l.n_ff * l.n_embd;   // (of one matrix)
     if (!(gate_up_by_entries(a) && down_by_entries(a))) return false;   // (the others want the entries grouped)
     if (l.gate_type == kIQ1_S) return weights <= 1ll << 27;
+    if (l.gate_type == kIQ2_S && a.k > 8 && l.n_embd % 1024 != 0) return weights <= 1ll << 26;
     if (l.gate_type == kIQ2_S) return weights <= 1ll << 27 || (weights <= 1ll << 28 && a.n_tokens <= 3);
     return l.gate_type == kQ4_K && (weights <= 1ll << 26 || (weights <= 1ll << 28 && 5 * entries <= 2 * n_expert && l.n_embd <= 4096));
 }

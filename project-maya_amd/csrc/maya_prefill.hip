@@ -63,10 +63,13 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
     int32_t* total = before + n_expert;              // (first the count of the entries behind the share)
     int32_t* base = total + n_expert;
     int32_t* tbase = base + n_expert + 1;
+    int32_t* wbase = tbase + n_expert + 1;
     __shared__ unsigned long long resident[MAYA_MAX_EXPERTS / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    uint64_t blob;   // (of expert tid)
     {
-        const unsigned long long r = __ballot(tid < n_expert && table[tid] != 0ull);   // (n_expert <= kPlanThreads: checked on the host)
+        blob = tid < n_expert ? table[tid] : 0ull;
+        const unsigned long long r = __ballot(blob != 0ull);   // (n_expert <= kPlanThreads: checked on the host)
         if (lane == 0) resident[wave] = r;
     }
     for (int i = tid; i < (kPlanWaves + 2) * n_expert; i += kPlanThreads) seg[i] = 0;
@@ -105,7 +108,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
         total[x] += run;
     }
     __syncthreads();
-    // the experts' first rows (wave 0) and first tiles (wave 1): a lane a run of experts, a scan over the lanes between two passes
+    // the experts' first rows (wave 0), tiles (wave 1) and items (wave 2): a lane a run of experts, a scan over the lanes between two passes
     auto first_of = [&](auto size, int32_t* o) {
         const int per_lane = (n_expert + 63) >> 6, x0 = lane * per_lane;
         int local = 0;
@@ -127,6 +130,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
     };
     if (wave == 0) first_of([&](int x) { return total[x]; }, base);
     if (wave == 1) first_of([&](int x) { return (total[x] + kPfRows - 1) / kPfRows; }, tbase);
+    if (wave == 2 && work.list != nullptr) first_of([&](int x) { return (total[x] + work.rows - 1) / work.rows; }, wbase);
     __syncthreads();
     if (blockIdx.x == 0) {
         for (int x = tid; x <= n_expert; x += kPlanThreads) p.bounds[x] = base[x];
@@ -139,14 +143,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
         if (tid == 0) *p.n_tiles = min(tbase[n_expert], max_tiles);
     }
     if (work.list != nullptr && blockIdx.x == min(1u, gridDim.x - 1)) {   // the GEMMs' work list: every expert's rows in runs of work.rows
-        __syncthreads();   // (tbase's readers above)
-        if (wave == 0) {
-            first_of([&](int x) { return (total[x] + work.rows - 1) / work.rows; }, tbase);
-            if (lane == 0) *work.n = tbase[n_expert];
-        }
-        __syncthreads();
-        for (int x = tid; x < n_expert; x += kPlanThreads)
-            for (int r = 0, t = tbase[x]; r < total[x]; r += work.rows, ++t) work.list[t] = {table[x], base[x] + r, min(work.rows, total[x] - r)};
+        if (tid == 0) *work.n = wbase[n_expert];
+        if (tid < n_expert)
+            for (int r = 0, t = wbase[tid]; r < total[tid]; r += work.rows, ++t) work.list[t] = {blob, base[tid] + r, min(work.rows, total[tid] - r)};
     }
     // the stable scatter: 64 entries a step, a lane's rank = the earlier lanes of the step with its expert
     for (int c0 = lo; c0 < hi; c0 += 64) {
@@ -873,8 +872,8 @@ static int pf_plan(const int32_t* ids, int n_entries, const uint64_t* expert_tab
     if (!ids || !expert_table || !plan_ok(plan)) return fail(MAYA_E_ARG, "prefill_plan: null pointer");
     if (n_entries <= 0 || n_entries > (1 << 20) || n_expert <= 0 || n_expert > MAYA_MAX_EXPERTS)
         return fail(MAYA_E_SHAPE, "prefill_plan: entries %d experts %d", n_entries, n_expert);
-    // (a wave's 64-bit lane masks an expert ride along while LDS holds them: up to 780 experts; ballots beyond)
-    size_t lds = sizeof(int32_t) * ((size_t) (kPlanWaves + 4) * n_expert + 2);
+    // (a wave's 64-bit lane masks an expert ride along while LDS holds them: up to 767 experts; ballots beyond)
+    size_t lds = sizeof(int32_t) * ((size_t) (kPlanWaves + 5) * n_expert + 3);
     const size_t masks = sizeof(unsigned long long) * (size_t) kPlanWaves * n_expert;
     const int with_masks = lds + masks + 1024 <= (size_t) st->lds_limit;
     if (with_masks) lds += masks;
