@@ -664,7 +664,10 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
 // dtype `mode & 255`, bias = the sigmoid router's (bit 8 of mode: the sigmoid router) or NULL; else p0 = the plan's blob
 // addresses (a.plan_ptr), p1 = the codes of x (a.x.q), p2 = their scales (a.x.d).  mode >> 16 = n_embd / 32, the
 // sub-blocks a row.
-template <int NW, int MINW, int HEAD>
+// MANY (with a head): several tokens, a row of the grid each.  One token's form knows no other row: with the row in it the compiler
+// waits for the grid's size before the first logits are asked for, a trip to memory on the way of every workgroup (7168 x 2048
+// top-8 of 256, one token, 29.3 us a layer, 29.8 with it).
+template <int NW, int MINW, int HEAD, bool MANY = false>
 __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_kernel(const void* __restrict__ p0, const void* __restrict__ p1,
                                                                                       const void* __restrict__ p2,
                                                                                       const uint64_t* __restrict__ iq2s_grid,
@@ -687,7 +690,7 @@ __global__ __launch_bounds__(NW > 4 ? 512 : 256, MINW) void gate_up_iq2s_tiles_k
     const bool on = lu < nu;
     const int u = on ? lu : nu - 1;
     // (n_ent = a.k: one token a row of the grid, entry = its plan slot)
-    const int tok = HEAD ? (int) blockIdx.y : 0;
+    const int tok = MANY ? (int) blockIdx.y : 0;
     int y[8];
     float dy8;
     int first_tile = blockIdx.x, tile_step = gridDim.x;

@@ -1670,7 +1670,8 @@ int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hip
     const unsigned walkers = (unsigned) (wgs < n_tiles ? wgs : n_tiles);
     const int nu = a.layout.n_embd >> 5;   // sub-blocks a row, in the upper half of `mode`
     if (hd) {   // workgroup 0 routes, the others walk the tiles
-        auto kern = hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8>;
+        auto kern = a.n_tokens == 1 ? (hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8>)
+                                    : (hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4, true> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8, true>);
         hipLaunchKernelGGL(kern, dim3(walkers + 1, (unsigned) a.n_tokens), dim3(64 * NW), 0, s, (const void*) hd->logits, (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias,
                            a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a, hd->out);
     } else {

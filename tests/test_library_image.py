@@ -2,17 +2,19 @@
 import os
 import re
 import struct
+import subprocess
 
 import pytest
 
 msgpack = pytest.importorskip("msgpack")
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+OBJDUMP = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
 CSRC = os.path.join(ROOT, "project-maya_amd", "csrc")
 
 
-def kernels(path):
-    """name -> metadata of every gfx950 kernel in a library's offload bundles."""
-    d, found, at = open(path, "rb").read(), {}, 0
+def code_objects(path):
+    """The gfx950 code objects in a library's offload bundles."""
+    d, at = open(path, "rb").read(), 0
     while (b := d.find(b"__CLANG_OFFLOAD_BUNDLE__", at)) >= 0:
         n, = struct.unpack_from("<Q", d, b + 24)
         at = b + 32
@@ -21,7 +23,25 @@ def kernels(path):
             name = d[at + 24:at + 24 + name_len]
             at += 24 + name_len
             if b"gfx950" in name:
-                found.update(code_object_kernels(d[b + off:b + off + size]))
+                yield d[b + off:b + off + size]
+
+
+def kernels(path):
+    """name -> metadata of every gfx950 kernel in a library's offload bundles."""
+    return {n: k for e in code_objects(path) for n, k in code_object_kernels(e)}
+
+
+def instructions(path, names, tmp_path):
+    """name -> the instructions of the kernels `names`, as the assembler writes them."""
+    found = {}
+    for i, e in enumerate(code_objects(path)):
+        co = tmp_path / ("%d.co" % i)
+        co.write_bytes(e)
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", "--disassemble-symbols=" + ",".join(names), str(co)],
+                              capture_output=True, text=True, check=True).stdout
+        for part in re.split(r"^(?=(?:[0-9a-f]+ )?<\S+>:$)", text, flags=re.M)[1:]:
+            head, *lines = part.splitlines()
+            found[re.search(r"<(\S+)>:", head).group(1)] = [l.split("//")[0].strip() for l in lines if l.strip()]
     return found
 
 
@@ -62,3 +82,15 @@ def test_the_iq2s_prompt_kernels_have_no_lds_but_their_array():
     assert len(got) == 2
     for n, k in got.items():
         assert k[".group_segment_fixed_size"] == lds, n
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no llvm-objdump")
+def test_one_token_of_iq2s_waits_for_nothing_before_its_first_loads(tmp_path):
+    """What the router is given arrives in registers with the dispatch: a wait in front of the first load is a trip to memory that every
+    workgroup makes first.  (In front of the body stands a prologue that loads and waits, for firmware that does not preload.)"""
+    names = [n for n in kernels(built()) if re.search(r"gate_up_iq2s_tiles_kernelILi\dELi\dELi[48]ELb0E", n)]
+    assert len(names) == 14
+    for n, code in instructions(built(), names, tmp_path).items():
+        body = code[next(i for i, c in enumerate(code) if c.startswith("s_branch")) + 1:]
+        first = next(i for i, c in enumerate(body) if c.startswith("global_load"))
+        assert not [c for c in body[:first] if c.startswith("s_waitcnt")], n
