@@ -521,8 +521,10 @@ struct LayerHeadIn {
 // slot blockIdx.y.  A lane past the row's last position (`on` false; u is then its own index, o0 and o1 the last
 // position's) gets zero codes and a zero scale.  False: the thread has nothing more to do in this launch.
 // R: the experts a lane of the picking wave holds: 4 (up to 256), 8 (up to 512: a chosen expert's blob address is then read from the
-// table's copy in LDS wherever the router needs it).
-template <int NW, int R>
+// table's copy in LDS wherever the router needs it).  MANY: several tokens, the grid's third dimension; one token's form does without
+// its index, three or four registers: with it Q4_K and IQ1_S rows that fill their lanes, and IQ1_S ones that do not, pass 72, 6 waves a
+// SIMD instead of 7.
+template <int NW, int R, bool MANY>
 __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent, const int32_t* skip, bool is_up, bool on, int u, int o0,
                                                 int o1, int (&y)[8], float& d, uint64_t& blob) {
     constexpr int NU = 32 * NW;
@@ -530,7 +532,7 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
     __shared__ float s_lv[64 * R];
     __shared__ uint64_t s_tab[64 * R];
     __shared__ int s_y[9][NU];
-    const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert, tok = (int) blockIdx.z;
+    const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert, tok = MANY ? (int) blockIdx.z : 0;
     const bool picker = t >= 64 * (NW - 1), sigm = hd.sigmoid != 0;
     float lv[R], bv[R];
     uint64_t tab[R];

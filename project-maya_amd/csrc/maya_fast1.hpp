@@ -88,8 +88,9 @@ __device__ __forceinline__ int sum32_codes(const int (&y)[8]) {
 // ---- gate/up: a workgroup of NW waves = 2 * 32 NW lanes for the sub-block positions of a (gate row, up row) pair (lanes past
 // the row's last position idle, as in the IQ2_S kernels);
 // grid (n_ff / ROWS, entries); entry e = token e / k, slot e % k.  Rows in batches of 8 (two quads), a quad ahead.
-// HEAD (4 or 8: a token's experts a lane): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k, tokens).
-template <int NW, int ROWS, int MINW, bool FIT, int HEAD = 0>
+// HEAD (4 or 8: a token's experts a lane): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k), of
+// several tokens (MANY) (n_ff / ROWS + 1, k, tokens).
+template <int NW, int ROWS, int MINW, bool FIT, int HEAD = 0, bool MANY = false>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(MAYA_HEAD_PARAMS, maya_moe_args a, Codebooks cb, LayerHead out) {
     static_assert(ROWS % 8 == 0, "a batch is two quads");
     constexpr int NU = 32 * NW;
@@ -100,14 +101,14 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(MAYA_HE
     const int nu = FIT ? NU : mode >> 16, lu = is_up ? t - NU : t;   // sub-blocks a row; the lane's position among 32 NW
     const bool on = FIT || lu < nu;
     const int u = on ? lu : nu - 1;
-    const int e = HEAD ? (int) blockIdx.z * n_ent + (int) blockIdx.y : (int) blockIdx.y;
+    const int e = MANY ? (int) blockIdx.z * n_ent + (int) blockIdx.y : (int) blockIdx.y;
     uint64_t blob;
     int y[8];
     float dy8;
     if constexpr (HEAD) {
         float d;
         const LayerHeadIn hd = {logits, table, x, bias, n_expert, mode & 255, (mode >> 8) & 1, out, mode >> 16 << 5};
-        if (!head_in_gate_up<NW, HEAD>(hd, n_ent, skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob)) return;
+        if (!head_in_gate_up<NW, HEAD, MANY>(hd, n_ent, skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob)) return;
         dy8 = d * 0.125f;
     } else {
         if (skip && *skip) return;

@@ -1862,10 +1862,13 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     }
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
+#define MAYA_IQ1H(NWV, MANY)                                                                                                    \
+    if (h.n_expert > 256) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, 8, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
+    else if (fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, 4, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);          \
+    else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, 4, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);
 #define MAYA_IQ1(NWV)                                                                                                          \
-    if (hd && hd->n_expert > 256) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, 8>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
-    else if (hd && fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, true, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);  \
-    else if (hd) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 6, false, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);   \
+    if (hd && a.n_tokens > 1) { MAYA_IQ1H(NWV, true) }                                                                          \
+    else if (hd) { MAYA_IQ1H(NWV, false) }                                                                                      \
     else if (fit) hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);         \
     else hipLaunchKernelGGL((gate_up_iq1s_pos_kernel<NWV, 16, 8, false>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, st.cb, h.out);
     switch (pos_waves(a.layout.n_embd)) {
@@ -1878,6 +1881,7 @@ int launch_gate_up_iq1s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
         default: MAYA_IQ1(8) break;
     }
 #undef MAYA_IQ1
+#undef MAYA_IQ1H
     MAYA_LAUNCHED("gate_up_iq1s_pos_kernel");
     return MAYA_OK;
 }
@@ -1964,18 +1968,20 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd ? 1u : 0u), (unsigned) (hd ? a.k : a.n_tokens * a.k), (unsigned) (hd ? a.n_tokens : 1));
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
-    const bool wide = hd && hd->n_expert > 256;   // (their rows take the form that any length has)
+#define MAYA_Q4H(NWV, F, HEAD, MANY)                                                                                        \
+    if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);   \
+    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
+#define MAYA_Q4HEAD(NWV, MANY)                                                                                              \
+    if (h.n_expert > 256) { MAYA_Q4H(NWV, false, 8, MANY) }   /* (their rows take the form that any length has) */           \
+    else if (fit) { MAYA_Q4H(NWV, true, 4, MANY) }                                                                          \
+    else { MAYA_Q4H(NWV, false, 4, MANY) }
 #define MAYA_Q4F(NWV, F)                                                                                                    \
-    if (hd && small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);      \
-    else if (hd) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, 4>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);        \
-    else if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);          \
+    if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);               \
     else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8, F>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
-#define MAYA_Q4W(NWV)                                                                                                       \
-    if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, false, true, 8>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);        \
-    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, false, false, 8>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
-#define MAYA_Q4(NWV)                         \
-    if (wide) { MAYA_Q4W(NWV) }             \
-    else if (fit) { MAYA_Q4F(NWV, true) }   \
+#define MAYA_Q4(NWV)                                       \
+    if (hd && a.n_tokens > 1) { MAYA_Q4HEAD(NWV, true) }  \
+    else if (hd) { MAYA_Q4HEAD(NWV, false) }              \
+    else if (fit) { MAYA_Q4F(NWV, true) }                 \
     else { MAYA_Q4F(NWV, false) }
     switch (pos_waves(a.layout.n_embd)) {
         case 2: MAYA_Q4(2) break;
@@ -1988,7 +1994,8 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     }
 #undef MAYA_Q4
 #undef MAYA_Q4F
-#undef MAYA_Q4W
+#undef MAYA_Q4H
+#undef MAYA_Q4HEAD
     MAYA_LAUNCHED("gate_up_q4k_pos_kernel");
     return MAYA_OK;
 }

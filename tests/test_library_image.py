@@ -94,3 +94,13 @@ def test_one_token_of_iq2s_waits_for_nothing_before_its_first_loads(tmp_path):
         body = code[next(i for i, c in enumerate(code) if c.startswith("s_branch")) + 1:]
         first = next(i for i, c in enumerate(body) if c.startswith("global_load"))
         assert not [c for c in body[:first] if c.startswith("s_waitcnt")], n
+
+
+def test_one_token_heads_leave_seven_waves_a_simd():
+    """Q4_K rows that fill their lanes (16 rows a workgroup) and IQ1_S rows of three waves and more, the layer's head in the launch: 72
+    registers at most, the form of several tokens has 75."""
+    got = {n: k for n, k in kernels(built()).items()
+           if re.search(r"gate_up_q4k_pos_kernelILi\dELi16ELi6ELb1ELb0ELi4ELb0E|gate_up_iq1s_pos_kernelILi[3-8]ELi16ELi6ELb[01]ELi[48]ELb0E", n)}
+    assert len(got) == 7 + 18
+    for n, k in got.items():
+        assert k[".vgpr_count"] <= 72 and k[".private_segment_fixed_size"] == 0, n
