@@ -722,26 +722,33 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, pf_lds8 lds, const PfTi
 
 // The workgroup's rows: a listed tile, and with it the next one on the list where that goes on with the expert's rows and starts in
 // the middle of 128 of them.  False where there are none: past the last tile, or the workgroup of the tile before takes them.
-// (Both sides read the list itself, so a caller's part of it is what is computed.)
+// (Both sides read the list itself, so a caller's part of it is what is computed.)  Every tile alone for a kernel that decodes its weights
+// once a group of 32 rows whatever it is given (PAIRS false).
 static_assert(2 * kPfRows == 4 * 32, "four row groups of a workgroup at most");
+template <bool PAIRS>
 __device__ __forceinline__ bool pf_my_tile(const PfGemm& a, PfTile& t) {
     const int tile = blockIdx.y, n = *a.plan.n_tiles;
     if (tile >= n) return false;
     const int ex = a.plan.tile_expert[tile];
     t.row0 = a.plan.tile_row0[tile];
+    t.blob = (const uint8_t*) a.table[ex];
+    if (!PAIRS) {
+        t.nrows = min(kPfRows, a.plan.bounds[ex + 1] - t.row0);
+        return true;
+    }
     const int before = max(tile - 1, 0), behind = min(tile + 1, n - 1);
     const int bx = a.plan.tile_expert[before], b0 = a.plan.tile_row0[before], nx = a.plan.tile_expert[behind], n0 = a.plan.tile_row0[behind];
     const int first = a.plan.bounds[ex], at = (t.row0 - first) % (2 * kPfRows);
     if (at == kPfRows && bx == ex && b0 == t.row0 - kPfRows) return false;
     const bool two = at == 0 && nx == ex && n0 == t.row0 + kPfRows;
     t.nrows = min(two ? 2 * kPfRows : kPfRows, a.plan.bounds[ex + 1] - t.row0);
-    t.blob = (const uint8_t*) a.table[ex];
     return true;
 }
 
 // the same from the work list where there is one
+template <bool PAIRS = true>
 __device__ __forceinline__ bool pf_my_rows(const PfGemm& a, PfTile& t) {
-    if (a.work.list == nullptr) return pf_my_tile(a, t);
+    if (a.work.list == nullptr) return pf_my_tile<PAIRS>(a, t);
     if ((int) blockIdx.y >= *a.work.n) return false;
     const PfItem i = a.work.list[blockIdx.y];
     t.blob = (const uint8_t*) i.blob, t.row0 = i.row0, t.nrows = i.nrows;

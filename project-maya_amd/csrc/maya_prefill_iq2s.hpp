@@ -199,7 +199,7 @@ template <bool GU>
 __global__ __launch_bounds__(256, 3) void prefill_iq2s_few_kernel(PfGemm a, Codebooks cb) {
     __shared__ __attribute__((aligned(256))) uint8_t lds[kIqFewLdsBytes];
     PfTile t;
-    if (!pf_my_rows(a, t)) return;
+    if (!pf_my_rows<false>(a, t)) return;
     pf_iq2s_tables(lds, cb, threadIdx.x);
     typedef PfIq2s<GU, kIqFewRing> W;
     for (int r = 0; r < t.nrows; r += 32) {

@@ -270,6 +270,39 @@ def test_layer_calls_equal_the_stages(pf, t, n_embd, n_ff):
     assert all(torch.equal(o.view(torch.int32), outs[0].view(torch.int32)) for o in outs)
 
 
+FEW_ROWS = [128, 97, 96, 65, 64, 33, 17, 8, 3, 1]   # (512 entries, of 128 tokens)
+
+
+@pytest.mark.parametrize("gate, down", [(Q4_K, 22), (22, Q4_K), (22, 22), (Q4_K, Q4_K)], ids=str)
+def test_layer_calls_equal_the_stages_on_few_rows(pf, gate, down):
+    """Chunks of few rows an expert on average, whose IQ2_S products run on a kernel of fewer rows and whose Q4_K ones do not: the
+    layer's list serves both, with the bits of the stage calls and of a chunk of more rows an expert, experts of 1 to 128 rows."""
+    from maya_amd import lib
+    import synth
+    gen = np.random.default_rng(100 * gate + down)
+    n_embd, n_ff, ne, k = 1024, 512, len(FEW_ROWS), 4
+    blobs = [synth.expert_blob(gate, down, n_embd, n_ff, gen) for _ in range(ne)]
+    layout, _ = lib.layout(gate, down, n_embd, n_ff)
+    store = lib.ExpertStore(blobs, pack_layout=layout)
+    layout = lib.copy_layout(layout, lib.PACK_STREAM)
+    ids = np.repeat(np.arange(ne, dtype=np.int32), FEW_ROWS)
+    gen.shuffle(ids)
+    nt = ids.size // k
+    x = dev(gen.standard_normal((nt, n_embd)).astype(np.float32))
+    weights = dev(gen.random((nt, k)).astype(np.float32) + 0.5)
+    outs = []
+    for idle in (0, 54, 290):   # (0: more than 8 rows an expert; 54: 8)
+        table = torch.cat([store.table, store.table[:1].expand(idle)]).contiguous()
+        p = pf.plan(dev(ids), table)
+        part = pf.down(layout, table, p, pf.gate_up(layout, table, p, pf.quant(x, p, k)))
+        want = pf.combine(p, weights, part, nt, k)
+        layer = pf.PrefillLayer(layout, ne + idle, k, nt, out_dtype=torch.float32)
+        got = layer.forward(table, None, x, routed=(dev(ids).view(nt, k), weights)).clone()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)) and bool((got != 0).any(1).all()), idle
+        outs.append(got)
+    assert all(torch.equal(o.view(torch.int32), outs[0].view(torch.int32)) for o in outs)
+
+
 @pytest.mark.parametrize("t, n_embd, n_ff", [(Q4_K, 512, 256), (22, 512, 512)], ids=str)
 def test_a_part_of_the_tile_list(pf, oracle, t, n_embd, n_ff):
     """A caller may hand on some of a plan's tiles - a chunk in two halves, every second tile, one tile, any order: their rows are the
