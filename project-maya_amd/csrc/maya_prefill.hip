@@ -51,6 +51,7 @@ struct PfWork {
     PfItem* list;
     int32_t* n;      // [1] items
     int rows;
+    bool few;        // IQ2_S products: on the kernel for few rows an expert
 };
 constexpr int kPlanMaxGroups = 64;   // (at 1 << 20 entries the counting would outweigh the scatter)
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_t* __restrict__ ids, int n_entries,
@@ -863,6 +864,12 @@ static bool act_ok(const maya_prefill_act& a) {
 static unsigned pf_grid_rows(const PfWork& work, int n_entries, int n_expert) {
     return work.list ? (unsigned) (n_entries / work.rows + std::min(n_entries, n_expert)) : (unsigned) maya_moe_prefill_max_tiles(n_entries, n_expert);
 }
+// A stage call's: no list; the slots of a token, which it is not told, taken as 8.
+static PfWork pf_stage_work(int n_entries, int n_expert) {
+    PfWork w{};
+    w.few = prefill_iq2s_few(n_entries / 8, n_entries, n_expert);
+    return w;
+}
 template <bool GU>
 static void pf_launch(const PfGemm& a, dim3 grid, hipStream_t s) {
     hipLaunchKernelGGL(prefill_q4k_kernel<GU>, grid, dim3(256), 0, s, a);
@@ -932,7 +939,7 @@ static int pf_gate_up(const maya_moe_layout* l, const uint64_t* expert_table, in
     a.work = work;
     const dim3 grid((unsigned) (l->n_ff / 64), pf_grid_rows(work, n_entries, n_expert));
     if (l->gate_type == kIQ2_S) {
-        prefill_iq2s_launch<true>(a, st->cb, grid, n_entries, n_expert, as_stream(stream));
+        prefill_iq2s_launch<true>(a, st->cb, grid, as_stream(stream));
         MAYA_LAUNCHED("prefill_iq2s_kernel<gate_up>");
     } else {
         pf_launch<true>(a, grid, as_stream(stream));
@@ -963,7 +970,7 @@ static int pf_down(const maya_moe_layout* l, const uint64_t* expert_table, int n
     a.work = work;
     const dim3 grid((unsigned) ((l->n_embd + 127) / 128), pf_grid_rows(work, n_entries, n_expert));
     if (l->down_type == kIQ2_S) {
-        prefill_iq2s_launch<false>(a, st->cb, grid, n_entries, n_expert, as_stream(stream));
+        prefill_iq2s_launch<false>(a, st->cb, grid, as_stream(stream));
         MAYA_LAUNCHED("prefill_iq2s_kernel<down>");
     } else {
         pf_launch<false>(a, grid, as_stream(stream));
@@ -1009,12 +1016,12 @@ int maya_moe_prefill_quant(const void* x, int x_dtype, int64_t x_stride, const m
 
 int maya_moe_prefill_gate_up(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan,
                              int n_entries, maya_prefill_act xq, float limit, float* h, maya_prefill_act hq, void* stream) {
-    return pf_gate_up(l, expert_table, n_expert, plan, n_entries, xq, limit, h, hq, PfWork{}, stream);
+    return pf_gate_up(l, expert_table, n_expert, plan, n_entries, xq, limit, h, hq, pf_stage_work(n_entries, n_expert), stream);
 }
 
 int maya_moe_prefill_down(const maya_moe_layout* l, const uint64_t* expert_table, int n_expert, const maya_prefill_plan* plan,
                           int n_entries, maya_prefill_act hq, float* part, void* stream) {
-    return pf_down(l, expert_table, n_expert, plan, n_entries, hq, part, PfWork{}, stream);
+    return pf_down(l, expert_table, n_expert, plan, n_entries, hq, part, pf_stage_work(n_entries, n_expert), stream);
 }
 
 int maya_moe_prefill_combine(const maya_prefill_plan* plan, const float* weights, const float* part, int n_tokens, int k,
@@ -1069,7 +1076,8 @@ static PrefillWs prefill_carve(const maya_moe_layout& l, int n_tokens, int k, in
     w.plan.tile_row0 = (int32_t*) take(4 * mt);
     w.plan.n_tiles = (int32_t*) take(4);
     // Items of 128 rows, a workgroup's most; of 64 where the IQ2_S kernel of few rows takes them.
-    w.work.rows = l.gate_type == kIQ2_S && prefill_iq2s_few((int) ne, n_expert) ? kPfRows : 2 * kPfRows;
+    w.work.few = prefill_iq2s_few(n_tokens, (int) ne, n_expert);
+    w.work.rows = l.gate_type == kIQ2_S && w.work.few ? kPfRows : 2 * kPfRows;
     w.work.list = (PfItem*) take(sizeof(PfItem) * mt);   // (fewer than the tiles)
     w.work.n = (int32_t*) take(4);
     auto take_act = [&](maya_prefill_act& a, size_t k) {

@@ -228,13 +228,22 @@ static int prefill_iq2s_lds_ok(const char* what) {
     if (!rc) rc = prefill_iq2s_kernel_lds_ok<prefill_iq2s_few_kernel<false>, kIqFewLdsBytes>(what);
     return rc;
 }
-// Whether a chunk's IQ2_S products run on the kernel for few rows an expert: on the average of them, as the host does not know the
-// routing.  Microseconds a layer call, 160 experts of 6144 x 1536, kernel of 128 rows and this one: 8 rows an expert on average 564 and 520
-// (routing skewed by 0.6 518 and 503, by 1.1 338 and 345), 12 rows 585 and 531 (590 and 578, 377 and 404), 24 rows 640 and 619 (714 and 760, 549 and
-// 618); of 3072 x 1536, 8 rows 301 and 278 (283 and 269, 188 and 185).
-static bool prefill_iq2s_few(int n_entries, int n_expert) { return n_entries <= 8 * n_expert; }
+// Whether a chunk's IQ2_S products run on the kernel for few rows an expert.  The host does not know the routing: an expert has 8 rows at most on
+// average, and the tokens are few enough that one which nearly all of them take, which this kernel decodes once a 32 of them, costs no more
+// than the others save.  Microseconds a layer call, kernel of 128 rows / this one, routing even, skewed by 0.6 and by 1.1:
+//   160 experts of 6144 x 1536 top-8, 75 tokens 520 / 485, 391 / 375, 233 / 224;  90 tokens 538 / 496, 423 / 402, 251 / 254;  110 tokens 537 / 497,
+//   465 / 440, 272 / 271;  top-4, 128 tokens by 0.6 342 / 330, by 1.1 168 / 164;  top-1, 250 tokens 195 / 183, 120 / 116;
+//   256 of 7168 x 2048 top-8, 80 tokens by 0.6 702 / 656, by 1.1 347 / 348;  80 of 7168 x 2048, 80 tokens 415 / 395, 317 / 320;
+//   256 of 4096 x 2048 top-8, 110 tokens 470 / 447, 244 / 247;  top-2, 250 tokens 281 / 271, 117 / 112;
+//   288 of 4096 x 1024 top-10, 88 tokens 275 / 264, 158 / 152;  64 of 3072 x 1536 top-6, 64 tokens 131 / 123, 131 / 121, 97 / 92
+// With more tokens even routing gains as much, but a skewed one loses: 160 experts of 6144 x 1536 top-8, 120 tokens by 1.1 276 / 288, 160 tokens
+// 554 / 510, 513 / 497, 320 / 332;  top-4, 220 tokens by 1.1 208 / 215;  top-1, 512 tokens 132 / 138;  256 of 4096 x 2048 top-8, 256 tokens
+// 774 / 712, 680 / 653, 355 / 376.
+static bool prefill_iq2s_few(int n_tokens, int n_entries, int n_expert) {
+    return n_entries <= 8 * n_expert && n_tokens <= (n_entries <= 512 ? 256 : 112);
+}
 template <bool GU>
-static void prefill_iq2s_launch(const PfGemm& a, const Codebooks& cb, dim3 grid, int n_entries, int n_expert, hipStream_t s) {
-    if (prefill_iq2s_few(n_entries, n_expert)) hipLaunchKernelGGL(prefill_iq2s_few_kernel<GU>, grid, dim3(256), 0, s, a, cb);
+static void prefill_iq2s_launch(const PfGemm& a, const Codebooks& cb, dim3 grid, hipStream_t s) {
+    if (a.work.few) hipLaunchKernelGGL(prefill_iq2s_few_kernel<GU>, grid, dim3(256), 0, s, a, cb);
     else hipLaunchKernelGGL(prefill_iq2s_kernel<GU>, grid, dim3(256), 0, s, a, cb);
 }
