@@ -107,8 +107,9 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_iq1s_pos_kernel(MAYA_HE
     float dy8;
     if constexpr (HEAD) {
         float d;
+        int slot;
         const LayerHeadIn hd = {logits, table, x, bias, n_expert, mode & 255, (mode >> 8) & 1, out, mode >> 16 << 5};
-        if (!head_in_gate_up<NW, HEAD, MANY>(hd, n_ent, skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob)) return;
+        if (!head_in_gate_up<NW, HEAD, MANY ? kTokenPlanes : kOneToken>(hd, n_ent, skip, is_up, on, lu, 32 * u, 32 * u + 16, y, d, blob, slot)) return;
         dy8 = d * 0.125f;
     } else {
         if (skip && *skip) return;

@@ -1964,8 +1964,9 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     // 16 rows a workgroup, 8 - all requested up front - when the call has so few entries that 16 would leave compute units idle
     const bool small = (long long) (a.layout.n_ff / 16) * a.n_tokens * a.k < 512;
     const int rows = small ? 8 : 16;
-    // (with the head in the launch: one more column, whose first workgroup is the token's router)
-    const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd ? 1u : 0u), (unsigned) (hd ? a.k : a.n_tokens * a.k), (unsigned) (hd ? a.n_tokens : 1));
+    // (with the head in the launch: one more column or, of several tokens, plane for the routers)
+    const bool many = hd && a.n_tokens > 1;
+    const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd && !many ? 1u : 0u), (unsigned) (many ? a.n_tokens : a.n_tokens * a.k), many ? a.k + 1u : 1u);
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_Q4H(NWV, F, HEAD, MANY)                                                                                        \
@@ -1979,7 +1980,7 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);               \
     else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 8, F>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
 #define MAYA_Q4(NWV)                                       \
-    if (hd && a.n_tokens > 1) { MAYA_Q4HEAD(NWV, true) }  \
+    if (many) { MAYA_Q4HEAD(NWV, true) }                  \
     else if (hd) { MAYA_Q4HEAD(NWV, false) }              \
     else if (fit) { MAYA_Q4F(NWV, true) }                 \
     else { MAYA_Q4F(NWV, false) }

@@ -450,3 +450,36 @@ def test_several_tokens_head_in_the_gate_up_launch(lib, ty, n_embd, n_ff, ne, k,
             assert torch.equal(got.ids, ids) and torch.equal(got.weights.view(torch.int32), w.view(torch.int32)), first
             assert torch.equal(got.out[:nt].view(torch.int32), want.view(torch.int32)), first
         assert torch.equal(out.view(torch.int32), want.view(torch.int32)), first
+
+
+@pytest.mark.parametrize("sigmoid", (False, True))
+@pytest.mark.parametrize("ty,n_embd,n_ff,ne,k,nt", ((12, 2048, 256, 40, 8, 2), (12, 3072, 512, 64, 6, 3), (12, 2304, 256, 300, 8, 5), (12, 4096, 1536, 128, 8, 5),
+                                                    (12, 7168, 2048, 16, 2, 2), (19, 2048, 256, 40, 8, 5), (22, 2048, 256, 40, 8, 5)))
+def test_windows_whose_tokens_take_the_same_experts(lib, ty, n_embd, n_ff, ne, k, nt, sigmoid):
+    """Tokens that share all or half of their experts, each in an order of its own, an expert of them not resident: every token's slots are
+    its own - the bits of the layer given the ids and weights, and of each token alone."""
+    blobs = make_experts(ty, ty, n_embd, n_ff, 9, 7 * ne + ty)
+    store = lib.ExpertStore(blobs, pack_layout=lib.layout(ty, ty, n_embd, n_ff)[0])
+    table = store.table[torch.arange(ne, device="cuda") % 9].contiguous()
+    rng = np.random.default_rng(n_embd + nt)
+    more = {}
+    if sigmoid:
+        bias = dev((rng.standard_normal(ne) * 0.1).astype(np.float32))
+        more = {"router": lib.Router(lib.ROUTER_SIGMOID, 1, bias.data_ptr(), 2.5)}
+    layer, given, alone = (lib.MoeLayer(ty, ty, n_embd, n_ff, ne, k, max_tokens=m, packing=1) for m in (nt, nt, 1))
+    x = torch.from_numpy(rng.standard_normal((nt, n_embd)).astype(np.float32)).cuda()
+    for share in (k, k // 2):
+        logits = rng.standard_normal((nt, ne)).astype(np.float32)
+        same = rng.permutation(ne)[:share]
+        logits[:, same] += np.float32(3.0 if sigmoid else 8.0)
+        table[int(same[0])] = 0
+        lg = dev(logits)
+        out = layer.forward(table, lg, x, **more).clone()
+        ids, w, _ = lib.route_plan(lg, k, table, more.get("router"))
+        want = given.forward(table, None, x, routed=(ids, w)).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(layer.ids, ids) and torch.equal(layer.weights.view(torch.int32), w.view(torch.int32)), share
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32)), share
+        for t in range(nt):
+            one = alone.forward(table, lg[t:t + 1].contiguous(), x[t:t + 1].contiguous(), **more)
+            assert torch.equal(one.view(torch.int32), out[t:t + 1].view(torch.int32)), (share, t)
