@@ -1641,45 +1641,49 @@ int launch_gate_up_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
     MAYA_LAUNCHED("gate_up_iq2s_pos_kernel");
     return MAYA_OK;
 }
-// One token: the tile-streaming form, launched with the workgroups the chip holds at once (asked of the runtime once a
-// shape), at most three a compute unit: measured on 7168 x 2048, top-8, 768 workgroups 18.5 us, 1024 (all resident, two
+// One token: the tile-streaming form, launched with the workgroups the chip holds at once, at most three a compute unit: measured on 7168 x 2048,
+// top-8, 768 workgroups 18.5 us, 1024 (all resident, two
 // tiles each) 20.1 us, 512 20.4 us, 256 24.1 us - a workgroup's cold start is paid per workgroup, latency hiding per wave.
 // (The layer at 4096 x 2048: 20.2 us with three a compute unit, 21.2 with six; 3072 x 1024: 15.6 and 15.7 with eight; only the
-// two-wave workgroups, whose three would leave a compute unit six waves, take twelve: 2048 x 2048 18.9 -> 16.8 us.)
+// two-wave workgroups, whose three would leave a compute unit six waves, take eight: 2048 x 2048 18.9 us with three -> 16.8, top-10 21.9,
+// 23.9 with ten, which its registers and LDS allow up to 256 experts.)
 // The kernel is compiled for 6 waves a SIMD - three workgroups of up to 8 waves a compute unit, what is launched; the small
 // workgroups of two and three waves for 5, which their registers want - not 8:
-// with the head's prologue in it the kernel needs 73-77 registers, and at 64 it spilled 36 bytes a lane to scratch
-// memory: 6.8 MB written and read back a launch, 2.1 us of the layer.  Windows keep gate_up_iq2s_pos_kernel: the tile
-// stream with the resident workgroups shared out among the tokens (a token's codes in a workgroup's registers) was built
-// and is slower on long ones (eight tokens of 7168 x 2048 260 us against 234); window_head_in_gate_up_pays says where it is not.
-template <int NW>
-int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd = nullptr) {
-    constexpr int kMinW = NW <= 3 ? 5 : 6, kMostPerCu = NW == 2 ? 12 : 3;
-    static int per_cu = 0;
+// with the head's prologue in it the kernel needs 74-79 registers (89 and 85 with two and three waves), and at 64 it spilled 36 bytes a lane
+// to scratch memory: 6.8 MB written and read back a launch, 2.1 us of the layer.  Windows of long calls keep gate_up_iq2s_pos_kernel: the tile
+// stream with the resident workgroups shared out among the tokens (a token's codes in a workgroup's registers)
+// is slower there (eight tokens of 7168 x 2048 260 us against 234); window_head_in_gate_up_pays says where it is not.
+static constexpr int iq2s_tiles_per_cu(int waves) { return waves == 2 ? 8 : 3; }
+template <int NW, int HEAD, bool MANY>
+int launch_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd) {
+    constexpr int kMinW = NW <= 3 ? 5 : 6, kMostPerCu = iq2s_tiles_per_cu(NW);
+    const auto kern = gate_up_iq2s_tiles_kernel<NW, kMinW, HEAD, MANY>;
+    static int per_cu = 0;   // (asked of the runtime once a form)
     if (per_cu == 0) {
-        int n = 0, m = 0;
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gate_up_iq2s_tiles_kernel<NW, kMinW, 0>, 64 * NW, 0));
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, kMinW, 4>, 64 * NW, 0));
-        n = m < n ? m : n;
-        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&m, gate_up_iq2s_tiles_kernel<NW, kMinW, 8>, 64 * NW, 0));
-        n = m < n ? m : n;
+        int n = 0;
+        MAYA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 64 * NW, 0));
         per_cu = n > kMostPerCu ? kMostPerCu : n > 0 ? n : 1;
     }
     const int n_tiles = a.k * (a.layout.n_ff / 8);
-    const int wgs = per_cu * st.n_cu / (hd ? a.n_tokens : 1);   // (the resident workgroups shared out among the tokens)
+    const int wgs = std::max(1, per_cu * st.n_cu / (MANY ? a.n_tokens : 1));   // (the resident workgroups shared out among the tokens)
     const unsigned walkers = (unsigned) (wgs < n_tiles ? wgs : n_tiles);
     const int nu = a.layout.n_embd >> 5;   // sub-blocks a row, in the upper half of `mode`
-    if (hd) {   // workgroup 0 routes, the others walk the tiles
-        auto kern = a.n_tokens == 1 ? (hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8>)
-                                    : (hd->n_expert <= 256 ? gate_up_iq2s_tiles_kernel<NW, kMinW, 4, true> : gate_up_iq2s_tiles_kernel<NW, kMinW, 8, true>);
-        hipLaunchKernelGGL(kern, dim3(walkers + 1, (unsigned) a.n_tokens), dim3(64 * NW), 0, s, (const void*) hd->logits, (const void*) hd->table, hd->x, st.cb.iq2s, hd->bias,
-                           a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a, hd->out);
+    if constexpr (HEAD) {   // workgroup 0 routes, the others walk the tiles
+        hipLaunchKernelGGL(kern, dim3(walkers + 1, (unsigned) (MANY ? a.n_tokens : 1)), dim3(64 * NW), 0, s, (const void*) hd->logits, (const void*) hd->table, hd->x, st.cb.iq2s,
+                           hd->bias, a.skip, hd->n_expert, hd->x_dtype | (hd->sigmoid << 8) | (nu << 16), a.k, a, hd->out);
     } else {
-        hipLaunchKernelGGL((gate_up_iq2s_tiles_kernel<NW, kMinW, 0>), dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
+        hipLaunchKernelGGL(kern, dim3(walkers), dim3(64 * NW), 0, s, (const void*) a.plan_ptr,
                            (const void*) a.x.q, (const void*) a.x.d, st.cb.iq2s, (const float*) nullptr, a.skip, 0, nu << 16, a.k, a, LayerHead{});
     }
     MAYA_LAUNCHED("gate_up_iq2s_tiles_kernel");
     return MAYA_OK;
+}
+template <int NW>
+int launch_gate_up_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd = nullptr) {
+    if (!hd) return launch_iq2s_tiles<NW, 0, false>(a, st, s, hd);
+    const bool wide = hd->n_expert > 256;
+    if (a.n_tokens == 1) return wide ? launch_iq2s_tiles<NW, 8, false>(a, st, s, hd) : launch_iq2s_tiles<NW, 4, false>(a, st, s, hd);
+    return wide ? launch_iq2s_tiles<NW, 8, true>(a, st, s, hd) : launch_iq2s_tiles<NW, 4, true>(a, st, s, hd);
 }
 // The layer whose head rides in the gate/up launch, one token's always, several tokens' where that pays (gate_up_iq2s_tiles_kernel<.., 4 or 8>,
 // gate_up_q4k_pos_kernel<.., 4 or 8>): either router over up to 512 experts with more experts than slots, x aligned for

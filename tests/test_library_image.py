@@ -104,3 +104,15 @@ def test_one_token_heads_leave_seven_waves_a_simd():
     assert len(got) == 7 + 18
     for n, k in got.items():
         assert k[".vgpr_count"] <= 72 and k[".private_segment_fixed_size"] == 0, n
+
+
+def test_the_iq2s_tile_walk_holds_the_workgroups_it_is_launched_with():
+    """Eight of two waves a compute unit, three of more, whichever form the layer's head has: 512 registers a lane of a SIMD in blocks
+    of 8, 160 KB of LDS."""
+    got = {n: k for n, k in kernels(built()).items() if "gate_up_iq2s_tiles_kernel" in n}
+    assert len(got) == 7 * 5
+    for n, k in got.items():
+        waves = int(re.search(r"kernelILi(\d)E", n).group(1))
+        wgs = 8 if waves == 2 else 3
+        assert wgs * k[".group_segment_fixed_size"] <= 160 * 1024, n
+        assert -(-wgs * waves // 4) <= 512 // (-(-k[".vgpr_count"] // 8) * 8), n
