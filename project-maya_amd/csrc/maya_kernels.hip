@@ -1697,34 +1697,50 @@ bool gate_up_iq1s_pos_ok(const maya_moe_args& a);
 bool gate_up_by_entries(const maya_moe_args& a);
 bool down_by_entries(const maya_moe_args& a);
 // The head of several tokens in the gate/up launch: a launch and its gap less (4 to 5 us), against a picking wave and the rounding
-// of x in every workgroup, fewer waves a compute unit (the registers of the head) and entries of one expert that no longer run side by side.
-// So: few weights to go through; IQ1_S up to 2^27 (its kernel is bound by vector instructions, which the head adds to); Q4_K up to 2^26, and up to
-// 2^28 where few of the tokens share experts and rows are of at most 4096 values (workgroups of up to four waves: those of five
-// or six lose a third of a compute unit's waves).  Microseconds a layer, head in a launch of its own / in this one:
-//   Q4_K 2048 x 768 top-8 of 128, 2 tokens 19.0 / 15.1, 4 24.1 / 20.3, 6 30.5 / 27.1, 16 (201 M) 51.8 / 54.9;  4096 x 512 of 200, 3 27.5 / 22.5;
-//   4096 x 1536 of 128, 2 36.7 / 32.2, 5 (252 M) 85.7 / 82.3;  4096 x 1024 top-4 of 64, 8 (experts shared) 36.9 / 37.4, 4096 x 512 top-6 of 96, 8 34.6 / 36.5;
-//   5120 x 1536 top-10 of 160, 2 54.3 / 55.2;  6144 x 1536 top-10 of 100, 3 96.2 / 99.6;  7168 x 2048 top-1 of 16, 4 (59 M) 27.3 / 25.1
-//   IQ1_S 2048 x 768, 2 18.8 / 14.6, 10 (126 M) 35.9 / 33.5;  4096 x 512, 4 25.6 / 21.8;  5120 x 1024 top-4 of 32, 4 (84 M) 23.9 / 24.1;
-//   6144 x 1536 top-10, 2 (189 M) 43.4 / 45.7;  7168 x 2048 top-8, 2 (235 M) 43.7 / 45.3, 4 75.5 / 82.5
-// IQ2_S rows share the resident workgroups of the tile walk out among the tokens: up to 2^27, two and three tokens up to 2^28 (the
-// kernel of a launch behind a head of its own has more waves a compute unit, which tells on longer launches).
-//   IQ2_S 2048 x 768 top-8 of 128, 2 18.9 / 15.5, 10 (126 M) 40.5 / 33.8;  4096 x 1536, 2 31.5 / 29.8, 3 (151 M) 41.4 / 36.1, 5 (252 M) 58.4 / 61.6;
-//   7168 x 2048 of 100, 2 (235 M) 53.0 / 49.5;  with Q4_K down rows 3 (352 M) 92.5 / 93.6, 8 197 / 206;  3072 x 1024 top-6, 8 (151 M) 39.1 / 40.2;
-//   more slots than eight and rows that leave lanes idle: top-10 2304 x 1792, 3 (124 M) 47.4 / 48.9, 4864 x 2048, 2 (199 M) 63.0 / 64.5
-static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert) {
+// of x in every workgroup, fewer waves a compute unit (the registers of the head) and entries of one expert that do not run side by side
+// (Q4_K's nearly do).  Microseconds a layer, head in a launch of its own / in this one, independent tokens unless a share of the slots is named.
+//   Q4_K: up to 2^26 weights of a matrix over the entries, and up to 2^28 where few of the tokens share experts by chance and rows are of at
+// most 4096 values (workgroups of up to four waves: those of five or six lose a third of a compute unit's waves):
+//   2048 x 768 top-8 of 128, 2 tokens 19.0 / 15.0, 5 27.9 / 23.7, all shared 24.9 / 21.1;  4096 x 512 of 200, 3 27.0 / 21.9;
+//   4096 x 1536 of 128, 2 40.5 / 36.7, half shared 33.3 / 29.6, all 29.0 / 25.2, 5 (252 M) 86.6 / 83.8, 73.9 / 70.4, 51.5 / 51.0;
+//   7168 x 2048 top-1 of 16, 4 (59 M) 25.8 / 23.8;  of longer rows: 5120 x 1536 top-10 of 160, 2 (157 M) 54.3 / 55.2;  6144 x 1536 top-10 of 100, 3 96.2 / 99.6
+//   IQ1_S: its kernel is bound by vector instructions, which the head adds to, and does not feel the sharing.  By the workgroups of 16 rows:
+// fewer than 4096 of two waves, 2048 of three and four, 1024 of more (two tokens) or 768 (three a compute unit, what the chip holds of seven
+// and eight waves):
+//   2048 x 768, 2 18.0 / 13.9, 10 (3840) 35.9 / 33.5;  2048 x 1024, 8 (4096) 32.0 / 32.4;  1024 x 1024, 16 (8192) 46.6 / 48.3;
+//   3072 x 1024 top-6, 5 (1920) 26.4 / 24.9, 6 (2304) 28.9 / 29.9;  4096 x 512, 8 (2048) 33.5 / 31.8;  4096 x 2048 top-4, 4 (2048) 29.4 / 28.4;
+//   two tokens: 5120 x 1024 (1024) 24.6 / 24.4, 7168 x 2048 top-4 (1024) 26.7 / 25.9;  5120 x 1024 top-4, 3 (768) 19.7 / 18.6, 4 (1024) 22.9 / 23.0, 5
+//   (1280) 27.1 / 27.5;  6144 x 2048 top-2, 4 (1024) 24.6 / 25.4;  7168 x 1024 top-4, 3 (768) 23.2 / 22.7, 4 (1024) 28.3 / 28.5
+//   IQ2_S: the resident workgroups of the tile walk are shared out among the tokens.  Up to 2^27 weights, two and three tokens up to 2^28 (the
+// kernel of a launch behind a head of its own has more waves a compute unit, which tells on longer launches); where a compute unit's three workgroups are
+// few waves (rows beyond 2048 values) four tiles a workgroup at most, two and three tokens more from four waves on:
+//   2048 x 768 top-8, 2 18.9 / 14.9, 10 (126 M) 39.7 / 33.7;  2048 x 2048 top-4, 8 39.0 / 36.1;  4096 x 1536, 2 31.1 / 29.6, 3 (151 M) 43.3 / 37.5, all shared 37.6 / 35.8;
+//   7168 x 2048 of 100, 2 (235 M) 58.1 / 56.2, all shared 50.5 / 48.8;  4096 x 768, 4 (4 tiles) 30.6 / 29.7;  3072 x 1024 top-6, 4 27.9 / 26.5, 6 (6 tiles)
+//   34.2 / 35.0;  2560 x 1024 top-6, 5 (5) 29.9 / 31.0;  4096 x 512, 8 (5.3) 40.4 / 41.3;  3072 x 2048, 3 (8, three waves) 43.1 / 43.3, half shared 39.7 / 40.6;
+//   5120 x 2048 top-5, 2 (3.3) 32.1 / 31.3, all shared 30.6 / 31.1, top-7, 2 (4.7) 42.7 / 37.6, 38.4 / 36.6;  5120 x 1280 top-4, 5 (4.2) 42.1 / 41.5, 40.4 / 41.0;
+//   four waves: 3584 x 2048 top-7, 2 (4.7) 32.2 / 30.2, 30.9 / 30.0, top-8 (32768 rows) 34.4 / 34.2, 33.0 / 33.7, 4096 x 2048, 3 (8) 51.2 / 49.6, 43.2 / 42.1;
+//   with Q4_K down rows 3 (352 M) 92.5 / 93.6, 8 197 / 206;
+//   more slots than eight and rows that leave lanes idle: top-10 2304 x 1280, 2 (59 M) 37.2 / 36.9, 3 (88 M) 40.7 / 41.9, 4864 x 2048, 2 (199 M) 63.0 / 64.5
+static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert, int n_cu) {
     const maya_moe_layout& l = a.layout;
-    const int entries = a.n_tokens * a.k;
-    const long long weights = (long long) entries * l.n_ff * l.n_embd;   // (of one matrix)
+    const int entries = a.n_tokens * a.k, waves = pos_waves(l.n_embd);
+    const long long rows = (long long) entries * l.n_ff, weights = rows * l.n_embd;   // (of one matrix)
     if (!(gate_up_by_entries(a) && down_by_entries(a))) return false;   // (the others want the entries grouped)
-    if (l.gate_type == kIQ1_S) return weights <= 1ll << 27;
+    if (l.gate_type == kIQ1_S) return waves == 2 ? rows < 16 * 4096 : rows <= 16 * (waves <= 4 ? 2048 : a.n_tokens == 2 ? 1024 : 768);
     if (l.gate_type == kIQ2_S && a.k > 8 && l.n_embd % 1024 != 0) return weights <= 1ll << 26;
-    if (l.gate_type == kIQ2_S) return weights <= 1ll << 27 || (weights <= 1ll << 28 && a.n_tokens <= 3);
+    if (l.gate_type == kIQ2_S) {
+        const bool few = a.n_tokens <= 3;
+        const int tiles = a.k * (l.n_ff / 8), walkers = std::max(1, iq2s_tiles_per_cu(waves) * n_cu / a.n_tokens);
+        if (weights > 1ll << (few ? 28 : 27)) return false;
+        if (waves == 2 || tiles <= 4 * walkers) return true;
+        return few && (waves > 4 || (waves == 4 && (a.n_tokens == 3 || rows < 32768)));
+    }
     return l.gate_type == kQ4_K && (weights <= 1ll << 26 || (weights <= 1ll << 28 && 5 * entries <= 2 * n_expert && l.n_embd <= 4096));
 }
 static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& rs, const float* logits, int n_expert, const void* x,
-                                     int x_dtype) {
+                                     int x_dtype, int n_cu) {
     const maya_moe_layout& l = a.layout;
-    if (!(logits && (a.n_tokens == 1 || window_head_in_gate_up_pays(a, n_expert)) && n_expert <= 512 && a.k < n_expert && x_dtype >= 0 && x_dtype <= 2 && ((uintptr_t) x & 15) == 0))
+    if (!(logits && (a.n_tokens == 1 || window_head_in_gate_up_pays(a, n_expert, n_cu)) && n_expert <= 512 && a.k < n_expert && x_dtype >= 0 && x_dtype <= 2 && ((uintptr_t) x & 15) == 0))
         return false;
     if (l.gate_type == kQ4_K) return gate_up_q4k_pos_ok(a);
     if (l.gate_type == kIQ1_S) return gate_up_iq1s_pos_ok(a);
@@ -2837,7 +2853,7 @@ static int layer_decode_core(const maya_moe_layout* l, const uint64_t* expert_ta
     }
     if (!head) {
         // (the second half of a call made in two: the plan, the groups and h are in the workspace)
-    } else if ((n_tokens == 1 || (!q80 && !join)) && layer_head_in_gate_up_ok(a, rs, logits, n_expert, x, x_dtype)) {
+    } else if ((n_tokens == 1 || (!q80 && !join)) && layer_head_in_gate_up_ok(a, rs, logits, n_expert, x, x_dtype, st->n_cu)) {
         // IQ2_S, Q4_K or IQ1_S experts: route, plan, Q8_K of x and gate/up in one launch (a window beside a shared expert keeps the head
         // of its own: it rounds x for a Q8_0 one too, and runs in the time of one on the second stream; where this runs, the down launch takes the entries one by one, ungrouped)
         const LayerHeadIn hd{logits, expert_table, x, rs.bias, n_expert, x_dtype, rs.kind == MAYA_ROUTER_SIGMOID ? 1 : 0,

@@ -454,7 +454,8 @@ def test_several_tokens_head_in_the_gate_up_launch(lib, ty, n_embd, n_ff, ne, k,
 
 @pytest.mark.parametrize("sigmoid", (False, True))
 @pytest.mark.parametrize("ty,n_embd,n_ff,ne,k,nt", ((12, 2048, 256, 40, 8, 2), (12, 3072, 512, 64, 6, 3), (12, 2304, 256, 300, 8, 5), (12, 4096, 1536, 128, 8, 5),
-                                                    (12, 7168, 2048, 16, 2, 2), (19, 2048, 256, 40, 8, 5), (22, 2048, 256, 40, 8, 5)))
+                                                    (12, 7168, 2048, 16, 2, 2), (19, 2048, 256, 40, 8, 5), (19, 2304, 256, 300, 8, 5), (19, 2048, 512, 400, 8, 15),
+                                                    (22, 2048, 256, 40, 8, 5), (22, 2304, 256, 300, 8, 3), (22, 2048, 256, 512, 8, 16)))
 def test_windows_whose_tokens_take_the_same_experts(lib, ty, n_embd, n_ff, ne, k, nt, sigmoid):
     """Tokens that share all or half of their experts, each in an order of its own, an expert of them not resident: every token's slots are
     its own - the bits of the layer given the ids and weights, and of each token alone."""
