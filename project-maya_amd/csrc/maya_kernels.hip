@@ -845,8 +845,9 @@ __device__ __forceinline__ void route_wave_sigmoid(const float (&p)[8], const fl
 }
 
 // The softmax router of many tokens, a wave each (up to 64 R experts): a workgroup a token, three of whose waves wait for one while it
-// adds and picks.  4096 tokens of 288 experts 40.3 -> 14.1 us, of 256 18.4 -> 11.6, 512 of 256 6.5 -> 5.7; one of 288 8.2 -> 6.2; up to
-// 256 tokens of up to 256 experts nothing in it (5.0 to 5.5 us, either way the shorter by 0.1), so these stay as they are.
+// adds and picks.  Microseconds a launch, a workgroup a token / a wave: of 256 experts 257 tokens 5.4 / 5.55, 384 6.0 / 5.55, 512 6.15 / 5.5, 1187 8.4 / 7.3, 4096
+// 18.8 / 11.3;  of 128, 257 tokens 4.5 / 4.4, 1187 5.95 / 5.5;  of 64, 257 tokens 3.8 / 3.5, 4096 8.8 / 5.7;  of 300, one token 8.2 / 6.2, 512 9.6 / 6.7; up
+// to 256 tokens of up to 256 experts nothing in it, so these stay as they are.
 template <int R>
 __global__ __launch_bounds__(256) void router_waves_kernel(const float* __restrict__ logits, int n_tokens, int n_expert, int k,
                                                            int32_t* __restrict__ ids, float* __restrict__ weights) {
@@ -2403,7 +2404,7 @@ static int route_impl(const char* what, const float* logits, int n_tokens, int n
     if (n_tokens <= 0 || n_tokens > 65535 || n_expert <= 0 || n_expert > MAYA_MAX_EXPERTS || k <= 0 || k > MAYA_MAX_K || k > n_expert)
         return fail(MAYA_E_SHAPE, "%s: tokens %d experts %d k %d (limits %d experts, k %d)", what, n_tokens, n_expert, k,
                     MAYA_MAX_EXPERTS, MAYA_MAX_K);
-    if (r.kind == MAYA_ROUTER_SOFTMAX && n_expert <= 512 && (n_expert > 256 || n_tokens > 256)) {
+    if (r.kind == MAYA_ROUTER_SOFTMAX && n_expert <= 512 && (n_expert > 256 || n_tokens > (n_expert > 128 ? 320 : 256))) {
         const dim3 grid((unsigned) ((n_tokens + 3) / 4));
         if (n_expert <= 256) hipLaunchKernelGGL(router_waves_kernel<4>, grid, dim3(256), 0, as_stream(stream), logits, n_tokens, n_expert, k, ids, weights);
         else hipLaunchKernelGGL(router_waves_kernel<8>, grid, dim3(256), 0, as_stream(stream), logits, n_tokens, n_expert, k, ids, weights);
