@@ -886,10 +886,12 @@ static int pf_plan(const int32_t* ids, int n_entries, const uint64_t* expert_tab
     if (!ids || !expert_table || !plan_ok(plan)) return fail(MAYA_E_ARG, "prefill_plan: null pointer");
     if (n_entries <= 0 || n_entries > (1 << 20) || n_expert <= 0 || n_expert > MAYA_MAX_EXPERTS)
         return fail(MAYA_E_SHAPE, "prefill_plan: entries %d experts %d", n_entries, n_expert);
-    // (a wave's 64-bit lane masks an expert ride along while LDS holds them: up to 767 experts; ballots beyond)
-    size_t lds = sizeof(int32_t) * ((size_t) (kPlanWaves + 5) * n_expert + 3);
+    // (a wave's 64-bit lane masks an expert ride along while LDS holds them beside the kernel's own 128 bytes: up to 771 experts with a
+    // work list, 786 without; ballots beyond)
+    size_t lds = sizeof(int32_t) * ((size_t) (kPlanWaves + 4) * n_expert + 2);
+    if (work.list != nullptr) lds += sizeof(int32_t) * ((size_t) n_expert + 1);
     const size_t masks = sizeof(unsigned long long) * (size_t) kPlanWaves * n_expert;
-    const int with_masks = lds + masks + 1024 <= (size_t) st->lds_limit;
+    const int with_masks = lds + masks + 256 <= (size_t) st->lds_limit;
     if (with_masks) lds += masks;
     if (lds > 65536) MAYA_HIP(hipFuncSetAttribute((const void*) prefill_plan_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
     const int groups = (n_entries + kPlanThreads - 1) / kPlanThreads;

@@ -270,6 +270,35 @@ def test_layer_calls_equal_the_stages(pf, t, n_embd, n_ff):
     assert all(torch.equal(o.view(torch.int32), outs[0].view(torch.int32)) for o in outs)
 
 
+@pytest.mark.parametrize("n_expert", [767, 768, 771, 772, 786, 787, 1024])
+def test_plans_of_many_experts(pf, oracle, n_expert):
+    """As many experts as the plan's lane masks have room for, with a work list and without, and more: the plan of the CPU path, and the
+    layer call's output that of the stages."""
+    from maya_amd import lib
+    rng = np.random.default_rng(n_expert)
+    n_tokens, k, n_embd, n_ff = 300, 8, 256, 256
+    logits = rng.standard_normal((n_tokens, n_expert)).astype(np.float32) + zipf_bias(n_expert)
+    ids = np.argsort(-logits, axis=1, kind="stable")[:, :k].astype(np.int32)
+    layout, _ = lib.layout(Q4_K, Q4_K, n_embd, n_ff)
+    store = lib.ExpertStore(make_blobs(oracle, 5, n_embd, n_ff, n_expert), pack_layout=layout)
+    layout = lib.copy_layout(layout, lib.PACK_STREAM)
+    table = store.table[torch.arange(n_expert, device="cuda") % 5].contiguous()
+    table[3::50] = 0
+    resident = np.ones(n_expert, dtype=bool)
+    resident[3::50] = False
+    x, weights = dev(rng.standard_normal((n_tokens, n_embd)).astype(np.float32)), dev(rng.random((n_tokens, k)).astype(np.float32) + 0.5)
+    p = pf.plan(dev(ids).reshape(-1), table)
+    part = pf.down(layout, table, p, pf.gate_up(layout, table, p, pf.quant(x, p, k)))
+    want = pf.combine(p, weights, part, n_tokens, k)
+    got = pf.PrefillLayer(layout, n_expert, k, n_tokens, out_dtype=torch.float32).forward(table, None, x, routed=(dev(ids), weights))
+    torch.cuda.synchronize()
+    bounds, row_entry, entry_row = oracle.prefill_plan(ids, n_expert, resident)
+    rows = int(bounds[-1])
+    assert np.array_equal(p.bounds.cpu().numpy(), bounds) and np.array_equal(p.row_entry.cpu().numpy()[:rows], row_entry)
+    assert np.array_equal(p.entry_row.cpu().numpy(), entry_row)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32)) and bool((got != 0).any())
+
+
 FEW_ROWS = [128, 97, 96, 65, 64, 33, 17, 8, 3, 1]   # (512 entries, of 128 tokens)
 
 
