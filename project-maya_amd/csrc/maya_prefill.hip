@@ -50,7 +50,7 @@ struct PfItem {
 struct PfWork {
     PfItem* list;
     int32_t* n;      // [1] items
-    int rows;
+    int rows;        // of an item at most: a power of two
     bool few;        // IQ2_S products: on the kernel for few rows an expert
 };
 constexpr int kPlanMaxGroups = 64;   // (at 1 << 20 entries the counting would outweigh the scatter)
@@ -131,7 +131,10 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(const int32_
     };
     if (wave == 0) first_of([&](int x) { return total[x]; }, base);
     if (wave == 1) first_of([&](int x) { return (total[x] + kPfRows - 1) / kPfRows; }, tbase);
-    if (wave == 2 && work.list != nullptr) first_of([&](int x) { return (total[x] + work.rows - 1) / work.rows; }, wbase);
+    if (wave == 2 && work.list != nullptr) {
+        const int log2_rows = __ffs(work.rows) - 1;   // (a division would make this wave the one that the others wait for)
+        first_of([&](int x) { return (total[x] + work.rows - 1) >> log2_rows; }, wbase);
+    }
     __syncthreads();
     if (blockIdx.x == 0) {
         for (int x = tid; x <= n_expert; x += kPlanThreads) p.bounds[x] = base[x];
