@@ -33,7 +33,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // 64-entry chunk) runs on as many workgroups as there are runs of 1024 entries.  32768 entries over 288 experts: 193 us with
 // one workgroup scattering all 32 chunks a wave, 11.9 us like this; 4096 entries over 256: 12 us, 7.5 us.
 // dynamic LDS: [kPlanWaves][n_expert] 64-bit lane masks (with_masks), seg[kPlanWaves][n_expert] counts -> bases,
-// before[n_expert], total[n_expert], base[n_expert + 1], tbase[n_expert + 1]
+// before[n_expert], total[n_expert], base[n_expert + 1], tbase[n_expert + 1], with a work list wbase[n_expert + 1]
+
 // What a layer call's GEMMs are to do, a row of their grids an item (a stage call has the plan's tiles only).  Every row of the grid
 // but the last ones has work.  With a workgroup for each tile of 64 rows, the second tile of every pair was a workgroup that
 // returned at once; workgroups go to an XCD's shader engines in turn whatever they do and in order, so with few bands of weight rows an

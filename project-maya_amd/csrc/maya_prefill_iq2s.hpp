@@ -13,9 +13,10 @@
 // Tiles of up to 128 rows keep a super-block's planes for their row groups, as Q4_K's do: the look-ups and the 200 vector
 // instructions of a decode are paid once.  1187 tokens top-8 of 256 experts of 7168 x 2048 under a skewed routing, gate/up 1388 -> 1232
 // us; 75 tokens of 160 experts of 6144 x 1536, where every tile has one group, 340 and 335.
-// What bounds it: few rows an expert, the decode's vector instructions (56 % of the cycles) and the matrix instructions (27 %),
-// which a SIMD's two waves overlap little.  Not LDS, though it is busy 69 %: with the signs' selectors made by a multiply
-// instead of a look-up (two reads of five less a sub-block) the 75 tokens took the same time.
+// Chunks of few rows an expert run on a form of one group of 32 rows, of which a compute unit holds three workgroups instead of two
+// (prefill_iq2s_few_kernel).  What bounds that one is LDS, busy 76 to 80 % of the cycles, 46 % of that with bank conflicts of the sign and digit
+// look-ups, which come at random.  What bounds the form of up to 128 rows: vector instructions (46 to 56 % of the cycles) and the matrix
+// instructions (27 to 35 %), which a SIMD's two waves overlap little.
 constexpr int kIqMags = 0, kIqSigns = 8192, kIqScales = kIqSigns + 2048, kIqTables = kIqScales + 256;   // byte offsets in LDS
 
 // A quad of rows (the stream packing's unit) holds, a super-block, 256 bytes of (index, sign) words [sub-block][row], 64 of (high

@@ -82,6 +82,9 @@ def test_the_iq2s_prompt_kernels_have_no_lds_but_their_array():
     assert len(got) == 2
     for n, k in got.items():
         assert k[".group_segment_fixed_size"] == lds, n
+    few = {n: k for n, k in kernels(built()).items() if "prefill_iq2s_few_kernel" in n}   # (the same tables, a shorter ring)
+    assert len(few) == 2 and len({k[".group_segment_fixed_size"] for k in few.values()}) == 1
+    assert all(k[".group_segment_fixed_size"] <= 160 * 1024 // 3 and k[".private_segment_fixed_size"] == 0 for k in few.values())
 
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no llvm-objdump")
