@@ -525,28 +525,29 @@ struct LayerHeadIn {
 // the token's index, three or four registers: with it Q4_K and IQ1_S rows that fill their lanes, and IQ1_S ones that do not, pass 72, 6
 // waves a SIMD instead of 7.
 //   kTokenPlanes: grid (row blocks + 1, k, tokens), a plane as one token's grid.
-//   kSlotPlanes: grid (row blocks, tokens, k + 1).  Workgroup (0, token) of the first plane is the token's router, the others of it leave;
-//   plane i + 1 is every token's slot of its i-th expert in the order of the experts.  Tokens that take the same experts so ask
-//   for the same rows one soon after the other, and on the same XCD (the row blocks are a multiple of 8): the rows come
-//   from its L2 but once.  What Q4_K wants, whose launches wait for memory.  Microseconds a layer, head in a launch of its own with the entries
-//   grouped / kTokenPlanes / kSlotPlanes, independent tokens, tokens that share half of their slots, and all:
-//     2048 x 768 top-8, 2 tokens 19.0 / 14.7 / 15.0, 18.8 / 14.5 / 14.7, 18.6 / 14.5 / 14.4;  8 tokens 37.4 / 34.3 / 33.4, 29.7 / 28.9 / 26.6, 28.6 / 28.2 / 25.8
-//     4096 x 1024 top-8, 2 tokens 28.2 / 24.8 / 24.0, 24.4 / 22.9 / 20.4, 23.1 / 23.4 / 19.0;  3072 x 1536, 3 tokens 47.8 / 45.7 / 45.8, 38.3 / 39.1 / 36.1, 33.2 / 36.1 / 30.7
-//     4096 x 1536 top-8, 2 tokens 40.5 / 36.2 / 36.7, 33.3 / 31.6 / 29.6, 29.0 / 30.8 / 25.2;  5 tokens 86.6 / 83.5 / 83.8, 73.9 / 73.0 / 70.4, 51.5 / 65.2 / 51.0
-//     7168 x 2048 top-2, 2 tokens 24.5 / 23.6 / 21.6, 21.9 / 23.0 / 19.4, 20.6 / 22.7 / 18.1;  top-1, 3 tokens 24.7 / 24.3 / 24.7, 24.7 / 24.3 / 24.7, 22.5 / 23.6 / 22.5
-//   IQ1_S, bound by vector instructions, does not feel the sharing and loses where the first plane is large (6144 x 2048 top-2, 4 tokens
-//   25.4 / 28.2, 7168 x 1024 top-8, 2 tokens 27.5 / 29.0).
-enum { kOneToken = 0, kTokenPlanes = 1, kSlotPlanes = 2 };
+//   kExpertOrder: grid (row blocks, tokens k + 1).  Workgroup t of the first row is token t's router (`rank` -1), the others of it leave; row
+// 1 + tokens i + t is token t's slot (`rank` i) of its i-th expert in the order of the experts.  Tokens that take the same experts so ask
+// for the same rows one soon after the other, and on the same XCD (the row blocks are a multiple of 8): the rows come
+// from its L2 but once.  What Q4_K wants, whose launches wait for memory.  Microseconds a layer, head in a launch of its own with the entries
+// grouped / kTokenPlanes / kExpertOrder, independent tokens, tokens that share half of their slots, and all:
+//     2048 x 768 top-8, 2 tokens 18.9 / 14.7 / 14.9, 18.8 / 14.5 / 14.6, 18.7 / 14.5 / 14.3;  5 tokens 27.6 / 24.2 / 23.2, 25.4 / 21.9 / 21.2, 24.8 / 21.7 / 20.6
+//     4096 x 1024 top-8, 2 tokens 28.2 / 24.8 / 24.0, 24.4 / 22.9 / 20.4, 22.9 / 23.4 / 18.7;  4 tokens 51.6 / 48.6 / 49.0, 37.8 / 38.2 / 36.3, 31.1 / 35.2 / 28.5
+//     4096 x 1536 top-8, 5 tokens 86.4 / 83.4 / 83.5, 73.8 / 73.0 / 69.8, 51.4 / 65.0 / 50.5;  7168 x 1024 top-4, 2 tokens 24.2 / 23.2 / 21.3, 21.9 / 22.9 / 19.0, 20.9 / 22.9 / 18.0
+//     7168 x 2048 top-1, 3 tokens 24.6 / 24.2 / 24.3, 24.7 / 24.2 / 24.2, 22.4 / 23.6 / 21.9;  4 tokens 25.6 / 25.2 / 22.6, 25.7 / 25.1 / 22.6, 23.1 / 24.4 / 20.3
+// (With the routers in a plane of their own, grid (row blocks, tokens, k + 1): row blocks x tokens workgroups for as many routers as tokens, 7168 x 2048
+// top-1, 4 tokens 23.8 instead of 22.6.)
+//   IQ1_S, bound by vector instructions, does not feel the sharing and keeps the planes.
+enum { kOneToken = 0, kTokenPlanes = 1, kExpertOrder = 2 };
 template <int NW, int R, int MANY>
 __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent, const int32_t* skip, bool is_up, bool on, int u, int o0,
-                                                int o1, int (&y)[8], float& d, uint64_t& blob, int& slot) {
+                                                int o1, int (&y)[8], float& d, uint64_t& blob, int& slot, int the_tok = 0, int rank = 0) {
     constexpr int NU = 32 * NW;
     __shared__ uint64_t s_blob[MAYA_MAX_K];
-    __shared__ int s_slot[MANY == kSlotPlanes ? MAYA_MAX_K : 1];
+    __shared__ int s_slot[MANY == kExpertOrder ? MAYA_MAX_K : 1];
     __shared__ float s_lv[64 * R];
     __shared__ uint64_t s_tab[64 * R];
     __shared__ int s_y[9][NU];
-    const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert, tok = MANY == kSlotPlanes ? (int) blockIdx.y : MANY ? (int) blockIdx.z : 0;
+    const int t = threadIdx.x, lane = t & 63, ne = hd.n_expert, tok = MANY == kExpertOrder ? the_tok : MANY ? (int) blockIdx.z : 0;
     const bool picker = t >= 64 * (NW - 1), sigm = hd.sigmoid != 0;
     float lv[R], bv[R];
     uint64_t tab[R];
@@ -565,8 +566,8 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
             for (int r = 0; r < R; ++r) s_tab[64 * r + lane] = tab[r];
         }
     }
-    if (MANY == kSlotPlanes ? blockIdx.z == 0 : blockIdx.x == gridDim.x - 1) {   // the router (it looks at no skip flag, like the head kernel)
-        if ((MANY == kSlotPlanes ? blockIdx.x : blockIdx.y) != 0 || !picker) return false;
+    if (MANY == kExpertOrder ? rank < 0 : blockIdx.x == gridDim.x - 1) {   // the router (it looks at no skip flag, like the head kernel)
+        if ((MANY != kExpertOrder && blockIdx.y != 0) || !picker) return false;
         int id;
         float w;
         uint64_t ptr;
@@ -613,10 +614,9 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
             if constexpr (R > 4) ptr = lane < n_ent && id >= 0 ? s_tab[id] : 0ull;
         }
         int at = lane;
-        if constexpr (MANY == kSlotPlanes) {   // the slots in their experts' order (the same expert twice, of a row that has no order: in the slots')
+        if constexpr (MANY == kExpertOrder) {   // the slots in their experts' order (the same expert twice, of a row that has no order: in the slots')
             const int key = id * 64 + lane;   // (k <= 64)
             at = 0;
-#pragma unroll 4
             for (int j = 0; j < n_ent; ++j) at += __builtin_amdgcn_readlane(key, j) < key ? 1 : 0;
             if (lane < n_ent) s_slot[at] = lane;
         }
@@ -675,9 +675,9 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
         for (int i = 0; i < 8; ++i) y[i] = s_y[i][u];
         d = __int_as_float(s_y[8][u]);
     }
-    if constexpr (MANY == kSlotPlanes) slot = __builtin_amdgcn_readfirstlane(s_slot[blockIdx.z - 1]);
+    if constexpr (MANY == kExpertOrder) slot = __builtin_amdgcn_readfirstlane(s_slot[rank]);
     else slot = (int) blockIdx.y;
-    const uint64_t bl = s_blob[MANY == kSlotPlanes ? blockIdx.z - 1 : blockIdx.y];
+    const uint64_t bl = s_blob[MANY == kExpertOrder ? rank : (int) blockIdx.y];
     const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) bl);
     const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (bl >> 32));
     blob = ((uint64_t) hi << 32) | lo;

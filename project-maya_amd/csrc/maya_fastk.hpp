@@ -72,7 +72,7 @@ __device__ __forceinline__ float pos_q4k_value(const PosQ4K& p, const u32x4 hdr,
 // AHEAD (8 rows): all of a lane's rows are requested up front - the launches of a few entries, whose workgroups do not fill
 // the chip and would otherwise run at the memory's latency a row.
 // HEAD (4 or 8: a token's experts a lane): the layer's head rides in this launch (head_in_gate_up) - grid (n_ff / ROWS + 1, k), of
-// several tokens (MANY) (n_ff / ROWS, tokens, k + 1).
+// several tokens (MANY) (n_ff / ROWS, tokens k + 1), with the tokens in bits 8 to 15 of n_ent and 2^16 / tokens, rounded up, above.
 // The leading arguments (MAYA_HEAD_ARGS) are what it asks of memory first, in scalar registers with the dispatch.
 template <int NW, int ROWS, int MINW, bool FIT, bool AHEAD = false, int HEAD = 0, bool MANY = false>
 __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(MAYA_HEAD_PARAMS, maya_moe_args a, LayerHead out) {
@@ -95,10 +95,20 @@ __global__ __launch_bounds__(64 * NW, MINW) void gate_up_q4k_pos_kernel(MAYA_HEA
         const int v0 = 256 * (u >> 3) + 64 * ((u & 7) >> 1) + 16 * (u & 1);
         int y[8];
         float d;
-        int slot;
+        int slot, tok = 0, rank = 0;
+        if constexpr (MANY) {
+            const int n_tok = (n_ent >> 8) & 0xff, i = (int) blockIdx.y - 1;
+            rank = (int) ((uint32_t) max(i, 0) * ((uint32_t) n_ent >> 16) >> 16);   // (i / n_tok: i < 256, 2 <= n_tok <= 16)
+            tok = i - rank * n_tok;
+            if (i < 0) {
+                if ((int) blockIdx.x >= n_tok) return;
+                tok = blockIdx.x, rank = -1;
+            }
+            n_ent &= 0xff;
+        }
         const LayerHeadIn hd = {logits, table, x, bias, n_expert, mode & 255, (mode >> 8) & 1, out, mode >> 16 << 5};
-        if (!head_in_gate_up<NW, HEAD, MANY ? kSlotPlanes : kOneToken>(hd, n_ent, skip, is_up, on, lu, v0, v0 + 32, y, d, blob, slot)) return;
-        e = MANY ? (int) blockIdx.y * n_ent + slot : slot;
+        if (!head_in_gate_up<NW, HEAD, MANY ? kExpertOrder : kOneToken>(hd, n_ent, skip, is_up, on, lu, v0, v0 + 32, y, d, blob, slot, tok, rank)) return;
+        e = MANY ? tok * n_ent + slot : slot;
 #pragma unroll
         for (int i = 0; i < 4; ++i) p.ylo[i] = y[i], p.yhi[i] = y[4 + i];
         p.dx = d;

@@ -1736,7 +1736,8 @@ static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert, in
         if (waves == 2 || tiles <= 4 * walkers) return true;
         return few && (waves > 4 || (waves == 4 && (a.n_tokens == 3 || rows < 32768)));
     }
-    return l.gate_type == kQ4_K && (weights <= 1ll << 26 || (weights <= 1ll << 28 && 5 * entries <= 2 * n_expert && l.n_embd <= 4096));
+    // (n_ff: the launch's first row of workgroups has the routers, one a token)
+    return l.gate_type == kQ4_K && l.n_ff >= 16 * MAYA_MAX_TOKENS && (weights <= 1ll << 26 || (weights <= 1ll << 28 && 5 * entries <= 2 * n_expert && l.n_embd <= 4096));
 }
 static bool layer_head_in_gate_up_ok(const maya_moe_args& a, const RouterSpec& rs, const float* logits, int n_expert, const void* x,
                                      int x_dtype, int n_cu) {
@@ -1985,14 +1986,15 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     // 16 rows a workgroup, 8 - all requested up front - when the call has so few entries that 16 would leave compute units idle
     const bool small = (long long) (a.layout.n_ff / 16) * a.n_tokens * a.k < 512;
     const int rows = small ? 8 : 16;
-    // (with the head in the launch: one more column or, of several tokens, plane for the routers)
+    // (with the head in the launch: one more column or, of several tokens, row for the routers)
     const bool many = hd && a.n_tokens > 1;
-    const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd && !many ? 1u : 0u), (unsigned) (many ? a.n_tokens : a.n_tokens * a.k), many ? a.k + 1u : 1u);
+    const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd && !many ? 1u : 0u), (unsigned) (a.n_tokens * a.k) + (many ? 1u : 0u));
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
+    const int n_tok = many ? (65535 + a.n_tokens) / a.n_tokens << 16 | a.n_tokens << 8 : 0;   // (in n_ent)
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_Q4H(NWV, F, HEAD, MANY)                                                                                        \
-    if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);   \
-    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a), a, h.out);
+    if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a) | n_tok, a, h.out);   \
+    else hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 16, 6, F, false, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a) | n_tok, a, h.out);
 #define MAYA_Q4HEAD(NWV, MANY)                                                                                              \
     if (h.n_expert > 256) { MAYA_Q4H(NWV, false, 8, MANY) }   /* (their rows take the form that any length has) */           \
     else if (fit) { MAYA_Q4H(NWV, true, 4, MANY) }                                                                          \
