@@ -1654,10 +1654,10 @@ int launch_gate_up_iq2s_pos(const maya_moe_args& a, const DeviceState& st, hipSt
 // to scratch memory: 6.8 MB written and read back a launch, 2.1 us of the layer.  Windows of long calls keep gate_up_iq2s_pos_kernel: the tile
 // stream with the resident workgroups shared out among the tokens (a token's codes in a workgroup's registers)
 // is slower there (eight tokens of 7168 x 2048 260 us against 234); window_head_in_gate_up_pays says where it is not.
-static constexpr int iq2s_tiles_per_cu(int waves) { return waves == 2 ? 8 : 3; }
+static constexpr int iq2s_walkers_per_cu(int waves) { return waves == 2 ? 8 : 3; }
 template <int NW, int HEAD, bool MANY>
 int launch_iq2s_tiles(const maya_moe_args& a, const DeviceState& st, hipStream_t s, const LayerHeadIn* hd) {
-    constexpr int kMinW = NW <= 3 ? 5 : 6, kMostPerCu = iq2s_tiles_per_cu(NW);
+    constexpr int kMinW = NW <= 3 ? 5 : 6, kMostPerCu = iq2s_walkers_per_cu(NW);
     const auto kern = gate_up_iq2s_tiles_kernel<NW, kMinW, HEAD, MANY>;
     static int per_cu = 0;   // (asked of the runtime once a form)
     if (per_cu == 0) {
@@ -1731,7 +1731,7 @@ static bool window_head_in_gate_up_pays(const maya_moe_args& a, int n_expert, in
     if (l.gate_type == kIQ2_S && a.k > 8 && l.n_embd % 1024 != 0) return weights <= 1ll << 26;
     if (l.gate_type == kIQ2_S) {
         const bool few = a.n_tokens <= 3;
-        const int tiles = a.k * (l.n_ff / 8), walkers = std::max(1, iq2s_tiles_per_cu(waves) * n_cu / a.n_tokens);
+        const int tiles = a.k * (l.n_ff / 8), walkers = std::max(1, iq2s_walkers_per_cu(waves) * n_cu / a.n_tokens);
         if (weights > 1ll << (few ? 28 : 27)) return false;
         if (waves == 2 || tiles <= 4 * walkers) return true;
         return few && (waves > 4 || (waves == 4 && (a.n_tokens == 3 || rows < 32768)));
