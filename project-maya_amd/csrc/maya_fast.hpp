@@ -530,8 +530,8 @@ struct LayerHeadIn {
 // for the same rows one soon after the other, and on the same XCD (the row blocks are a multiple of 8): the rows come
 // from its L2 but once.  What Q4_K wants, whose launches wait for memory.  Microseconds a layer, head in a launch of its own with the entries
 // grouped / kTokenPlanes / kExpertOrder, independent tokens, tokens that share half of their slots, and all:
-//     2048 x 768 top-8, 2 tokens 18.9 / 14.7 / 14.9, 18.8 / 14.5 / 14.6, 18.7 / 14.5 / 14.3;  5 tokens 27.6 / 24.2 / 23.2, 25.4 / 21.9 / 21.2, 24.8 / 21.7 / 20.6
-//     4096 x 1024 top-8, 2 tokens 28.2 / 24.8 / 24.0, 24.4 / 22.9 / 20.4, 22.9 / 23.4 / 18.7;  4 tokens 51.6 / 48.6 / 49.0, 37.8 / 38.2 / 36.3, 31.1 / 35.2 / 28.5
+//     2048 x 768 top-8, 2 tokens 18.9 / 14.7 / 14.8, 18.8 / 14.5 / 14.6, 18.7 / 14.5 / 14.3;  5 tokens 27.6 / 24.2 / 23.2, 25.4 / 21.9 / 21.2, 24.8 / 21.7 / 20.6
+//     4096 x 1024 top-8, 2 tokens 28.2 / 24.8 / 24.0, 24.4 / 22.9 / 20.4, 22.9 / 23.4 / 18.7;  4 tokens 51.6 / 48.6 / 48.8, 37.8 / 38.2 / 36.3, 31.1 / 35.2 / 28.5
 //     4096 x 1536 top-8, 5 tokens 86.4 / 83.4 / 83.5, 73.8 / 73.0 / 69.8, 51.4 / 65.0 / 50.5;  7168 x 1024 top-4, 2 tokens 24.2 / 23.2 / 21.3, 21.9 / 22.9 / 19.0, 20.9 / 22.9 / 18.0
 //     7168 x 2048 top-1, 3 tokens 24.6 / 24.2 / 24.3, 24.7 / 24.2 / 24.2, 22.4 / 23.6 / 21.9;  4 tokens 25.6 / 25.2 / 22.6, 25.7 / 25.1 / 22.6, 23.1 / 24.4 / 20.3
 // (With the routers in a plane of their own, grid (row blocks, tokens, k + 1): row blocks x tokens workgroups for as many routers as tokens, 7168 x 2048
@@ -615,9 +615,16 @@ __device__ __forceinline__ bool head_in_gate_up(const LayerHeadIn& hd, int n_ent
         }
         int at = lane;
         if constexpr (MANY == kExpertOrder) {   // the slots in their experts' order (the same expert twice, of a row that has no order: in the slots')
-            const int key = id * 64 + lane;   // (k <= 64)
+            // (no loop over the slots that there are: a trip of it costs more than three counts)
+            static_assert(MAYA_MAX_K == 16, "two runs of eight");
+            const int key = lane < n_ent ? id * 64 + lane : 0x7fffffff;
             at = 0;
-            for (int j = 0; j < n_ent; ++j) at += __builtin_amdgcn_readlane(key, j) < key ? 1 : 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) at += __builtin_amdgcn_readlane(key, j) < key ? 1 : 0;
+            if (n_ent > 8) {
+#pragma unroll
+                for (int j = 8; j < 16; ++j) at += __builtin_amdgcn_readlane(key, j) < key ? 1 : 0;
+            }
             if (lane < n_ent) s_slot[at] = lane;
         }
         if (lane < n_ent) s_blob[at] = ptr;
