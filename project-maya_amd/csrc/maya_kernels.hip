@@ -1990,7 +1990,7 @@ int launch_gate_up_q4k_pos(const maya_moe_args& a, hipStream_t s, const LayerHea
     const bool many = hd && a.n_tokens > 1;
     const dim3 grid((unsigned) (a.layout.n_ff / rows) + (hd && !many ? 1u : 0u), (unsigned) (a.n_tokens * a.k) + (many ? 1u : 0u));
     const LayerHeadIn h = hd ? *hd : LayerHeadIn{};
-    const int n_tok = many ? (65535 + a.n_tokens) / a.n_tokens << 16 | a.n_tokens << 8 : 0;   // (in n_ent)
+    const int n_tok = many ? (int) ((65535u + (unsigned) a.n_tokens) / (unsigned) a.n_tokens << 16 | (unsigned) a.n_tokens << 8) : 0;   // (in n_ent)
     const bool fit = a.layout.n_embd == 1024 * pos_waves(a.layout.n_embd);
 #define MAYA_Q4H(NWV, F, HEAD, MANY)                                                                                        \
     if (small) hipLaunchKernelGGL((gate_up_q4k_pos_kernel<NWV, 8, 4, F, true, HEAD, MANY>), grid, dim3(64 * NWV), 0, s, MAYA_HEAD_ARGS(h, a) | n_tok, a, h.out);   \
